@@ -1,4 +1,8 @@
-"""ctypes binding of libmoespresso_amd.so (the C-ABI in include/moespresso_amd.h).
+"""Bindings of libmoespresso_amd.so (the C-ABI in include/moespresso_amd.h).
+
+``dispatch`` is the native call path (``_dispatch.so``): an operator asks it first, with its arguments by position,
+and goes on in Python (checks, conversions, error messages, the ctypes call) only when it answers ``None``, which is
+what it does for anything but dense operands of the plain types on one HIP device.
 
 The library is loaded lazily and only from this package directory. There is no
 fallback: a missing library or a tensor that is not on a HIP device raises.
@@ -13,6 +17,20 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmoespresso_amd.so")
+DISPATCH_PATH = os.path.join(os.path.dirname(LIB_PATH), "_dispatch.so")
+
+
+class _NotBuilt:
+    """Stands where the native call path would: every operator goes on to ``lib()``, which says what is missing."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+if os.path.exists(DISPATCH_PATH):
+    from moespresso_amd import _dispatch as dispatch
+else:
+    dispatch = _NotBuilt()
 
 MSPR_OK = 0
 MSPR_ERR_ARG = -1
@@ -134,17 +152,17 @@ _LIB = None
 
 
 def library_available() -> bool:
-    """True when the shared library exists on disk (it is not loaded here)."""
-    return os.path.exists(LIB_PATH)
+    """True when the shared library and its native call path exist on disk (the library is not loaded here)."""
+    return os.path.exists(LIB_PATH) and os.path.exists(DISPATCH_PATH)
 
 
 def lib() -> ctypes.CDLL:
     """Load (once) and return the shared library; raises if it was never built."""
     global _LIB
     if _LIB is None:
-        if not os.path.exists(LIB_PATH):
+        if not library_available():
             raise RuntimeError(
-                f"{LIB_PATH} is missing: build it with `python -m moespresso_amd.build` "
+                f"{LIB_PATH} or {DISPATCH_PATH} is missing: build it with `python -m moespresso_amd.build` "
                 "(there is no CPU or PyTorch fallback for these operators)")
         handle = ctypes.CDLL(LIB_PATH)
         for name, (restype, argtypes) in SIGNATURES.items():

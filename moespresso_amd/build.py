@@ -1,7 +1,8 @@
-"""Build libmoespresso_amd.so from the HIP sources in ``csrc/`` with hipcc for gfx950.
+"""Build libmoespresso_amd.so from the HIP sources in ``csrc/`` with hipcc for gfx950, and the Python extension
+``_dispatch.so`` (``binding/dispatch.cpp``) that calls it with torch tensors.
 
 ``python -m moespresso_amd.build`` compiles every source to an object file (in
-parallel) and links the shared library in-tree next to this file. hipcc
+parallel) and links both in-tree next to this file. hipcc
 cross-compiles without a GPU.
 """
 
@@ -16,6 +17,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "_obj")
 LIB_PATH = os.path.join(HERE, "libmoespresso_amd.so")
+DISPATCH_SRC = os.path.join(HERE, "binding", "dispatch.cpp")
+DISPATCH_PATH = os.path.join(HERE, "_dispatch.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON_FLAGS = [
@@ -52,17 +55,47 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build(verbose: bool = True) -> str:
-    os.makedirs(OBJ_DIR, exist_ok=True)
-    srcs = sources()
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as pool:
-        objs = list(pool.map(_compile, srcs))
-    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
+def _compile_dispatch() -> str:
+    """Object file of the Python extension: host code only, against the headers of the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(OBJ_DIR, "dispatch.o")
+    cmd = [HIPCC, "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{p}" for p in cpp_extension.include_paths("cuda")), f"-I{sysconfig.get_paths()['include']}",
+           "-w", "-c", DISPATCH_SRC, "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
+        raise RuntimeError(f"hipcc failed on {DISPATCH_SRC}:\n{proc.stderr}")
+    return obj
+
+
+def _link(out: str, args: list[str]) -> None:
+    proc = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *args], capture_output=True,
+                          text=True)
+    if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
+
+
+def build(verbose: bool = True) -> str:
+    from torch.utils import cpp_extension
+
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    srcs = sources()
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as pool:
+        dispatch = pool.submit(_compile_dispatch)
+        objs = list(pool.map(_compile, srcs))
+        dispatch = dispatch.result()
+    _link(LIB_PATH, [*objs, "-Wl,-soname," + os.path.basename(LIB_PATH)])
+    # the library is found next to the extension; torch's own libraries are loaded before the extension is imported
+    _link(DISPATCH_PATH, [dispatch, LIB_PATH, "-Wl,-rpath,$ORIGIN",
+                          *(f"-L{p}" for p in cpp_extension.library_paths("cuda")[:1]), "-lc10", "-lc10_hip",
+                          "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"])
     if verbose:
-        print(f"built {LIB_PATH} from {len(srcs)} sources")
+        print(f"built {LIB_PATH} from {len(srcs)} sources, and {DISPATCH_PATH}")
     return LIB_PATH
 
 

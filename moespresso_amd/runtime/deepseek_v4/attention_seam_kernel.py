@@ -94,6 +94,12 @@ def partial_rope_eligible(x, inv_freq, *, offset, positions) -> bool:
     return True
 
 
+def _note_rope_launch(form: str, inverse) -> None:
+    key = (form, bool(inverse))
+    if key not in _ROPE_KERNELS:
+        _ROPE_KERNELS[key] = f"mspr_fused_partial_rope[{form},{'inv' if inverse else 'fwd'}]"
+
+
 def fused_partial_rope(x, inv_freq, *, offset=0, inverse=False, positions=None):
     """Apply the DS4 partial rope in one launch (reference :247).
 
@@ -108,6 +114,11 @@ def fused_partial_rope(x, inv_freq, *, offset=0, inverse=False, positions=None):
     Returns:
         A tensor of the same shape and dtype.
     """
+    out = _lib.dispatch.fused_partial_rope(x, inv_freq, offset, inverse, positions,
+                                           _MAX_ROWS_PREFILL if prefill_rope_seam_enabled() else _MAX_ROWS_DECODE)
+    if out is not None:
+        _note_rope_launch("off" if positions is None else "pos", inverse)
+        return out
     if not partial_rope_eligible(x, inv_freq, offset=offset, positions=positions):
         raise ValueError("operands are outside the fused partial-rope contract")
     _lib.require_device(x, inv_freq, positions)
@@ -118,11 +129,10 @@ def fused_partial_rope(x, inv_freq, *, offset=0, inverse=False, positions=None):
     out = torch.empty_like(xc)
     inv = inv_freq.contiguous()
     pos = None if positions is None else positions.reshape(seq_len).contiguous()
-    form = "off" if positions is None else "pos"
     dtype_code = _lib.DTYPE_CODE[x.dtype]
     rc = _lib.lib().mspr_fused_partial_rope(_lib.ptr(xc), dtype_code, rows // seq_len, seq_len, width, _lib.ptr(inv),
                                             _lib.ptr(pos), 0 if positions is not None else int(offset),
                                             1 if inverse else 0, _lib.ptr(out), _lib.stream_ptr())
     _lib.check(rc, "fused_partial_rope")
-    _ROPE_KERNELS[(form, bool(inverse))] = f"mspr_fused_partial_rope[{form},{'inv' if inverse else 'fwd'}]"
+    _note_rope_launch("off" if positions is None else "pos", inverse)
     return out.reshape(x.shape)

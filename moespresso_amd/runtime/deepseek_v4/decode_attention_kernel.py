@@ -89,6 +89,10 @@ def fused_decode_prep(q_idx, pooled_qat, weights, kv_row, inv_freq, params, *, s
         ascending row order, then boundary ties by ascending row), float16
         ``[512]`` roped + FP8-rounded KV row, float32 ``[n_rows]`` scores.
     """
+    done = _lib.dispatch.fused_decode_prep(q_idx, pooled_qat, weights, kv_row, inv_freq, params, scale, topk,
+                                           pool_rows_in_params)
+    if done is not None:
+        return done
     if q_idx.ndim != 2 or int(q_idx.shape[1]) != _INDEX_HEAD_DIM:
         raise ValueError("q_idx must have shape [n_heads, 128]")
     n_heads = int(q_idx.shape[0])
@@ -157,6 +161,10 @@ def fused_decode_sdpa(q, window, row, pooled, sel, sinks, inv_freq, params, *, s
     Returns:
         float16 ``[n_heads, 512]`` attention output after the inverse rope.
     """
+    out = _lib.dispatch.fused_decode_sdpa(q, window, row, pooled, sel, sinks, inv_freq, params, scale,
+                                          pool_rows_in_params, workspace)
+    if out is not None:
+        return out
     if q.ndim != 2 or int(q.shape[1]) != _HEAD_DIM or q.dtype != torch.float16:
         raise ValueError("q must be float16 [n_heads, 512]")
     n_heads = int(q.shape[0])

@@ -141,6 +141,10 @@ def sparse_mla_decode(q, kv, rows, *, scale: float, v_dim: int = 512, window_sta
     Returns:
         ``[batch, n_heads, v_dim]`` in the input dtype.
     """
+    out = _lib.dispatch.sparse_mla_decode(q, kv, rows, scale, v_dim, window_start, window_rows, sinks, workspace, row_mul,
+                                          row_add)
+    if out is not None:
+        return out
     if q.ndim != 3 or kv.ndim != 3 or rows.ndim != 2:
         raise ValueError("q must be [batch, n_heads, k_dim], kv [batch, n_pool, k_dim], rows [batch, n_rows]")
     batch, n_heads, k_dim = (int(v) for v in q.shape)
@@ -297,6 +301,9 @@ def _launch_live(q, raw_kv, comp_kv, topk, sinks, dims, *, pos0, window, ratio, 
         topk = topk.to(torch.int32)
     if sinks.dtype != torch.float32:
         sinks = sinks.to(torch.float32)
+    out = _lib.dispatch.prefill_live(q, raw_kv, comp_kv, topk, sinks, pos0, window, ratio, raw_start)
+    if out is not None:
+        return out
     return _run_prefill(q.contiguous(), raw_kv.contiguous(), comp_kv.contiguous(), topk.contiguous(),
                         sinks.contiguous(), batch=batch, n_heads=n_heads, n_tokens=n_tokens,
                         strides=(n_heads * n_tokens * head_dim, n_tokens * head_dim, head_dim), raw_cap=raw_cap,
@@ -379,6 +386,10 @@ def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int =
     Returns:
         float32 ``[batch, tokens, n_comp]``, ``-inf`` where the row is not yet visible to the token.
     """
+    scores = _lib.dispatch.indexer_scores_tiled_live(q, weights, index_comp, pos0, ratio)
+    if scores is not None:
+        _SCORES_TILED_CALL_COUNTS["f16" if q.dtype == torch.float16 else "f32"] += 1
+        return scores
     if q.ndim != 4 or weights.ndim != 3 or index_comp.ndim != 3:
         raise ValueError("q, weights, and index_comp must be BHLD/BLH/BPD")
     batch, n_heads, n_tokens, head_dim = (int(v) for v in q.shape)
@@ -418,6 +429,9 @@ def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int =
 
 def indexer_q_qat_live(q):
     """Hadamard-128 + FP4 QAT of live BHLD query rows, prefill-side rules (reference :1989)."""
+    out = _lib.dispatch.indexer_q_qat_live(q)
+    if out is not None:
+        return out
     if q.ndim != 4:
         raise ValueError("q must have shape [batch, n_heads, tokens, 128]")
     batch, n_heads, n_tokens, head_dim = (int(v) for v in q.shape)

@@ -60,6 +60,9 @@ def indexer_qat_rows(x: torch.Tensor) -> torch.Tensor:
     Returns:
         float32 tensor of the same shape.
     """
+    out = _lib.dispatch.indexer_qat_rows(x)
+    if out is not None:
+        return out
     if x.ndim < 1 or int(x.shape[-1]) != _HEAD_DIM:
         raise ValueError("indexer QAT expects 128-wide rows")
     if x.dtype not in _query_dtypes():
@@ -113,6 +116,9 @@ def fused_qat_indexer_scores(q, pooled_qat, weights, scale) -> torch.Tensor:
         float32 ``[n_rows]``:
         ``scores[r] = sum_h max(qat(q_h) . pooled_r, 0) * scale * weights[h]``.
     """
+    scores = _lib.dispatch.fused_qat_indexer_scores(q, pooled_qat, weights, scale)
+    if scores is not None:
+        return scores
     if q.ndim != 4:
         raise ValueError("q must have shape [1, n_heads, 1, 128]")
     batch, n_heads, tokens, head_dim = (int(v) for v in q.shape)
@@ -240,6 +246,9 @@ def topk_select(scores: torch.Tensor, topk: int) -> torch.Tensor:
     Returns:
         int32 ``[..., topk]``.
     """
+    sel = _lib.dispatch.topk_select(scores, topk)
+    if sel is not None:
+        return sel
     if scores.ndim < 1:
         raise ValueError("scores must have a row axis")
     if scores.dtype != torch.float32:
@@ -274,6 +283,9 @@ def indexer_scores_fp8(q, keys, key_scales, weights) -> torch.Tensor:
     Returns:
         float32 ``[batch, n_rows]``.
     """
+    scores = _lib.dispatch.indexer_scores_fp8(q, keys, key_scales, weights)
+    if scores is not None:
+        return scores
     if q.ndim != 3 or int(q.shape[2]) != _HEAD_DIM:
         raise ValueError("q must have shape [batch, n_heads, 128]")
     batch, n_heads, _ = (int(v) for v in q.shape)

@@ -76,6 +76,9 @@ def quantize(x, group_size: int = 64, bits: int = 8):
     """
     if group_size != 64 or bits != 8:
         raise ValueError("quantize supports group_size=64, bits=8 only")
+    done = _lib.dispatch.quantize(x)
+    if done is not None:
+        return done
     if x.dtype not in _lib.DTYPE_CODE:
         raise ValueError("x must be float32, float16 or bfloat16")
     if x.ndim < 1 or int(x.shape[-1]) % 64 != 0 or x.numel() == 0:
@@ -97,6 +100,9 @@ def dequantize(wq, scales, biases, group_size: int = 64, bits: int = 8):
     """``code * scale + bias`` in the dtype of ``scales`` (the role of ``mx.dequantize``)."""
     if group_size != 64 or bits != 8:
         raise ValueError("dequantize supports group_size=64, bits=8 only")
+    out = _lib.dispatch.dequantize(wq, scales, biases)
+    if out is not None:
+        return out
     if scales.dtype not in _lib.DTYPE_CODE or biases.dtype != scales.dtype:
         raise ValueError("scales and biases must share a float32/float16/bfloat16 dtype")
     if wq.dtype not in (torch.uint32, torch.int32):
@@ -192,6 +198,9 @@ def sdpa_decode_q8(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases, 
     """
     if group_size != 64 or bits != 8:
         raise ValueError("sdpa_decode_q8 supports group_size=64, bits=8 only")
+    out = _lib.dispatch.sdpa_decode_q8(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases, scale, workspace)
+    if out is not None:
+        return out
     if queries.ndim != 4 or int(queries.shape[2]) != 1:
         raise ValueError("queries must be [B, Hq, 1, D] (single-token decode)")
     if int(queries.shape[3]) != _HEAD_DIM:
@@ -232,6 +241,9 @@ def sdpa_decode_q8_0(queries, k_codes, k_scales, v_codes, v_scales, scale, *, wo
     Returns:
         ``[B, Hq, 256]`` in the dtype of ``queries``.
     """
+    out = _lib.dispatch.sdpa_decode_q8_0(queries, k_codes, k_scales, v_codes, v_scales, scale, workspace)
+    if out is not None:
+        return out
     if queries.ndim != 3 or int(queries.shape[2]) != _HEAD_DIM:
         raise ValueError("queries must be [B, Hq, 256]")
     if queries.dtype not in _lib.DTYPE_CODE:
@@ -281,6 +293,10 @@ def sdpa_fa_prefill_q8(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, p
     """
     if group_size != 64 or bits != 8:
         raise ValueError("sdpa_fa_prefill_q8 supports group_size=64, bits=8 only")
+    out = _lib.dispatch.sdpa_fa_prefill_q8(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, pv_biases, self_k, self_v,
+                                           scale, workspace)
+    if out is not None:
+        return out
     if queries.ndim != 4 or int(queries.shape[3]) != _HEAD_DIM:
         raise ValueError("queries must be [B, Hq, L, 256]")
     if queries.dtype != torch.float32:
