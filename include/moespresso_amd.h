@@ -242,6 +242,14 @@ int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer, int64_t s
 
 /* ------------------------------------------------------------------ Qwen/Ornith GQA attention, 8-bit KV */
 
+/* The same quantisation of new rows straight into a cache, keys and values in one launch (the append of
+ * mlx_lm's QuantizedKVCache, src/moespresso/runtime/qwen/full_attention.py:352-369). keys, values: [n_heads][n_rows][width]
+ * of `dtype` (n_heads = batch x KV heads), width a multiple of 64; the buffers hold cap_rows rows per head in the layout
+ * above (scales and biases of `dtype`), row r of a head goes to row offset_rows + r. */
+int mspr_affine_q8_append(const void* keys, const void* values, int dtype, int n_heads, int64_t n_rows, int width,
+                          void* k_wq, void* k_scales, void* k_biases, void* v_wq, void* v_scales, void* v_biases,
+                          int64_t cap_rows, int64_t offset_rows, void* stream);
+
 /* Affine 8-bit quantisation in groups of 64 over the last axis and its inverse: the cache write
  * path in front of the two attention operators below.
  * Stands in for mx.quantize / mx.dequantize (group_size=64, bits=8) as used by the quantised KV

@@ -86,6 +86,9 @@ SIGNATURES = {
         c_int, [c_void_p, c_int, c_int64, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p]),
     "mspr_affine_q8_quantize": (
         c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p]),
+    "mspr_affine_q8_append": (
+        c_int, [c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                c_void_p, c_int64, c_int64, c_void_p]),
     "mspr_affine_q8_dequantize": (
         c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_void_p, c_int, c_int, c_void_p]),
     "mspr_sdpa_decode_q8_workspace_bytes": (c_size_t, [c_int, c_int, c_int64]),

@@ -480,6 +480,63 @@ bool affine_cache(PyObject* const* a, const Tensor* (&t)[6], int64_t B, int64_t*
   return *cap >= *N;
 }
 
+// The three tensors of a cache side, capacity buffers [B, H, cap, *].
+bool cache_side(PyObject* o, const Tensor* (&t)[3]) {
+  if (!PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) != 3) return false;
+  for (int i = 0; i < 3; i++)
+    if (!(t[i] = cache_part(PyTuple_GET_ITEM(o, i)))) return false;
+  return true;
+}
+
+// (keys [B, H, L, D], values, key side, value side, offset): quantises the rows into the buffers of both sides behind the
+// first `offset` rows of every head -> True
+PyObject* q8_append(PyObject* const* a, Py_ssize_t nargs) {
+  MSPR_NARGS(5)
+  const Tensor *k = dense(a[0], 4), *v = dense(a[1], 4), *ks[3], *vs[3];
+  int64_t offset;
+  if (!k || !v || !cache_side(a[2], ks) || !cache_side(a[3], vs) || !whole(a[4], &offset)) return none();
+  const int code = type_code(k->scalar_type());
+  const int64_t B = k->size(0), H = k->size(1), L = k->size(2), D = k->size(3), cap = ks[0]->size(2);
+  if (code == kNoType || v->scalar_type() != k->scalar_type() || k->sizes() != v->sizes() || k->numel() == 0 || D % 64 != 0 ||
+      D > 4096 || B * H > 65535 || offset < 0 || offset + L > cap || !same_device({k, v, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2]}))
+    return none();
+  for (const Tensor** side : {ks, vs})
+    for (int i = 0; i < 3; i++) {
+      const Tensor& t = *side[i];
+      const bool codes = i == 0;
+      if (!t.is_contiguous() || t.size(0) != B || t.size(1) != H || t.size(2) != cap || t.size(3) != (codes ? D / 4 : D / 64) ||
+          t.scalar_type() != (codes ? at::kUInt32 : k->scalar_type()))
+        return none();
+    }
+  const int rc = launch([&](void* st) {
+    return mspr_affine_q8_append(k->const_data_ptr(), v->const_data_ptr(), code, (int)(B * H), L, (int)D, ks[0]->data_ptr(),
+                                 ks[1]->data_ptr(), ks[2]->data_ptr(), vs[0]->data_ptr(), vs[1]->data_ptr(),
+                                 vs[2]->data_ptr(), cap, offset, st);
+  });
+  if (failed(rc, "q8_append")) return nullptr;
+  Py_RETURN_TRUE;
+}
+
+// (key side, value side, n) -> both sides as views of the first n rows of every head
+PyObject* leading_rows(PyObject* const* a, Py_ssize_t nargs) {
+  MSPR_NARGS(3)
+  const Tensor* t[2][3];
+  int64_t n;
+  if (!cache_side(a[0], t[0]) || !cache_side(a[1], t[1]) || !whole(a[2], &n)) return none();
+  for (const auto& side : t)
+    for (const Tensor* p : side)
+      if (n < 0 || n > p->size(2)) return none();
+  PyObject* sides[2];
+  for (int s = 0; s < 2; s++) {
+    sides[s] = wrap_tuple(t[s][0]->narrow(2, 0, n), t[s][1]->narrow(2, 0, n), t[s][2]->narrow(2, 0, n));
+    if (!sides[s]) return nullptr;
+  }
+  PyObject* r = PyTuple_Pack(2, sides[0], sides[1]);
+  Py_DECREF(sides[0]);
+  Py_DECREF(sides[1]);
+  return r;
+}
+
 // (queries f32 [B, Hq, 1, 256], six cache parts, scale, workspace) -> f32 like queries
 PyObject* sdpa_decode_q8(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(9)
@@ -576,6 +633,8 @@ PyMethodDef kMethods[] = {
     MSPR_METHOD(prefill_live),
     MSPR_METHOD(quantize),
     MSPR_METHOD(dequantize),
+    MSPR_METHOD(q8_append),
+    MSPR_METHOD(leading_rows),
     MSPR_METHOD(sdpa_decode_q8),
     MSPR_METHOD(sdpa_decode_q8_0),
     MSPR_METHOD(sdpa_fa_prefill_q8),

@@ -141,10 +141,10 @@ class QuantizedKVCache:
         self.values = None
 
     def _grow(self, like, need: int):
-        B, H, _, D = (int(v) for v in like.shape)
         cap = 0 if self.keys is None else int(self.keys[0].shape[2])
         if need <= cap:
             return
+        B, H, _, D = (int(v) for v in like.shape)
         new_cap = (need + self.step - 1) // self.step * self.step
 
         def alloc():
@@ -159,29 +159,38 @@ class QuantizedKVCache:
                     old[:, :, :self.offset].view(torch.int32 if old.dtype == torch.uint32 else old.dtype))
         self.keys, self.values = new_k, new_v
 
-    def _trimmed(self, triplet):
-        return tuple(t[:, :, :self.offset] for t in triplet)
+    def _views(self):
+        """Both sides trimmed to the rows in use."""
+        views = _lib.dispatch.leading_rows(self.keys, self.values, self.offset)
+        if views is not None:
+            return views
+        return (tuple(t[:, :, :self.offset] for t in self.keys), tuple(t[:, :, :self.offset] for t in self.values))
 
     @property
     def state(self):
         if self.keys is None:
             return None, None
-        return self._trimmed(self.keys), self._trimmed(self.values)
+        return self._views()
 
     def update_and_fetch(self, keys, values):
-        """Append ``keys``/``values`` ``[B, Hkv, L, D]`` and return the quantised cache up to the new length."""
-        if keys.ndim != 4 or tuple(keys.shape) != tuple(values.shape):
+        """Append ``keys``/``values`` ``[B, Hkv, L, D]`` and return the quantised cache up to the new length.
+
+        Rows in the cache's own layout and type are quantised straight into its buffers, keys and values in one
+        launch; others take a quantised copy that is moved behind the prefix.
+        """
+        if keys.ndim != 4 or keys.shape != values.shape:
             raise ValueError("keys and values must be [B, Hkv, L, D] of one shape")
         L = int(keys.shape[2])
         self._grow(keys, self.offset + L)
-        for src, dst in ((keys, self.keys), (values, self.values)):
-            wq, sc, bi = quantize(src)
-            lo, hi = self.offset, self.offset + L
-            dst[0][:, :, lo:hi].view(torch.int32).copy_(wq.view(torch.int32))
-            dst[1][:, :, lo:hi].copy_(sc)
-            dst[2][:, :, lo:hi].copy_(bi)
+        if _lib.dispatch.q8_append(keys, values, self.keys, self.values, self.offset) is None:
+            for src, dst in ((keys, self.keys), (values, self.values)):
+                wq, sc, bi = quantize(src)
+                lo, hi = self.offset, self.offset + L
+                dst[0][:, :, lo:hi].view(torch.int32).copy_(wq.view(torch.int32))
+                dst[1][:, :, lo:hi].copy_(sc)
+                dst[2][:, :, lo:hi].copy_(bi)
         self.offset += L
-        return self._trimmed(self.keys), self._trimmed(self.values)
+        return self._views()
 
 
 def sdpa_decode_q8(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases, scale, *, group_size: int = 64,
