@@ -128,6 +128,14 @@ int mspr_indexer_q_qat_live(const float* q, int64_t n_rows, float* out, void* st
 int mspr_indexer_scores_tiled_live(const void* q, const float* weights, const void* index_comp, int dtype,
                                    int batch, int n_heads, int n_tokens, int64_t n_comp, int64_t pos0,
                                    int ratio, float* scores, void* stream);
+/* The same with scratch of mspr_indexer_scores_tiled_live_workspace_bytes (16-byte aligned; NULL = none): the pool is
+ * packed into it as fp4 groups, and tokens whose operands are exact in that format (what the indexer's QAT produces) are
+ * multiplied in it, with the same scores. */
+size_t mspr_indexer_scores_tiled_live_workspace_bytes(int batch, int n_heads, int n_tokens, int64_t n_comp);
+int mspr_indexer_scores_tiled_live_ws(const void* q, const float* weights, const void* index_comp, int dtype,
+                                      int batch, int n_heads, int n_tokens, int64_t n_comp, int64_t pos0, int ratio,
+                                      float* scores, void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* ------------------------------------------------------------------ DS4 sparse attention */
 

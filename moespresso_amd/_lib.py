@@ -64,6 +64,10 @@ SIGNATURES = {
     "mspr_indexer_scores_tiled_live": (
         c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int, c_void_p,
                 c_void_p]),
+    "mspr_indexer_scores_tiled_live_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int64]),
+    "mspr_indexer_scores_tiled_live_ws": (
+        c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int, c_void_p,
+                c_void_p, c_size_t, c_void_p]),
     "mspr_indexed_mixed_attention_prefill": (
         c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64,
                 c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -226,9 +226,11 @@ PyObject* indexer_scores_tiled_live(PyObject* const* a, Py_ssize_t nargs) {
       P < 1 || H > 64)
     return none();
   Tensor scores = empty({B, T, P}, at::kFloat, *q);
+  Tensor ws = scratch(mspr_indexer_scores_tiled_live_workspace_bytes((int)B, (int)H, (int)T, P), *q);
   const int rc = launch([&](void* st) {
-    return mspr_indexer_scores_tiled_live(q->const_data_ptr(), (const float*)w->const_data_ptr(), c->const_data_ptr(), code,
-                                          (int)B, (int)H, (int)T, P, pos0, ratio, (float*)scores.data_ptr(), st);
+    return mspr_indexer_scores_tiled_live_ws(q->const_data_ptr(), (const float*)w->const_data_ptr(), c->const_data_ptr(),
+                                             code, (int)B, (int)H, (int)T, P, pos0, ratio, (float*)scores.data_ptr(),
+                                             ws.data_ptr(), ws.nbytes(), st);
   });
   return failed(rc, "indexer_scores_tiled_live") ? nullptr : wrap(scores);
 }

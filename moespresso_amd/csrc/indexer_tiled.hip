@@ -4,8 +4,23 @@
 // on v_mfma_f32_32x32x16_f16 with heads = M and pool rows = N, so the relu / weight / head sum runs on
 // the accumulator registers of one lane column per pool row.
 //
-// Workgroup = 4 waves = 4 consecutive tokens of one batch entry walking the same block of pool rows, which
-// it stages tile by tile in LDS; the token's 64 x 128 query block stays in registers.
+// Workgroup = 4 waves = 4 consecutive tokens of one batch entry walking the same block of pool rows; the token's
+// 64 x 128 query block stays in registers.
+//
+// Two forms of the product:
+//  * Operands that came out of the indexer's QAT are, group of 32 by group of 32, values of the e2m1 lattice times a power
+//    of two: exactly the operand format of v_mfma_scale_f32_32x32x64_f8f6f4 (fp4 with one e8m0 scale per 32), which
+//    multiplies four times as many of them per cycle as the float16 form. Both operands are packed once per call into MFMA
+//    operand order (pack_operands_kernel), where each value is checked by converting it back; the products are exact and
+//    so are their sums (some 18 significant bits), so the scores are those of the float16 form bit for bit. With the
+//    products this cheap the relu-weighted head sum on the vector units is the bound (two instructions per score and
+//    head: 256 cycles of a wave's 32-row tile against 128 of the matrix pipe). Its tiles need no LDS and no barrier, so
+//    the four waves drift apart and one wave's sums run under another's products.
+//    3844 tokens x 7961 rows from position 28000: 24 us packing + 157 us (float16 form 633), vector units busy three
+//    quarters of it; x 961 rows from position 0: 24 + 21 us (75); 517 tokens x 2053 rows: 7 + 14 us (46).
+//  * Where a value is outside that lattice (a pool row, or a query of the workgroup's tokens) the float16 form does the
+//    work, with pool tiles staged in LDS. It is a launch of its own behind the first, whose workgroups leave at once where
+//    nothing is left to do: in one kernel the two forms' registers held it to two waves per SIMD.
 #include "common.h"
 #include "profile.h"
 
@@ -28,7 +43,298 @@ __device__ __forceinline__ u32x4_t load8_as_f16(const void* base, int64_t off) {
   }
 }
 
-// A workgroup = 4 waves = 4 consecutive tokens walks `rows_per_block` pool rows (a multiple of 32) in tiles of 32.
+// ---- fp4 form of the operands
+
+typedef __attribute__((ext_vector_type(8))) int i32x8_t;
+
+// A packed block: 64 rows of 128 (the heads of one token, or 64 pool rows) in MFMA operand order, [row / 32][k-step][lane]
+// [16 bytes] with lane (n, g) holding columns 64 step + 32 g .. +31 of row n (+32), and one word of e8m0 scales per lane,
+// byte 2 (row / 32) + step.
+constexpr int kBlockRows = 64;
+constexpr int kBlockCodeBytes = kBlockRows * 64;
+constexpr int kBlockScaleBytes = 64 * 4;
+
+// four consecutive elements, widened to float32
+template <int DT>
+__device__ __forceinline__ f32x4_t load4_as_f32(const void* base, int64_t off) {
+  if constexpr (DT == MSPR_F16) {
+    const u32x2_t x = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const uint16_t*>(base) + off);
+    return f32x4_t{f16_bits_to_f32((uint16_t)(x.x & 0xFFFFu)), f16_bits_to_f32((uint16_t)(x.x >> 16)),
+                   f16_bits_to_f32((uint16_t)(x.y & 0xFFFFu)), f16_bits_to_f32((uint16_t)(x.y >> 16))};
+  } else {
+    return *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(base) + off);
+  }
+}
+
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor_max(uint32_t v) {
+  const uint32_t o = (uint32_t)__float_as_int(lane_xor<M>(__int_as_float((int)v)));
+  return o > v ? o : v;
+}
+
+// The packed operands in the workspace.
+struct PackedOperands {
+  uint8_t* pool_codes;   // [batch][pool blocks] blocks
+  uint8_t* q_codes;      // [batch][tokens] blocks
+  uint8_t* pool_scales;
+  uint8_t* q_scales;
+  int32_t* pool_exact;   // one flag per block: every value is of the lattice
+  int32_t* q_exact;
+};
+
+__host__ __device__ __forceinline__ int64_t pool_blocks(int64_t n_comp) { return (n_comp + kBlockRows - 1) / kBlockRows; }
+
+inline size_t packed_bytes(int batch, int n_tokens, int64_t n_comp) {
+  const size_t blocks = (size_t)batch * (pool_blocks(n_comp) + n_tokens);
+  return blocks * (kBlockCodeBytes + kBlockScaleBytes + sizeof(int32_t));
+}
+
+inline PackedOperands packed_operands(void* workspace, int batch, int n_tokens, int64_t n_comp) {
+  const int64_t pb = batch * pool_blocks(n_comp), qb = (int64_t)batch * n_tokens;
+  PackedOperands o;
+  o.pool_codes = reinterpret_cast<uint8_t*>(workspace);
+  o.q_codes = o.pool_codes + pb * kBlockCodeBytes;
+  o.pool_scales = o.q_codes + qb * kBlockCodeBytes;
+  o.q_scales = o.pool_scales + pb * kBlockScaleBytes;
+  o.pool_exact = reinterpret_cast<int32_t*>(o.q_scales + qb * kBlockScaleBytes);
+  o.q_exact = o.pool_exact + pb;
+  return o;
+}
+
+// Packs one block per workgroup. grid: (pool blocks + tokens, batch), 256 threads. Bound by the read of the queries, so all
+// accesses are whole lines: eight neighbouring lanes read a group of 32 (16 bytes each in float32), find its largest
+// magnitude by lane exchanges and convert four values each; the codes change to operand order in LDS.
+//
+// A group is stored times 2^e with the largest magnitude in [4, 8) * 2^e. (Lattice values times a power of two survive the
+// shift to that range: doubling maps the lattice below 4 into itself.) A block is exact if every value converts back to
+// itself and float16 could hold its groups exactly too.
+template <int DT>
+__global__ __launch_bounds__(256) void pack_operands_kernel(const void* __restrict__ q, const void* __restrict__ comp,
+                                                            int n_heads, int n_tokens, int64_t n_comp, PackedOperands out) {
+  __shared__ __attribute__((aligned(16))) uint16_t codes[kBlockCodeBytes / 2];
+  __shared__ __attribute__((aligned(16))) uint8_t scales[kBlockScaleBytes];
+  const int tid = threadIdx.x;
+  const int64_t n_pool = pool_blocks(n_comp), b = blockIdx.y;
+  const bool is_pool = (int64_t)blockIdx.x < n_pool;
+  const int64_t x = is_pool ? blockIdx.x : blockIdx.x - n_pool;  // pool block, or token
+  const void* src = is_pool ? comp : q;
+  const int64_t row0 = is_pool ? b * n_comp + x * kBlockRows : b * n_heads * n_tokens + x;
+  const int64_t row_step = is_pool ? 1 : n_tokens;
+  const int64_t left = is_pool ? n_comp - x * kBlockRows : n_heads;
+  const int n_rows = left < kBlockRows ? (int)left : kBlockRows;
+  const int col = (tid & 31) * 4;  // 32 lanes a row: eight rows per pass of the workgroup
+  f32x4_t v[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int r = 8 * i + (tid >> 5);
+    v[i] = r < n_rows ? load4_as_f32<DT>(src, (row0 + r * row_step) * 128 + col) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  bool exact = true;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int r = 8 * i + (tid >> 5);
+    uint32_t top = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const uint32_t a = __float_as_uint(v[i][j]) & 0x7FFFFFFFu;
+      top = a > top ? a : top;
+    }
+    top = lane_xor_max<4>(lane_xor_max<2>(lane_xor_max<1>(top)));
+    const int e = top == 0u ? 0 : (int)(top >> 23) - 127 - 2;
+    exact = exact && e >= -13 && e <= 13;
+    const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
+    uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[i].x, v[i].y, scale, 0);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v[i].z, v[i].w, scale, 1);
+    const f32x2_t b0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0), b1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 1);
+    exact = exact && b0.x == v[i].x && b0.y == v[i].y && b1.x == v[i].z && b1.y == v[i].w;
+    const int group = (tid & 31) >> 3, k = tid & 7;
+    const int lane = (r & 31) + 32 * (group & 1), part = 2 * (r >> 5) + (group >> 1);
+    codes[(part * 64 + lane) * 8 + k] = (uint16_t)c;
+    if (k == 0) scales[lane * 4 + part] = (uint8_t)(e + 127);
+  }
+  const int all = __syncthreads_and(exact);
+  const int64_t block = is_pool ? b * n_pool + x : b * n_tokens + x;
+  uint8_t* cp = (is_pool ? out.pool_codes : out.q_codes) + block * kBlockCodeBytes;
+  uint8_t* sp = (is_pool ? out.pool_scales : out.q_scales) + block * kBlockScaleBytes;
+  reinterpret_cast<u32x4_t*>(cp)[tid] = reinterpret_cast<const u32x4_t*>(codes)[tid];
+  if (tid < 64) reinterpret_cast<uint32_t*>(sp)[tid] = reinterpret_cast<const uint32_t*>(scales)[tid];
+  if (tid == 0) (is_pool ? out.pool_exact : out.q_exact)[block] = all;
+}
+
+// Whether all operands of the workgroup (the whole pool of its batch entry, its four tokens) are exact; every thread calls it.
+__device__ __forceinline__ bool operands_exact(const PackedOperands& o, int n_tokens, int64_t n_comp) {
+  const int64_t n = pool_blocks(n_comp);
+  bool exact = true;
+  for (int64_t i = threadIdx.x; i < n; i += 256) exact = exact && o.pool_exact[blockIdx.z * n + i] != 0;
+  const int t = blockIdx.y * 4 + (threadIdx.x & 3);
+  if (t < n_tokens) exact = exact && o.q_exact[(int64_t)blockIdx.z * n_tokens + t] != 0;
+  return __syncthreads_and(exact);
+}
+
+// max(x, 0) of a number that is no NaN, as one integer maximum (fmaxf costs a second instruction that quiets NaNs)
+__device__ __forceinline__ float relu_finite(float x) {
+  const int b = __float_as_int(x);
+  return __int_as_float(b > 0 ? b : 0);
+}
+
+// What one wave of a score workgroup works on: its token and the workgroup's block of pool rows.
+struct ScoreJob {
+  int lane, n, g;  // lane; operand row (head or pool row) and half
+  int b, t;        // batch entry, token (the last one where the chunk ends inside the workgroup: t_live is false)
+  bool t_live;
+  int64_t row_begin, row_end, visible;
+  int n_live;   // tiles of the block that hold a row visible to the token
+  int n_fetch;  // the same for the workgroup's last token, which sees the most
+  float* out_row;
+
+  __device__ __forceinline__ ScoreJob(int n_tokens, int64_t n_comp, uint32_t pos0, uint32_t ratio, int rows_per_block,
+                                      float* scores) {
+    lane = threadIdx.x & 63;
+    n = lane & 31;
+    g = lane >> 5;
+    b = blockIdx.z;
+    t = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    t_live = t < n_tokens;
+    if (!t_live) t = n_tokens - 1;
+    row_begin = (int64_t)blockIdx.x * rows_per_block;
+    row_end = row_begin + rows_per_block;
+    if (row_end > n_comp) row_end = n_comp;
+    auto visible_of = [&](int tok) -> int64_t {
+      const uint32_t qpos1 = pos0 + (uint32_t)tok + 1u;
+      const int64_t v = ratio == 0u ? n_comp : (int64_t)(qpos1 / ratio);
+      return v < n_comp ? v : n_comp;
+    };
+    auto live_tiles = [&](int64_t vis) -> int {
+      const int64_t live_end = vis < row_end ? vis : row_end;
+      return live_end > row_begin ? (int)((live_end - row_begin + 31) / 32) : 0;
+    };
+    visible = visible_of(t);
+    n_live = live_tiles(visible);
+    int t_last = blockIdx.y * 4 + 3;
+    if (t_last > n_tokens - 1) t_last = n_tokens - 1;
+    n_fetch = live_tiles(visible_of(t_last));
+    out_row = scores + ((int64_t)b * n_tokens + t) * n_comp;
+  }
+
+  // rows of the block behind the `n_done` tiles that were multiplied: not visible to this token
+  __device__ __forceinline__ void mask_rest(int n_done) const {
+    if (!t_live) return;
+    for (int64_t c = row_begin + (int64_t)n_done * 32 + lane; c < row_end; c += 64) out_row[c] = -__builtin_inff();
+  }
+
+  // weights of the heads this lane's accumulator registers hold: head = 32 hb + 8 (i/4) + 4 g + i%4
+  __device__ __forceinline__ void head_weights(const float* __restrict__ w, int n_tokens, int n_heads,
+                                               float (&wv)[2][16]) const {
+    const float* w_row = w + ((int64_t)b * n_tokens + t) * n_heads;
+    if (n_heads == 64 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {  // (four consecutive heads per load)
+#pragma unroll
+      for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(w_row + 32 * hb + 8 * j + 4 * g);
+          wv[hb][4 * j] = v.x;
+          wv[hb][4 * j + 1] = v.y;
+          wv[hb][4 * j + 2] = v.z;
+          wv[hb][4 * j + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+      for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const int head = 32 * hb + 8 * (i / 4) + 4 * g + (i % 4);
+          wv[hb][i] = head < n_heads ? w_row[head] : 0.0f;
+        }
+    }
+  }
+};
+
+// fp4 form. grid: (row blocks, token blocks, batch); a wave walks its rows in pairs of tiles, one packed block at a time.
+__global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restrict__ w, int n_heads, int n_tokens,
+                                                            int64_t n_comp, uint32_t pos0, uint32_t ratio,
+                                                            int rows_per_block, PackedOperands ops,
+                                                            float* __restrict__ scores) {
+  const ScoreJob j(n_tokens, n_comp, pos0, ratio, rows_per_block, scores);
+  if (j.n_fetch == 0) {  // no row of the block is visible to any of the four tokens, whatever the operands are
+    j.mask_rest(0);
+    return;
+  }
+  const int n_pairs = (j.n_live + 1) / 2;
+  const int64_t block0 = j.b * pool_blocks(n_comp) + j.row_begin / kBlockRows;
+  const u32x4_t* cp = reinterpret_cast<const u32x4_t*>(ops.pool_codes + block0 * kBlockCodeBytes) + j.lane;
+  const uint32_t* sp = reinterpret_cast<const uint32_t*>(ops.pool_scales + block0 * kBlockScaleBytes) + j.lane;
+  struct Rows {
+    u32x4_t c[2][2];
+    uint32_t s;
+  } even, odd;
+  auto fetch = [&](Rows& k, int pair) {
+    if (pair >= n_pairs) pair = n_pairs - 1;  // (a last fetch that nothing uses)
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) k.c[u][s] = cp[pair * (kBlockCodeBytes / 16) + (2 * u + s) * 64];
+    k.s = sp[pair * 64];
+  };
+  if (n_pairs > 0) fetch(even, 0);
+  u32x4_t qa[2][2];
+  const int64_t token = (int64_t)j.b * n_tokens + j.t;
+  const u32x4_t* qp = reinterpret_cast<const u32x4_t*>(ops.q_codes + token * kBlockCodeBytes) + j.lane;
+#pragma unroll
+  for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+    for (int s = 0; s < 2; s++) qa[hb][s] = qp[(2 * hb + s) * 64];
+  const uint32_t qs = reinterpret_cast<const uint32_t*>(ops.q_scales + token * kBlockScaleBytes)[j.lane];
+  float wv[2][16];
+  j.head_weights(w, n_tokens, n_heads, wv);
+  if (!operands_exact(ops, n_tokens, n_comp)) return;
+
+  float* out = j.out_row + j.row_begin + j.lane;
+  int left = (int)(j.row_end - j.row_begin) - j.lane, seen = (int)(j.visible - j.row_begin) - j.lane;
+  if (!j.t_live) left = 0;
+  auto step = [&](const Rows& k, int pair) {
+    f32x16_t acc[2][2];
+#define MSPR_FP4_STEP(u, hb, st)                                                                                   \
+  acc[u][hb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(                                                    \
+      i32x8_t{(int)qa[hb][st].x, (int)qa[hb][st].y, (int)qa[hb][st].z, (int)qa[hb][st].w, 0, 0, 0, 0},             \
+      i32x8_t{(int)k.c[u][st].x, (int)k.c[u][st].y, (int)k.c[u][st].z, (int)k.c[u][st].w, 0, 0, 0, 0},             \
+      st == 0 ? f32x16_t{0} : acc[u][hb], 4, 4, 2 * hb + st, (int)qs, 2 * u + st, (int)k.s)
+    MSPR_FP4_STEP(0, 0, 0);
+    MSPR_FP4_STEP(0, 1, 0);
+    MSPR_FP4_STEP(0, 0, 1);
+    MSPR_FP4_STEP(0, 1, 1);
+    MSPR_FP4_STEP(1, 0, 0);
+    MSPR_FP4_STEP(1, 1, 0);
+    MSPR_FP4_STEP(1, 0, 1);
+    MSPR_FP4_STEP(1, 1, 1);
+#undef MSPR_FP4_STEP
+    float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        sum[u] += relu_finite(acc[u][0][i]) * wv[0][i];
+        sum[u] += relu_finite(acc[u][1][i]) * wv[1][i];
+      }
+    // the exchange adds the two halves of a tile's heads and leaves the first tile's scores in the lower half-wave, the
+    // second's in the upper one: 256 bytes are stored at once
+    half_wave_exchange(sum[0], sum[1]);
+    const int c = 64 * pair;
+    if (c < left) out[c] = c < seen ? sum[0] + sum[1] : -__builtin_inff();
+  };
+  for (int i = 0; i < n_pairs; i += 2) {
+    fetch(odd, i + 1);
+    __builtin_amdgcn_sched_barrier(0);  // (requested before the products it hides behind, not after them)
+    step(even, i);
+    if (i + 1 >= n_pairs) break;
+    fetch(even, i + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    step(odd, i + 1);
+  }
+  j.mask_rest(2 * n_pairs);
+}
+
+// A workgroup = 4 waves = 4 consecutive tokens walks `rows_per_block` pool rows (a multiple of 64) in tiles of 32. Float16
+// form:
 // A tile is fetched once per workgroup (every thread 32 bytes of it, rounded to float16) into one of two LDS buffers,
 // a tile ahead of its use, and the four waves read their B operands from there: fetched by each wave for itself, the
 // 16-byte pieces of 32 rows keep a CU's address path busier than its matrix pipes. Rows past a token's visible
@@ -40,38 +346,14 @@ template <int DT>
 __global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __restrict__ q, const float* __restrict__ w,
                                                            const void* __restrict__ comp, int n_heads, int n_tokens,
                                                            int64_t n_comp, uint32_t pos0, uint32_t ratio,
-                                                           int rows_per_block, float* __restrict__ scores) {
+                                                           int rows_per_block, PackedOperands packed,
+                                                           float* __restrict__ scores) {
   __shared__ __attribute__((aligned(16))) unsigned char tile_lds[2][32 * kTilePitch];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int n = lane & 31;
-  const int g = lane >> 5;
-  const int b = blockIdx.z;
-  int t = blockIdx.y * 4 + wave;
-  const bool t_live = t < n_tokens;
-  if (!t_live) t = n_tokens - 1;
-
-  const int64_t row_begin = (int64_t)blockIdx.x * rows_per_block;
-  int64_t row_end = row_begin + rows_per_block;
-  if (row_end > n_comp) row_end = n_comp;
-  // tiles of this block that hold a row visible to token `tok`
-  auto visible_of = [&](int tok) -> int64_t {
-    const uint32_t qpos1 = pos0 + (uint32_t)tok + 1u;
-    const int64_t v = ratio == 0u ? n_comp : (int64_t)(qpos1 / ratio);
-    return v < n_comp ? v : n_comp;
-  };
-  auto live_tiles = [&](int64_t vis) -> int {
-    const int64_t live_end = vis < row_end ? vis : row_end;
-    return live_end > row_begin ? (int)((live_end - row_begin + 31) / 32) : 0;
-  };
-  const int64_t visible = visible_of(t);
-  const int n_live = live_tiles(visible);
-  // the workgroup's last token sees the most rows: it sets the number of tiles the workgroup fetches
-  int t_last = blockIdx.y * 4 + 3;
-  if (t_last > n_tokens - 1) t_last = n_tokens - 1;
-  const int n_fetch = live_tiles(visible_of(t_last));
-  float* out_row = scores + ((int64_t)b * n_tokens + t) * n_comp;
+  if (packed.pool_codes && operands_exact(packed, n_tokens, n_comp)) return;  // the fp4 form has done the work
+  const ScoreJob j(n_tokens, n_comp, pos0, ratio, rows_per_block, scores);
+  const int tid = threadIdx.x, n = j.n, g = j.g, b = j.b, t = j.t;
+  const int n_live = j.n_live, n_fetch = j.n_fetch;
+  const int64_t row_begin = j.row_begin;
 
   if (n_fetch > 0) {  // (the same in every wave of the workgroup: the barriers below are met by all)
     const void* comp_b =
@@ -106,29 +388,8 @@ __global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __rest
         qa[hb][s] = live ? v : u32x4_t{0, 0, 0, 0};
       }
     }
-    // weights of the heads this lane's accumulator registers hold: head = 32 hb + 8 (i/4) + 4 g + i%4
     float wv[2][16];
-    const float* w_row = w + ((int64_t)b * n_tokens + t) * n_heads;
-    if (n_heads == 64 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {  // (four consecutive heads per load)
-#pragma unroll
-      for (int hb = 0; hb < 2; hb++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(w_row + 32 * hb + 8 * j + 4 * g);
-          wv[hb][4 * j] = v.x;
-          wv[hb][4 * j + 1] = v.y;
-          wv[hb][4 * j + 2] = v.z;
-          wv[hb][4 * j + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-      for (int hb = 0; hb < 2; hb++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const int head = 32 * hb + 8 * (i / 4) + 4 * g + (i % 4);
-          wv[hb][i] = head < n_heads ? w_row[head] : 0.0f;
-        }
-    }
+    j.head_weights(w, n_tokens, n_heads, wv);
     stash(0, st);
     __syncthreads();
 
@@ -154,23 +415,26 @@ __global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __rest
         }
         sum += __shfl_xor(sum, 32, MSPR_WAVE);
         const int64_t c = row_begin + 32 * (int64_t)i + n;
-        if (t_live && g == 0 && c < row_end) out_row[c] = c < visible ? sum : -__builtin_inff();
+        if (j.t_live && g == 0 && c < j.row_end) j.out_row[c] = c < j.visible ? sum : -__builtin_inff();
       }
       if (i + 1 < n_fetch) stash((i + 1) & 1, st);
       __syncthreads();  // tile i+1 written by every thread; tile i read by every wave
     }
   }
-  // rows of the block behind the last multiplied tile: not visible to this token
-  if (t_live) {
-    for (int64_t c = row_begin + (int64_t)n_live * 32 + lane; c < row_end; c += 64) out_row[c] = -__builtin_inff();
-  }
+  j.mask_rest(n_live);
 }
 
 }  // namespace
 
-extern "C" int mspr_indexer_scores_tiled_live(const void* q, const float* weights, const void* index_comp, int dtype,
-                                              int batch, int n_heads, int n_tokens, int64_t n_comp, int64_t pos0,
-                                              int ratio, float* scores, void* stream) {
+extern "C" size_t mspr_indexer_scores_tiled_live_workspace_bytes(int batch, int n_heads, int n_tokens, int64_t n_comp) {
+  if (batch < 1 || n_heads < 1 || n_tokens < 1 || n_comp < 1) return 0;
+  return packed_bytes(batch, n_tokens, n_comp);
+}
+
+extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* weights, const void* index_comp, int dtype,
+                                                 int batch, int n_heads, int n_tokens, int64_t n_comp, int64_t pos0,
+                                                 int ratio, float* scores, void* workspace, size_t workspace_bytes,
+                                                 void* stream) {
   MSPR_REQUIRE(q && weights && index_comp && scores, "indexer_scores_tiled_live: null pointer");
   MSPR_REQUIRE(dtype == MSPR_F32 || dtype == MSPR_F16,
                "indexer_scores_tiled_live: q and index_comp must both be float32 or both be float16");
@@ -181,25 +445,62 @@ extern "C" int mspr_indexer_scores_tiled_live(const void* q, const float* weight
                "indexer_scores_tiled_live: bad size argument");
   MSPR_REQUIRE(mspr_aligned(q, 16) && mspr_aligned(index_comp, 16),
                "indexer_scores_tiled_live: pointers must be 16-byte aligned");
+  MSPR_REQUIRE(!workspace || (workspace_bytes >= packed_bytes(batch, n_tokens, n_comp) && mspr_aligned(workspace, 16)),
+               "indexer_scores_tiled_live: workspace of %zu bytes (16-byte aligned) needed, %zu given",
+               packed_bytes(batch, n_tokens, n_comp), workspace_bytes);
   // Four tokens per workgroup; the pool rows are split over several workgroups only as far as it takes to have
-  // about three workgroups for each of the 256 CUs (every workgroup fetches its tokens' query blocks anew).
+  // `want` workgroups, and no finer than `least` pairs of tiles.
   const int64_t tok_blocks = (n_tokens + 3) / 4;
-  int64_t row_blocks = (768 + tok_blocks * batch - 1) / (tok_blocks * batch);
-  const int64_t row_tiles = (n_comp + 31) / 32;
-  if (row_blocks > row_tiles) row_blocks = row_tiles;
-  if (row_blocks < 1) row_blocks = 1;
-  const int64_t rows_per_block = (row_tiles + row_blocks - 1) / row_blocks * 32;
-  row_blocks = (n_comp + rows_per_block - 1) / rows_per_block;
-  MSPR_REQUIRE(row_blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && rows_per_block < ((int64_t)1 << 31),
-               "indexer_scores_tiled_live: grid too large");
-  dim3 grid((unsigned)row_blocks, (unsigned)tok_blocks, (unsigned)batch), block(256);
+  const int64_t row_pairs = (n_comp + 63) / 64;
+  auto rows_per_workgroup = [&](int64_t want, int64_t least) -> int64_t {
+    int64_t blocks = (want + tok_blocks * batch - 1) / (tok_blocks * batch);
+    if (blocks > row_pairs / least) blocks = row_pairs / least;
+    if (blocks < 1) blocks = 1;
+    return (row_pairs + blocks - 1) / blocks * 64;
+  };
   hipStream_t st = (hipStream_t)stream;
+  dim3 block(256);
+  PackedOperands packed = {};
+  if (workspace) {
+    packed = packed_operands(workspace, batch, n_tokens, n_comp);
+    const int64_t blocks = pool_blocks(n_comp) + n_tokens;
+    MSPR_REQUIRE(blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && n_comp < ((int64_t)1 << 31),
+                 "indexer_scores_tiled_live: grid too large");
+    dim3 pgrid((unsigned)blocks, (unsigned)batch);
+    if (dtype == MSPR_F16)
+      pack_operands_kernel<MSPR_F16><<<pgrid, block, 0, st>>>(q, index_comp, n_heads, n_tokens, n_comp, packed);
+    else
+      pack_operands_kernel<MSPR_F32><<<pgrid, block, 0, st>>>(q, index_comp, n_heads, n_tokens, n_comp, packed);
+    // A workgroup's start (operands, flags: some 3 us) has to be carried by its tiles: at least 16 pairs of them, or 8 where
+    // the chip is not full otherwise. Three rounds of workgroups level the last one: 3844 tokens x 7961 rows took 164, 160,
+    // 157, 168 us with 1, 2, 3, 4 row blocks, x 961 rows from position 0 took 21, 25, 31 us with 1, 2, 4; 517 tokens x
+    // 2053 rows 15.5 us with 2 and 13.7 us with 4.
+    int64_t rows = rows_per_workgroup(2304, 16);
+    if ((n_comp + rows - 1) / rows * tok_blocks * batch < 768) rows = rows_per_workgroup(768, 8);
+    dim3 grid((unsigned)((n_comp + rows - 1) / rows), (unsigned)tok_blocks, (unsigned)batch);
+    scores_fp4_kernel<<<grid, block, 0, st>>>(weights, n_heads, n_tokens, n_comp, (uint32_t)pos0, (uint32_t)ratio,
+                                              (int)rows, packed, scores);
+    MSPR_CHECK_LAUNCH("indexer_scores_tiled_live (fp4)");
+  }
+  // float16 form: about three workgroups for each of the 256 CUs (every workgroup fetches its tokens' query blocks anew)
+  const int64_t rows = rows_per_workgroup(768, 1);
+  const int64_t row_blocks = (n_comp + rows - 1) / rows;
+  MSPR_REQUIRE(row_blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && rows < ((int64_t)1 << 31),
+               "indexer_scores_tiled_live: grid too large");
+  dim3 grid((unsigned)row_blocks, (unsigned)tok_blocks, (unsigned)batch);
   if (dtype == MSPR_F16)
-    scores_tiled_kernel<MSPR_F16><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp,
-                                                          (uint32_t)pos0, (uint32_t)ratio, (int)rows_per_block, scores);
+    scores_tiled_kernel<MSPR_F16><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp, (uint32_t)pos0,
+                                                          (uint32_t)ratio, (int)rows, packed, scores);
   else
-    scores_tiled_kernel<MSPR_F32><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp,
-                                                          (uint32_t)pos0, (uint32_t)ratio, (int)rows_per_block, scores);
+    scores_tiled_kernel<MSPR_F32><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp, (uint32_t)pos0,
+                                                          (uint32_t)ratio, (int)rows, packed, scores);
   MSPR_CHECK_LAUNCH("indexer_scores_tiled_live");
   return MSPR_OK;
+}
+
+extern "C" int mspr_indexer_scores_tiled_live(const void* q, const float* weights, const void* index_comp, int dtype,
+                                              int batch, int n_heads, int n_tokens, int64_t n_comp, int64_t pos0,
+                                              int ratio, float* scores, void* stream) {
+  return mspr_indexer_scores_tiled_live_ws(q, weights, index_comp, dtype, batch, n_heads, n_tokens, n_comp, pos0, ratio,
+                                           scores, nullptr, 0, stream);
 }

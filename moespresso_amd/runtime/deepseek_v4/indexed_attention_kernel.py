@@ -420,9 +420,11 @@ def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int =
     _SCORES_TILED_CALL_COUNTS[operand_form] += 1
     qc, wc, cc = q.contiguous(), weights.contiguous(), index_comp.contiguous()
     scores = torch.empty((batch, n_tokens, n_comp), dtype=torch.float32, device=dev)
-    rc = _lib.lib().mspr_indexer_scores_tiled_live(
+    nbytes = int(_lib.lib().mspr_indexer_scores_tiled_live_workspace_bytes(batch, n_heads, n_tokens, n_comp))
+    ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=dev)
+    rc = _lib.lib().mspr_indexer_scores_tiled_live_ws(
         _lib.ptr(qc), _lib.ptr(wc), _lib.ptr(cc), _lib.DTYPE_CODE[qc.dtype], batch, n_heads, n_tokens, n_comp,
-        int(pos0), int(ratio), _lib.ptr(scores), _lib.stream_ptr())
+        int(pos0), int(ratio), _lib.ptr(scores), _lib.ptr(ws), ws.numel() * 4, _lib.stream_ptr())
     _lib.check(rc, "indexer_scores_tiled_live")
     return scores
 

@@ -1,0 +1,59 @@
+"""The fp4 form of the tiled scores: the same scores as the float16 form (bit for bit on QAT'd operands), and operands of
+which only a part is exact in fp4."""
+
+import pytest
+import torch
+
+from moespresso_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(batch, heads, tokens, rows, dtype, seed=3):
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+    from moespresso_amd.runtime.deepseek_v4 import indexer_score_kernel as isk
+
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    q = iak.indexer_q_qat_live(torch.randn((batch, heads, tokens, 128), device="cuda", generator=gen))
+    comp = isk.indexer_qat_rows(torch.randn((batch, rows, 128), device="cuda", generator=gen))
+    w = torch.randn((batch, tokens, heads), device="cuda", generator=gen)
+    return q.to(dtype), w, comp.to(dtype)
+
+
+def _both(q, w, comp, pos0, ratio=4):
+    """(the operator's scores, the float16 form's scores)"""
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+    got = iak.indexer_scores_tiled_live(q, w, comp, pos0=pos0, ratio=ratio)
+    want = torch.empty_like(got)
+    _lib.check(_lib.lib().mspr_indexer_scores_tiled_live(
+        _lib.ptr(q), _lib.ptr(w), _lib.ptr(comp), _lib.DTYPE_CODE[q.dtype], q.shape[0], q.shape[1], q.shape[2],
+        comp.shape[1], pos0, ratio, _lib.ptr(want), _lib.stream_ptr()), "float16 form")
+    return got, want
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("batch,heads,tokens,rows,pos0,ratio", [
+    (1, 64, 1, 1, 3, 4), (1, 64, 4, 31, 200, 4), (2, 64, 5, 33, 60, 4), (1, 64, 9, 63, 0, 0), (1, 64, 6, 64, 250, 4),
+    (3, 64, 3, 65, 300, 4), (1, 40, 7, 130, 512, 4), (1, 1, 2, 97, 400, 4), (1, 64, 37, 2011, 7900, 4), (1, 64, 801, 1000, 0, 1)])
+def test_qat_operands_give_the_float16_form_bit_for_bit(dtype, batch, heads, tokens, rows, pos0, ratio):
+    got, want = _both(*_operands(batch, heads, tokens, rows, dtype), pos0, ratio)
+    assert got.equal(want)
+    assert ratio != 0 or bool(torch.isfinite(got).all())
+
+
+@pytest.mark.parametrize("spoil", ["query", "pool", "tiny", "huge", "nan"])
+def test_operands_outside_the_format_take_the_float16_form(spoil):
+    q, w, comp = _operands(1, 64, 13, 200, torch.float32)
+    if spoil == "query":
+        q[0, 5, 6, 70] += 0.03125  # one token of the second workgroup
+    elif spoil == "pool":
+        comp[0, 199, 127] = 0.3
+    elif spoil == "tiny":
+        comp[0, 64, :32] *= 2.0 ** -20
+    elif spoil == "huge":
+        q[0, :, 2, 32:64] *= 2.0 ** 13
+    else:
+        comp[0, 3, 3] = float("nan")
+    got, want = _both(q, w, comp, 900)
+    assert torch.equal(torch.nan_to_num(got, nan=12345.0), torch.nan_to_num(want, nan=12345.0))
