@@ -172,11 +172,11 @@ int mspr_indexed_mixed_attention_decode(const float* q, int n_heads, const void*
  * 512 contiguous values of q_dtype (f32 rounded to half on load, or f16); raw_kv: f16
  * [batch,raw_cap,512]; comp_kv: f16 [batch,n_comp,512]; topk: int32 [batch,n_tokens,top_k]
  * (top_k may be 0); sinks: f32 [n_heads]; out: f32 with the strides of q.
- * Calls whose slot count fits 22 tiles of 32 (window and ids each rounded up to whole tiles) run on one
- * persistent workgroup per CU that streams consecutive tokens; float32 queries are first rounded to half into
- * the workspace. Other calls take one workgroup per token and key range (every call does with
- * MSPR_PREFILL_PERSISTENT=0 in the environment, read per call). The arguments and the workspace size asked
- * for are the same either way.
+ * Id lists of up to 3520 ids run on the kernel of prefill_attn.hip (one workgroup per token and 64 heads, two per CU,
+ * no workspace), longer ones on the split kernel, one workgroup per token and key range. MSPR_PREFILL_PERSISTENT in
+ * the environment, read per call, keeps every call on a form to compare with: 1 = one persistent workgroup per CU that
+ * streams consecutive tokens (slots of up to 22 tiles; float32 queries are rounded to half into the workspace), 0 = the
+ * split kernel. The workspace query follows the same variable.
  * Workspace: mspr_indexed_mixed_attention_prefill_workspace_bytes(q_dtype, batch, n_heads, n_tokens,
  * min(window or raw_cap, raw_cap), top_k). */
 int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, int batch, int n_heads, int n_tokens,

@@ -1,0 +1,25 @@
+// Launch interface of the indexed prefill attention kernel (prefill_attn.hip).
+#pragma once
+#include "common.h"
+
+struct IndexedPrefillArgs {
+  const void* q;  // element (b, t, head, d) at b*q_batch_stride + t*q_token_stride + head*q_head_stride + d
+  int q_dtype;    // MSPR_F16 or MSPR_F32 (rounded to float16 on load)
+  int64_t q_batch_stride, q_head_stride, q_token_stride;
+  int batch, n_tokens, n_heads;
+  const void* win;  // float16 ring [batch][raw_cap][512]
+  int raw_cap, raw_start;
+  int max_win;      // most ring rows any token visits
+  const void* pool;  // float16 [batch][n_pool][512]
+  int64_t n_pool;
+  const int32_t* idx;  // [batch][n_tokens][n_idx]
+  int n_idx;
+  uint32_t pos0, window, ratio;
+  const float* sinks;  // [n_heads] or null
+  float scale_log2;
+  float* out;  // strides as q
+};
+
+// Whether the kernel takes the call: the ids of a token are staged in LDS next to the row tiles.
+bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx);
+int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, hipStream_t st);

@@ -1,0 +1,323 @@
+// Indexed prefill attention: every token of a chunk attends the rows of its sliding window (a ring) and pool rows that its
+// own id list names. K == V, 512 wide float16 rows shared by all heads; a per-head sink joins the denominator.
+//
+// Visit rules (reference: indexed_attention_kernel.py:120-173 of src/moespresso/runtime/deepseek_v4): ring rows for positions
+// [max(first_raw, pos+1-window), min(pos, last)], then the ids in order; a negative id is skipped and the first id at or
+// behind min((pos+1)/ratio, n_pool) ends the walk.
+//
+// Split: a workgroup is four waves and owns one token and 64 heads; a wave owns 16 of the heads outright: the 16 x 512 query
+// block (64 registers), the whole 512-wide output (128 registers) and the softmax state of its heads. Nothing but the row
+// tiles is shared between the waves, so a tile costs one barrier: tiles of 32 rows lie in two LDS buffers, the copies of
+// tile t+1 (asynchronous, one 1 KB row per instruction, its address scalar) are issued behind the barrier of tile t and land
+// under its arithmetic. S^T = K.Q^T leaves a wave's weights in the registers that O^T += V^T.P^T wants as its B operand
+// (the key order inside a tile is free as long as V^T uses the same), V^T comes out of the row-major tile by transpose reads.
+//
+// Two such workgroups share a CU (80 KB of LDS and 256 registers a lane each) and drift apart: one multiplies while the
+// other waits for its barrier, its ids, or takes its exponentials. The price is LDS traffic: each wave reads the whole tile
+// for both products, 256 KB per tile and workgroup, which bounds the kernel: the two products alone need 2800 cycles of a
+// pair of workgroups' tiles, the matrix pipes 2050, and it takes 3100 (2.15 GHz).
+//
+// 3844 tokens, 64 heads, 128 + 512 rows each: from position 28000 426 us with float32 queries (before, with eight waves of
+// a persistent workgroup on one token and the queries rounded to half in a pass of their own: 620 + 130), from position 0
+// 324 us (542); 517 tokens 76 us (121). Without the tile copies 355 / 295 us, without the stores 360 / 276, with neither
+// 303 / 240, which is the products and the softmax. Measured and not kept: one wave for 128 output columns of all heads
+// (V^T read once per workgroup, weights exchanged through LDS behind a second barrier) 500 / 397; persistent workgroups
+// that request the next token's ids, rows and queries under the last tile 471 / 351 with the stores as they were (464 / 361
+// without).
+#include "prefill_attn.h"
+#include "profile.h"
+
+namespace {
+
+constexpr int kTile = 32;
+constexpr int kThreads = 256;
+constexpr int kD = 512;
+constexpr int kPitch = kD * 2 + 32;  // bytes between rows in LDS: both read patterns run fastest at this distance
+constexpr int kTileBytes = kTile * kPitch;
+constexpr int kOffIds = 2 * kTileBytes;
+constexpr int kLdsBytes = 80 * 1024;                       // half of a CU's
+constexpr int kMaxIds = (kLdsBytes - kOffIds - 64) / 4 / 64 * 64;
+constexpr int kOffStop = kOffIds + kMaxIds * 4;
+static_assert(kOffStop + 4 <= kLdsBytes, "LDS map");
+constexpr int kQSteps = kD / 32;
+constexpr int kOutPitch = 256 + 4;  // floats between rows of the output staging: 16 heads' stores fall on 16 bank groups
+static_assert(4 * 16 * kOutPitch * 4 <= 2 * kTileBytes, "output staging lies in the tile buffers");
+constexpr int kAheadK = 8, kAheadV = 6;  // operand reads in flight (6/4 measures the same, 10/8 9 % slower)
+
+__device__ __attribute__((aligned(16))) const unsigned char g_prefill_zero_row[kD * 2] = {0};
+
+__device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) _Float16 h2_t;
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, h2_t));
+}
+
+// One 1 KB row to LDS: lane l's 16 bytes go to lds_base + 16 l. Through asm so that the compiler does not drain it in front
+// of LDS reads; the tile loop waits for all copies of a tile at its barrier.
+__device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_base) : "memory", "m0");
+}
+
+template <int QDT>
+__global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPrefillArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  int* ids = reinterpret_cast<int*>(lds + kOffIds);
+  int* stop_sh = reinterpret_cast<int*>(lds + kOffStop);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15;  // head of the wave (MFMA column), or row of an operand block
+  const int kg = lane >> 4;
+
+  // The tokens with the most rows (the last ones, at the start of a context) are started first.
+  const int n_hblk = (a.n_heads + 63) / 64;
+  const int unit = (int)(gridDim.x - 1u - blockIdx.x);
+  const int hb = unit % n_hblk;
+  const int seq = unit / n_hblk;
+  const int b = seq / a.n_tokens;
+  const int t = seq - b * a.n_tokens;
+
+  // window rows and visible pool prefix, in the unsigned 32-bit arithmetic of the reference kernel
+  const uint32_t qpos = a.pos0 + (uint32_t)t, n_raw = (uint32_t)a.raw_cap;
+  const uint32_t last_pos = a.pos0 + (uint32_t)a.n_tokens - 1u;
+  const uint32_t first_raw_pos = last_pos + 1u - n_raw;
+  const uint32_t window_first = (a.window != 0u && qpos + 1u > a.window) ? qpos + 1u - a.window : 0u;
+  const uint32_t first = first_raw_pos > window_first ? first_raw_pos : window_first;
+  const uint32_t last = qpos < last_pos ? qpos : last_pos;
+  int n_win = first <= last ? (int)(last - first + 1u) : 0;
+  if (n_win > a.max_win) n_win = a.max_win;
+  const int win_first = first <= last ? (int)(first - first_raw_pos) : 0;
+  int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
+  if (visible > a.n_pool) visible = a.n_pool;
+  const int wt = (n_win + kTile - 1) / kTile;
+  const uint64_t win_base = reinterpret_cast<uint64_t>(a.win) + (uint64_t)b * (uint64_t)a.raw_cap * (kD * 2);
+  const uint64_t pool_base = reinterpret_cast<uint64_t>(a.pool) + (uint64_t)b * (uint64_t)a.n_pool * (kD * 2);
+
+  // Copies of a tile: this wave's eight rows. `row` holds, per lane l < 32, the row of slot l (-1: no row, zeros).
+  const uint32_t lane_off = (uint32_t)lane * 16u;
+  const uint32_t my_rows_lds =
+      __builtin_amdgcn_readfirstlane((uint32_t)(size_t)MSPR_LDS_PTR(unsigned char, lds) + (uint32_t)(8 * wave * kPitch));
+  auto copy_rows = [&](int tile, uint64_t base, int row) {
+    const uint32_t dst = my_rows_lds + (uint32_t)((tile & 1) * kTileBytes);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int r = __builtin_amdgcn_readlane(row, 8 * wave + j);
+      const uint64_t p = r >= 0 ? base + (uint64_t)(uint32_t)r * (kD * 2) : reinterpret_cast<uint64_t>(&g_prefill_zero_row[0]);
+      async_row(p, lane_off, dst + (uint32_t)(j * kPitch));
+    }
+  };
+  auto window_row = [&](int tile) -> int {
+    const int ls = tile * kTile + (lane & 31);
+    uint32_t r = (uint32_t)a.raw_start + (uint32_t)win_first + (uint32_t)ls;
+    if (r >= n_raw) r -= n_raw;
+    return ls < n_win ? (int)r : -1;
+  };
+
+  // ---- the first window tile needs no ids: on its way before anything else
+  if (wt > 0) copy_rows(0, win_base, window_row(0));
+
+  // ---- ids to LDS, position of the first one that ends the walk
+  if (tid == 0) *stop_sh = a.n_idx;
+  __syncthreads();
+  {
+    const int32_t* src = a.idx + ((int64_t)b * a.n_tokens + t) * a.n_idx;
+    int found = a.n_idx;
+    for (int i = tid; i < a.n_idx; i += kThreads) {
+      const int id = src[i];
+      ids[i] = id;
+      if (id >= 0 && (int64_t)id >= visible && i < found) found = i;
+    }
+    if (found < a.n_idx) atomicMin(stop_sh, found);
+  }
+
+  // ---- query operand: lane (head c16, kg) holds q[head][32 ks + 8 kg .. +7], zero rows past n_heads
+  const int head = hb * 64 + 16 * wave + c16;
+  const bool live = head < a.n_heads;
+  const int64_t qoff = (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
+                       (int64_t)(live ? head : 0) * a.q_head_stride + 8 * kg;
+  u32x4_t qf[kQSteps];
+#pragma unroll
+  for (int ks = 0; ks < kQSteps; ks++) {
+    if constexpr (QDT == MSPR_F16) {
+      qf[ks] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(a.q) + qoff + 32 * ks);
+    } else {
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff + 32 * ks);
+      const f32x4_t lo = p[0], hi = p[1];
+      qf[ks] = u32x4_t{pack_h2(lo.x, lo.y), pack_h2(lo.z, lo.w), pack_h2(hi.x, hi.y), pack_h2(hi.z, hi.w)};
+    }
+    if (!live) qf[ks] = u32x4_t{0u, 0u, 0u, 0u};
+  }
+  const float sink = live && a.sinks ? a.sinks[head] * 1.4426950408889634f : -__builtin_inff();
+  __syncthreads();
+  const int stop = __builtin_amdgcn_readfirstlane(*stop_sh);
+  const int n_tiles = wt + (stop + kTile - 1) / kTile;
+
+  auto pool_row = [&](int tile) -> int {
+    const int gi = (tile - wt) * kTile + (lane & 31);
+    const int id = ids[gi < kMaxIds ? gi : 0];
+    return gi < stop ? (id >= 0 ? id : -1) : -1;  // (an id in front of the stop is inside the visible prefix)
+  };
+  // rows and validity word of a tile
+  auto rows_of = [&](int tile) -> int { return tile < wt ? window_row(tile) : pool_row(tile); };
+  int row = rows_of(0);
+  if (wt == 0 && n_tiles > 0) copy_rows(0, pool_base, row);
+
+  f32x4_t oacc[32];
+#pragma unroll
+  for (int mt = 0; mt < 32; mt++) oacc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -__builtin_inff();  // reference maximum of head c16 (log2 domain), the same in its four lanes
+  float l_run = 0.0f;               // this lane's share of the denominator: its eight keys of every tile
+  constexpr float kGrow = 8.0f;     // float16 weights stay below 2^8
+
+  const int a_off = c16 * kPitch + 16 * kg;
+  const int tr_off = (4 * kg + (c16 >> 2)) * kPitch + 8 * (c16 & 3);
+
+  for (int tile = 0; tile < n_tiles; tile++) {
+    const uint32_t valid = (uint32_t)__ballot(row >= 0);  // bit l: slot l (both halves of the wave hold the 32 slots)
+    // the copies of this tile have landed (they are the only vector-memory operations in flight), and every wave is done
+    // with the tile before it, whose buffer the next copies overwrite
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tile + 1 < n_tiles) {
+      row = rows_of(tile + 1);
+      copy_rows(tile + 1, tile + 1 < wt ? win_base : pool_base, row);
+    }
+    const unsigned char* kt = lds + (tile & 1) * kTileBytes;
+
+    // ---- S^T blocks: keys 16 u + 4 kg + i of head c16. The operand reads run kAheadK matrix instructions in front of their
+    //      use (stated to the scheduler, which keeps two in flight otherwise; an LDS read takes as long as eight of them).
+    f32x4_t sacc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < kQSteps; ks++)
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+        sacc[u] = mfma16(*reinterpret_cast<const u32x4_t*>(kt + a_off + u * (16 * kPitch) + ks * 64), qf[ks], sacc[u]);
+    __builtin_amdgcn_sched_group_barrier(0x100, kAheadK, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * kQSteps - kAheadK; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAheadK, 0);
+
+    // ---- online softmax in the log2 domain
+    float sv[8];
+    float tmax = -__builtin_inff();
+    {
+      const uint32_t v0 = valid >> (4 * kg), v1 = valid >> (16 + 4 * kg);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        sv[i] = (v0 >> i) & 1u ? sacc[0][i] * a.scale_log2 : -__builtin_inff();
+        sv[4 + i] = (v1 >> i) & 1u ? sacc[1][i] * a.scale_log2 : -__builtin_inff();
+        tmax = fmaxf(tmax, fmaxf(sv[i], sv[4 + i]));
+      }
+    }
+    tmax = half_wave_max(row_pair_max(tmax));
+    const bool grow = tmax > m_run + kGrow;
+    if (__any(grow)) {
+      const float m_new = grow ? tmax : m_run;
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+      l_run *= alpha;
+      m_run = m_new;
+#pragma unroll
+      for (int mt = 0; mt < 32; mt++) oacc[mt] = oacc[mt] * alpha;
+    }
+    const float m_safe = m_run == -__builtin_inff() ? 0.0f : m_run;
+    u32x4_t pf;
+    {
+      float p[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        p[i] = __builtin_amdgcn_exp2f(sv[i] - m_safe);
+        l_run += p[i];
+      }
+      pf = u32x4_t{pack_h2(p[0], p[1]), pack_h2(p[2], p[3]), pack_h2(p[4], p[5]), pack_h2(p[6], p[7])};
+    }
+
+    // ---- O^T += V^T.P^T: output columns 16 mt + 4 kg + i of head c16
+#pragma unroll
+    for (int mt = 0; mt < 32; mt++) {
+      const unsigned char* base = kt + tr_off + mt * 32;
+      const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MSPR_LDS_PTR(s16x4_t, base));
+      const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MSPR_LDS_PTR(s16x4_t, base + 16 * kPitch));
+      const u32x2_t lo2 = __builtin_bit_cast(u32x2_t, lo), hi2 = __builtin_bit_cast(u32x2_t, hi);
+      oacc[mt] = mfma16(u32x4_t{lo2.x, lo2.y, hi2.x, hi2.y}, pf, oacc[mt]);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 0);
+#pragma unroll
+    for (int i = 0; i < 32 - kAheadV; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAheadV, 0);
+  }
+
+  // ---- sink, normalisation, output
+  float l = l_run;
+  l += __shfl_xor(l, 16, MSPR_WAVE);
+  l += __shfl_xor(l, 32, MSPR_WAVE);
+  const float m_all = fmaxf(m_run, sink);
+  const float m_safe = m_all == -__builtin_inff() ? 0.0f : m_all;
+  const float w = __builtin_amdgcn_exp2f(m_run - m_safe);
+  l = l * w + __builtin_amdgcn_exp2f(sink - m_safe);
+  const float f = l == 0.0f ? 0.0f : w / l;
+  // The accumulators hold 64-byte pieces of 16 heads' rows. They change places through LDS (the tile buffers are free), half
+  // of the columns at a time, so that every store writes 1 KB of one row; and as nobody reads 128 KB per token back before
+  // the chunk is through, past the caches.
+  __syncthreads();
+  float* stage = reinterpret_cast<float*>(lds) + wave * (16 * kOutPitch);  // [16 heads][kOutPitch], this wave's own
+  float* out = a.out + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
+               (int64_t)(hb * 64 + 16 * wave) * a.q_head_stride + 4 * lane;
+  const int n_live = a.n_heads - (hb * 64 + 16 * wave);
+#pragma unroll
+  for (int half = 0; half < 2; half++) {
+#pragma unroll
+    for (int mt = 0; mt < 16; mt++)
+      *reinterpret_cast<f32x4_t*>(stage + c16 * kOutPitch + 16 * mt + 4 * kg) = oacc[16 * half + mt] * f;
+    f32x4_t r[16];
+#pragma unroll
+    for (int h = 0; h < 16; h++) r[h] = *reinterpret_cast<const f32x4_t*>(stage + h * kOutPitch + 4 * lane);
+    if (n_live >= 16) {
+#pragma unroll
+      for (int h = 0; h < 16; h++)
+        __builtin_nontemporal_store(r[h], reinterpret_cast<f32x4_t*>(out + h * a.q_head_stride + 256 * half));
+    } else {
+#pragma unroll
+      for (int h = 0; h < 16; h++)
+        if (h < n_live) *reinterpret_cast<f32x4_t*>(out + h * a.q_head_stride + 256 * half) = r[h];
+    }
+  }
+}
+
+template <int QDT>
+int launch(const IndexedPrefillArgs& a, hipStream_t st) {
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    if (e != hipSuccess) {
+      mspr_set_error("indexed prefill attention: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
+      return MSPR_ERR_LAUNCH;
+    }
+    attr_set = true;
+  }
+  dim3 grid((unsigned)((int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64))), block(kThreads);
+  {
+    MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
+    indexed_prefill_kernel<QDT><<<grid, block, kLdsBytes, st>>>(a);
+  }
+  MSPR_CHECK_LAUNCH("indexed prefill attention");
+  return MSPR_OK;
+}
+
+}  // namespace
+
+bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx) {
+  return n_idx <= kMaxIds && (int64_t)batch * n_tokens * ((n_heads + 63) / 64) < ((int64_t)1 << 31);
+}
+
+int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, hipStream_t st) {
+  return a.q_dtype == MSPR_F32 ? launch<MSPR_F32>(a, st) : launch<MSPR_F16>(a, st);
+}

@@ -23,6 +23,7 @@
 // column = l % 32, row = 8*(i/4) + 4*(l/32) + i%4. In S^T the column is the head and the row the
 // key, so softmax statistics are per lane; P^T registers feed the next MFMA's B operand unchanged.
 #include "common.h"
+#include "prefill_attn.h"
 #include "profile.h"
 
 #include <cstdlib>
@@ -1485,6 +1486,17 @@ int launch_split(const SparseAttnArgs& a, hipStream_t st) {
   return MSPR_OK;
 }
 
+// Which kernel runs the prefill form: by default the one of prefill_attn.hip, which takes id lists of up to what its LDS
+// holds next to the tiles (longer ones: the split kernel below, one workgroup per token). MSPR_PREFILL_PERSISTENT in the
+// environment, read per call like the reference's consumer switches, keeps calls on the forms to compare it with: 1 the
+// persistent kernel of this file, 0 the split kernel.
+enum PrefillForm { kPrefillSplit = 0, kPrefillPersistent = 1, kPrefillWaves = 2 };
+PrefillForm prefill_form() {
+  const char* gate = getenv("MSPR_PREFILL_PERSISTENT");
+  if (!gate || gate[0] == '\0' || gate[1] != '\0') return kPrefillWaves;
+  return gate[0] == '0' ? kPrefillSplit : gate[0] == '1' ? kPrefillPersistent : kPrefillWaves;
+}
+
 // The persistent prefill consumer takes at most PrefillGeometry::kMaxTiles tiles per token (float32 queries go
 // through a half-precision copy in the workspace first); longer slot lists go through the split kernel, one
 // workgroup per token.
@@ -1492,10 +1504,7 @@ bool prefill_consumer_fits(const SparseAttnArgs& a, int kv_dtype, int k_dim) {
   if (!a.prefill || kv_dtype != MSPR_F16 || k_dim != 512 || (a.q_dtype != MSPR_F16 && a.q_dtype != MSPR_F32) || a.rope ||
       a.out_dtype != MSPR_F32)
     return false;
-  // MSPR_PREFILL_PERSISTENT=0 (read per call, like the reference's consumer switches) keeps every prefill call on
-  // the split kernel, one workgroup per token: the form to compare the persistent consumer with
-  const char* gate = getenv("MSPR_PREFILL_PERSISTENT");
-  if (gate && gate[0] == '0' && gate[1] == '\0') return false;
+  if (prefill_form() != kPrefillPersistent) return false;
   if (a.subst_row || a.subst_from_params || a.pool_rows_dev) return false;
   const int tiles = (a.n_win + kTile - 1) / kTile + (a.n_idx + kTile - 1) / kTile;
   return tiles <= PrefillGeometry::kMaxTiles;
@@ -1607,10 +1616,12 @@ extern "C" size_t mspr_sparse_attention_workspace_bytes(int batch, int n_heads, 
 extern "C" size_t mspr_indexed_mixed_attention_prefill_workspace_bytes(int q_dtype, int batch, int n_heads,
                                                                        int n_tokens, int window_rows, int top_k) {
   if (batch < 1 || n_heads < 1 || n_tokens < 1 || window_rows < 0 || top_k < 0) return 0;
+  const PrefillForm form = prefill_form();
+  if (form == kPrefillWaves && mspr_indexed_prefill_fits(batch, n_heads, n_tokens, top_k)) return 0;
   // the per-range partials of the split kernel (slot lists too long for the persistent consumer), or the
   // half-precision copy of float32 queries for the persistent consumer, whichever is larger
   size_t need = workspace_bytes(batch * n_tokens, n_heads, (int64_t)window_rows + top_k);
-  if (q_dtype == MSPR_F32) {
+  if (form == kPrefillPersistent && q_dtype == MSPR_F32) {
     const size_t copy = (size_t)batch * n_tokens * n_heads * 512 * sizeof(uint16_t);
     if (copy > need) need = copy;
   }
@@ -1806,6 +1817,36 @@ extern "C" int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, 
                "%s: q strides must be multiples of 8 elements", what);
   MSPR_REQUIRE(mspr_aligned(q, 16) && mspr_aligned(raw_kv, 16) && mspr_aligned(comp_kv, 16) && mspr_aligned(out, 16),
                "%s: pointers must be 16-byte aligned", what);
+  // slot space: at most min(window, raw_cap, tokens seen so far) ring rows per token
+  int64_t max_win = window != 0 && window < raw_cap ? window : raw_cap;
+  if (max_win > pos0 + n_tokens) max_win = pos0 + n_tokens;
+  if (prefill_form() == kPrefillWaves && n_comp < ((int64_t)1 << 31) &&
+      mspr_indexed_prefill_fits(batch, n_heads, n_tokens, top_k)) {
+    IndexedPrefillArgs p = {};
+    p.q = q;
+    p.q_dtype = q_dtype;
+    p.q_batch_stride = q_batch_stride;
+    p.q_head_stride = q_head_stride;
+    p.q_token_stride = q_token_stride;
+    p.batch = batch;
+    p.n_tokens = n_tokens;
+    p.n_heads = n_heads;
+    p.win = raw_kv;
+    p.raw_cap = raw_cap;
+    p.raw_start = raw_start;
+    p.max_win = (int)max_win;
+    p.pool = comp_kv;
+    p.n_pool = n_comp;
+    p.idx = topk;
+    p.n_idx = top_k;
+    p.pos0 = (uint32_t)pos0;
+    p.window = (uint32_t)window;
+    p.ratio = (uint32_t)ratio;
+    p.sinks = sinks;
+    p.scale_log2 = (float)(1.4426950408889634 / sqrt(512.0));
+    p.out = out;
+    return mspr_launch_indexed_prefill(p, (hipStream_t)stream);
+  }
   SparseAttnArgs a = {};
   a.q = q;
   a.q_dtype = q_dtype;
@@ -1821,9 +1862,6 @@ extern "C" int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, 
   a.ratio = (uint32_t)ratio;
   a.win = raw_kv;
   a.win_batch_stride = (int64_t)raw_cap * 512;
-  // slot space: at most min(window, raw_cap, tokens seen so far) ring rows per token
-  int64_t max_win = window != 0 && window < raw_cap ? window : raw_cap;
-  if (max_win > pos0 + n_tokens) max_win = pos0 + n_tokens;
   a.n_win = (int)max_win;
   a.win_first = 0;
   a.raw_start = raw_start;

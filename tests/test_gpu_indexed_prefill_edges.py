@@ -1,0 +1,39 @@
+"""The prefill attention kernel at the edges of its tiles, head blocks and id staging, in all three forms of the dispatch."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ds4
+
+pytestmark = pytest.mark.gpu
+
+
+# tokens, heads, top_k, window, raw_cap, pos0, ratio: no ids; one row more or less than a tile of 32; heads of a partly
+# filled wave and of a second block; the longest id list the kernel stages, and one that goes to the split kernel
+@pytest.mark.parametrize("tokens,heads,top_k,window,raw_cap,pos0,ratio", [
+    (1, 8, 0, 128, 1, 0, 4), (3, 16, 1, 1, 3, 9, 4), (5, 24, 31, 31, 40, 200, 4), (4, 64, 32, 32, 36, 300, 1),
+    (2, 72, 33, 33, 37, 400, 4), (2, 136, 65, 128, 130, 1000, 4), (2, 16, 3520, 64, 70, 20000, 4), (2, 16, 3521, 64, 70, 20000, 4),
+    (6, 32, 100, 0, 6, 0, 0)])
+@pytest.mark.parametrize("form", [None, "1", "0"])
+def test_edges_match_the_oracle(monkeypatch, form, tokens, heads, top_k, window, raw_cap, pos0, ratio):
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+    monkeypatch.delenv("MSPR_PREFILL_PERSISTENT", raising=False)
+    if form is not None:
+        monkeypatch.setenv("MSPR_PREFILL_PERSISTENT", form)
+    rng = np.random.default_rng(17)
+    n_comp = max(8, top_k + 9)
+    q = rng.standard_normal((tokens, heads, 512), dtype=np.float32)
+    raw = rng.standard_normal((raw_cap, 512), dtype=np.float32).astype(np.float16)
+    comp = rng.standard_normal((n_comp, 512), dtype=np.float32).astype(np.float16)
+    ids = np.stack([np.sort(rng.choice(n_comp, top_k, replace=False)) for _ in range(tokens)]).astype(np.int32).reshape(tokens, top_k)
+    ids[rng.random(ids.shape) < 0.1] = -1
+    sinks = rng.standard_normal((heads,), dtype=np.float32)
+    raw_start = raw_cap // 3
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    got = iak.indexed_mixed_attention_prefill(to(q), to(raw), to(comp), to(ids), to(sinks), pos0=pos0, window=window, ratio=ratio,
+                                              raw_start=raw_start)
+    want = ds4.indexed_mixed_attention_prefill(q, raw, comp, ids, sinks, pos0=pos0, window=window, ratio=ratio,
+                                               raw_start=raw_start)
+    np.testing.assert_allclose(got.cpu().numpy(), want, rtol=2e-3, atol=2e-3)
