@@ -5,10 +5,9 @@
 // inverse form negates the float32 sine first); every product and every sum of the rotation is
 // rounded to the element type on its own (float32 rows: float32 operations, never contracted).
 //
-// A workgroup owns one sequence position and a slab of the outer rows (batch x heads): the 32
-// cosine / sine pairs of the position are worked out once, by the first 32 threads, and shared
-// through LDS, so the transcendental work does not grow with the head count; the rows then stream
-// through with 16-byte (float32) or 8-byte (16-bit) accesses.
+// A workgroup owns one sequence position (the wide form below: a few) and a slab of the outer rows (batch x heads): the
+// cosine / sine pairs of the position are worked out once and shared through LDS, so the transcendental work does not
+// grow with the head count; the rows then stream through. Both forms are bound by memory.
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -112,6 +111,101 @@ __global__ __launch_bounds__(kThreads) void partial_rope_kernel(const void* __re
   }
 }
 
+// Wide form, for rows of whole 16-byte chunks that divide the workgroup (64 to 1024 channels of 16 bits, 64 to 512 of
+// 32): the workgroup covers kThreads chunks = kThreads / chunks-per-row consecutive positions of one outer row at a time,
+// 4 KB of contiguous memory, and walks its slab of outer rows at the same positions. A thread keeps its place in the row
+// and its position, so its cosines and sines stay in registers and no index arithmetic is left in the loop.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void* __restrict__ x, int n_outer, int seq_len,
+                                                                    int chunks_log2, const float* __restrict__ inv_freq,
+                                                                    const float* __restrict__ positions, int64_t offset,
+                                                                    int inverse, int rows_per_wg, void* __restrict__ out) {
+  constexpr int kPairs = DT == MSPR_F32 ? 2 : 4;  // of a 16-byte chunk
+  constexpr int kMaxPos = kThreads * kPairs * 2 / kRopeDim;
+  __shared__ float cs[kMaxPos * kRopeFreqs], sn[kMaxPos * kRopeFreqs];
+  const int tid = threadIdx.x;
+  const int n_pos = kThreads >> chunks_log2;
+  const int l0 = blockIdx.x * n_pos;
+  for (int i = tid; i < n_pos * kRopeFreqs; i += kThreads) {
+    const int l = l0 + i / kRopeFreqs;
+    const float pos = positions ? positions[l < seq_len ? l : seq_len - 1] : (float)(offset + l);
+    const float theta = pos * inv_freq[i % kRopeFreqs];
+    // float32 cosine and sine of the float32 angle, correctly rounded
+    const float c = (float)cos((double)theta);
+    float s = (float)sin((double)theta);
+    if (inverse) s = -s;
+    cs[i] = round_to<DT>(c);
+    sn[i] = round_to<DT>(s);
+  }
+  __syncthreads();
+  const int chunk = tid & ((1 << chunks_log2) - 1), lp = tid >> chunks_log2;
+  if (l0 + lp >= seq_len) return;
+  const int tail_chunk = (1 << chunks_log2) - kRopeDim / (2 * kPairs);
+  const bool tail = chunk >= tail_chunk;
+  float c[kPairs], s[kPairs];
+#pragma unroll
+  for (int p = 0; p < kPairs; p++) {
+    const int f = lp * kRopeFreqs + (tail ? (chunk - tail_chunk) * kPairs + p : 0);
+    c[p] = cs[f];
+    s[p] = sn[f];
+  }
+  const int64_t row_step = (int64_t)seq_len << chunks_log2;  // chunks between outer rows at one position
+  int o = blockIdx.y * rows_per_wg;
+  int n = n_outer - o;
+  if (n > rows_per_wg) n = rows_per_wg;
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(x) + o * row_step + ((int64_t)(l0 + lp) << chunks_log2) + chunk;
+  u32x4_t* dst = reinterpret_cast<u32x4_t*>(out) + (src - reinterpret_cast<const u32x4_t*>(x));
+  auto pair = [&](float x0, float x1, int p, float* y0, float* y1) {
+    const float m0 = round_to<DT>(x0 * c[p]), m1 = round_to<DT>(x1 * s[p]);
+    const float m2 = round_to<DT>(x0 * s[p]), m3 = round_to<DT>(x1 * c[p]);
+    *y0 = round_to<DT>(m0 - m1);
+    *y1 = round_to<DT>(m2 + m3);
+  };
+  auto rotate = [&](u32x4_t v) -> u32x4_t {
+#pragma unroll
+    for (int p = 0; p < kPairs; p++) {
+      float y0, y1;
+      if constexpr (DT == MSPR_F32) {
+        pair(__uint_as_float(v[2 * p]), __uint_as_float(v[2 * p + 1]), p, &y0, &y1);
+        v[2 * p] = __float_as_uint(y0);
+        v[2 * p + 1] = __float_as_uint(y1);
+      } else if constexpr (DT == MSPR_F16) {
+        pair(f16_bits_to_f32((uint16_t)(v[p] & 0xFFFFu)), f16_bits_to_f32((uint16_t)(v[p] >> 16)), p, &y0, &y1);
+        v[p] = (uint32_t)f32_to_f16_bits(y0) | ((uint32_t)f32_to_f16_bits(y1) << 16);
+      } else {
+        pair(bf16_bits_to_f32((uint16_t)(v[p] & 0xFFFFu)), bf16_bits_to_f32((uint16_t)(v[p] >> 16)), p, &y0, &y1);
+        v[p] = (uint32_t)f32_to_bf16_bits(y0) | ((uint32_t)f32_to_bf16_bits(y1) << 16);
+      }
+    }
+    return v;
+  };
+  // (16-bit rows past the caches: 504 MB in and out in 88 us against 91; float32 rows measured slower that way)
+  auto put = [](u32x4_t v, u32x4_t* p) {
+    if constexpr (DT == MSPR_F32) *p = v;
+    else __builtin_nontemporal_store(v, p);
+  };
+  constexpr int kAtOnce = 4;  // rows in flight per thread
+  for (; n >= kAtOnce; n -= kAtOnce) {
+    u32x4_t v[kAtOnce];
+#pragma unroll
+    for (int j = 0; j < kAtOnce; j++) v[j] = src[j * row_step];
+#pragma unroll
+    for (int j = 0; j < kAtOnce; j++) {
+      if (tail) v[j] = rotate(v[j]);
+      put(v[j], dst + j * row_step);
+    }
+    src += kAtOnce * row_step;
+    dst += kAtOnce * row_step;
+  }
+  for (; n > 0; n--) {
+    u32x4_t v = *src;
+    if (tail) v = rotate(v);
+    put(v, dst);
+    src += row_step;
+    dst += row_step;
+  }
+}
+
 }  // namespace
 
 extern "C" int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer, int64_t seq_len, int width,
@@ -127,6 +221,31 @@ extern "C" int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer
                "fused_partial_rope: positions must stay exact in float32");
   MSPR_REQUIRE(mspr_aligned(x, 16) && mspr_aligned(out, 16), "fused_partial_rope: rows must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
+  // The wide form where its blocks of positions are filled, in many small workgroups of four outer rows or more: 1008 MB of
+  // float32 rows took 175, 169, 165, 160 us with 2048, 8192, 16384, 32768 workgroups (171 in the form below), 504 MB of
+  // float16 rows 88 us (108), 126 MB of 128-wide float16 rows 24 us (30).
+  const int chunk_elems = dtype == MSPR_F32 ? 4 : 8;
+  const int chunks = width / chunk_elems;
+  if (width % chunk_elems == 0 && (chunks & (chunks - 1)) == 0 && chunks <= kThreads && seq_len >= kThreads / chunks) {
+    const int log2 = __builtin_ctz(chunks);
+    const int64_t pos_blocks = (seq_len + (kThreads >> log2) - 1) / (kThreads >> log2);
+    int64_t slabs = (32768 + pos_blocks - 1) / pos_blocks;
+    int64_t rows = (n_outer + slabs - 1) / slabs;
+    if (rows < 4) rows = n_outer < 4 ? n_outer : 4;
+    slabs = (n_outer + rows - 1) / rows;
+    if (slabs <= 65535) {
+      dim3 grid((unsigned)pos_blocks, (unsigned)slabs), block(kThreads);
+#define MSPR_ROPE_WIDE(DT)                                                                                          \
+  partial_rope_wide_kernel<DT><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, offset, \
+                                                       inverse, (int)rows, out)
+      if (dtype == MSPR_F32) MSPR_ROPE_WIDE(MSPR_F32);
+      else if (dtype == MSPR_F16) MSPR_ROPE_WIDE(MSPR_F16);
+      else MSPR_ROPE_WIDE(MSPR_BF16);
+#undef MSPR_ROPE_WIDE
+      MSPR_CHECK_LAUNCH("fused_partial_rope");
+      return MSPR_OK;
+    }
+  }
   // slabs: enough workgroups to cover the chip, at least one quad per thread and pass
   const int quads = width / 4;
   int64_t rows_per_wg = (kThreads * 4 + quads - 1) / quads;  // about four passes of the thread block
