@@ -1,0 +1,31 @@
+"""Decode attention of few sequences, where a key range is whole tiles of the window and then of the ids."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ds4
+from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+pytestmark = pytest.mark.gpu
+
+
+# (batch, window, ids): one id; a tile each; window tile alone in a range; ragged window and ids; the last range ragged;
+# a range that starts in the window and ends in the ids; two tiles a range; no window
+@pytest.mark.parametrize("batch,window,ids", [(1, 1, 1), (1, 32, 32), (1, 33, 640), (2, 97, 513), (1, 128, 2047),
+                                              (5, 100, 1985), (1, 128, 2048), (3, 0, 1200), (8, 31, 2000)])
+def test_decode_ranges_of_whole_tiles(batch, window, ids):
+    rng = np.random.default_rng(window + ids)
+    n = 9000
+    gen = torch.Generator(device="cuda").manual_seed(ids)
+    kv = torch.randn((batch, n, 512), device="cuda", generator=gen).to(torch.bfloat16)
+    q = torch.randn((batch, 64, 512), device="cuda", generator=gen).to(torch.bfloat16)
+    sel = np.stack([rng.choice((n - window) // 4, ids, replace=False) for _ in range(batch)]).astype(np.int32)
+    got = iak.sparse_mla_decode(q, kv, torch.from_numpy(sel).cuda(), scale=512 ** -0.5, window_start=n - window,
+                                window_rows=window, row_mul=4, row_add=3).float().cpu().numpy()
+    rows = np.concatenate([np.tile(np.arange(n - window, n), (batch, 1)), 4 * sel + 3], axis=1)
+    gathered = np.stack([kv[b].float().cpu().numpy()[rows[b]] for b in range(batch)])
+    local = np.tile(np.arange(rows.shape[1]), (batch, 1))
+    want = ds4.sparse_mla_decode(q.float().cpu().numpy(), gathered, local, scale=512 ** -0.5, sinks=None)
+    # bfloat16 output, and probabilities of 8 significant bits: errors of single keys average out over many
+    bound = 1e-3 + 2e-2 * (window + ids) ** -0.5 + 2.0 ** -7 * np.abs(want)
+    assert (np.abs(got - want) <= bound).all(), (np.abs(got - want) - bound).max()
