@@ -520,134 +520,119 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   }
 }
 
-// Float16 tail rows of the quantised-prefix form: key 32 q8_tiles + j for j in [0, tail_rows), the
-// last (past_len % 32) prefix rows dequantised, then the chunk's own rows converted.
-template <int SDT, int ODT>
-__global__ __launch_bounds__(256) void prefill_q8_tail_kernel(PrefillArgs a, const void* self_k, const void* self_v,
-                                                              int self_dtype, uint16_t* tail_k, uint16_t* tail_v,
-                                                              int tail_rows, int first_row) {
-  const int d = threadIdx.x;
-  const int j = first_row + blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int b = blockIdx.z;
-  const int64_t bh = (int64_t)b * a.n_kv_heads + kvh;
-  const int64_t key = (int64_t)a.q8_tiles * kTile + j;
-  float kx, vx;
-  if (key < a.past_len) {
-    const int64_t row = bh * a.past_rows + key;
-    const float ks = load_as_f32<SDT>(a.pk_s, row * 4 + d / 64), kb = load_as_f32<SDT>(a.pk_b, row * 4 + d / 64);
-    const float vs = load_as_f32<SDT>(a.pv_s, row * 4 + d / 64), vb = load_as_f32<SDT>(a.pv_b, row * 4 + d / 64);
-    kx = (float)reinterpret_cast<const uint8_t*>(a.pk_wq)[row * kD + d] * ks + kb;
-    vx = (float)reinterpret_cast<const uint8_t*>(a.pv_wq)[row * kD + d] * vs + vb;
-  } else {
-    const int64_t off = (bh * a.q_len + (key - a.past_len)) * kD + d;
-    if (self_dtype == MSPR_F32) {
-      kx = load_as_f32<MSPR_F32>(self_k, off);
-      vx = load_as_f32<MSPR_F32>(self_v, off);
-    } else if (self_dtype == MSPR_F16) {
-      kx = load_as_f32<MSPR_F16>(self_k, off);
-      vx = load_as_f32<MSPR_F16>(self_v, off);
-    } else {
-      kx = load_as_f32<MSPR_BF16>(self_k, off);
-      vx = load_as_f32<MSPR_BF16>(self_v, off);
-    }
-  }
-  // 16-bit staging: values beyond the range of the staging type saturate instead of becoming infinite (an
-  // infinite key or value turns the whole output row into NaN)
-  if constexpr (ODT == MSPR_F16) {
-    kx = __builtin_amdgcn_fmed3f(kx, -65504.0f, 65504.0f);
-    vx = __builtin_amdgcn_fmed3f(vx, -65504.0f, 65504.0f);
-    tail_k[(bh * tail_rows + j) * kD + d] = f32_to_f16_bits(kx);
-    tail_v[(bh * tail_rows + j) * kD + d] = f32_to_f16_bits(vx);
-  } else {
-    constexpr float kBf16Max = 0x1.fep127f;
-    kx = __builtin_amdgcn_fmed3f(kx, -kBf16Max, kBf16Max);
-    vx = __builtin_amdgcn_fmed3f(vx, -kBf16Max, kBf16Max);
-    tail_k[(bh * tail_rows + j) * kD + d] = f32_to_bf16_bits(kx);
-    tail_v[(bh * tail_rows + j) * kD + d] = f32_to_bf16_bits(vx);
-  }
-}
-
-// Prefix rows [0, n_rows) of the quantised cache as float16 rows of the dense K/V buffers (the form taken for
-// long chunks: the attention kernel then reads every tile as a dense one). Same arithmetic as the in-kernel
-// unpacking (float16 code * scale + bias), so both forms attend the same values. A thread converts 16 codes
-// of K and of V; 16 threads a row, 16 rows a workgroup.
-// 16 unsigned 8-bit codes -> 16 bfloat16 values: code * scale + bias in float32 (one fused multiply-add, scale and
-// bias at their float32 values), rounded once
-__device__ __forceinline__ void dequant16_bf16(u32x4_t c, float sc, float bi, u32x4_t& p0, u32x4_t& p1) {
-#pragma unroll
-  for (int w = 0; w < 4; w++) {
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = __builtin_fmaf((float)((c[w] >> (8 * j)) & 0xFFu), sc, bi);
-    const uint32_t lo = pack2<MSPR_BF16>(v[0], v[1]), hi = pack2<MSPR_BF16>(v[2], v[3]);
-    if (w < 2) {
-      p0[2 * w] = lo;
-      p0[2 * w + 1] = hi;
-    } else {
-      p1[2 * (w - 2)] = lo;
-      p1[2 * (w - 2) + 1] = hi;
-    }
-  }
-}
-template <int SDT>
-__device__ __forceinline__ float sb_to_f32(uint32_t bits) {
-  if constexpr (SDT == MSPR_F32) return __builtin_bit_cast(float, bits);
-  else if constexpr (SDT == MSPR_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
-  else return __builtin_bit_cast(float, bits << 16);
-}
-
-template <int SDT, int ODT>
-__global__ __launch_bounds__(256) void prefill_q8_dequant_kernel(PrefillArgs a, uint16_t* out_k, uint16_t* out_v,
-                                                                 int64_t n_rows, int64_t out_rows) {
-  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int pp = threadIdx.x & 15;
-  if (row >= n_rows) return;
-  const int64_t bh = (int64_t)blockIdx.z * a.n_kv_heads + blockIdx.y;
-  const int64_t src = bh * a.past_rows + row;
-  const u32x4_t rk = reinterpret_cast<const u32x4_t*>(a.pk_wq)[src * 16 + pp];
-  const u32x4_t rv = reinterpret_cast<const u32x4_t*>(a.pv_wq)[src * 16 + pp];
-  uint32_t rs[4];
-  const void* arrs[4] = {a.pk_s, a.pk_b, a.pv_s, a.pv_b};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if constexpr (SDT == MSPR_F32) rs[i] = reinterpret_cast<const uint32_t*>(arrs[i])[src * 4 + (pp >> 2)];
-    else rs[i] = reinterpret_cast<const uint16_t*>(arrs[i])[src * 4 + (pp >> 2)];
-  }
-  u32x4_t p0, p1;
-  const int64_t dst = (bh * out_rows + row) * kD + 16 * pp;
-  if constexpr (ODT == MSPR_F16) dequant16(rk, sb_to_h2<SDT>(rs[0]), sb_to_h2<SDT>(rs[1]), p0, p1);
-  else dequant16_bf16(rk, sb_to_f32<SDT>(rs[0]), sb_to_f32<SDT>(rs[1]), p0, p1);
-  *reinterpret_cast<u32x4_t*>(out_k + dst) = p0;
-  *reinterpret_cast<u32x4_t*>(out_k + dst + 8) = p1;
-  if constexpr (ODT == MSPR_F16) dequant16(rv, sb_to_h2<SDT>(rs[2]), sb_to_h2<SDT>(rs[3]), p0, p1);
-  else dequant16_bf16(rv, sb_to_f32<SDT>(rs[2]), sb_to_f32<SDT>(rs[3]), p0, p1);
-  *reinterpret_cast<u32x4_t*>(out_v + dst) = p0;
-  *reinterpret_cast<u32x4_t*>(out_v + dst + 8) = p1;
-}
-
-// Merge of the key-range partials of one query row: 64 lanes x 4 columns, four rows per workgroup.
+// Dense rows of the quantised-prefix form: row j is key 32 q8_tiles + j, for the prefix rows that the attention kernel
+// does not unpack itself (all of them, or the last past_len % 32) and then the chunk's own rows. A thread makes 16
+// values of K and of V, 16 threads a row, 16 rows a workgroup, so one launch moves both kinds in 16-byte pieces: it is
+// bound by its bytes (2 * 36000 rows 23 us). code * scale + bias is one float32 multiply-add, rounded once.
+// Values beyond the range of the staging type saturate instead of becoming infinite (an infinite key or value
+// turns the whole output row into NaN).
 template <int ODT>
+__device__ __forceinline__ void store_row16(float (&v)[16], uint16_t* dst) {
+  constexpr float kMax = ODT == MSPR_F16 ? 65504.0f : 0x1.fep127f;
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j] = __builtin_amdgcn_fmed3f(v[j], -kMax, kMax);
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+    reinterpret_cast<u32x4_t*>(dst)[h] = u32x4_t{pack2<ODT>(v[8 * h], v[8 * h + 1]), pack2<ODT>(v[8 * h + 2], v[8 * h + 3]),
+                                                 pack2<ODT>(v[8 * h + 4], v[8 * h + 5]), pack2<ODT>(v[8 * h + 6], v[8 * h + 7])};
+}
+// 16 elements of the chunk's own rows (of which only the element's own alignment is known)
+template <int DT>
+__device__ __forceinline__ void load_row16(const void* base, int64_t off, float (&v)[16]) {
+  if constexpr (DT == MSPR_F32) {
+    typedef f32x4_t any_t __attribute__((aligned(4)));
+    const any_t* p = reinterpret_cast<const any_t*>(reinterpret_cast<const float*>(base) + off);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f32x4_t x = p[i];
+      v[4 * i] = x.x;
+      v[4 * i + 1] = x.y;
+      v[4 * i + 2] = x.z;
+      v[4 * i + 3] = x.w;
+    }
+  } else {
+    typedef u32x4_t any_t __attribute__((aligned(2)));
+    const any_t* p = reinterpret_cast<const any_t*>(reinterpret_cast<const uint16_t*>(base) + off);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const u32x4_t x = p[i];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint16_t lo = (uint16_t)(x[j] & 0xFFFFu), hi = (uint16_t)(x[j] >> 16);
+        v[8 * i + 2 * j] = DT == MSPR_F16 ? f16_bits_to_f32(lo) : bf16_bits_to_f32(lo);
+        v[8 * i + 2 * j + 1] = DT == MSPR_F16 ? f16_bits_to_f32(hi) : bf16_bits_to_f32(hi);
+      }
+    }
+  }
+}
+
+template <int SDT, int ODT>
+__global__ __launch_bounds__(256) void prefill_q8_rows_kernel(PrefillArgs a, const void* self_k, const void* self_v,
+                                                              int self_dtype, uint16_t* out_k, uint16_t* out_v) {
+  const int64_t j = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int pp = threadIdx.x & 15;
+  if (j >= a.kv_rows) return;
+  const int64_t bh = (int64_t)blockIdx.z * a.n_kv_heads + blockIdx.y;
+  const int64_t key = (int64_t)a.q8_tiles * kTile + j;
+  float kx[16], vx[16];
+  if (key < a.past_len) {
+    const int64_t src = bh * a.past_rows + key;
+    const u32x4_t rk = reinterpret_cast<const u32x4_t*>(a.pk_wq)[src * 16 + pp];
+    const u32x4_t rv = reinterpret_cast<const u32x4_t*>(a.pv_wq)[src * 16 + pp];
+    const float ks = load_as_f32<SDT>(a.pk_s, src * 4 + (pp >> 2)), kb = load_as_f32<SDT>(a.pk_b, src * 4 + (pp >> 2));
+    const float vs = load_as_f32<SDT>(a.pv_s, src * 4 + (pp >> 2)), vb = load_as_f32<SDT>(a.pv_b, src * 4 + (pp >> 2));
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      kx[i] = __builtin_fmaf((float)((rk[i >> 2] >> (8 * (i & 3))) & 0xFFu), ks, kb);
+      vx[i] = __builtin_fmaf((float)((rv[i >> 2] >> (8 * (i & 3))) & 0xFFu), vs, vb);
+    }
+  } else {
+    const int64_t off = (bh * a.q_len + (key - a.past_len)) * kD + 16 * pp;
+    if (self_dtype == MSPR_F32) {
+      load_row16<MSPR_F32>(self_k, off, kx);
+      load_row16<MSPR_F32>(self_v, off, vx);
+    } else if (self_dtype == MSPR_F16) {
+      load_row16<MSPR_F16>(self_k, off, kx);
+      load_row16<MSPR_F16>(self_v, off, vx);
+    } else {
+      load_row16<MSPR_BF16>(self_k, off, kx);
+      load_row16<MSPR_BF16>(self_v, off, vx);
+    }
+  }
+  const int64_t dst = (bh * a.kv_rows + j) * kD + 16 * pp;
+  store_row16<ODT>(kx, out_k + dst);
+  store_row16<ODT>(vx, out_v + dst);
+}
+
+// Merge of the key-range partials of one query row: 64 lanes x 4 columns. SHARE waves take every SHARE-th range of the
+// row, eight at once, and meet in LDS, so that up to 8 SHARE ranges are one trip to memory; a workgroup is 4 / SHARE
+// rows. The time is the partials' bytes (16 ranges of 3248 rows 10 us) or, for few rows, that trip (17 ranges of 528
+// rows 4.2 us, with one wave a row 7.1); with few ranges a wave per row keeps more loads in flight (4 ranges of 14400
+// rows: four waves a row took 13 us more).
+template <int ODT, int SHARE>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  __shared__ float xm[4], xl[4];
+  __shared__ f32x4_t xo[4][64];
   const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
   const int64_t n_rows = (int64_t)a.batch * a.n_q_heads * a.q_len;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= n_rows) return;
+  const int64_t row = (int64_t)blockIdx.x * (4 / SHARE) + wave / SHARE;
+  const bool live = row < n_rows;
   float m_run = -__builtin_inff(), l = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
   constexpr int kChunk = 8;
-  for (int s0 = 0; s0 < a.n_splits; s0 += kChunk) {
+  for (int s0 = live ? wave % SHARE : a.n_splits; s0 < a.n_splits; s0 += SHARE * kChunk) {
     float mv[kChunk], lv[kChunk];
     f32x4_t ov[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; j++) {
-      const int sj = s0 + j < a.n_splits ? s0 + j : 0;
+      const int sj = s0 + SHARE * j < a.n_splits ? s0 + SHARE * j : s0;
       const int64_t r = (int64_t)sj * n_rows + row;
       mv[j] = a.ws_ml[r * 2];
       lv[j] = a.ws_ml[r * 2 + 1];
       ov[j] = *reinterpret_cast<const f32x4_t*>(a.ws_o + r * kD + 4 * lane);
       // a range that saw no key of this row contributes nothing (its O is whatever the registers held)
-      if (s0 + j >= a.n_splits || !(lv[j] > 0.0f)) {
+      if (s0 + SHARE * j >= a.n_splits || !(lv[j] > 0.0f)) {
         mv[j] = -__builtin_inff();
         lv[j] = 0.0f;
         ov[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -668,6 +653,29 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     }
     m_run = m_new;
   }
+  if constexpr (SHARE > 1) {
+    xo[wave][lane] = o;
+    if (lane == 0) {
+      xm[wave] = m_run;
+      xl[wave] = l;
+    }
+    __syncthreads();
+    if (wave % SHARE != 0) return;
+    float m_all = m_run;
+#pragma unroll
+    for (int w = 1; w < SHARE; w++) m_all = fmaxf(m_all, xm[wave + w]);
+    const float m_safe = m_all == -__builtin_inff() ? 0.0f : m_all;
+    float e = __builtin_amdgcn_exp2f(m_run - m_safe);
+    l *= e;
+    o = o * e;
+#pragma unroll
+    for (int w = 1; w < SHARE; w++) {
+      e = __builtin_amdgcn_exp2f(xm[wave + w] - m_safe);
+      l += xl[wave + w] * e;
+      o += xo[wave + w][lane] * e;
+    }
+  }
+  if (!live) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + row * kD + 4 * lane) = o * inv;
@@ -687,22 +695,26 @@ int prefill_q_blocks(int rep, int q_len) {
   return n_pairs * (rep / heads_per_group);
 }
 
-// enough workgroups for the 256 CUs but not more (one fits a CU, so a count just above 256 means a second
-// round for a few of them), at least 16 tiles (512 keys) per range
-int prefill_choose_splits(int batch, int n_kv_heads, int q_blocks, int64_t past_len, int q_len) {
+// Enough workgroups for the 256 CUs but not more (one fits a CU, so a count just above 256 means a second round for a
+// few of them), and as many ranges as the partials are worth: tiles / ranges of about 1.3 us each against 1 KB per row
+// and range, written and read again at about 5 TB/s and partly under the tiles of other workgroups. The sum is
+// smallest near ranges^2 = 6000 * tiles / rows (3000 and 1500 measured up to 10 and 20 % slower). At least two tiles
+// per range: 33 queries of 16 heads over 9000 keys 39 -> 31 us (17 ranges before, 56 now), 203 over 2000 43 -> 33 us.
+int prefill_choose_splits(int batch, int n_q_heads, int n_kv_heads, int q_blocks, int64_t past_len, int q_len) {
   const int64_t wgs = (int64_t)batch * n_kv_heads * q_blocks;
   if (wgs >= 192) return 1;
-  int64_t want = 256 / wgs;
   const int64_t tiles = (past_len + q_len + kTile - 1) / kTile;
-  if (want > tiles / 16) want = tiles / 16;
-  if (want > 32) want = 32;
+  int64_t want = (int64_t)sqrt(6000.0 * (double)tiles / ((double)batch * n_q_heads * q_len));
+  if (want > 256 / wgs) want = 256 / wgs;
+  if (want > tiles / 2) want = tiles / 2;
+  if (want > 64) want = 64;
   return want < 1 ? 1 : (int)want;
 }
 
 size_t prefill_split_bytes(int batch, int n_q_heads, int n_kv_heads, int q_len, int64_t past_len) {
   const int rep = n_q_heads / n_kv_heads;
   const int q_blocks = prefill_q_blocks(rep, q_len);
-  const int splits = prefill_choose_splits(batch, n_kv_heads, q_blocks, past_len, q_len);
+  const int splits = prefill_choose_splits(batch, n_q_heads, n_kv_heads, q_blocks, past_len, q_len);
   if (splits == 1) return 0;
   return (size_t)splits * batch * n_q_heads * q_len * (kD + 2) * sizeof(float);
 }
@@ -727,9 +739,12 @@ int prefill_launch(const PrefillArgs& a, hipStream_t st) {
   MSPR_CHECK_LAUNCH("flash_prefill");
   if (a.n_splits > 1) {
     const int64_t n_rows = (int64_t)a.batch * a.n_q_heads * a.q_len;
-    dim3 mgrid((unsigned)((n_rows + 3) / 4)), mblock(256);
-    if (IO32) prefill_merge_kernel<MSPR_F32><<<mgrid, mblock, 0, st>>>(a);
-    else prefill_merge_kernel<KDT><<<mgrid, mblock, 0, st>>>(a);
+    const int share = a.n_splits <= 8 ? 1 : a.n_splits <= 16 ? 2 : 4;
+    dim3 mgrid((unsigned)((n_rows * share + 3) / 4)), mblock(256);
+    constexpr int ODT = IO32 ? (int)MSPR_F32 : KDT;
+    if (share == 1) prefill_merge_kernel<ODT, 1><<<mgrid, mblock, 0, st>>>(a);
+    else if (share == 2) prefill_merge_kernel<ODT, 2><<<mgrid, mblock, 0, st>>>(a);
+    else prefill_merge_kernel<ODT, 4><<<mgrid, mblock, 0, st>>>(a);
     MSPR_CHECK_LAUNCH("flash_prefill (merge)");
   }
   return MSPR_OK;
@@ -774,7 +789,7 @@ extern "C" int mspr_flash_prefill(const void* q, const void* k, const void* v, i
   a.scale_log2 = (float)((double)scale * 1.4426950408889634);
   a.rep_shift = rep == 1 ? 0 : rep == 2 ? 1 : rep == 4 ? 2 : 3;
   a.q_blocks = prefill_q_blocks(rep, q_len);
-  a.n_splits = prefill_choose_splits(batch, n_kv_heads, a.q_blocks, past_len, q_len);
+  a.n_splits = prefill_choose_splits(batch, n_q_heads, n_kv_heads, a.q_blocks, past_len, q_len);
   MSPR_REQUIRE((int64_t)a.q_blocks * n_kv_heads * batch * a.n_splits < ((int64_t)1 << 31), "flash_prefill: grid too large");
   if (a.n_splits > 1) {
     const size_t need = prefill_split_bytes(batch, n_q_heads, n_kv_heads, q_len, past_len);
@@ -788,11 +803,12 @@ extern "C" int mspr_flash_prefill(const void* q, const void* k, const void* v, i
   return prefill_launch<MSPR_F16, false, MSPR_F32>(a, st);
 }
 
-// Prefix tiles unpacked inside the attention kernel. Unpacking costs a fifth of a tile's time for every
-// workgroup that passes the tile; converting the prefix once costs about 1.4 ns per row. From a thousand
-// queries per chunk on, the prefix is therefore converted to float16 rows first (a scratch of 1 KB per key and
-// KV head) and the attention kernel runs on dense tiles only.
-static int prefill_q8_tiles(int q_len, int64_t past_len) { return q_len >= 1024 ? 0 : (int)(past_len / kTile); }
+// Prefix tiles unpacked inside the attention kernel. Unpacking costs every workgroup that passes a tile 0.7 us next to
+// the 1.3 us of its attention; converting the prefix once (1 KB per key and KV head of scratch) costs a launch and
+// about 0.6 ns per row. From five 32-query blocks on, the prefix is therefore converted first and the attention
+// kernel runs on dense tiles only (at 128 queries both forms are within 5 % of each other from 2000 to 32000 keys;
+// 517 over 9000: 124 -> 114 us).
+static int prefill_q8_tiles(int q_len, int64_t past_len) { return q_len > 128 ? 0 : (int)(past_len / kTile); }
 
 extern "C" size_t mspr_sdpa_fa_prefill_q8_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int q_len,
                                                           int64_t past_len) {
@@ -854,7 +870,7 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   a.q_blocks = prefill_q_blocks(rep, q_len);
   a.q8_tiles = q8_tiles;
   a.past_rows = past_rows;
-  a.n_splits = prefill_choose_splits(batch, n_kv_heads, a.q_blocks, past_len, q_len);
+  a.n_splits = prefill_choose_splits(batch, n_q_heads, n_kv_heads, a.q_blocks, past_len, q_len);
   if (a.n_splits > 1) {
     const size_t tail = ((size_t)batch * n_kv_heads * tail_rows * kRowBytes * 2 + 255) / 256 * 256;
     a.ws_o = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(workspace) + tail);
@@ -867,38 +883,23 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   a.pv_s = pv_scales;
   a.pv_b = pv_biases;
   hipStream_t st = (hipStream_t)stream;
-  // rows of the dense buffers: prefix rows not left to the attention kernel, then the chunk's own rows
-  const int64_t dq_rows = q8_tiles == 0 ? past_len : 0;  // converted 16 codes at a time
-  const int first_row = (int)dq_rows;                   // the rest element by element (at most 31 prefix rows + chunk)
-#ifndef MSPR_Q8_LONG_BF16
-#define MSPR_Q8_LONG_BF16 1
-#endif
-  // Long chunks (prefix converted beforehand) stage K/V and the queries as bfloat16 and run the bfloat16 matrix
+  // Long chunks stage K/V and the queries as bfloat16 and run the bfloat16 matrix
   // instructions: the device holds a higher clock under them than under the float16 ones, and the 8-bit codes
-  // leave the rounding of the staging type (2^-9 of a value) below their own step. Short chunks unpack the
-  // prefix inside the attention kernel with packed float16 arithmetic and stay float16 throughout.
-  const bool bf16_staging = MSPR_Q8_LONG_BF16 && q_len >= 1024;  // (then q8_tiles == 0)
-#define MSPR_LAUNCH_BY_SB(KERNEL, GRID, ...)                                                          \
-  do {                                                                                                \
-    if (bf16_staging) {                                                                               \
-      if (sb_dtype == MSPR_F32) KERNEL<MSPR_F32, MSPR_BF16><<<GRID, 256, 0, st>>>(__VA_ARGS__);        \
-      else if (sb_dtype == MSPR_F16) KERNEL<MSPR_F16, MSPR_BF16><<<GRID, 256, 0, st>>>(__VA_ARGS__);   \
-      else KERNEL<MSPR_BF16, MSPR_BF16><<<GRID, 256, 0, st>>>(__VA_ARGS__);                            \
-    } else {                                                                                          \
-      if (sb_dtype == MSPR_F32) KERNEL<MSPR_F32, MSPR_F16><<<GRID, 256, 0, st>>>(__VA_ARGS__);         \
-      else if (sb_dtype == MSPR_F16) KERNEL<MSPR_F16, MSPR_F16><<<GRID, 256, 0, st>>>(__VA_ARGS__);    \
-      else KERNEL<MSPR_BF16, MSPR_F16><<<GRID, 256, 0, st>>>(__VA_ARGS__);                             \
-    }                                                                                                 \
+  // leave the rounding of the staging type (2^-9 of a value) below their own step. Shorter chunks stay float16.
+  const bool bf16_staging = q_len >= 1024;
+  dim3 rgrid((unsigned)((tail_rows + 15) / 16), (unsigned)n_kv_heads, (unsigned)batch);
+#define MSPR_ROWS_LAUNCH(SDT)                                                                                        \
+  do {                                                                                                               \
+    if (bf16_staging)                                                                                                \
+      prefill_q8_rows_kernel<SDT, MSPR_BF16><<<rgrid, 256, 0, st>>>(a, self_k, self_v, self_dtype, tail_k, tail_v);   \
+    else                                                                                                             \
+      prefill_q8_rows_kernel<SDT, MSPR_F16><<<rgrid, 256, 0, st>>>(a, self_k, self_v, self_dtype, tail_k, tail_v);    \
   } while (0)
-  if (dq_rows > 0) {
-    dim3 dgrid((unsigned)((dq_rows + 15) / 16), (unsigned)n_kv_heads, (unsigned)batch);
-    MSPR_LAUNCH_BY_SB(prefill_q8_dequant_kernel, dgrid, a, tail_k, tail_v, dq_rows, tail_rows);
-    MSPR_CHECK_LAUNCH("sdpa_fa_prefill_q8 (prefix rows)");
-  }
-  dim3 tgrid((unsigned)(tail_rows - first_row), (unsigned)n_kv_heads, (unsigned)batch);
-  MSPR_LAUNCH_BY_SB(prefill_q8_tail_kernel, tgrid, a, self_k, self_v, self_dtype, tail_k, tail_v, tail_rows, first_row);
-#undef MSPR_LAUNCH_BY_SB
-  MSPR_CHECK_LAUNCH("sdpa_fa_prefill_q8 (tail rows)");
+  if (sb_dtype == MSPR_F32) MSPR_ROWS_LAUNCH(MSPR_F32);
+  else if (sb_dtype == MSPR_F16) MSPR_ROWS_LAUNCH(MSPR_F16);
+  else MSPR_ROWS_LAUNCH(MSPR_BF16);
+#undef MSPR_ROWS_LAUNCH
+  MSPR_CHECK_LAUNCH("sdpa_fa_prefill_q8 (dense rows)");
   // (prefix converted beforehand: the dense kernel, with float32 queries and output)
   if (q8_tiles == 0) {
     if (bf16_staging) return prefill_launch<MSPR_BF16, false, MSPR_F32, true>(a, st);
