@@ -682,83 +682,198 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
   }
 }
 
-// Short rows, one row per workgroup of 256 threads. A prefill chunk selects for thousands of tokens at once over a
-// pool of a few hundred to two thousand rows: with 1024 threads a row a CU holds two of them, with 256 it holds
-// eight, and each spends less on barriers. Thread t owns the C consecutive rows [C t, C t + C) (read coalesced,
-// handed over through LDS); four 8-bit digit passes, each with a histogram of its own (zeroed once, so a pass costs
-// one barrier), votes of a wave for one bin merged into one atomic; every wave derives the select state from the
-// same totals. Rows past n_rows get key 0 as in the blocked kernel. Emission as there.
-constexpr int kSmallThreads = 256;
-template <int C>
-__global__ __launch_bounds__(kSmallThreads) void topk_small_kernel(const float* __restrict__ scores_all,
-                                                                   int64_t score_stride, int n_rows, int topk,
-                                                                   int32_t* __restrict__ sel_all) {
-  __shared__ __attribute__((aligned(16))) uint32_t stage[C * kSmallThreads];
-  __shared__ uint32_t hist[4][256];
-  __shared__ uint32_t wave_tot[kSmallThreads / 64];
+// Rows of up to C * THREADS scores, one a workgroup: key j * THREADS + t in register j of thread t. The selection is by
+// value range instead of by digit: 1024 bins over the span from a lower bound of the k-th key to the highest key, then the
+// bin with the k-th key becomes the span, until it holds 64 keys or fewer, which every wave ranks for itself. The scores
+// of a row share their leading bits, so a digit's votes meet on a few counters and take a pass each for four digits;
+// the bins of the span spread the votes, and one round is nearly always enough. The lower bound is the lowest of the
+// maxima of k or more disjoint groups of keys, or the lowest finite key; -inf (a row that a token may not see yet) is
+// counted on the side and does not stretch the span. Keys past n_rows are 0: they can only tie with the lowest
+// possible key and lose every tie to a real row. Emission order comes from ballots: the hits of (chunk, wave) pairs
+// are scanned and a wave stores its own side by side.
+// What is left is instructions per key and barriers. Four 8-bit digit passes with merged votes took, k = 512: 1 row of
+// 961 scores 7.0 us (now 4.5), 189 of 3974 20 (6.9), 517 of 2053 22 (8.3), 3844 of 961 24 (13), 3844 of 4000 78 (37).
+constexpr uint32_t kRowBins = 1024;
+constexpr uint32_t kNegInfKey = 0x007FFFFFu;
+
+template <int OFF>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, OFF, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t umin(uint32_t a, uint32_t b) { return a < b ? a : b; }
+// maximum over the wave, in every lane
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = umax(v, dpp_u32<0x128>(v));  // row_ror:8
+  v = umax(v, dpp_u32<0x124>(v));  // row_ror:4
+  v = umax(v, dpp_u32<0x122>(v));  // row_ror:2
+  v = umax(v, dpp_u32<0x121>(v));  // row_ror:1
+  uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+  r = umax(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 16));
+  r = umax(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 32));
+  return umax(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 48));
+}
+
+template <int C, int THREADS>
+__global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restrict__ scores_all, int64_t score_stride,
+                                                           int n_rows, int topk, int32_t* __restrict__ sel_all) {
+  constexpr int kW = THREADS / 64;
+  static_assert(C <= 32 && kRowBins % THREADS == 0, "a lane per chunk, whole zeroing rounds");
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kRowBins];
+  __shared__ __attribute__((aligned(16))) uint32_t cnt[C * kW];  // hits per (chunk, wave): above low, ties high
+  __shared__ uint32_t red_max[kW], red_not_min[kW], red_not_bound[kW], red_count[kW];
+  __shared__ uint32_t list[64];
+  __shared__ uint32_t list_n;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float* scores = scores_all + (int64_t)blockIdx.x * score_stride;
   int32_t* sel = sel_all + (int64_t)blockIdx.x * topk;
 
-#pragma unroll
-  for (int i = 0; i < 4; i++) (&hist[0][0])[i * kSmallThreads + tid] = 0u;
+  uint32_t key[C];
 #pragma unroll
   for (int j = 0; j < C; j++) {
-    const int e = j * kSmallThreads + tid;
-    stage[e] = e < n_rows ? score_key(scores[e]) : 0u;
+    const int e = j * THREADS + tid;
+    key[j] = e < n_rows ? score_key(scores[e]) : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < (int)kRowBins / THREADS; i++) hist[i * THREADS + tid] = 0u;
+  if (tid == 0) list_n = 0u;
+  uint32_t top4[4] = {0u, 0u, 0u, 0u}, not_lo = 0u, n_fin = 0u, n_inf = 0u;  // not_lo: complement of the lowest finite key
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    const bool fin = key[j] > kNegInfKey;
+    top4[j & 3] = umax(key[j], top4[j & 3]);
+    not_lo = umax(fin ? ~key[j] : 0u, not_lo);
+    n_fin += (uint32_t)__popcll(__ballot(fin));
+    n_inf += (uint32_t)__popcll(__ballot(key[j] == kNegInfKey));
+  }
+  const uint32_t even = umax(top4[0], top4[2]), odd = umax(top4[1], top4[3]);
+  uint32_t hi = umax(even, odd);
+  // the lowest of the maxima of disjoint groups of keys, of which there are at least k, is not above the k-th key
+  const uint32_t group = topk <= THREADS ? hi : topk <= 2 * THREADS ? umin(even, odd) :
+                         topk <= 4 * THREADS ? umin(umin(top4[0], top4[1]), umin(top4[2], top4[3])) : 0u;
+  hi = wave_max(hi);
+  not_lo = wave_max(not_lo);
+  const uint32_t not_bound = wave_max(~group);
+  if (lane == 0) {
+    red_max[wave] = hi;
+    red_not_min[wave] = not_lo;
+    red_not_bound[wave] = not_bound;
+    red_count[wave] = n_fin | (n_inf << 16);
   }
   __syncthreads();
-  uint32_t kreg[C];
-#pragma unroll
-  for (int i = 0; i < C; i++) kreg[i] = stage[C * tid + i];
+  hi = wave_max(red_max[lane % kW]);
+  not_lo = wave_max(red_not_min[lane % kW]);
+  const uint32_t bound = ~wave_max(red_not_bound[lane % kW]);
+  const uint32_t counts = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(lane < kW ? red_count[lane] : 0u), 63);
+  n_fin = counts & 0xFFFFu;
+  n_inf = counts >> 16;
 
-  uint32_t prefix = 0u, need = (uint32_t)topk;
+  uint32_t need = (uint32_t)topk;
+  uint32_t lo = umax(~not_lo, bound), span = hi - lo, threshold = kNegInfKey;
+  bool found = false;
+  if (need > n_fin) {  // the k-th key is -inf, or one of the negative NaNs below it
+    need -= n_fin;
+    found = need <= n_inf;
+    if (!found) need -= n_inf;
+    lo = 0u;
+    span = kNegInfKey - 1u;
+  }
+  while (!found) {
+    const int shift = span >= kRowBins ? 22 - __builtin_clz(span) : 0;
 #pragma unroll
-  for (int pass = 0; pass < 4; pass++) {
-    const uint32_t shift = 24u - 8u * (uint32_t)pass;
-    const uint32_t mask_hi = pass == 0 ? 0u : 0xFFFFFFFFu << (shift + 8u);
-#pragma unroll
-    for (int i = 0; i < C; i++) {
-      const int bin = (kreg[i] & mask_hi) == prefix ? (int)((kreg[i] >> shift) & 0xFFu) : -1;
-      wave_hist_add(hist[pass], bin, lane);
+    for (int j = 0; j < C; j++) {
+      const uint32_t d = key[j] - lo;
+      if (d <= span) atomicAdd(&hist[d >> shift], 1u);
     }
     __syncthreads();
-    const Pick p = pick_bucket(hist[pass], need, lane);
-    prefix |= p.digit << shift;
-    need = p.need;
-  }
-  const uint32_t threshold = prefix;
-  const uint32_t need_ties = need;
-  const uint32_t n_above = (uint32_t)topk - need_ties;
-
-  // ---- ordered emission: per-thread masks, one packed block scan (above count low, tie count high)
-  uint32_t above_mask = 0u, tie_mask = 0u;
+    // lane l holds the sixteen bins below 1024 - 16 l, so that a prefix sum over lanes counts from the top
+    uint32_t t[16];
 #pragma unroll
-  for (int i = 0; i < C; i++) {
-    above_mask |= (kreg[i] > threshold ? 1u : 0u) << i;
-    tie_mask |= (kreg[i] == threshold ? 1u : 0u) << i;
+    for (int i = 0; i < 4; i++) {
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&hist[16 * (63 - lane) + 4 * i]);
+#pragma unroll
+      for (int c = 0; c < 4; c++) t[4 * i + c] = v[c];
+    }
+    uint32_t sum = 0u;
+#pragma unroll
+    for (int i = 0; i < 16; i++) sum += t[i];
+    const uint32_t incl = wave_prefix_sum(sum);
+    uint32_t run = incl - sum, left = 0u, held = 0u, bin = 0u;
+#pragma unroll
+    for (int i = 15; i >= 0; i--) {
+      const bool here = run < need && run + t[i] >= need;
+      bin = here ? (uint32_t)(16 * (63 - lane) + i) : bin;
+      left = here ? need - run : left;
+      held = here ? t[i] : held;
+      run += t[i];
+    }
+    const int src = (int)__builtin_ctzll(__ballot(held != 0u));
+    bin = (uint32_t)__builtin_amdgcn_readlane((int)bin, src);
+    need = (uint32_t)__builtin_amdgcn_readlane((int)left, src);
+    held = (uint32_t)__builtin_amdgcn_readlane((int)held, src);
+    lo += bin << shift;
+    const uint32_t rest = span - (bin << shift), width = (1u << shift) - 1u;
+    span = rest < width ? rest : width;
+    if (span == 0u) {
+      threshold = lo;
+      break;
+    }
+    if (held <= 64u) {
+#pragma unroll
+      for (int j = 0; j < C; j++) {
+        const bool in = key[j] - lo <= span;
+        if (in) list[atomicAdd(&list_n, 1u)] = key[j];
+      }
+      __syncthreads();
+      const uint32_t mine = list[lane];
+      uint32_t above = 0u, ties = 0u;
+      for (int i = 0; i < (int)held; i++) {
+        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
+        above += o > mine ? 1u : 0u;
+        ties += o == mine ? 1u : 0u;
+      }
+      const int at = (int)__builtin_ctzll(__ballot(lane < (int)held && above < need && above + ties >= need));
+      threshold = (uint32_t)__builtin_amdgcn_readlane((int)mine, at);
+      need -= (uint32_t)__builtin_amdgcn_readlane((int)above, at);
+      break;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (int)kRowBins / THREADS; i++) hist[i * THREADS + tid] = 0u;
+    __syncthreads();
   }
-  const uint32_t mine = (uint32_t)__popc(above_mask) | ((uint32_t)__popc(tie_mask) << 16);
-  const uint32_t incl = wave_prefix_sum(mine);
-  if (lane == 63) wave_tot[wave] = incl;
+  const uint32_t n_above = (uint32_t)topk - need;
+
+  uint32_t hits = 0u;
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    const uint32_t a = (uint32_t)__popcll(__ballot(key[j] > threshold)), t = (uint32_t)__popcll(__ballot(key[j] == threshold));
+    hits = lane == j ? a | (t << 16) : hits;
+  }
+  if (lane < C) cnt[lane * kW + wave] = hits;
   __syncthreads();
-  uint32_t base = 0u;
-  for (int w = 0; w < wave; w++) base += wave_tot[w];
-  const uint32_t excl = base + incl - mine;
-  uint32_t slot_a = excl & 0xFFFFu;
-  uint32_t rank_t = excl >> 16;
-  const int row0 = C * tid;
-  while (above_mask) {
-    const int i = __builtin_ctz(above_mask);
-    above_mask &= above_mask - 1u;
-    sel[slot_a++] = row0 + i;
+  uint32_t row_sum = 0u, before = 0u;  // of chunk `lane`: all waves, the waves in front of this one
+  if (lane < C) {
+#pragma unroll
+    for (int w = 0; w < kW; w++) {
+      const uint32_t c = cnt[lane * kW + w];
+      row_sum += c;
+      before += w < wave ? c : 0u;
+    }
   }
-  while (tie_mask && rank_t < need_ties) {
-    const int i = __builtin_ctz(tie_mask);
-    tie_mask &= tie_mask - 1u;
-    sel[n_above + rank_t++] = row0 + i;
+  before += wave_prefix_sum(row_sum) - row_sum;
+  asm volatile("" : "+s"(threshold));  // the votes below are taken again, not kept in 4 C scalar registers
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)before, j);
+    const bool above = key[j] > threshold, tie = key[j] == threshold;
+    const uint64_t ba = __ballot(above), bt = __ballot(tie);
+    const uint32_t ra = __builtin_amdgcn_mbcnt_hi((uint32_t)(ba >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ba, 0u));
+    const uint32_t rt = __builtin_amdgcn_mbcnt_hi((uint32_t)(bt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bt, 0u));
+    if (above) sel[(base & 0xFFFFu) + ra] = j * THREADS + tid;
+    else if (tie && (base >> 16) + rt < need) sel[n_above + (base >> 16) + rt] = j * THREADS + tid;
   }
 }
 
@@ -781,14 +896,18 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
                      hipStream_t st) {
   dim3 grid((unsigned)batch), block(kThreads);
   MsprProfScope prof(MSPR_K_TOPK, st);
-  if (n_rows <= 4 * kSmallThreads)
-    topk_small_kernel<4><<<grid, dim3(kSmallThreads), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel);
-  else if (n_rows <= 8 * kSmallThreads)
-    topk_small_kernel<8><<<grid, dim3(kSmallThreads), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel);
-  // (many rows of up to 4096 scores: more rows resident per CU beats more threads per row; measured at 3844 rows,
-  // k = 512: 84 against 111 us at 2500 scores, 92 against 113 at 4000, but 218 against 145 at 7961)
-  else if (batch >= 128 && n_rows <= 16 * kSmallThreads)
-    topk_small_kernel<16><<<grid, dim3(kSmallThreads), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel);
+  // Up to 4096 scores a row: 256 threads a row keep the most rows in flight; a row of more than 2048 that has a CU for
+  // itself is better off with 512 (189 rows of 3974 scores: 6.9 against 8.7 us; 517 of 2053: 9.5 against 8.3). Past that
+  // the blocked form's work per key is less (3844 rows of 7961 scores: 67 us, 84 with a longer row kernel; 16 of
+  // 32768: 10 against 22).
+#define MSPR_TOPK_ROW(C, THREADS) \
+  topk_row_kernel<C, THREADS><<<grid, dim3(THREADS), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel)
+  if (n_rows <= 1024) MSPR_TOPK_ROW(4, 256);
+  else if (n_rows <= 2048) MSPR_TOPK_ROW(8, 256);
+  else if (n_rows <= 4096 && batch <= 256) MSPR_TOPK_ROW(8, 512);
+  else if (n_rows <= 3072) MSPR_TOPK_ROW(12, 256);
+  else if (n_rows <= 4096) MSPR_TOPK_ROW(16, 256);
+#undef MSPR_TOPK_ROW
   else if (n_rows <= 8 * 1024)
     topk_blocked_kernel<8><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, pivot_sample_rank(8, topk), sel);
   else if (n_rows <= 32 * 1024)
