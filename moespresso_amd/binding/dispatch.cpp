@@ -490,21 +490,35 @@ bool cache_side(PyObject* o, const Tensor* (&t)[3]) {
   return true;
 }
 
+// both sides as views of the first n rows of every head
+PyObject* wrap_leading_rows(const Tensor* const (&t)[2][3], int64_t n) {
+  PyObject* sides[2];
+  for (int s = 0; s < 2; s++) {
+    sides[s] = wrap_tuple(t[s][0]->slice(2, 0, n), t[s][1]->slice(2, 0, n), t[s][2]->slice(2, 0, n));
+    if (!sides[s]) return nullptr;
+  }
+  PyObject* r = PyTuple_Pack(2, sides[0], sides[1]);
+  Py_DECREF(sides[0]);
+  Py_DECREF(sides[1]);
+  return r;
+}
+
 // (keys [B, H, L, D], values, key side, value side, offset): quantises the rows into the buffers of both sides behind the
-// first `offset` rows of every head -> True
+// first `offset` rows of every head -> ((key side, value side) up to the new length, the new length)
 PyObject* q8_append(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(5)
-  const Tensor *k = dense(a[0], 4), *v = dense(a[1], 4), *ks[3], *vs[3];
+  const Tensor *k = dense(a[0], 4), *v = dense(a[1], 4), *side[2][3];
   int64_t offset;
-  if (!k || !v || !cache_side(a[2], ks) || !cache_side(a[3], vs) || !whole(a[4], &offset)) return none();
+  if (!k || !v || !cache_side(a[2], side[0]) || !cache_side(a[3], side[1]) || !whole(a[4], &offset)) return none();
+  const Tensor *const(&ks)[3] = side[0], *const(&vs)[3] = side[1];
   const int code = type_code(k->scalar_type());
   const int64_t B = k->size(0), H = k->size(1), L = k->size(2), D = k->size(3), cap = ks[0]->size(2);
   if (code == kNoType || v->scalar_type() != k->scalar_type() || k->sizes() != v->sizes() || k->numel() == 0 || D % 64 != 0 ||
       D > 4096 || B * H > 65535 || offset < 0 || offset + L > cap || !same_device({k, v, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2]}))
     return none();
-  for (const Tensor** side : {ks, vs})
+  for (const auto& half : side)
     for (int i = 0; i < 3; i++) {
-      const Tensor& t = *side[i];
+      const Tensor& t = *half[i];
       const bool codes = i == 0;
       if (!t.is_contiguous() || t.size(0) != B || t.size(1) != H || t.size(2) != cap || t.size(3) != (codes ? D / 4 : D / 64) ||
           t.scalar_type() != (codes ? at::kUInt32 : k->scalar_type()))
@@ -516,7 +530,12 @@ PyObject* q8_append(PyObject* const* a, Py_ssize_t nargs) {
                                  vs[2]->data_ptr(), cap, offset, st);
   });
   if (failed(rc, "q8_append")) return nullptr;
-  Py_RETURN_TRUE;
+  PyObject* views = wrap_leading_rows(side, offset + L);
+  PyObject* length = views ? PyLong_FromLongLong(offset + L) : nullptr;
+  PyObject* r = length ? PyTuple_Pack(2, views, length) : nullptr;
+  Py_XDECREF(views);
+  Py_XDECREF(length);
+  return r;
 }
 
 // (key side, value side, n) -> both sides as views of the first n rows of every head
@@ -528,15 +547,7 @@ PyObject* leading_rows(PyObject* const* a, Py_ssize_t nargs) {
   for (const auto& side : t)
     for (const Tensor* p : side)
       if (n < 0 || n > p->size(2)) return none();
-  PyObject* sides[2];
-  for (int s = 0; s < 2; s++) {
-    sides[s] = wrap_tuple(t[s][0]->narrow(2, 0, n), t[s][1]->narrow(2, 0, n), t[s][2]->narrow(2, 0, n));
-    if (!sides[s]) return nullptr;
-  }
-  PyObject* r = PyTuple_Pack(2, sides[0], sides[1]);
-  Py_DECREF(sides[0]);
-  Py_DECREF(sides[1]);
-  return r;
+  return wrap_leading_rows(t, n);
 }
 
 // (queries f32 [B, Hq, 1, 256], six cache parts, scale, workspace) -> f32 like queries

@@ -178,19 +178,24 @@ class QuantizedKVCache:
         Rows in the cache's own layout and type are quantised straight into its buffers, keys and values in one
         launch; others take a quantised copy that is moved behind the prefix.
         """
-        if keys.ndim != 4 or keys.shape != values.shape:
-            raise ValueError("keys and values must be [B, Hkv, L, D] of one shape")
-        L = int(keys.shape[2])
-        self._grow(keys, self.offset + L)
-        if _lib.dispatch.q8_append(keys, values, self.keys, self.values, self.offset) is None:
+        appended = _lib.dispatch.q8_append(keys, values, self.keys, self.values, self.offset)
+        if appended is None:
+            if keys.ndim != 4 or keys.shape != values.shape:
+                raise ValueError("keys and values must be [B, Hkv, L, D] of one shape")
+            L = int(keys.shape[2])
+            self._grow(keys, self.offset + L)
+            appended = _lib.dispatch.q8_append(keys, values, self.keys, self.values, self.offset)
+        if appended is None:
             for src, dst in ((keys, self.keys), (values, self.values)):
                 wq, sc, bi = quantize(src)
                 lo, hi = self.offset, self.offset + L
                 dst[0][:, :, lo:hi].view(torch.int32).copy_(wq.view(torch.int32))
                 dst[1][:, :, lo:hi].copy_(sc)
                 dst[2][:, :, lo:hi].copy_(bi)
-        self.offset += L
-        return self._views()
+            self.offset += L
+            return self._views()
+        views, self.offset = appended
+        return views
 
 
 def sdpa_decode_q8(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases, scale, *, group_size: int = 64,
