@@ -687,12 +687,12 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
 // bin with the k-th key becomes the span, until it holds 64 keys or fewer, which every wave ranks for itself. The scores
 // of a row share their leading bits, so a digit's votes meet on a few counters and take a pass each for four digits;
 // the bins of the span spread the votes, and one round is nearly always enough. The lower bound is the lowest of the
-// maxima of k or more disjoint groups of keys, or the lowest finite key; -inf (a row that a token may not see yet) is
-// counted on the side and does not stretch the span. Keys past n_rows are 0: they can only tie with the lowest
-// possible key and lose every tie to a real row. Emission order comes from ballots: the hits of (chunk, wave) pairs
-// are scanned and a wave stores its own side by side.
+// maxima of k or more disjoint groups of keys, or, where a group holds nothing finite, the lowest finite key; -inf (a row
+// that a token may not see yet) is then counted on the side and does not stretch the span. Keys past n_rows are 0: they
+// can only tie with the lowest possible key and lose every tie to a real row. Emission order comes from ballots: the
+// hits of (chunk, wave) pairs are scanned and a wave stores its own side by side.
 // What is left is instructions per key and barriers. Four 8-bit digit passes with merged votes took, k = 512: 1 row of
-// 961 scores 7.0 us (now 4.5), 189 of 3974 20 (6.9), 517 of 2053 22 (8.3), 3844 of 961 24 (13), 3844 of 4000 78 (37).
+// 961 scores 7.0 us (now 4.1), 189 of 3974 20 (6.2), 517 of 2053 22 (6.7), 3844 of 961 24 (12), 3844 of 4000 78 (32).
 constexpr uint32_t kRowBins = 1024;
 constexpr uint32_t kNegInfKey = 0x007FFFFFu;
 
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
   static_assert(C <= 32 && kRowBins % THREADS == 0, "a lane per chunk, whole zeroing rounds");
   __shared__ __attribute__((aligned(16))) uint32_t hist[kRowBins];
   __shared__ __attribute__((aligned(16))) uint32_t cnt[C * kW];  // hits per (chunk, wave): above low, ties high
-  __shared__ uint32_t red_max[kW], red_not_min[kW], red_not_bound[kW], red_count[kW];
+  __shared__ uint32_t red_max[kW], red_not_low[kW], red_count[kW];
   __shared__ uint32_t list[64];
   __shared__ uint32_t list_n;
   const int tid = threadIdx.x;
@@ -739,47 +739,55 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
 #pragma unroll
   for (int i = 0; i < (int)kRowBins / THREADS; i++) hist[i * THREADS + tid] = 0u;
   if (tid == 0) list_n = 0u;
-  uint32_t top4[4] = {0u, 0u, 0u, 0u}, not_lo = 0u, n_fin = 0u, n_inf = 0u;  // not_lo: complement of the lowest finite key
+  uint32_t top4[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int j = 0; j < C; j++) {
-    const bool fin = key[j] > kNegInfKey;
-    top4[j & 3] = umax(key[j], top4[j & 3]);
-    not_lo = umax(fin ? ~key[j] : 0u, not_lo);
-    n_fin += (uint32_t)__popcll(__ballot(fin));
-    n_inf += (uint32_t)__popcll(__ballot(key[j] == kNegInfKey));
-  }
+  for (int j = 0; j < C; j++) top4[j & 3] = umax(key[j], top4[j & 3]);
   const uint32_t even = umax(top4[0], top4[2]), odd = umax(top4[1], top4[3]);
   uint32_t hi = umax(even, odd);
   // the lowest of the maxima of disjoint groups of keys, of which there are at least k, is not above the k-th key
   const uint32_t group = topk <= THREADS ? hi : topk <= 2 * THREADS ? umin(even, odd) :
                          topk <= 4 * THREADS ? umin(umin(top4[0], top4[1]), umin(top4[2], top4[3])) : 0u;
   hi = wave_max(hi);
-  not_lo = wave_max(not_lo);
   const uint32_t not_bound = wave_max(~group);
   if (lane == 0) {
     red_max[wave] = hi;
-    red_not_min[wave] = not_lo;
-    red_not_bound[wave] = not_bound;
-    red_count[wave] = n_fin | (n_inf << 16);
+    red_not_low[wave] = not_bound;
   }
   __syncthreads();
   hi = wave_max(red_max[lane % kW]);
-  not_lo = wave_max(red_not_min[lane % kW]);
-  const uint32_t bound = ~wave_max(red_not_bound[lane % kW]);
-  const uint32_t counts = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(lane < kW ? red_count[lane] : 0u), 63);
-  n_fin = counts & 0xFFFFu;
-  n_inf = counts >> 16;
+  uint32_t lo = ~wave_max(red_not_low[lane % kW]);
 
-  uint32_t need = (uint32_t)topk;
-  uint32_t lo = umax(~not_lo, bound), span = hi - lo, threshold = kNegInfKey;
+  uint32_t need = (uint32_t)topk, threshold = kNegInfKey;
   bool found = false;
-  if (need > n_fin) {  // the k-th key is -inf, or one of the negative NaNs below it
-    need -= n_fin;
-    found = need <= n_inf;
-    if (!found) need -= n_inf;
-    lo = 0u;
-    span = kNegInfKey - 1u;
+  if (lo <= kNegInfKey) {  // not bounded by finite groups: the lowest finite key, or what lies below
+    uint32_t not_low = 0u, n_fin = 0u, n_inf = 0u;
+#pragma unroll
+    for (int j = 0; j < C; j++) {
+      const bool fin = key[j] > kNegInfKey;
+      not_low = umax(fin ? ~key[j] : 0u, not_low);
+      n_fin += (uint32_t)__popcll(__ballot(fin));
+      n_inf += (uint32_t)__popcll(__ballot(key[j] == kNegInfKey));
+    }
+    not_low = wave_max(not_low);
+    __syncthreads();  // every wave has read the bounds
+    if (lane == 0) {
+      red_not_low[wave] = not_low;
+      red_count[wave] = n_fin | (n_inf << 16);
+    }
+    __syncthreads();
+    lo = ~wave_max(red_not_low[lane % kW]);
+    const uint32_t counts = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(lane < kW ? red_count[lane] : 0u), 63);
+    n_fin = counts & 0xFFFFu;
+    n_inf = counts >> 16;
+    if (need > n_fin) {  // the k-th key is -inf, or one of the negative NaNs below it
+      need -= n_fin;
+      found = need <= n_inf;
+      if (!found) need -= n_inf;
+      lo = 0u;
+      hi = kNegInfKey - 1u;
+    }
   }
+  uint32_t span = hi - lo;
   while (!found) {
     const int shift = span >= kRowBins ? 22 - __builtin_clz(span) : 0;
 #pragma unroll
@@ -870,10 +878,12 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
     const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)before, j);
     const bool above = key[j] > threshold, tie = key[j] == threshold;
     const uint64_t ba = __ballot(above), bt = __ballot(tie);
-    const uint32_t ra = __builtin_amdgcn_mbcnt_hi((uint32_t)(ba >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ba, 0u));
-    const uint32_t rt = __builtin_amdgcn_mbcnt_hi((uint32_t)(bt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bt, 0u));
-    if (above) sel[(base & 0xFFFFu) + ra] = j * THREADS + tid;
-    else if (tie && (base >> 16) + rt < need) sel[n_above + (base >> 16) + rt] = j * THREADS + tid;
+    const uint32_t ra = __builtin_amdgcn_mbcnt_hi((uint32_t)(ba >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ba, base & 0xFFFFu));
+    if (above) sel[ra] = j * THREADS + tid;
+    if (bt != 0ull) {
+      const uint32_t rt = __builtin_amdgcn_mbcnt_hi((uint32_t)(bt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bt, base >> 16));
+      if (tie && rt < need) sel[n_above + rt] = j * THREADS + tid;
+    }
   }
 }
 
@@ -897,9 +907,10 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
   dim3 grid((unsigned)batch), block(kThreads);
   MsprProfScope prof(MSPR_K_TOPK, st);
   // Up to 4096 scores a row: 256 threads a row keep the most rows in flight; a row of more than 2048 that has a CU for
-  // itself is better off with 512 (189 rows of 3974 scores: 6.9 against 8.7 us; 517 of 2053: 9.5 against 8.3). Past that
-  // the blocked form's work per key is less (3844 rows of 7961 scores: 67 us, 84 with a longer row kernel; 16 of
-  // 32768: 10 against 22).
+  // itself is better off with 512 (189 rows of 3974 scores: 6.2 against 7.4 us; 517 of 2053: 7.7 against 6.7). Up to 8192
+  // many rows take the row kernel too (3844 rows of 7961 scores, k = 512: 58 against 67 us, 517 11.4 against 15.2), few take
+  // the blocked form, whose sample bounds a large k better (1 row, k = 2048: 8.6 against 7.9; 20 rows are equal). Past
+  // that its work per key is less (16 rows of 32768: 10 against 17 us).
 #define MSPR_TOPK_ROW(C, THREADS) \
   topk_row_kernel<C, THREADS><<<grid, dim3(THREADS), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel)
   if (n_rows <= 1024) MSPR_TOPK_ROW(4, 256);
@@ -907,6 +918,7 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
   else if (n_rows <= 4096 && batch <= 256) MSPR_TOPK_ROW(8, 512);
   else if (n_rows <= 3072) MSPR_TOPK_ROW(12, 256);
   else if (n_rows <= 4096) MSPR_TOPK_ROW(16, 256);
+  else if (n_rows <= 8192 && batch > 32) MSPR_TOPK_ROW(16, 512);
 #undef MSPR_TOPK_ROW
   else if (n_rows <= 8 * 1024)
     topk_blocked_kernel<8><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, pivot_sample_rank(8, topk), sel);

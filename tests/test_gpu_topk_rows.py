@@ -1,4 +1,4 @@
-"""Top-k of rows of up to 4096 scores at the widths of the kernel, with values that move its bins: rows mostly -inf (with
+"""Top-k of rows of up to 8192 scores at the widths of the kernel, with values that move its bins: rows mostly -inf (with
 more wanted than finite scores), NaN of both signs, one huge value over close ones, a k-th key inside ties."""
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows", [5, 257])  # 257: past one row per compute unit
 @pytest.mark.parametrize("n,k", [(1, 1), (513, 512), (1024, 513), (1025, 64), (2048, 1), (2049, 2049), (3072, 512),
-                                 (3073, 1025), (4096, 2048), (4095, 4000)])
+                                 (3073, 1025), (4096, 2048), (4095, 4000), (4097, 512), (8192, 2049)])
 def test_topk_rows(rows, n, k):
     rng = np.random.default_rng(n + k + rows)
     s = rng.standard_normal((rows, n)).astype(np.float32)
