@@ -115,7 +115,10 @@ __global__ __launch_bounds__(kThreads) void partial_rope_kernel(const void* __re
 // 32): the workgroup covers kThreads chunks = kThreads / chunks-per-row consecutive positions of one outer row at a time,
 // 4 KB of contiguous memory, and walks its slab of outer rows at the same positions. A thread keeps its place in the row
 // and its position, so its cosines and sines stay in registers and no index arithmetic is left in the loop.
-template <int DT>
+// STREAM: the rows are read past the caches, and 16-bit ones written past them. Bound by memory: 3844 tokens of 64 x 512,
+// 504 MB of float16 in and out 112 -> 86 us, 1008 MB of float32 162 -> 148 and 176 -> 173; 126 MB of float16 24.8 -> 23.6.
+// (Float32 rows written past the caches too: 163 and 163 us.)
+template <int DT, bool STREAM>
 __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void* __restrict__ x, int n_outer, int seq_len,
                                                                     int chunks_log2, const float* __restrict__ inv_freq,
                                                                     const float* __restrict__ positions, int64_t offset,
@@ -179,16 +182,19 @@ __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void*
     }
     return v;
   };
-  // (16-bit rows past the caches: 504 MB in and out in 88 us against 91; float32 rows measured slower that way)
+  auto get = [](const u32x4_t* p) -> u32x4_t {
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
   auto put = [](u32x4_t v, u32x4_t* p) {
-    if constexpr (DT == MSPR_F32) *p = v;
-    else __builtin_nontemporal_store(v, p);
+    if constexpr (STREAM && DT != MSPR_F32) __builtin_nontemporal_store(v, p);
+    else *p = v;
   };
   constexpr int kAtOnce = 4;  // rows in flight per thread
   for (; n >= kAtOnce; n -= kAtOnce) {
     u32x4_t v[kAtOnce];
 #pragma unroll
-    for (int j = 0; j < kAtOnce; j++) v[j] = src[j * row_step];
+    for (int j = 0; j < kAtOnce; j++) v[j] = get(src + j * row_step);
 #pragma unroll
     for (int j = 0; j < kAtOnce; j++) {
       if (tail) v[j] = rotate(v[j]);
@@ -198,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void*
     dst += kAtOnce * row_step;
   }
   for (; n > 0; n--) {
-    u32x4_t v = *src;
+    u32x4_t v = get(src);
     if (tail) v = rotate(v);
     put(v, dst);
     src += row_step;
@@ -222,8 +228,9 @@ extern "C" int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer
   MSPR_REQUIRE(mspr_aligned(x, 16) && mspr_aligned(out, 16), "fused_partial_rope: rows must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   // The wide form where its blocks of positions are filled, in many small workgroups of four outer rows or more: 1008 MB of
-  // float32 rows took 175, 169, 165, 160 us with 2048, 8192, 16384, 32768 workgroups (171 in the form below), 504 MB of
-  // float16 rows 88 us (108), 126 MB of 128-wide float16 rows 24 us (30).
+  // float32 rows took 175, 169, 165, 160 us with 2048, 8192, 16384, 32768 workgroups (171 in the form below).
+  // Past the caches from 24 M elements on: 31 M (3844 tokens of 64 x 128) gain by it, 17 M (517 of 64 x 512) in float32 lose
+  // 4 %, for their rows still lie in the last-level cache.
   const int chunk_elems = dtype == MSPR_F32 ? 4 : 8;
   const int chunks = width / chunk_elems;
   if (width % chunk_elems == 0 && (chunks & (chunks - 1)) == 0 && chunks <= kThreads && seq_len >= kThreads / chunks) {
@@ -235,9 +242,16 @@ extern "C" int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer
     slabs = (n_outer + rows - 1) / rows;
     if (slabs <= 65535) {
       dim3 grid((unsigned)pos_blocks, (unsigned)slabs), block(kThreads);
-#define MSPR_ROPE_WIDE(DT)                                                                                          \
-  partial_rope_wide_kernel<DT><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, offset, \
-                                                       inverse, (int)rows, out)
+      const bool stream_rows = n_outer * seq_len * width >= ((int64_t)24 << 20);
+#define MSPR_ROPE_WIDE(DT)                                                                                               \
+  do {                                                                                                                   \
+    if (stream_rows)                                                                                                     \
+      partial_rope_wide_kernel<DT, true><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, \
+                                                                 offset, inverse, (int)rows, out);                       \
+    else                                                                                                                 \
+      partial_rope_wide_kernel<DT, false><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, \
+                                                                  offset, inverse, (int)rows, out);                      \
+  } while (0)
       if (dtype == MSPR_F32) MSPR_ROPE_WIDE(MSPR_F32);
       else if (dtype == MSPR_F16) MSPR_ROPE_WIDE(MSPR_F16);
       else MSPR_ROPE_WIDE(MSPR_BF16);

@@ -25,3 +25,14 @@ def test_rows_bit_identical(dtype_name, shape):
         want = ds4.fused_partial_rope(x.float().numpy(), inv, offset=offset, inverse=inverse, positions=positions, dtype=dtype_name)
         bits = torch.int32 if dtype_name == "float32" else torch.int16
         assert got.cpu().view(bits).equal(torch.from_numpy(want).to(_TORCH[dtype_name]).view(bits))
+
+
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_rows_past_the_caches_are_those_of_smaller_calls(dtype_name, inverse):
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn((65, 3027, 128), device="cuda", generator=gen).to(_TORCH[dtype_name])    # 24.02 M elements
+    inv = torch.from_numpy(ds4.rope_inverse_frequencies(64, 10000.0).astype(np.float32)).cuda()
+    got = seam.fused_partial_rope(x, inv, offset=71, inverse=inverse)
+    for part, want in ((x[:32], got[:32]), (x[32:], got[32:])):
+        assert seam.fused_partial_rope(part, inv, offset=71, inverse=inverse).equal(want)
