@@ -698,7 +698,7 @@ int prefill_q_blocks(int rep, int q_len) {
 // Enough workgroups for the 256 CUs but not more (one fits a CU, so a count just above 256 means a second round for a
 // few of them), and as many ranges as the partials are worth: tiles / ranges of about 1.3 us each against 1 KB per row
 // and range, written and read again at about 5 TB/s and partly under the tiles of other workgroups. The sum is
-// smallest near ranges^2 = 6000 * tiles / rows (3000 and 1500 measured up to 10 and 20 % slower). At least two tiles
+// smallest near ranges^2 = 6000 * tiles / rows (3000 and 1500 measured up to 10 and 20 % slower). At least two or three tiles
 // per range: 33 queries of 16 heads over 9000 keys 39 -> 31 us (17 ranges before, 56 now), 203 over 2000 43 -> 33 us.
 int prefill_choose_splits(int batch, int n_q_heads, int n_kv_heads, int q_blocks, int64_t past_len, int q_len) {
   const int64_t wgs = (int64_t)batch * n_kv_heads * q_blocks;
@@ -706,7 +706,8 @@ int prefill_choose_splits(int batch, int n_q_heads, int n_kv_heads, int q_blocks
   const int64_t tiles = (past_len + q_len + kTile - 1) / kTile;
   int64_t want = (int64_t)sqrt(6000.0 * (double)tiles / ((double)batch * n_q_heads * q_len));
   if (want > 256 / wgs) want = 256 / wgs;
-  if (want > tiles / 2) want = tiles / 2;
+  const int64_t fewest = q_len > 96 ? 3 : 2;  // tiles per range
+  if (want > tiles / fewest) want = tiles / fewest;
   if (want > 64) want = 64;
   return want < 1 ? 1 : (int)want;
 }
@@ -809,8 +810,11 @@ extern "C" int mspr_flash_prefill(const void* q, const void* k, const void* v, i
 // the 1.3 us of its attention; converting the prefix once (1 KB per key and KV head of scratch) costs a launch and
 // about 0.6 ns per row. From five 32-query blocks on, the prefix is therefore converted first and the attention
 // kernel runs on dense tiles only (at 128 queries both forms are within 5 % of each other from 2000 to 32000 keys;
-// 517 over 9000: 124 -> 114 us).
-static int prefill_q8_tiles(int q_len, int64_t past_len) { return q_len > 128 ? 0 : (int)(past_len / kTile); }
+// 517 over 9000: 124 -> 114 us); behind a long prefix only from nine on (203 over 32768: 148 us unpacked, 150 converted).
+static int prefill_q8_tiles(int q_len, int64_t past_len) {
+  const bool converted = q_len > 256 || (q_len > 128 && past_len <= 16384);
+  return converted ? 0 : (int)(past_len / kTile);
+}
 
 extern "C" size_t mspr_sdpa_fa_prefill_q8_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int q_len,
                                                           int64_t past_len) {
