@@ -18,8 +18,13 @@ struct IndexedPrefillArgs {
   const float* sinks;  // [n_heads] or null
   float scale_log2;
   float* out;  // strides as q
+  // filled in by the launch: units (token and block of 64 heads) that are cut into key ranges, and their partials
+  int split_units, ranges;
+  float* parts;
 };
 
 // Whether the kernel takes the call: the ids of a token are staged in LDS next to the row tiles.
 bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx);
-int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, hipStream_t st);
+// Room for the partials of a part-filled last round; without it every token is one workgroup's.
+size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int n_idx);
+int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, void* workspace, size_t workspace_bytes, hipStream_t st);

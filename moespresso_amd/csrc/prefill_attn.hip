@@ -19,7 +19,7 @@
 //
 // 3844 tokens, 64 heads, 128 + 512 rows each: from position 28000 426 us with float32 queries (before, with eight waves of
 // a persistent workgroup on one token and the queries rounded to half in a pass of their own: 620 + 130), from position 0
-// 324 us (542); 517 tokens 76 us (121). Without the tile copies 355 / 295 us, without the stores 360 / 276, with neither
+// 324 us (542); 517 tokens 62 us (121). Without the tile copies 355 / 295 us, without the stores 360 / 276, with neither
 // 303 / 240, which is the products and the softmax. Measured and not kept: one wave for 128 output columns of all heads
 // (V^T read once per workgroup, weights exchanged through LDS behind a second barrier) 500 / 397; persistent workgroups
 // that request the next token's ids, rows and queries under the last tile 471 / 351 with the stores as they were (464 / 361
@@ -42,6 +42,7 @@ static_assert(kOffStop + 4 <= kLdsBytes, "LDS map");
 constexpr int kQSteps = kD / 32;
 constexpr int kOutPitch = 256 + 4;  // floats between rows of the output staging: 16 heads' stores fall on 16 bank groups
 static_assert(4 * 16 * kOutPitch * 4 <= 2 * kTileBytes, "output staging lies in the tile buffers");
+constexpr int kMaxRanges = 8;
 constexpr int kAheadK = 8, kAheadV = 6;  // operand reads in flight (6/4 measures the same, 10/8 9 % slower)
 
 __device__ __attribute__((aligned(16))) const unsigned char g_prefill_zero_row[kD * 2] = {0};
@@ -61,7 +62,8 @@ __device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint3
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_base) : "memory", "m0");
 }
 
-template <int QDT>
+// CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
+template <int QDT, bool CUT>
 __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int* ids = reinterpret_cast<int*>(lds + kOffIds);
@@ -74,7 +76,16 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
 
   // The tokens with the most rows (the last ones, at the start of a context) are started first.
   const int n_hblk = (a.n_heads + 63) / 64;
-  const int unit = (int)(gridDim.x - 1u - blockIdx.x);
+  // The first a.split_units units, a part-filled last round, are cut into a.ranges key ranges each and come last.
+  int unit = (int)(gridDim.x - 1u - blockIdx.x), range = 0;
+  bool split = false;
+  if constexpr (CUT) {
+    const int whole = a.batch * a.n_tokens * n_hblk - a.split_units;
+    split = (int)blockIdx.x >= whole;
+    const int i = (int)blockIdx.x - whole;
+    unit = split ? i / a.ranges : a.split_units - 1 - i;
+    range = split ? i - unit * a.ranges : 0;
+  }
   const int hb = unit % n_hblk;
   const int seq = unit / n_hblk;
   const int b = seq / a.n_tokens;
@@ -93,6 +104,12 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
   if (visible > a.n_pool) visible = a.n_pool;
   const int wt = (n_win + kTile - 1) / kTile;
+  // this workgroup's tiles: all of them, or its share of what the token has at most
+  int t_begin = 0, t_share = 0x7FFFFFFF;
+  if (CUT && split) {
+    t_share = (wt + (a.n_idx + kTile - 1) / kTile + a.ranges - 1) / a.ranges;
+    t_begin = range * t_share;
+  }
   const uint64_t win_base = reinterpret_cast<uint64_t>(a.win) + (uint64_t)b * (uint64_t)a.raw_cap * (kD * 2);
   const uint64_t pool_base = reinterpret_cast<uint64_t>(a.pool) + (uint64_t)b * (uint64_t)a.n_pool * (kD * 2);
 
@@ -117,7 +134,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   };
 
   // ---- the first window tile needs no ids: on its way before anything else
-  if (wt > 0) copy_rows(0, win_base, window_row(0));
+  if (t_begin < wt) copy_rows(t_begin, win_base, window_row(t_begin));
 
   // ---- ids to LDS, position of the first one that ends the walk
   if (tid == 0) *stop_sh = a.n_idx;
@@ -153,7 +170,8 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   const float sink = live && a.sinks ? a.sinks[head] * 1.4426950408889634f : -__builtin_inff();
   __syncthreads();
   const int stop = __builtin_amdgcn_readfirstlane(*stop_sh);
-  const int n_tiles = wt + (stop + kTile - 1) / kTile;
+  int n_tiles = wt + (stop + kTile - 1) / kTile;
+  if (CUT && n_tiles - t_begin > t_share) n_tiles = t_begin + t_share;
 
   auto pool_row = [&](int tile) -> int {
     const int gi = (tile - wt) * kTile + (lane & 31);
@@ -162,8 +180,8 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   };
   // rows and validity word of a tile
   auto rows_of = [&](int tile) -> int { return tile < wt ? window_row(tile) : pool_row(tile); };
-  int row = rows_of(0);
-  if (wt == 0 && n_tiles > 0) copy_rows(0, pool_base, row);
+  int row = rows_of(t_begin);
+  if (t_begin >= wt && t_begin < n_tiles) copy_rows(t_begin, pool_base, row);
 
   f32x4_t oacc[32];
 #pragma unroll
@@ -175,7 +193,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   const int a_off = c16 * kPitch + 16 * kg;
   const int tr_off = (4 * kg + (c16 >> 2)) * kPitch + 8 * (c16 & 3);
 
-  for (int tile = 0; tile < n_tiles; tile++) {
+  for (int tile = t_begin; tile < n_tiles; tile++) {
     const uint32_t valid = (uint32_t)__ballot(row >= 0);  // bit l: slot l (both halves of the wave hold the 32 slots)
     // the copies of this tile have landed (they are the only vector-memory operations in flight), and every wave is done
     // with the tile before it, whose buffer the next copies overwrite
@@ -258,6 +276,18 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   float l = l_run;
   l += __shfl_xor(l, 16, MSPR_WAVE);
   l += __shfl_xor(l, 32, MSPR_WAVE);
+  if (CUT && split) {  // unnormalised, as the registers hold it
+    const int part = unit * a.ranges + range;
+    float* po = a.parts + (int64_t)part * (64 * kD) + (wave * 32 * 64 + lane) * 4;
+#pragma unroll
+    for (int mt = 0; mt < 32; mt++) *reinterpret_cast<f32x4_t*>(po + mt * 256) = oacc[mt];
+    if (kg == 0) {
+      float* ml = a.parts + (int64_t)a.split_units * a.ranges * (64 * kD) + ((int64_t)part * 64 + 16 * wave + c16) * 2;
+      ml[0] = m_run;
+      ml[1] = l;
+    }
+    return;
+  }
   const float m_all = fmaxf(m_run, sink);
   const float m_safe = m_all == -__builtin_inff() ? 0.0f : m_all;
   const float w = __builtin_amdgcn_exp2f(m_run - m_safe);
@@ -291,11 +321,53 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   }
 }
 
-template <int QDT>
+// The ranges of the cut units and the sink, normalised. A wave takes one accumulator register quad (16 heads, 16 columns) of
+// a unit: every range's is 1 KB, and all are requested at once.
+__global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(IndexedPrefillArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int c16 = lane & 15, kg = lane >> 4;
+  const int piece = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  const int unit = piece >> 7, wave = (piece >> 5) & 3, mt = piece & 31;
+  const int n_hblk = (a.n_heads + 63) / 64;
+  const int hb = unit % n_hblk, seq = unit / n_hblk;
+  const int b = seq / a.n_tokens, t = seq - b * a.n_tokens;
+  const int head = hb * 64 + 16 * wave + c16;
+  const float* po = a.parts + (int64_t)unit * a.ranges * (64 * kD) + ((wave * 32 + mt) * 64 + lane) * 4;
+  const float* ml = a.parts + (int64_t)a.split_units * a.ranges * (64 * kD) + ((int64_t)unit * a.ranges * 64 + 16 * wave + c16) * 2;
+  float m[kMaxRanges], l[kMaxRanges];
+  f32x4_t o[kMaxRanges];
+#pragma unroll
+  for (int r = 0; r < kMaxRanges; r++) {
+    const int rr = r < a.ranges ? r : 0;
+    m[r] = ml[rr * 128];
+    l[r] = ml[rr * 128 + 1];
+    o[r] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)rr * (64 * kD));
+    if (r >= a.ranges) m[r] = -__builtin_inff();
+  }
+  const float sink = head < a.n_heads && a.sinks ? a.sinks[head] * 1.4426950408889634f : -__builtin_inff();
+  float m_all = sink;
+#pragma unroll
+  for (int r = 0; r < kMaxRanges; r++) m_all = fmaxf(m_all, m[r]);
+  const float m_safe = m_all == -__builtin_inff() ? 0.0f : m_all;
+  float den = __builtin_amdgcn_exp2f(sink - m_safe);
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < kMaxRanges; r++) {
+    const float w = __builtin_amdgcn_exp2f(m[r] - m_safe);
+    den += l[r] * w;
+    acc += o[r] * w;
+  }
+  const float f = den == 0.0f ? 0.0f : 1.0f / den;
+  if (head < a.n_heads)
+    *reinterpret_cast<f32x4_t*>(a.out + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
+                                (int64_t)head * a.q_head_stride + 16 * mt + 4 * kg) = acc * f;
+}
+
+template <int QDT, bool CUT>
 int launch(const IndexedPrefillArgs& a, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) {
       mspr_set_error("indexed prefill attention: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
@@ -303,12 +375,18 @@ int launch(const IndexedPrefillArgs& a, hipStream_t st) {
     }
     attr_set = true;
   }
-  dim3 grid((unsigned)((int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64))), block(kThreads);
+  const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
+  dim3 grid((unsigned)(units - a.split_units + a.split_units * a.ranges)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
-    indexed_prefill_kernel<QDT><<<grid, block, kLdsBytes, st>>>(a);
+    indexed_prefill_kernel<QDT, CUT><<<grid, block, kLdsBytes, st>>>(a);
   }
   MSPR_CHECK_LAUNCH("indexed prefill attention");
+  if constexpr (CUT) {
+    MsprProfScope prof(MSPR_K_SPARSE_MERGE, st);
+    indexed_prefill_merge_kernel<<<dim3((unsigned)(a.split_units * 32)), block, 0, st>>>(a);
+    MSPR_CHECK_LAUNCH("indexed prefill attention (merge)");
+  }
   return MSPR_OK;
 }
 
@@ -318,6 +396,39 @@ bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx) 
   return n_idx <= kMaxIds && (int64_t)batch * n_tokens * ((n_heads + 63) / 64) < ((int64_t)1 << 31);
 }
 
-int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, hipStream_t st) {
-  return a.q_dtype == MSPR_F32 ? launch<MSPR_F32>(a, st) : launch<MSPR_F16>(a, st);
+// Two workgroups on each of 256 CUs are a round; what is left of the last one runs one to a CU, and if it is few units the
+// chip is idle. Up to 80 of them are cut into key ranges, as many as keep the partials (128 KB each) under 24 MB, with at
+// least two id tiles in each. With the merge, 128 + 512 rows each: 1 token 29 -> 13 us, 20 29.5 -> 21, 64 30 -> 25, 513
+// 75 -> 62; 96 would gain nothing. (Partials under 16 MB: 64 tokens 28; under 32 MB: 544 tokens 73 instead of 68.)
+static void cut_last_round(IndexedPrefillArgs& a) {
+  const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
+  const int left = (int)(units % 512);
+  int ranges = left == 0 || left > 80 ? 1 : 192 / left;
+  if (ranges > a.n_idx / (2 * kTile)) ranges = a.n_idx / (2 * kTile);
+  if (ranges > kMaxRanges) ranges = kMaxRanges;
+  a.split_units = ranges > 1 ? left : 0;
+  a.ranges = ranges > 1 ? ranges : 1;
+}
+
+static size_t part_bytes(const IndexedPrefillArgs& a) {
+  return (size_t)a.split_units * a.ranges * (64 * kD + 64 * 2) * sizeof(float);
+}
+
+size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int n_idx) {
+  IndexedPrefillArgs a = {};
+  a.batch = batch;
+  a.n_heads = n_heads;
+  a.n_tokens = n_tokens;
+  a.n_idx = n_idx;
+  cut_last_round(a);
+  return part_bytes(a);
+}
+
+int mspr_launch_indexed_prefill(const IndexedPrefillArgs& call, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  IndexedPrefillArgs a = call;
+  cut_last_round(a);
+  a.parts = static_cast<float*>(workspace);
+  if (!workspace || workspace_bytes < part_bytes(a) || !mspr_aligned(workspace, 16)) a.split_units = 0;
+  if (a.split_units > 0) return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, true>(a, st) : launch<MSPR_F16, true>(a, st);
+  return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, false>(a, st) : launch<MSPR_F16, false>(a, st);
 }

@@ -1672,7 +1672,8 @@ extern "C" size_t mspr_indexed_mixed_attention_prefill_workspace_bytes(int q_dty
                                                                        int n_tokens, int window_rows, int top_k) {
   if (batch < 1 || n_heads < 1 || n_tokens < 1 || window_rows < 0 || top_k < 0) return 0;
   const PrefillForm form = prefill_form();
-  if (form == kPrefillWaves && mspr_indexed_prefill_fits(batch, n_heads, n_tokens, top_k)) return 0;
+  if (form == kPrefillWaves && mspr_indexed_prefill_fits(batch, n_heads, n_tokens, top_k))
+    return mspr_indexed_prefill_workspace_bytes(batch, n_heads, n_tokens, top_k);
   // the per-range partials of the split kernel (slot lists too long for the persistent consumer), or the
   // half-precision copy of float32 queries for the persistent consumer, whichever is larger
   size_t need = workspace_bytes(batch * n_tokens, n_heads, (int64_t)window_rows + top_k);
@@ -1900,7 +1901,7 @@ extern "C" int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, 
     p.sinks = sinks;
     p.scale_log2 = (float)(1.4426950408889634 / sqrt(512.0));
     p.out = out;
-    return mspr_launch_indexed_prefill(p, (hipStream_t)stream);
+    return mspr_launch_indexed_prefill(p, workspace, workspace_bytes_given, (hipStream_t)stream);
   }
   SparseAttnArgs a = {};
   a.q = q;

@@ -37,3 +37,23 @@ def test_edges_match_the_oracle(monkeypatch, form, tokens, heads, top_k, window,
     want = ds4.indexed_mixed_attention_prefill(q, raw, comp, ids, sinks, pos0=pos0, window=window, ratio=ratio,
                                                raw_start=raw_start)
     np.testing.assert_allclose(got.cpu().numpy(), want, rtol=2e-3, atol=2e-3)
+
+
+# a part-filled last round of workgroups in key ranges: alone, behind a whole round, in two head blocks, ids that end early,
+# tokens whose last ranges hold nothing, the most tokens that are cut and one more
+@pytest.mark.parametrize("batch,tokens,heads,top_k,pos0", [(1, 1, 64, 512, 3000), (1, 20, 64, 512, 0), (1, 515, 16, 130, 900),
+                                                          (2, 7, 72, 300, 500), (1, 80, 32, 512, 2100), (1, 81, 32, 512, 2100)])
+def test_last_round_in_key_ranges(monkeypatch, batch, tokens, heads, top_k, pos0):
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    q = torch.randn((batch, heads, tokens, 512), device="cuda", generator=gen)
+    raw = torch.randn((batch, 1, min(127, pos0) + tokens, 512), device="cuda", generator=gen).half()
+    comp = torch.randn((batch, 900, 512), device="cuda", generator=gen).half()
+    ids = torch.rand((batch, tokens, 900), device="cuda", generator=gen).topk(top_k, dim=2).indices.sort(dim=2).values.to(torch.int32)
+    sinks = torch.randn(heads, device="cuda", generator=gen)
+    run = lambda: iak.indexed_mixed_attention_prefill_live_f32(q, raw, comp, ids, sinks, pos0=pos0, window=128, ratio=4)
+    monkeypatch.delenv("MSPR_PREFILL_PERSISTENT", raising=False)
+    got = run()
+    monkeypatch.setenv("MSPR_PREFILL_PERSISTENT", "1")
+    torch.testing.assert_close(got, run(), rtol=2e-3, atol=2e-3)
