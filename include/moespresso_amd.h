@@ -142,9 +142,9 @@ int mspr_indexer_scores_tiled_live_ws(const void* q, const float* weights, const
 /* Scratch bytes for the gathered-attention entry points below. */
 size_t mspr_sparse_attention_workspace_bytes(int batch, int n_heads, int64_t n_keys);
 
-/* Scratch bytes for mspr_indexed_mixed_attention_prefill: the per-range partials of calls that take one workgroup
- * per token, or the half-precision copy of float32 queries (batch*n_tokens*n_heads*512*2 bytes), whichever is
- * larger. window_rows is the largest number of ring rows a token attends. No counterpart in the reference
+/* Scratch bytes for mspr_indexed_mixed_attention_prefill: the per-range partials of a last round of workgroups that
+ * would leave CUs idle, those of the split kernel, or (persistent form) the half-precision copy of float32 queries;
+ * 0 where none applies. window_rows is the largest number of ring rows a token attends. No counterpart in the reference
  * (its kernels allocate through MLX). */
 size_t mspr_indexed_mixed_attention_prefill_workspace_bytes(int q_dtype, int batch, int n_heads, int n_tokens,
                                                             int window_rows, int top_k);
@@ -172,11 +172,12 @@ int mspr_indexed_mixed_attention_decode(const float* q, int n_heads, const void*
  * 512 contiguous values of q_dtype (f32 rounded to half on load, or f16); raw_kv: f16
  * [batch,raw_cap,512]; comp_kv: f16 [batch,n_comp,512]; topk: int32 [batch,n_tokens,top_k]
  * (top_k may be 0); sinks: f32 [n_heads]; out: f32 with the strides of q.
- * Id lists of up to 3520 ids run on the kernel of prefill_attn.hip (one workgroup per token and 64 heads, two per CU,
- * no workspace), longer ones on the split kernel, one workgroup per token and key range. MSPR_PREFILL_PERSISTENT in
- * the environment, read per call, keeps every call on a form to compare with: 1 = one persistent workgroup per CU that
- * streams consecutive tokens (slots of up to 22 tiles; float32 queries are rounded to half into the workspace), 0 = the
- * split kernel. The workspace query follows the same variable.
+ * Id lists of up to 3520 ids run on the kernel of prefill_attn.hip (one workgroup per token and 64 heads, two per CU; a
+ * last round that would leave CUs idle is cut into key ranges when the workspace is given), longer ones on the split
+ * kernel, one workgroup per token and key range. MSPR_PREFILL_PERSISTENT in the environment, read per call, keeps every
+ * call on a form to compare with: 1 = one persistent workgroup per CU that streams consecutive tokens (slots of up to 22
+ * tiles; float32 queries are rounded to half into the workspace), 0 = the split kernel. The workspace query follows the
+ * same variable.
  * Workspace: mspr_indexed_mixed_attention_prefill_workspace_bytes(q_dtype, batch, n_heads, n_tokens,
  * min(window or raw_cap, raw_cap), top_k). */
 int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, int batch, int n_heads, int n_tokens,
