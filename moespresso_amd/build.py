@@ -167,5 +167,22 @@ def inline_asm_register_loads(lines: list[str]) -> list[str]:
     return found
 
 
+def m0_hazards(lines: list[str]) -> list[str]:
+    """Asynchronous copies into LDS that directly follow the scalar instruction that writes M0, from which they take
+    their LDS address. gfx950 wants an instruction between the two; the compiler puts one there for its own copies
+    but does not look inside an inline asm statement."""
+    import re
+
+    found, previous = [], ""
+    for line in lines:
+        text = line.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        if "_load_lds_" in text and re.match(r"s_\w+ m0\b", previous):
+            found.append(f"{previous} / {text}")
+        previous = text
+    return found
+
+
 if __name__ == "__main__":
     build()

@@ -113,15 +113,16 @@ __device__ __forceinline__ void wait_vm_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 // lane i's 16 bytes at `src` land at lds_base + 16 i (lds_base wave-uniform); issued through asm so
-// that the compiler's wait-count pass does not drain it in front of LDS transpose reads
+// that the compiler's wait-count pass does not drain it in front of LDS transpose reads (s_nop: the copy needs
+// one instruction between it and the scalar write of M0, which the compiler does not add inside an asm statement)
 __device__ __forceinline__ void async_load_16(uint64_t base, uint32_t offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(offset), "s"(lds_base)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(offset), "s"(lds_base)
                : "memory", "m0");
 }
 
 // the same with 4 bytes per lane: lane i's dword lands at lds_base + 4 i
 __device__ __forceinline__ void async_load_4(uint64_t base, uint32_t offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %1, %0" ::"s"(base), "v"(offset), "s"(lds_base)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" ::"s"(base), "v"(offset), "s"(lds_base)
                : "memory", "m0");
 }
 

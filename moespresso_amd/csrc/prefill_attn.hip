@@ -57,9 +57,12 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 }
 
 // One 1 KB row to LDS: lane l's 16 bytes go to lds_base + 16 l. Through asm so that the compiler does not drain it in front
-// of LDS reads; the tile loop waits for all copies of a tile at its barrier.
+// of LDS reads; the tile loop waits for all copies of a tile at its barrier. (An instruction has to stand between a scalar
+// write of M0 and the copy that takes its LDS address from it; the compiler, which sees to that elsewhere, does not look
+// inside an asm statement.)
 __device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_base)
+               : "memory", "m0");
 }
 
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).

@@ -173,9 +173,10 @@ __device__ __forceinline__ void wait_vm_and_barrier() {
 // One wave-wide asynchronous copy global -> LDS: lane i's 16 bytes at `src` land at lds_base + 16 i
 // (lds_base is wave-uniform). Issued through asm so that the compiler's wait-count pass does not
 // see LDS writes in flight (it would drain them in front of every LDS transpose read); completion
-// is awaited explicitly through wait_vm_and_barrier.
+// is awaited explicitly through wait_vm_and_barrier. (s_nop: the copy needs one instruction between it and
+// the scalar write of M0, which the compiler does not add inside an asm statement; so in every copy below.)
 __device__ __forceinline__ void async_load_16(uint64_t src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -917,7 +918,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_prefill_kernel(Sparse
       gi = gi < 0 ? 0 : (gi >= a.n_idx ? a.n_idx - 1 : gi);
       const int32_t* p = idx_b + gi;
       // lane i's dword lands at ids_lds[64 wave + 512 j + i] = ids_lds[tid + 512 j]
-      asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(ids_lds_wave + j * (kThreads * 4))
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(ids_lds_wave + j * (kThreads * 4))
                    : "memory", "m0");
     }
     issued += 2;
@@ -1039,7 +1040,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_prefill_kernel(Sparse
     const uint16_t* p = reinterpret_cast<const uint16_t*>(a.q) + (int64_t)m.b * a.q_batch_stride +
                         (int64_t)m.t * a.q_token_stride + (int64_t)(head < a.n_heads ? head : 0) * a.q_head_stride +
                         (tid & 7) * 64;
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(warm_lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(warm_lds) : "memory", "m0");
     issued += 1;
   };
   static_assert(PG::kQSteps == 16, "the query wait below names sixteen registers");

@@ -68,3 +68,15 @@ def test_prefill_consumer_store_count_matches_what_its_waits_assume(sparse_assem
     loads = [l.split()[0] for l in lines if l.strip().startswith(("global_load", "flat_load", "buffer_load", "scratch_load"))
              and "_lds_" not in l]
     assert loads.count("global_load_dwordx4") == 32 and len(loads) == 36, loads
+
+
+@pytest.mark.parametrize("source", ["sparse_attn.hip", "prefill_attn.hip", "flash_prefill.hip"])
+def test_no_copy_into_lds_directly_follows_the_write_of_its_address_register(source):
+    bodies = build.kernel_bodies(build.device_assembly(os.path.join(build.CSRC, source)))
+    assert any("_load_lds_" in l for lines in bodies.values() for l in lines)
+    for name, lines in bodies.items():
+        assert build.m0_hazards(lines) == [], name
+    copy = "\tglobal_load_lds_dwordx4 v2, s[4:5]"
+    assert len(build.m0_hazards(["\ts_mov_b32 m0, s8", "\t;;#ASMSTART", copy])) == 1
+    assert len(build.m0_hazards(["\ts_add_i32 m0, s8, 0x400", copy])) == 1
+    assert build.m0_hazards(["\ts_mov_b32 m0, s8", "\ts_nop 0", copy, copy]) == []
