@@ -501,7 +501,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     }
     return;
   }
-  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  const float inv = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
   if (active && q0 + n < a.q_len) {
     const int64_t ooff = (((int64_t)b * a.n_q_heads + head) * a.q_len + q0 + n) * kD;
 #pragma unroll
@@ -525,13 +525,14 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
 // does not unpack itself (all of them, or the last past_len % 32) and then the chunk's own rows. A thread makes 16
 // values of K and of V, 16 threads a row, 16 rows a workgroup, so one launch moves both kinds in 16-byte pieces: it is
 // bound by its bytes (2 * 36000 rows 23 us). code * scale + bias is one float32 multiply-add, rounded once.
-// Values beyond the range of the staging type saturate instead of becoming infinite (an infinite key or value
-// turns the whole output row into NaN).
+// Finite values beyond the range of the staging type saturate instead of becoming infinite (an infinite key or value
+// turns the whole output row into NaN). Infinities and NaN stay (v_med3 alone would make a NaN the lowest finite value): a
+// cache that holds them gives NaN in decode and has to here.
 template <int ODT>
 __device__ __forceinline__ void store_row16(float (&v)[16], uint16_t* dst) {
   constexpr float kMax = ODT == MSPR_F16 ? 65504.0f : 0x1.fep127f;
 #pragma unroll
-  for (int j = 0; j < 16; j++) v[j] = __builtin_amdgcn_fmed3f(v[j], -kMax, kMax);
+  for (int j = 0; j < 16; j++) v[j] = __builtin_isfinite(v[j]) ? __builtin_amdgcn_fmed3f(v[j], -kMax, kMax) : v[j];
 #pragma unroll
   for (int h = 0; h < 2; h++)
     reinterpret_cast<u32x4_t*>(dst)[h] = u32x4_t{pack2<ODT>(v[8 * h], v[8 * h + 1]), pack2<ODT>(v[8 * h + 2], v[8 * h + 3]),
@@ -599,6 +600,17 @@ __global__ __launch_bounds__(256) void prefill_q8_rows_kernel(PrefillArgs a, con
       load_row16<MSPR_BF16>(self_k, off, kx);
       load_row16<MSPR_BF16>(self_v, off, vx);
     }
+    // Queries in front of this row do not see it, but its tile is theirs: their weight for it is zero, and zero times a
+    // value that is not finite is NaN. Such a value is therefore made finite and the row's key NaN instead, whose score
+    // those queries mask and the others turn into NaN.
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      finite = finite && __builtin_isfinite(vx[i]);
+      vx[i] = __builtin_isfinite(vx[i]) ? vx[i] : 0.0f;
+    }
+    const uint64_t row_finite = __ballot(finite) >> (threadIdx.x & 48);  // (the row's sixteen lanes are here together)
+    if ((row_finite & 0xFFFFu) != 0xFFFFu) kx[0] = __builtin_nanf("");
   }
   const int64_t dst = (bh * a.kv_rows + j) * kD + 16 * pp;
   store_row16<ODT>(kx, out_k + dst);
@@ -632,8 +644,9 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
       mv[j] = a.ws_ml[r * 2];
       lv[j] = a.ws_ml[r * 2 + 1];
       ov[j] = *reinterpret_cast<const f32x4_t*>(a.ws_o + r * kD + 4 * lane);
-      // a range that saw no key of this row contributes nothing (its O is whatever the registers held)
-      if (s0 + SHARE * j >= a.n_splits || !(lv[j] > 0.0f)) {
+      // a range that saw no key of this row contributes nothing (its O may be zero times a value that is not finite); one
+      // whose denominator is NaN makes the row NaN
+      if (s0 + SHARE * j >= a.n_splits || lv[j] == 0.0f) {
         mv[j] = -__builtin_inff();
         lv[j] = 0.0f;
         ov[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -677,7 +690,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     }
   }
   if (!live) return;
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const float inv = l == 0.0f ? 0.0f : 1.0f / l;
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + row * kD + 4 * lane) = o * inv;
   } else {

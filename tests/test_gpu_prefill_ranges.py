@@ -37,3 +37,47 @@ def test_quantised_prefix_rows(tokens, past, dtype):
     want = qwen.causal_prefill_attention(q[:, :, past:].float().cpu().numpy(), dk.float().cpu().numpy(),
                                          dv.float().cpu().numpy(), 256 ** -0.5, past=past)
     assert np.abs(got.cpu().numpy() - want).max() < 2e-3
+
+
+# unpacked in the attention kernel; converted to float16; to bfloat16: one key range, several, and merges of two waves a row
+@pytest.mark.parametrize("tokens,past", [(17, 40), (17, 5000), (203, 301), (300, 9000), (1024, 70)])
+@pytest.mark.parametrize("side", ["key", "value"])
+@pytest.mark.parametrize("bad", ["infinite activation", "infinite bias", "NaN scale"])
+def test_infinities_and_nan_of_a_quantised_prefix_reach_the_output(tokens, past, side, bad):
+    """As in decode over the same cache: a key that is not a number makes its KV head's rows NaN, a value its group's columns."""
+    gen = torch.Generator(device="cuda").manual_seed(tokens + past)
+    q, k, v = (torch.randn((1, h, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (8, 2, 2))
+    dirty_k, dirty_v = k.clone(), v.clone()
+    at = (0, 1, past // 2)                                               # second head
+    if bad == "infinite activation":
+        (dirty_k if side == "key" else dirty_v)[(*at, 70)] = float("inf")  # second group: columns 64 to 127
+    prefix = [t[:, :, :past] for t in (*kquant.quantize(dirty_k), *kquant.quantize(dirty_v))]
+    scales, biases = prefix[1:3] if side == "key" else prefix[4:6]
+    if bad == "infinite bias":
+        biases[(*at, 1)] = float("inf")
+    elif bad == "NaN scale":
+        scales[(*at, 1)] = float("nan")
+    dk, dv = (kquant.dequantize(*kquant.quantize(x)) for x in (k, v))
+    got = kquant.sdpa_fa_prefill_q8(q[:, :, past:], *prefix, dk[:, :, past:], dv[:, :, past:], 256 ** -0.5).cpu().numpy()
+    step = kquant.sdpa_decode_q8(q[:, :, past:past + 1].contiguous(), *prefix, 256 ** -0.5).cpu().numpy()
+    hit = ~np.isfinite(step)
+    assert hit[0, 4:, :, 64:128].all() and not hit[0, :4].any() and bool(hit[0, 4:].all()) == (side == "key")
+    np.testing.assert_array_equal(~np.isfinite(got), np.broadcast_to(hit, got.shape))
+    want = qwen.causal_prefill_attention(q[:, :, past:].cpu().numpy(), dk.cpu().numpy(), dv.cpu().numpy(), 256 ** -0.5, past=past)
+    assert np.abs(np.where(np.isfinite(got), got - want, 0.0)).max() < 2e-3
+
+
+@pytest.mark.parametrize("tokens", [40, 200, 1030])
+@pytest.mark.parametrize("side", ["key", "value"])
+def test_a_chunk_row_that_is_not_finite_reaches_the_queries_that_see_it_and_no_other(tokens, side):
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    q, k, v = (torch.randn((1, h, 33 + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (8, 2, 2))
+    dk, dv = (kquant.dequantize(*kquant.quantize(x)) for x in (k, v))
+    prefix = [t[:, :, :33] for t in (*kquant.quantize(k), *kquant.quantize(v))]
+    want = qwen.causal_prefill_attention(q[:, :, 33:].cpu().numpy(), dk.cpu().numpy(), dv.cpu().numpy(), 256 ** -0.5, past=33)
+    row = tokens // 2 + 3
+    (dk if side == "key" else dv)[0, 1, 33 + row, 64:128] = float("inf") if tokens == 40 else float("nan")
+    got = kquant.sdpa_fa_prefill_q8(q[:, :, 33:], *prefix, dk[:, :, 33:], dv[:, :, 33:], 256 ** -0.5).cpu().numpy()
+    assert np.isnan(got[0, 4:, row:]).all()
+    rest = np.abs(got - want)
+    assert rest[0, :4].max() < 2e-3 and rest[0, 4:, :row].max() < 2e-3
