@@ -163,6 +163,15 @@ __device__ __attribute__((aligned(16))) float g_store_sink[64 * 512];
 
 #define MSPR_GLB_PTR(T, p) ((__attribute__((address_space(1))) T*)(p))
 
+// Infinities of a packed float16 pair become the largest finite values. (IEEE 754-2019 minimum and maximum: a NaN stays one,
+// which v_med3 on the float32 values made the lowest finite value.)
+__device__ __forceinline__ uint32_t h2_saturate(uint32_t w) {
+  typedef __attribute__((ext_vector_type(2))) _Float16 h2_t;
+  const h2_t most = {(_Float16)65504.0f, (_Float16)65504.0f};
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_maximum(
+                                          __builtin_elementwise_minimum(__builtin_bit_cast(h2_t, w), most), -most));
+}
+
 // Wait until at most N of this wave's vector-memory operations are outstanding and all of its LDS
 // operations are done, then meet the other waves. Written as one asm statement so that no
 // compiler-inserted full drain (as a fence would add) sits between the asynchronous tile loads.
@@ -723,12 +732,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
       uint32_t w[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        float x = oacc[mt][4 * c + 2 * j] * inv_l, y = oacc[mt][4 * c + 2 * j + 1] * inv_l;
-        if constexpr (KDT == MSPR_BF16) {
-          x = __builtin_amdgcn_fmed3f(x, -65504.0f, 65504.0f);
-          y = __builtin_amdgcn_fmed3f(y, -65504.0f, 65504.0f);
-        }
-        w[j] = pack2<MSPR_F16>(x, y);
+        w[j] = pack2<MSPR_F16>(oacc[mt][4 * c + 2 * j] * inv_l, oacc[mt][4 * c + 2 * j + 1] * inv_l);
+        if constexpr (KDT == MSPR_BF16) w[j] = h2_saturate(w[j]);
       }
       // registers 4c..4c+7 of this lane: 16 bytes, lane-contiguous
       *reinterpret_cast<u32x4_t*>(wo + ((mt * 2 + c / 2) * 64 + lane) * 8) = u32x4_t{w[0], w[1], w[2], w[3]};

@@ -29,3 +29,21 @@ def test_decode_ranges_of_whole_tiles(batch, window, ids):
     # bfloat16 output, and probabilities of 8 significant bits: errors of single keys average out over many
     bound = 1e-3 + 2e-2 * (window + ids) ** -0.5 + 2.0 ** -7 * np.abs(want)
     assert (np.abs(got - want) <= bound).all(), (np.abs(got - want) - bound).max()
+
+
+@pytest.mark.parametrize("ids", [20, 2000])          # one key range, written directly; many, merged
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_row_that_is_not_finite_makes_its_columns_nan(ids, dtype):
+    """An infinite element whose score is -inf has weight zero, and zero times infinity is NaN in that column alone; a score
+    of +inf makes the whole row NaN. A partial stored as float16 must not turn either into a finite value."""
+    gen = torch.Generator(device="cuda").manual_seed(ids)
+    kv = torch.randn((2, 4000, 512), device="cuda", generator=gen).to(dtype)
+    q = torch.randn((2, 64, 512), device="cuda", generator=gen).to(dtype)
+    sel = torch.arange(ids, dtype=torch.int32, device="cuda").expand(2, ids).contiguous()
+    kv[1, ids // 2, 300] = float("inf")
+    q[1, :, 300] = torch.where(torch.arange(64, device="cuda") % 2 == 0, -1.0, 1.0).to(dtype)
+    got = iak.sparse_mla_decode(q, kv, sel, scale=512 ** -0.5)
+    want = torch.zeros((2, 64, 512), dtype=torch.bool, device="cuda")
+    want[1, 0::2, 300] = True
+    want[1, 1::2] = True
+    assert got.isnan().equal(want) and bool(got[~want].isfinite().all())
