@@ -11,8 +11,13 @@
 //  * Operands that came out of the indexer's QAT are, group of 32 by group of 32, values of the e2m1 lattice times a power
 //    of two: exactly the operand format of v_mfma_scale_f32_32x32x64_f8f6f4 (fp4 with one e8m0 scale per 32), which
 //    multiplies four times as many of them per cycle as the float16 form. Both operands are packed once per call into MFMA
-//    operand order (pack_operands_kernel), where each value is checked by converting it back; the products are exact and
-//    so are their sums (some 18 significant bits), so the scores are those of the float16 form bit for bit. With the
+//    operand order (pack_operands_kernel), where each value is checked by converting it back; the products are exact. Their
+//    sums are exact too, and the scores those of the float16 form bit for bit, where the exponents of a dot product's four
+//    group products lie within 9 of each other: in units of the smallest group's least product (a quarter, as lattice
+//    values are multiples of one half) 32 products of at most 36 from each of four groups are at most 4 * 32 * 144 * 2^9 <
+//    2^24 of them. (Rows of Gaussian values: within 2 per operand.) Groups further apart round in float32 in either form,
+//    here once per 64 products and there once per 16: with group exponents drawn evenly from -13 .. 13 a dot product is off
+//    by at most 0.9e-7 of the sum of its products' magnitudes, and by 2.0e-7 in the float16 form. With the
 //    products this cheap the relu-weighted head sum on the vector units is the bound (two instructions per score and
 //    head: 256 cycles of a wave's 32-row tile against 128 of the matrix pipe). Its tiles need no LDS and no barrier, so
 //    the four waves drift apart and one wave's sums run under another's products.

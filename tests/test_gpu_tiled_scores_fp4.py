@@ -1,5 +1,5 @@
-"""The fp4 form of the tiled scores: the same scores as the float16 form (bit for bit on QAT'd operands), and operands of
-which only a part is exact in fp4."""
+"""The fp4 form of the tiled scores: the same scores as the float16 form (bit for bit where the sums are exact), sums that
+round, and operands of which only a part is exact in fp4."""
 
 import pytest
 import torch
@@ -57,3 +57,36 @@ def test_operands_outside_the_format_take_the_float16_form(spoil):
         comp[0, 3, 3] = float("nan")
     got, want = _both(q, w, comp, 900)
     assert torch.equal(torch.nan_to_num(got, nan=12345.0), torch.nan_to_num(want, nan=12345.0))
+
+
+def _lattice_rows(rows, low, high, gen):
+    """[rows, 128] of e2m1 lattice values, each group of 32 times a power of two with an exponent in [low, high]."""
+    v = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6], device="cuda")[torch.randint(0, 8, (rows, 128), device="cuda", generator=gen)]
+    v *= torch.randint(0, 2, v.shape, device="cuda", generator=gen) * 2 - 1
+    v[:, ::32] = 6.0                                 # (a group is stored by its largest magnitude)
+    e = torch.randint(low, high + 1, (rows, 4), device="cuda", generator=gen)
+    return v * torch.exp2(e.float()).repeat_interleave(32, dim=1)
+
+
+@pytest.mark.parametrize("q_exp,comp_exp", [((0, 5), (-4, 0)), ((-13, -8), (9, 13))])
+def test_group_exponents_within_nine_give_exact_sums(q_exp, comp_exp):
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    q, comp = _lattice_rows(70, *q_exp, gen), _lattice_rows(300, *comp_exp, gen)
+    got, want = _both(q.reshape(1, 1, 70, 128), torch.ones((1, 70, 1), device="cuda"), comp.reshape(1, 300, 128), 0, 0)
+    assert got.equal(want)
+    exact = torch.relu(q.double().cpu() @ comp.double().cpu().T)
+    assert got[0].cpu().double().equal(exact)
+
+
+def test_group_exponents_far_apart_round_in_float32():
+    """One head of weight one, so that a score is a dot product. Either form adds its 128 products in at most eight
+    instructions, each rounding its sum, at most the sum of magnitudes, to float32 (2^-23 allows a truncated sum)."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, comp = _lattice_rows(300, -13, 13, gen), _lattice_rows(500, -13, 13, gen)
+    got, f16 = _both(q.reshape(1, 1, 300, 128), torch.ones((1, 300, 1), device="cuda"), comp.reshape(1, 500, 128), 0, 0)
+    assert not got.equal(f16)                        # (the fp4 form did the work)
+    q, comp = q.double().cpu(), comp.double().cpu()
+    exact, size = torch.relu(q @ comp.T), q.abs() @ comp.abs().T
+    errors = [(x[0].cpu().double() - exact).abs() for x in (got, f16)]
+    assert all(bool((e <= 8 * 2.0 ** -23 * size).all()) for e in errors)
+    assert errors[0].norm() <= errors[1].norm()      # no less precise than the form it takes the place of
