@@ -25,7 +25,9 @@
 //    quarters of it; x 961 rows from position 0: 24 + 21 us (75); 517 tokens x 2053 rows: 7 + 14 us (46).
 //  * Where a value is outside that lattice (a pool row, or a query of the workgroup's tokens) the float16 form does the
 //    work, with pool tiles staged in LDS. It is a launch of its own behind the first, whose workgroups leave at once where
-//    nothing is left to do: in one kernel the two forms' registers held it to two waves per SIMD.
+//    nothing is left to do: in one kernel the two forms' registers held it to two waves per SIMD. What the first launch costs
+//    such operands: 3844 float32 tokens x 961 rows 68 us in the float16 form alone, 78 with it (97 when every row was
+//    packed before a block was found not exact); x 7961 rows 557 and 574 (602); 517 x 2053 rows 45 and 54 (58).
 #include "common.h"
 #include "profile.h"
 
@@ -128,53 +130,71 @@ __global__ __launch_bounds__(256) void pack_operands_kernel(const void* __restri
   const int64_t left = is_pool ? n_comp - x * kBlockRows : n_heads;
   const int n_rows = left < kBlockRows ? (int)left : kBlockRows;
   const int col = (tid & 31) * 4;  // 32 lanes a row: eight rows per pass of the workgroup
-  f32x4_t v[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
+  auto load = [&](int i) -> f32x4_t {
     const int r = 8 * i + (tid >> 5);
-    v[i] = r < n_rows ? load4_as_f32<DT>(src, (row0 + r * row_step) * 128 + col) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  bool exact = true;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
+    return r < n_rows ? load4_as_f32<DT>(src, (row0 + r * row_step) * 128 + col) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  auto pack = [&](int i, const f32x4_t& v) -> bool {
     const int r = 8 * i + (tid >> 5);
     uint32_t top = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const uint32_t a = __float_as_uint(v[i][j]) & 0x7FFFFFFFu;
+      const uint32_t a = __float_as_uint(v[j]) & 0x7FFFFFFFu;
       top = a > top ? a : top;
     }
     top = lane_xor_max<4>(lane_xor_max<2>(lane_xor_max<1>(top)));
     const int e = top == 0u ? 0 : (int)(top >> 23) - 127 - 2;
-    exact = exact && e >= -13 && e <= 13;
     const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
-    uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[i].x, v[i].y, scale, 0);
-    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v[i].z, v[i].w, scale, 1);
+    uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v.x, v.y, scale, 0);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v.z, v.w, scale, 1);
     const f32x2_t b0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0), b1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 1);
-    exact = exact && b0.x == v[i].x && b0.y == v[i].y && b1.x == v[i].z && b1.y == v[i].w;
     const int group = (tid & 31) >> 3, k = tid & 7;
     const int lane = (r & 31) + 32 * (group & 1), part = 2 * (r >> 5) + (group >> 1);
     codes[(part * 64 + lane) * 8 + k] = (uint16_t)c;
     if (k == 0) scales[lane * 4 + part] = (uint8_t)(e + 127);
-  }
-  const int all = __syncthreads_and(exact);
+    return e >= -13 && e <= 13 && b0.x == v.x && b0.y == v.y && b1.x == v.z && b1.y == v.w;
+  };
   const int64_t block = is_pool ? b * n_pool + x : b * n_tokens + x;
+  int32_t* flag = (is_pool ? out.pool_exact : out.q_exact) + block;
+  // The first eight rows decide whether the rest is read at all: values that did not come out of the QAT end here.
+  bool exact = pack(0, load(0));
+  if (!__syncthreads_and(exact)) {
+    if (tid == 0) *flag = 0;
+    return;
+  }
+  f32x4_t v[8];
+#pragma unroll
+  for (int i = 1; i < 8; i++) v[i] = load(i);
+#pragma unroll
+  for (int i = 1; i < 8; i++) exact = pack(i, v[i]) && exact;
+  const int all = __syncthreads_and(exact);
   uint8_t* cp = (is_pool ? out.pool_codes : out.q_codes) + block * kBlockCodeBytes;
   uint8_t* sp = (is_pool ? out.pool_scales : out.q_scales) + block * kBlockScaleBytes;
   reinterpret_cast<u32x4_t*>(cp)[tid] = reinterpret_cast<const u32x4_t*>(codes)[tid];
   if (tid < 64) reinterpret_cast<uint32_t*>(sp)[tid] = reinterpret_cast<const uint32_t*>(scales)[tid];
-  if (tid == 0) (is_pool ? out.pool_exact : out.q_exact)[block] = all;
+  if (tid == 0) *flag = all;
 }
 
-// Whether all operands of the workgroup (the whole pool of its batch entry, its four tokens) are exact; every thread calls it.
-__device__ __forceinline__ bool operands_exact(const PackedOperands& o, int n_tokens, int64_t n_comp) {
-  const int64_t n = pool_blocks(n_comp);
-  bool exact = true;
-  for (int64_t i = threadIdx.x; i < n; i += 256) exact = exact && o.pool_exact[blockIdx.z * n + i] != 0;
-  const int t = blockIdx.y * 4 + (threadIdx.x & 3);
-  if (t < n_tokens) exact = exact && o.q_exact[(int64_t)blockIdx.z * n_tokens + t] != 0;
-  return __syncthreads_and(exact);
-}
+// Whether all operands of the workgroup (the whole pool of its batch entry, its four tokens) are exact. Every thread makes
+// one and asks it once; the flags are requested in between, ahead of what the caller loads meanwhile.
+struct OperandsExact {
+  const int32_t* pool;
+  int64_t n;
+  int32_t pool_flag, q_flag;
+
+  __device__ __forceinline__ OperandsExact(const PackedOperands& o, int n_tokens, int64_t n_comp) {
+    n = pool_blocks(n_comp);
+    pool = o.pool_exact + blockIdx.z * n;
+    const int t = blockIdx.y * 4 + (threadIdx.x & 3);
+    pool_flag = pool[(int64_t)threadIdx.x < n ? threadIdx.x : 0];
+    q_flag = o.q_exact[(int64_t)blockIdx.z * n_tokens + (t < n_tokens ? t : n_tokens - 1)];
+  }
+  __device__ __forceinline__ bool all() const {
+    bool exact = pool_flag != 0 && q_flag != 0;
+    for (int64_t i = threadIdx.x + 256; i < n; i += 256) exact = exact && pool[i] != 0;
+    return __syncthreads_and(exact);
+  }
+};
 
 // max(x, 0) of a number that is no NaN, as one integer maximum (fmaxf costs a second instruction that quiets NaNs)
 __device__ __forceinline__ float relu_finite(float x) {
@@ -264,6 +284,7 @@ __global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restr
     j.mask_rest(0);
     return;
   }
+  const OperandsExact exact(ops, n_tokens, n_comp);  // (first, so that a workgroup without work waits for nothing else)
   const int n_pairs = (j.n_live + 1) / 2;
   const int64_t block0 = j.b * pool_blocks(n_comp) + j.row_begin / kBlockRows;
   const u32x4_t* cp = reinterpret_cast<const u32x4_t*>(ops.pool_codes + block0 * kBlockCodeBytes) + j.lane;
@@ -291,7 +312,7 @@ __global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restr
   const uint32_t qs = reinterpret_cast<const uint32_t*>(ops.q_scales + token * kBlockScaleBytes)[j.lane];
   float wv[2][16];
   j.head_weights(w, n_tokens, n_heads, wv);
-  if (!operands_exact(ops, n_tokens, n_comp)) return;
+  if (!exact.all()) return;
 
   float* out = j.out_row + j.row_begin + j.lane;
   int left = (int)(j.row_end - j.row_begin) - j.lane, seen = (int)(j.visible - j.row_begin) - j.lane;
@@ -354,7 +375,7 @@ __global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __rest
                                                            int rows_per_block, PackedOperands packed,
                                                            float* __restrict__ scores) {
   __shared__ __attribute__((aligned(16))) unsigned char tile_lds[2][32 * kTilePitch];
-  if (packed.pool_codes && operands_exact(packed, n_tokens, n_comp)) return;  // the fp4 form has done the work
+  if (packed.pool_codes && OperandsExact(packed, n_tokens, n_comp).all()) return;  // the fp4 form has done the work
   const ScoreJob j(n_tokens, n_comp, pos0, ratio, rows_per_block, scores);
   const int tid = threadIdx.x, n = j.n, g = j.g, b = j.b, t = j.t;
   const int n_live = j.n_live, n_fetch = j.n_fetch;

@@ -375,18 +375,20 @@ def banded_prefill_attention_live(q, raw_kv, comp_kv, topk, sinks, *, pos0: int,
     return _launch_live(q, raw_kv, comp_kv, topk, sinks, dims, pos0=pos0, window=window, ratio=ratio, raw_start=0)
 
 
-def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int = 4):
+def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int = 4, qat_operands: bool = True):
     """Ratio-4 indexer scores over a prefill chunk (reference :1888).
 
     Args:
         q: float32 or float16 ``[batch, n_heads, tokens, 128]`` QAT indexer queries (staged as half).
         weights: float32 ``[batch, tokens, n_heads]`` head weights including the DS4 scale factors.
         index_comp: ``[batch, n_comp, 128]`` QAT compressed index rows, same dtype as ``q``.
+        qat_operands: False for operands that did not come out of the QAT. Such are recognised and scored all the same;
+            said beforehand, it saves looking at them (a seventh of the call at 3844 tokens and 961 rows).
 
     Returns:
         float32 ``[batch, tokens, n_comp]``, ``-inf`` where the row is not yet visible to the token.
     """
-    scores = _lib.dispatch.indexer_scores_tiled_live(q, weights, index_comp, pos0, ratio)
+    scores = _lib.dispatch.indexer_scores_tiled_live(q, weights, index_comp, pos0, ratio) if qat_operands else None
     if scores is not None:
         _SCORES_TILED_CALL_COUNTS["f16" if q.dtype == torch.float16 else "f32"] += 1
         return scores
@@ -420,11 +422,13 @@ def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int =
     _SCORES_TILED_CALL_COUNTS[operand_form] += 1
     qc, wc, cc = q.contiguous(), weights.contiguous(), index_comp.contiguous()
     scores = torch.empty((batch, n_tokens, n_comp), dtype=torch.float32, device=dev)
-    nbytes = int(_lib.lib().mspr_indexer_scores_tiled_live_workspace_bytes(batch, n_heads, n_tokens, n_comp))
-    ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=dev)
+    ws, nbytes = None, 0
+    if qat_operands:
+        nbytes = int(_lib.lib().mspr_indexer_scores_tiled_live_workspace_bytes(batch, n_heads, n_tokens, n_comp))
+        ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=dev)
     rc = _lib.lib().mspr_indexer_scores_tiled_live_ws(
         _lib.ptr(qc), _lib.ptr(wc), _lib.ptr(cc), _lib.DTYPE_CODE[qc.dtype], batch, n_heads, n_tokens, n_comp,
-        int(pos0), int(ratio), _lib.ptr(scores), _lib.ptr(ws), ws.numel() * 4, _lib.stream_ptr())
+        int(pos0), int(ratio), _lib.ptr(scores), _lib.ptr(ws), nbytes, _lib.stream_ptr())
     _lib.check(rc, "indexer_scores_tiled_live")
     return scores
 

@@ -59,6 +59,23 @@ def test_operands_outside_the_format_take_the_float16_form(spoil):
     assert torch.equal(torch.nan_to_num(got, nan=12345.0), torch.nan_to_num(want, nan=12345.0))
 
 
+# (a block of 64 heads or pool rows is read on only if its first eight are of the format)
+@pytest.mark.parametrize("operand,row", [("query", 0), ("query", 7), ("query", 8), ("query", 63), ("pool", 64 + 7), ("pool", 64 + 8),
+                                         ("pool", 199), ("pool", 192)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_one_value_outside_the_format_anywhere_in_a_block(operand, row, dtype):
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+    q, w, comp = _operands(1, 64, 701, 200, dtype)
+    if operand == "query":
+        q[0, row, 633, 127] = 0.3
+    else:
+        comp[0, row, 127] = 0.3
+    got, want = _both(q, w, comp, 900)
+    assert got.equal(want)
+    assert iak.indexer_scores_tiled_live(q, w, comp, pos0=900, qat_operands=False).equal(want)
+
+
 def _lattice_rows(rows, low, high, gen):
     """[rows, 128] of e2m1 lattice values, each group of 32 times a power of two with an exponent in [low, high]."""
     v = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6], device="cuda")[torch.randint(0, 8, (rows, 128), device="cuda", generator=gen)]
