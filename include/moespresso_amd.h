@@ -130,7 +130,7 @@ int mspr_indexer_scores_tiled_live(const void* q, const float* weights, const vo
                                    int ratio, float* scores, void* stream);
 /* The same with scratch of mspr_indexer_scores_tiled_live_workspace_bytes (16-byte aligned; NULL = none): the pool is
  * packed into it as fp4 groups, and tokens whose operands are exact in that format (what the indexer's QAT produces) are
- * multiplied in it. Products are exact; scores are the same bit for bit where the exponents of a dot product's group
+ * multiplied in it where there are enough scores for that to pay. Products are exact; scores are the same bit for bit where the exponents of a dot product's group
  * products lie within 9 of each other, else they differ by the float32 rounding of its sum. */
 size_t mspr_indexer_scores_tiled_live_workspace_bytes(int batch, int n_heads, int n_tokens, int64_t n_comp);
 int mspr_indexer_scores_tiled_live_ws(const void* q, const float* weights, const void* index_comp, int dtype,

@@ -487,7 +487,11 @@ extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* wei
   hipStream_t st = (hipStream_t)stream;
   dim3 block(256);
   PackedOperands packed = {};
-  if (workspace) {
+  // The fp4 form is two launches more, some 5 us, which cheaper products have to earn. It does so from 2^17 scores on with
+  // float32 operands, which the float16 form rounds as it loads them (us without and with it: 64 tokens x 2000 rows 12.1 and
+  // 12.9, 128 x 1000 12.4 and 13.0, 96 x 2000 17.5 and 13.6, 17 x 8000 16.7 and 14.1, 517 x 500 22.6 and 15.1), and from 450
+  // thousand with float16 ones (384 x 1000 14.2 and 14.8, 128 x 4000 15.1 and 15.1, 517 x 1000 19.0 and 17.5).
+  if (workspace && (int64_t)batch * n_tokens * n_comp >= (dtype == MSPR_F32 ? 1 << 17 : 450000)) {
     packed = packed_operands(workspace, batch, n_tokens, n_comp);
     const int64_t blocks = pool_blocks(n_comp) + n_tokens;
     MSPR_REQUIRE(blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && n_comp < ((int64_t)1 << 31),

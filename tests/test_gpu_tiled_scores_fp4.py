@@ -42,6 +42,20 @@ def test_qat_operands_give_the_float16_form_bit_for_bit(dtype, batch, heads, tok
     assert ratio != 0 or bool(torch.isfinite(got).all())
 
 
+# Enough scores for the fp4 form (2^17 of float32 operands, 450 thousand of float16 ones), and the last numbers below them:
+# ragged blocks of rows, tokens and heads, several sequences, the whole pool visible.
+@pytest.mark.parametrize("dtype,batch,heads,tokens,rows,pos0,ratio", [
+    (torch.float32, 1, 64, 4097, 33, 0, 4), (torch.float32, 2, 64, 1025, 64, 60, 4), (torch.float32, 1, 40, 1031, 130, 512, 4),
+    (torch.float32, 3, 64, 46, 1000, 3800, 4), (torch.float32, 1, 1, 45, 3001, 11980, 4), (torch.float32, 1, 64, 6, 22011, 0, 0),
+    (torch.float32, 1, 64, 2, 65535, 0, 0), (torch.float32, 1, 64, 2, 65536, 0, 0),
+    (torch.float16, 1, 64, 4097, 129, 0, 4), (torch.float16, 2, 64, 1001, 255, 60, 4), (torch.float16, 1, 40, 3511, 130, 512, 4),
+    (torch.float16, 3, 64, 150, 1024, 3800, 4), (torch.float16, 1, 1, 151, 2999, 11900, 4), (torch.float16, 1, 64, 22, 22011, 0, 0),
+    (torch.float16, 1, 64, 18, 24999, 0, 0), (torch.float16, 1, 64, 18, 25000, 0, 0)])
+def test_both_forms_agree_where_the_fp4_form_is_taken(dtype, batch, heads, tokens, rows, pos0, ratio):
+    got, want = _both(*_operands(batch, heads, tokens, rows, dtype), pos0, ratio)
+    assert got.equal(want)
+
+
 @pytest.mark.parametrize("spoil", ["query", "pool", "tiny", "huge", "nan"])
 def test_operands_outside_the_format_take_the_float16_form(spoil):
     q, w, comp = _operands(1, 64, 13, 200, torch.float32)
@@ -66,7 +80,7 @@ def test_operands_outside_the_format_take_the_float16_form(spoil):
 def test_one_value_outside_the_format_anywhere_in_a_block(operand, row, dtype):
     from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
 
-    q, w, comp = _operands(1, 64, 701, 200, dtype)
+    q, w, comp = _operands(1, 64, 2301, 200, dtype)
     if operand == "query":
         q[0, row, 633, 127] = 0.3
     else:
@@ -74,6 +88,19 @@ def test_one_value_outside_the_format_anywhere_in_a_block(operand, row, dtype):
     got, want = _both(q, w, comp, 900)
     assert got.equal(want)
     assert iak.indexer_scores_tiled_live(q, w, comp, pos0=900, qat_operands=False).equal(want)
+
+
+@pytest.mark.parametrize("spoil", ["tiny", "huge", "nan"])
+def test_groups_outside_the_scales_and_nan_among_many_scores(spoil):
+    q, w, comp = _operands(1, 64, 701, 200, torch.float32)
+    if spoil == "tiny":
+        comp[0, 64, :32] *= 2.0 ** -20
+    elif spoil == "huge":
+        q[0, :, 2, 32:64] *= 2.0 ** 13
+    else:
+        comp[0, 103, 3] = float("nan")
+    got, want = _both(q, w, comp, 900)
+    assert torch.equal(torch.nan_to_num(got, nan=12345.0), torch.nan_to_num(want, nan=12345.0))
 
 
 def _lattice_rows(rows, low, high, gen):
@@ -88,8 +115,8 @@ def _lattice_rows(rows, low, high, gen):
 @pytest.mark.parametrize("q_exp,comp_exp", [((0, 5), (-4, 0)), ((-13, -8), (9, 13))])
 def test_group_exponents_within_nine_give_exact_sums(q_exp, comp_exp):
     gen = torch.Generator(device="cuda").manual_seed(4)
-    q, comp = _lattice_rows(70, *q_exp, gen), _lattice_rows(300, *comp_exp, gen)
-    got, want = _both(q.reshape(1, 1, 70, 128), torch.ones((1, 70, 1), device="cuda"), comp.reshape(1, 300, 128), 0, 0)
+    q, comp = _lattice_rows(470, *q_exp, gen), _lattice_rows(300, *comp_exp, gen)
+    got, want = _both(q.reshape(1, 1, 470, 128), torch.ones((1, 470, 1), device="cuda"), comp.reshape(1, 300, 128), 0, 0)
     assert got.equal(want)
     exact = torch.relu(q.double().cpu() @ comp.double().cpu().T)
     assert got[0].cpu().double().equal(exact)
