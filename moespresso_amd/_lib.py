@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 import torch
@@ -20,17 +21,35 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmoespres
 DISPATCH_PATH = os.path.join(os.path.dirname(LIB_PATH), "_dispatch.so")
 
 
-class _NotBuilt:
-    """Stands where the native call path would: every operator goes on to ``lib()``, which says what is missing."""
+class _NoNativePath:
+    """Stands where the native call path would: every operator goes on in Python."""
 
     def __getattr__(self, name):
         return lambda *args: None
 
 
-if os.path.exists(DISPATCH_PATH):
-    from moespresso_amd import _dispatch as dispatch
-else:
-    dispatch = _NotBuilt()
+def _load_dispatch():
+    """The native call path. It is compiled against torch's own C++ interface, so it is used only with the torch of its
+    build; the library itself needs none, and without the native path the operators call it from Python."""
+    if not os.path.exists(DISPATCH_PATH):
+        why = f"{DISPATCH_PATH} is missing"
+        if not os.path.exists(LIB_PATH):  # nothing is built: lib() says so
+            return _NoNativePath()
+    else:
+        try:
+            from moespresso_amd import _dispatch
+        except ImportError as e:
+            why = f"it cannot be loaded ({e})"
+        else:
+            if _dispatch.torch_version == torch.__version__:
+                return _dispatch
+            why = f"it was built for torch {_dispatch.torch_version}, this is {torch.__version__}"
+    warnings.warn(f"operators are called without the native call path: {why}; `python -m moespresso_amd.build` builds it",
+                  RuntimeWarning, stacklevel=2)
+    return _NoNativePath()
+
+
+dispatch = _load_dispatch()
 
 MSPR_OK = 0
 MSPR_ERR_ARG = -1
@@ -159,8 +178,8 @@ _LIB = None
 
 
 def library_available() -> bool:
-    """True when the shared library and its native call path exist on disk (the library is not loaded here)."""
-    return os.path.exists(LIB_PATH) and os.path.exists(DISPATCH_PATH)
+    """True when the shared library exists on disk (it is not loaded here)."""
+    return os.path.exists(LIB_PATH)
 
 
 def lib() -> ctypes.CDLL:
@@ -169,7 +188,7 @@ def lib() -> ctypes.CDLL:
     if _LIB is None:
         if not library_available():
             raise RuntimeError(
-                f"{LIB_PATH} or {DISPATCH_PATH} is missing: build it with `python -m moespresso_amd.build` "
+                f"{LIB_PATH} is missing: build it with `python -m moespresso_amd.build` "
                 "(there is no CPU or PyTorch fallback for these operators)")
         handle = ctypes.CDLL(LIB_PATH)
         for name, (restype, argtypes) in SIGNATURES.items():

@@ -658,4 +658,11 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dispatch", "Native call path of 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__dispatch(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__dispatch(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "torch_version", MSPR_TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

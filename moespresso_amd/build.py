@@ -64,7 +64,7 @@ def _compile_dispatch() -> str:
 
     obj = os.path.join(OBJ_DIR, "dispatch.o")
     cmd = [HIPCC, "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DMSPR_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-I{p}" for p in cpp_extension.include_paths("cuda")), f"-I{sysconfig.get_paths()['include']}",
            "-w", "-c", DISPATCH_SRC, "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
