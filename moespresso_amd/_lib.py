@@ -2,7 +2,7 @@
 
 ``dispatch`` is the native call path (``_dispatch.so``): an operator asks it first, with its arguments by position,
 and goes on in Python (checks, conversions, error messages, the ctypes call) only when it answers ``None``, which is
-what it does for anything but dense operands of the plain types on one HIP device.
+what it does for anything but dense operands of the plain types on the current HIP device.
 
 The library is loaded lazily and only from this package directory. There is no
 fallback: a missing library or a tensor that is not on a HIP device raises.
@@ -235,6 +235,14 @@ def ptr(t: torch.Tensor | None) -> c_void_p:
     if t is None:
         return c_void_p(0)
     return c_void_p(t.data_ptr())
+
+
+def launch(dev: torch.device, entry: str, *args) -> int:
+    """One entry point of the library on the current stream of ``dev``, the device of its operands."""
+    if dev.index == torch.cuda.current_device():
+        return getattr(lib(), entry)(*args, stream_ptr())
+    with torch.cuda.device(dev):
+        return getattr(lib(), entry)(*args, stream_ptr())
 
 
 def stream_ptr() -> c_void_p:

@@ -3,7 +3,7 @@
 // At batch 1 a decode layer is a handful of kernels of 4 to 12 us, and a call made in Python (shape checks, two
 // allocations, twenty converted arguments) costs the host as much as its kernels cost the device: three such calls of
 // the DS4 decode layer took 42 us of host time against 30 us of kernels. Each function here takes the arguments of one
-// Python operator by position, checks the plain case (types, shapes, dense layout, one device) and makes the call.
+// Python operator by position, checks the plain case (types, shapes, dense layout, the current device) and makes the call.
 // Whatever is not that case (another layout, a type to convert, a mistake) makes it return None, and the Python operator
 // goes through its own checks, conversions and messages; so nothing is rejected or converted here.
 //
@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -42,11 +43,17 @@ const Tensor* dense(PyObject* o, int64_t ndim, at::ScalarType type) {
   return t && t->scalar_type() == type ? t : nullptr;
 }
 
-bool same_device(std::initializer_list<const Tensor*> ts) {
+// Launches go to the current device's stream: operands of another one are the Python path's, which changes devices.
+bool here(const Tensor& t) {
+  c10::DeviceIndex current;
+  return t.is_cuda() && c10::hip::GetDevice(&current) == hipSuccess && t.get_device() == current;
+}
+
+bool here(std::initializer_list<const Tensor*> ts) {
   const Tensor* first = *ts.begin();
   for (const Tensor* t : ts)
     if (t->get_device() != first->get_device()) return false;
-  return true;
+  return here(*first);
 }
 
 // Whole numbers and real numbers that are Python's own; anything else (NumPy scalars, tensors) is the Python path's.
@@ -145,7 +152,7 @@ PyObject* qat_rows(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(1)
   if (!THPVariable_Check(a[0])) return none();
   const Tensor& x = THPVariable_Unpack(a[0]);
-  if (!x.is_cuda() || x.dim() < 1 || x.size(-1) != 128 || x.numel() == 0 || !x.is_contiguous()) return none();
+  if (!here(x) || x.dim() < 1 || x.size(-1) != 128 || x.numel() == 0 || !x.is_contiguous()) return none();
   const int code = type_code(x.scalar_type());
   if (code == kNoType || (LIVE && (code != MSPR_F32 || x.dim() != 4))) return none();
   Tensor out = empty(x.sizes(), at::kFloat, x);
@@ -163,7 +170,7 @@ PyObject* topk_select(PyObject* const* a, Py_ssize_t nargs) {
   int64_t k;
   if (!THPVariable_Check(a[0]) || !whole(a[1], &k)) return none();
   const Tensor& s = THPVariable_Unpack(a[0]);
-  if (!s.is_cuda() || s.dim() < 1 || s.scalar_type() != at::kFloat || !s.is_contiguous()) return none();
+  if (!here(s) || s.dim() < 1 || s.scalar_type() != at::kFloat || !s.is_contiguous()) return none();
   const int64_t n = s.size(-1);
   if (k < 1 || k > n || s.numel() == 0) return none();
   at::DimVector shape(s.sizes());
@@ -180,7 +187,7 @@ PyObject* indexer_scores_fp8(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(4)
   const Tensor *q = dense(a[0], 3, at::kBFloat16), *keys = dense(a[1], 3), *ks = dense(a[2], 2, at::kFloat),
                *w = dense(a[3], 2, at::kFloat);
-  if (!q || !keys || !ks || !w || !same_device({q, keys, ks, w})) return none();
+  if (!q || !keys || !ks || !w || !here({q, keys, ks, w})) return none();
   if (keys->scalar_type() != at::kFloat8_e4m3fn && keys->scalar_type() != at::kByte) return none();
   const int64_t B = q->size(0), H = q->size(1), N = keys->size(1);
   if (B < 1 || H < 1 || H > 64 || N < 1 || q->size(2) != 128 || keys->size(0) != B || keys->size(2) != 128 ||
@@ -199,7 +206,7 @@ PyObject* fused_qat_indexer_scores(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(4)
   const Tensor *q = dense(a[0], 4), *p = dense(a[1], 3, at::kFloat), *w = dense(a[2], 3, at::kFloat);
   float scale;
-  if (!q || !p || !w || !real(a[3], &scale) || !same_device({q, p, w})) return none();
+  if (!q || !p || !w || !real(a[3], &scale) || !here({q, p, w})) return none();
   const int code = type_code(q->scalar_type());
   const int64_t H = q->size(1), N = p->size(1);
   if (code == kNoType || q->size(0) != 1 || q->size(2) != 1 || q->size(3) != 128 || H < 1 || H > 64 || p->size(0) != 1 ||
@@ -218,7 +225,7 @@ PyObject* indexer_scores_tiled_live(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(5)
   const Tensor *q = dense(a[0], 4), *w = dense(a[1], 3, at::kFloat), *c = dense(a[2], 3);
   int pos0, ratio;
-  if (!q || !w || !c || !whole32(a[3], &pos0) || !whole32(a[4], &ratio) || !same_device({q, w, c})) return none();
+  if (!q || !w || !c || !whole32(a[3], &pos0) || !whole32(a[4], &ratio) || !here({q, w, c})) return none();
   const int code = type_code(q->scalar_type());
   const int64_t B = q->size(0), H = q->size(1), T = q->size(2), P = c->size(1);
   if ((code != MSPR_F32 && code != MSPR_F16) || c->scalar_type() != q->scalar_type() || q->size(3) != 128 ||
@@ -246,7 +253,7 @@ PyObject* fused_partial_rope(PyObject* const* a, Py_ssize_t nargs) {
       !whole(a[5], &max_rows))
     return none();
   const Tensor& x = THPVariable_Unpack(a[0]);
-  if (!x.is_cuda() || x.dim() < 2 || !x.is_contiguous() || !same_device({&x, inv})) return none();
+  if (!x.is_cuda() || x.dim() < 2 || !x.is_contiguous() || !here({&x, inv})) return none();
   const int code = type_code(x.scalar_type());
   const int64_t W = x.size(-1), T = x.size(-2);
   if (code == kNoType || W < 64 || W % 4 != 0 || x.numel() == 0) return none();
@@ -256,7 +263,7 @@ PyObject* fused_partial_rope(PyObject* const* a, Py_ssize_t nargs) {
   } else {
     if (!THPVariable_Check(a[4])) return none();
     const Tensor& p = THPVariable_Unpack(a[4]);
-    if (!p.is_cuda() || !p.is_contiguous() || p.scalar_type() != at::kFloat || p.numel() != T || !same_device({&x, &p}))
+    if (!p.is_cuda() || !p.is_contiguous() || p.scalar_type() != at::kFloat || p.numel() != T || !here({&x, &p}))
       return none();
     positions = (const float*)p.const_data_ptr();
     offset = 0;
@@ -281,7 +288,7 @@ PyObject* fused_decode_prep(PyObject* const* a, Py_ssize_t nargs) {
   float scale;
   int64_t topk;
   if (!q || !p || !w || !kv || !inv || !prm || !real(a[6], &scale) || !whole(a[7], &topk) || !PyBool_Check(a[8]) ||
-      !same_device({q, p, w, kv, inv, prm}))
+      !here({q, p, w, kv, inv, prm}))
     return none();
   const bool fixed = a[8] == Py_True;
   const int code = type_code(q->scalar_type());
@@ -308,7 +315,7 @@ PyObject* fused_decode_sdpa(PyObject* const* a, Py_ssize_t nargs) {
                *inv = dense(a[6], 1, at::kFloat), *prm = dense(a[7], 1, at::kInt);
   float scale;
   if (!q || !win || !row || !pool || !sel || !sinks || !inv || !prm || !real(a[8], &scale) || !PyBool_Check(a[9]) ||
-      !same_device({q, win, row, pool, sel, sinks, inv, prm}))
+      !here({q, win, row, pool, sel, sinks, inv, prm}))
     return none();
   const bool fixed = a[9] == Py_True;
   const int64_t H = q->size(0), W = win->size(0), N = pool->size(0), K = sel->size(0);
@@ -336,13 +343,13 @@ PyObject* sparse_mla_decode(PyObject* const* a, Py_ssize_t nargs) {
   int v_dim, win_rows, row_mul, row_add;
   int64_t win_start = 0;
   if (!q || !kv || !rows || !real(a[3], &scale) || !whole32(a[4], &v_dim) || !whole32(a[6], &win_rows) ||
-      !whole32(a[9], &row_mul) || !whole32(a[10], &row_add) || !same_device({q, kv, rows}))
+      !whole32(a[9], &row_mul) || !whole32(a[10], &row_add) || !here({q, kv, rows}))
     return none();
   if (a[5] != Py_None && !whole(a[5], &win_start)) return none();
   const int64_t B = q->size(0), H = q->size(1), D = q->size(2), P = kv->size(1), K = rows->size(1);
   if (a[7] != Py_None) {
     sinks = dense(a[7], 1, at::kFloat);
-    if (!sinks || sinks->size(0) != H || !same_device({q, sinks})) return none();
+    if (!sinks || sinks->size(0) != H || !here({q, sinks})) return none();
   }
   if ((q->scalar_type() != at::kHalf && q->scalar_type() != at::kBFloat16) || kv->scalar_type() != q->scalar_type() ||
       B < 1 || B > 65535 || H < 1 || H > 128 || (D != 512 && D != 576) || v_dim != 512 || kv->size(0) != B ||
@@ -369,7 +376,7 @@ PyObject* prefill_live(PyObject* const* a, Py_ssize_t nargs) {
                *topk = dense(a[3], 3, at::kInt), *sinks = dense(a[4], 1, at::kFloat);
   int pos0, window, ratio, raw_start;
   if (!q || !raw || !comp || !topk || !sinks || !whole32(a[5], &pos0) || !whole32(a[6], &window) ||
-      !whole32(a[7], &ratio) || !whole32(a[8], &raw_start) || !same_device({q, raw, comp, topk, sinks}))
+      !whole32(a[7], &ratio) || !whole32(a[8], &raw_start) || !here({q, raw, comp, topk, sinks}))
     return none();
   const int code = type_code(q->scalar_type());
   const int64_t B = q->size(0), H = q->size(1), T = q->size(2), R = raw->size(2), P = comp->size(1), K = topk->size(2);
@@ -397,7 +404,7 @@ PyObject* quantize(PyObject* const* a, Py_ssize_t nargs) {
   MSPR_NARGS(1)
   if (!THPVariable_Check(a[0])) return none();
   const Tensor& x = THPVariable_Unpack(a[0]);
-  if (!x.is_cuda() || x.dim() < 1 || x.numel() == 0 || !x.is_contiguous() || x.size(-1) % 64 != 0) return none();
+  if (!here(x) || x.dim() < 1 || x.numel() == 0 || !x.is_contiguous() || x.size(-1) % 64 != 0) return none();
   const int code = type_code(x.scalar_type());
   if (code == kNoType) return none();
   at::DimVector shape(x.sizes());
@@ -422,7 +429,7 @@ PyObject* dequantize(PyObject* const* a, Py_ssize_t nargs) {
     return none();
   const int code = type_code(s.scalar_type());
   if (code == kNoType || b.scalar_type() != s.scalar_type() || w.numel() == 0 || w.dim() < 1 || w.dim() != s.dim() ||
-      s.sizes() != b.sizes() || (w.scalar_type() != at::kUInt32 && w.scalar_type() != at::kInt) || !same_device({&w, &s, &b}))
+      s.sizes() != b.sizes() || (w.scalar_type() != at::kUInt32 && w.scalar_type() != at::kInt) || !here({&w, &s, &b}))
     return none();
   at::DimVector shape(w.sizes());
   for (int64_t d = 0; d + 1 < w.dim(); d++)
@@ -477,7 +484,7 @@ bool affine_cache(PyObject* const* a, const Tensor* (&t)[6], int64_t B, int64_t*
               : t[i]->scalar_type() != t[1]->scalar_type())
       return false;
   }
-  if (!same_device({t[0], t[1], t[2], t[3], t[4], t[5]})) return false;
+  if (!here({t[0], t[1], t[2], t[3], t[4], t[5]})) return false;
   *cap = common_row_capacity({t[0], t[1], t[2], t[3], t[4], t[5]});
   return *cap >= *N;
 }
@@ -514,7 +521,7 @@ PyObject* q8_append(PyObject* const* a, Py_ssize_t nargs) {
   const int code = type_code(k->scalar_type());
   const int64_t B = k->size(0), H = k->size(1), L = k->size(2), D = k->size(3), cap = ks[0]->size(2);
   if (code == kNoType || v->scalar_type() != k->scalar_type() || k->sizes() != v->sizes() || k->numel() == 0 || D % 64 != 0 ||
-      D > 4096 || B * H > 65535 || offset < 0 || offset + L > cap || !same_device({k, v, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2]}))
+      D > 4096 || B * H > 65535 || offset < 0 || offset + L > cap || !here({k, v, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2]}))
     return none();
   for (const auto& half : side)
     for (int i = 0; i < 3; i++) {
@@ -560,7 +567,7 @@ PyObject* sdpa_decode_q8(PyObject* const* a, Py_ssize_t nargs) {
   int64_t Hkv, N, cap;
   int sb;
   if (!affine_cache(a + 1, t, B, &Hkv, &N, &sb, &cap) || N < 1 || B < 1 || B > 65535 || Hq < 1 || Hq % Hkv != 0 ||
-      Hq / Hkv > 16 || !same_device({q, t[0]}))
+      Hq / Hkv > 16 || !here({q, t[0]}))
     return none();
   Tensor ws;
   if (!take_workspace(a[8], mspr_sdpa_decode_q8_workspace_bytes((int)B, (int)Hkv, N), *q, &ws)) return none();
@@ -580,7 +587,7 @@ PyObject* sdpa_decode_q8_0(PyObject* const* a, Py_ssize_t nargs) {
   const Tensor *q = dense(a[0], 3), *kc = cache_part(a[1]), *ks = cache_part(a[2]), *vc = cache_part(a[3]),
                *vs = cache_part(a[4]);
   float scale;
-  if (!q || !kc || !ks || !vc || !vs || !real(a[5], &scale) || !same_device({q, kc, ks, vc, vs})) return none();
+  if (!q || !kc || !ks || !vc || !vs || !real(a[5], &scale) || !here({q, kc, ks, vc, vs})) return none();
   const int code = type_code(q->scalar_type());
   const int64_t B = q->size(0), Hq = q->size(1), Hkv = kc->size(1), N = kc->size(2);
   if (code == kNoType || q->size(2) != 256 || B < 1 || B > 65535 || Hkv < 1 || Hq < 1 || Hq % Hkv != 0 || Hq / Hkv > 16 ||
@@ -613,7 +620,7 @@ PyObject* sdpa_fa_prefill_q8(PyObject* const* a, Py_ssize_t nargs) {
   const int self_code = type_code(sk->scalar_type());
   if (!affine_cache(a + 1, t, B, &Hkv, &P, &sb, &cap) || self_code == kNoType || sv->scalar_type() != sk->scalar_type() ||
       sk->sizes() != sv->sizes() || sk->size(0) != B || sk->size(1) != Hkv || sk->size(2) != L || sk->size(3) != 256 ||
-      B < 1 || L < 1 || L > 0x7FFFFFFF || Hq < 1 || Hq > 4096 || !same_device({q, t[0], sk, sv}))
+      B < 1 || L < 1 || L > 0x7FFFFFFF || Hq < 1 || Hq > 4096 || !here({q, t[0], sk, sv}))
     return none();
   const int64_t rep = Hq / Hkv;
   if (Hq % Hkv != 0 || (rep != 1 && rep != 2 && rep != 4 && rep != 8)) return none();

@@ -121,7 +121,7 @@ def fused_partial_rope(x, inv_freq, *, offset=0, inverse=False, positions=None):
         return out
     if not partial_rope_eligible(x, inv_freq, offset=offset, positions=positions):
         raise ValueError("operands are outside the fused partial-rope contract")
-    _lib.require_device(x, inv_freq, positions)
+    dev = _lib.require_device(x, inv_freq, positions)
     width = int(x.shape[-1])
     seq_len = int(x.shape[-2])
     rows = x.numel() // width
@@ -130,9 +130,9 @@ def fused_partial_rope(x, inv_freq, *, offset=0, inverse=False, positions=None):
     inv = inv_freq.contiguous()
     pos = None if positions is None else positions.reshape(seq_len).contiguous()
     dtype_code = _lib.DTYPE_CODE[x.dtype]
-    rc = _lib.lib().mspr_fused_partial_rope(_lib.ptr(xc), dtype_code, rows // seq_len, seq_len, width, _lib.ptr(inv),
-                                            _lib.ptr(pos), 0 if positions is not None else int(offset),
-                                            1 if inverse else 0, _lib.ptr(out), _lib.stream_ptr())
+    rc = _lib.launch(dev, "mspr_fused_partial_rope", _lib.ptr(xc), dtype_code, rows // seq_len, seq_len, width,
+                     _lib.ptr(inv), _lib.ptr(pos), 0 if positions is not None else int(offset),
+                     1 if inverse else 0, _lib.ptr(out))
     _lib.check(rc, "fused_partial_rope")
     _note_rope_launch("off" if positions is None else "pos", inverse)
     return out.reshape(x.shape)

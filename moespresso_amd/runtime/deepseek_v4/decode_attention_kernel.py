@@ -57,10 +57,10 @@ def fp8_kv_prefix_rows(x: torch.Tensor) -> torch.Tensor:
     n_rows = x.numel() // _HEAD_DIM
     if n_rows == 0:
         raise ValueError("fp8 rows expect at least one row")
-    _lib.require_device(x)
+    dev = _lib.require_device(x)
     rows2d = x.reshape(-1, _HEAD_DIM).contiguous()
     out = torch.empty_like(rows2d)
-    rc = _lib.lib().mspr_fp8_kv_prefix_rows(_lib.ptr(rows2d), n_rows, _lib.ptr(out), _lib.stream_ptr())
+    rc = _lib.launch(dev, "mspr_fp8_kv_prefix_rows", _lib.ptr(rows2d), n_rows, _lib.ptr(out))
     _lib.check(rc, "fp8_kv_prefix_rows")
     return out.reshape(x.shape)
 
@@ -130,11 +130,12 @@ def fused_decode_prep(q_idx, pooled_qat, weights, kv_row, inv_freq, params, *, s
     sel = torch.empty((topk,), dtype=torch.int32, device=dev)
     row = torch.empty((_HEAD_DIM,), dtype=torch.float16, device=dev)
     scores = torch.empty((n_rows,), dtype=torch.float32, device=dev)
-    entry = _lib.lib().mspr_fused_decode_prep_fixed if pool_rows_in_params else _lib.lib().mspr_fused_decode_prep
-    rc = entry(
+    entry = "mspr_fused_decode_prep_fixed" if pool_rows_in_params else "mspr_fused_decode_prep"
+    rc = _lib.launch(
+        dev, entry,
         _lib.ptr(qc), _lib.DTYPE_CODE[q_idx.dtype], n_heads, _lib.ptr(pc), n_rows, _lib.ptr(wc),
         _lib.ptr(kc), _lib.ptr(fc), _lib.ptr(prm), float(scale), topk, _lib.ptr(sel), _lib.ptr(row),
-        _lib.ptr(scores), _lib.stream_ptr())
+        _lib.ptr(scores))
     _lib.check(rc, "fused_decode_prep")
     return sel, row, scores
 
@@ -194,11 +195,12 @@ def fused_decode_sdpa(q, window, row, pooled, sel, sinks, inv_freq, params, *, s
     sc, kc, fc, prm = sel.contiguous(), sinks.contiguous(), inv_freq.reshape(-1).contiguous(), params.reshape(-1).contiguous()
     out = torch.empty((n_heads, _HEAD_DIM), dtype=torch.float16, device=dev)
     ws = workspace if workspace is not None else _lib.sparse_attention_workspace(1, n_heads, window_rows + n_sel, dev)
-    entry = _lib.lib().mspr_fused_decode_sdpa_fixed if pool_rows_in_params else _lib.lib().mspr_fused_decode_sdpa
-    rc = entry(
+    entry = "mspr_fused_decode_sdpa_fixed" if pool_rows_in_params else "mspr_fused_decode_sdpa"
+    rc = _lib.launch(
+        dev, entry,
         _lib.ptr(qc), n_heads, _lib.ptr(wc), window_rows, _lib.ptr(rc_), _lib.ptr(pc), n_rows, _lib.ptr(sc),
         n_sel, _lib.ptr(kc), _lib.ptr(fc), _lib.ptr(prm), float(scale), _lib.ptr(out), _lib.ptr(ws),
-        ws.numel() * 4, _lib.stream_ptr())
+        ws.numel() * 4)
     _lib.check(rc, "fused_decode_sdpa")
     return out
 

@@ -109,10 +109,11 @@ def indexed_mixed_attention_decode(q, raw_kv, comp_kv, topk, sinks, *, pos0: int
     qc, rc_, cc, tc, sc = (t.contiguous() for t in (q, raw_kv, comp_kv, topk, sinks))
     out = torch.empty((n_heads, head_dim), dtype=torch.float32, device=dev)
     ws = _lib.sparse_attention_workspace(1, n_heads, raw_cap + top_k, dev)
-    rc = _lib.lib().mspr_indexed_mixed_attention_decode(
+    rc = _lib.launch(
+        dev, "mspr_indexed_mixed_attention_decode",
         _lib.ptr(qc), n_heads, _lib.ptr(rc_), raw_cap, _lib.ptr(cc), n_comp, _lib.ptr(tc), top_k,
         _lib.ptr(sc), int(pos0), int(window), int(ratio), int(raw_start), _lib.ptr(out), _lib.ptr(ws),
-        ws.numel() * 4, _lib.stream_ptr())
+        ws.numel() * 4)
     _lib.check(rc, "indexed_mixed_attention_decode")
     return out
 
@@ -178,10 +179,11 @@ def sparse_mla_decode(q, kv, rows, *, scale: float, v_dim: int = 512, window_sta
     qc, kc, rc_ = q.contiguous(), kv.contiguous(), rows.contiguous()
     out = torch.empty((batch, n_heads, 512), dtype=q.dtype, device=dev)
     ws = workspace if workspace is not None else _lib.sparse_attention_workspace(batch, n_heads, n_rows + window_rows, dev)
-    rc = _lib.lib().mspr_sparse_mla_decode(
+    rc = _lib.launch(
+        dev, "mspr_sparse_mla_decode",
         _lib.ptr(qc), _lib.ptr(kc), _lib.ptr(rc_), _lib.ptr(sinks), _lib.DTYPE_CODE[q.dtype], batch, n_heads,
         k_dim, 512, n_pool, n_rows, int(row_mul), int(row_add), win_start, window_rows, float(scale), _lib.ptr(out), _lib.ptr(ws),
-        ws.numel() * 4, _lib.stream_ptr())
+        ws.numel() * 4)
     _lib.check(rc, "sparse_mla_decode")
     return out
 
@@ -195,11 +197,12 @@ def _run_prefill(q, raw_kv, comp_kv, topk, sinks, *, batch, n_heads, n_tokens, s
     out = torch.empty(q.shape, dtype=torch.float32, device=dev)
     max_win = min(int(window), raw_cap) if int(window) != 0 else raw_cap
     ws = _lib.prefill_attention_workspace(q.dtype, batch, n_heads, n_tokens, max_win, top_k, dev)
-    rc = _lib.lib().mspr_indexed_mixed_attention_prefill(
+    rc = _lib.launch(
+        dev, "mspr_indexed_mixed_attention_prefill",
         _lib.ptr(q), _lib.DTYPE_CODE[q.dtype], batch, n_heads, n_tokens, strides[0], strides[1], strides[2],
         _lib.ptr(raw_kv), raw_cap, _lib.ptr(comp_kv), n_comp, _lib.ptr(topk) if top_k else None, top_k,
         _lib.ptr(sinks), int(pos0), int(window), int(ratio), int(raw_start), _lib.ptr(out), _lib.ptr(ws),
-        ws.numel() * 4, _lib.stream_ptr())
+        ws.numel() * 4)
     _lib.check(rc, "indexed_mixed_attention_prefill")
     return out
 
@@ -426,9 +429,10 @@ def indexer_scores_tiled_live(q, weights, index_comp, *, pos0: int, ratio: int =
     if qat_operands:
         nbytes = int(_lib.lib().mspr_indexer_scores_tiled_live_workspace_bytes(batch, n_heads, n_tokens, n_comp))
         ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=dev)
-    rc = _lib.lib().mspr_indexer_scores_tiled_live_ws(
+    rc = _lib.launch(
+        dev, "mspr_indexer_scores_tiled_live_ws",
         _lib.ptr(qc), _lib.ptr(wc), _lib.ptr(cc), _lib.DTYPE_CODE[qc.dtype], batch, n_heads, n_tokens, n_comp,
-        int(pos0), int(ratio), _lib.ptr(scores), _lib.ptr(ws), nbytes, _lib.stream_ptr())
+        int(pos0), int(ratio), _lib.ptr(scores), _lib.ptr(ws), nbytes)
     _lib.check(rc, "indexer_scores_tiled_live")
     return scores
 
@@ -450,8 +454,7 @@ def indexer_q_qat_live(q):
     dev = _lib.require_device(q)
     qc = q.contiguous()
     out = torch.empty(qc.shape, dtype=torch.float32, device=dev)
-    rc = _lib.lib().mspr_indexer_q_qat_live(_lib.ptr(qc), batch * n_heads * n_tokens, _lib.ptr(out),
-                                            _lib.stream_ptr())
+    rc = _lib.launch(dev, "mspr_indexer_q_qat_live", _lib.ptr(qc), batch * n_heads * n_tokens, _lib.ptr(out))
     _lib.check(rc, "indexer_q_qat_live")
     return out
 

@@ -70,11 +70,12 @@ def indexer_qat_rows(x: torch.Tensor) -> torch.Tensor:
     n_rows = x.numel() // _HEAD_DIM
     if n_rows == 0:
         raise ValueError("indexer QAT expects at least one row")
-    _lib.require_device(x)
+    dev = _lib.require_device(x)
     rows2d = x.reshape(-1, _HEAD_DIM).contiguous()
     out = torch.empty((n_rows, _HEAD_DIM), dtype=torch.float32, device=x.device)
-    rc = _lib.lib().mspr_indexer_qat_rows(
-        _lib.ptr(rows2d), _lib.DTYPE_CODE[x.dtype], n_rows, _lib.ptr(out), _lib.stream_ptr())
+    rc = _lib.launch(
+        dev, "mspr_indexer_qat_rows",
+        _lib.ptr(rows2d), _lib.DTYPE_CODE[x.dtype], n_rows, _lib.ptr(out))
     _lib.check(rc, "indexer_qat_rows")
     return out.reshape(x.shape)
 
@@ -139,14 +140,15 @@ def fused_qat_indexer_scores(q, pooled_qat, weights, scale) -> torch.Tensor:
         raise ValueError("q must be float32, float16, or bfloat16")
     if pooled_qat.dtype != torch.float32 or weights.dtype != torch.float32:
         raise ValueError("pooled_qat and weights must be float32")
-    _lib.require_device(q, pooled_qat, weights)
+    dev = _lib.require_device(q, pooled_qat, weights)
     qc = q.reshape(n_heads, head_dim).contiguous()
     pc = pooled_qat.reshape(n_rows, head_dim).contiguous()
     wc = weights.reshape(n_heads).contiguous()
     scores = torch.empty((n_rows,), dtype=torch.float32, device=q.device)
-    rc = _lib.lib().mspr_fused_qat_indexer_scores(
+    rc = _lib.launch(
+        dev, "mspr_fused_qat_indexer_scores",
         _lib.ptr(qc), _lib.DTYPE_CODE[q.dtype], n_heads, _lib.ptr(pc), n_rows, _lib.ptr(wc),
-        float(scale), _lib.ptr(scores), _lib.stream_ptr())
+        float(scale), _lib.ptr(scores))
     _lib.check(rc, "fused_qat_indexer_scores")
     return scores
 
@@ -214,14 +216,15 @@ def fused_score_tail(scores, weights_raw, params, *, scale) -> torch.Tensor:
         raise ValueError("weights_raw must be float32, float16, or bfloat16")
     if params.dtype != torch.int32 or params.numel() < 2:
         raise ValueError("params must be int32 with the row count at index 1")
-    _lib.require_device(scores, weights_raw, params)
+    dev = _lib.require_device(scores, weights_raw, params)
     sc = scores.reshape(n_heads, capacity).contiguous()
     wc = weights_raw.reshape(n_heads).contiguous()
     pc = params.reshape(-1).contiguous()
     neg = torch.empty((capacity,), dtype=torch.float32, device=scores.device)
-    rc = _lib.lib().mspr_indexer_score_tail(
+    rc = _lib.launch(
+        dev, "mspr_indexer_score_tail",
         _lib.ptr(sc), n_heads, capacity, _lib.ptr(wc), _lib.DTYPE_CODE[weights_raw.dtype],
-        _lib.ptr(pc), float(scale), _lib.ptr(neg), _lib.stream_ptr())
+        _lib.ptr(pc), float(scale), _lib.ptr(neg))
     _lib.check(rc, "fused_score_tail")
     return neg.reshape(1, 1, capacity)
 
@@ -257,12 +260,11 @@ def topk_select(scores: torch.Tensor, topk: int) -> torch.Tensor:
     topk = int(topk)
     if not 0 < topk <= n_rows:
         raise ValueError("topk must be positive and at most n_rows")
-    _lib.require_device(scores)
+    dev = _lib.require_device(scores)
     s2 = scores.reshape(-1, n_rows).contiguous()
     batch = int(s2.shape[0])
     sel = torch.empty((batch, topk), dtype=torch.int32, device=scores.device)
-    rc = _lib.lib().mspr_topk_select(_lib.ptr(s2), n_rows, batch, n_rows, topk, _lib.ptr(sel),
-                                     _lib.stream_ptr())
+    rc = _lib.launch(dev, "mspr_topk_select", _lib.ptr(s2), n_rows, batch, n_rows, topk, _lib.ptr(sel))
     _lib.check(rc, "topk_select")
     return sel.reshape(*scores.shape[:-1], topk)
 
@@ -307,7 +309,7 @@ def indexer_scores_fp8(q, keys, key_scales, weights) -> torch.Tensor:
     dev = _lib.require_device(q, keys, key_scales, weights)
     qc, kc, sc, wc = q.contiguous(), keys.contiguous(), key_scales.contiguous(), weights.contiguous()
     scores = torch.empty((batch, n_rows), dtype=torch.float32, device=dev)
-    rc = _lib.lib().mspr_indexer_scores_fp8(_lib.ptr(qc), _lib.ptr(kc), _lib.ptr(sc), _lib.ptr(wc), batch,
-                                            n_heads, n_rows, _lib.ptr(scores), _lib.stream_ptr())
+    rc = _lib.launch(dev, "mspr_indexer_scores_fp8", _lib.ptr(qc), _lib.ptr(kc), _lib.ptr(sc), _lib.ptr(wc), batch,
+                     n_heads, n_rows, _lib.ptr(scores))
     _lib.check(rc, "indexer_scores_fp8")
     return scores

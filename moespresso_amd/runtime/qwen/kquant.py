@@ -90,9 +90,10 @@ def quantize(x, group_size: int = 64, bits: int = 8):
     wq = torch.empty(lead + (d // 4,), dtype=torch.int32, device=dev).view(torch.uint32)
     scales = torch.empty(lead + (d // 64,), dtype=xc.dtype, device=dev)
     biases = torch.empty_like(scales)
-    _lib.check(_lib.lib().mspr_affine_q8_quantize(
+    _lib.check(_lib.launch(
+        dev, "mspr_affine_q8_quantize",
         _lib.ptr(xc), _lib.DTYPE_CODE[xc.dtype], xc.numel() // 64, _lib.ptr(wq), _lib.ptr(scales), _lib.ptr(biases),
-        64, 8, _lib.stream_ptr()), "quantize")
+        64, 8), "quantize")
     return wq, scales, biases
 
 
@@ -113,9 +114,9 @@ def dequantize(wq, scales, biases, group_size: int = 64, bits: int = 8):
     dev = _lib.require_device(wq, scales, biases)
     w, s, b = wq.contiguous(), scales.contiguous(), biases.contiguous()
     out = torch.empty(tuple(w.shape[:-1]) + (int(w.shape[-1]) * 4,), dtype=s.dtype, device=dev)
-    _lib.check(_lib.lib().mspr_affine_q8_dequantize(
-        _lib.ptr(w), _lib.ptr(s), _lib.ptr(b), _lib.DTYPE_CODE[s.dtype], s.numel(), _lib.ptr(out), 64, 8,
-        _lib.stream_ptr()), "dequantize")
+    _lib.check(_lib.launch(
+        dev, "mspr_affine_q8_dequantize",
+        _lib.ptr(w), _lib.ptr(s), _lib.ptr(b), _lib.DTYPE_CODE[s.dtype], s.numel(), _lib.ptr(out), 64, 8), "dequantize")
     return out
 
 
@@ -232,16 +233,17 @@ def sdpa_decode_q8(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases, 
         raise ValueError("key and value scales must share a dtype")
     if N < 1:
         raise ValueError("the cache must hold at least one token")
-    _lib.require_device(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases)
+    dev = _lib.require_device(queries, k_wq, k_scales, k_biases, v_wq, v_scales, v_biases)
     q = queries.contiguous()
     (kw, ks, kb, vw, vs, vb), kv_rows = _cache_operands((k_wq, k_scales, k_biases, v_wq, v_scales, v_biases), N)
     out = torch.empty_like(q)
     if workspace is None:
         workspace = _lib.q8_decode_workspace(B, Hkv, N, q.device)
-    _lib.check(_lib.lib().mspr_sdpa_decode_q8(
+    _lib.check(_lib.launch(
+        dev, "mspr_sdpa_decode_q8",
         _lib.ptr(q), _lib.DTYPE_CODE[q.dtype], _lib.ptr(kw), _lib.ptr(ks), _lib.ptr(kb), _lib.ptr(vw), _lib.ptr(vs),
         _lib.ptr(vb), _lib.DTYPE_CODE[ks.dtype], B, Hq, Hkv, _HEAD_DIM, N, kv_rows, float(scale), 64, 8, _lib.ptr(out),
-        _lib.ptr(workspace), workspace.numel() * workspace.element_size(), _lib.stream_ptr()), "sdpa_decode_q8")
+        _lib.ptr(workspace), workspace.numel() * workspace.element_size()), "sdpa_decode_q8")
     return out
 
 
@@ -277,16 +279,17 @@ def sdpa_decode_q8_0(queries, k_codes, k_scales, v_codes, v_scales, scale, *, wo
         raise ValueError("query heads must be a multiple (at most 16x) of the KV heads")
     if N < 1:
         raise ValueError("the cache must hold at least one token")
-    _lib.require_device(queries, k_codes, k_scales, v_codes, v_scales)
+    dev = _lib.require_device(queries, k_codes, k_scales, v_codes, v_scales)
     q = queries.contiguous()
     (kc, ks, vc, vs), kv_rows = _cache_operands((k_codes, k_scales, v_codes, v_scales), N)
     out = torch.empty_like(q)
     if workspace is None:
         workspace = _lib.q8_decode_workspace(B, Hkv, N, q.device)
-    _lib.check(_lib.lib().mspr_sdpa_decode_q8_0(
+    _lib.check(_lib.launch(
+        dev, "mspr_sdpa_decode_q8_0",
         _lib.ptr(q), _lib.DTYPE_CODE[q.dtype], _lib.ptr(kc), _lib.ptr(ks), _lib.ptr(vc), _lib.ptr(vs), B, Hq, Hkv,
         _HEAD_DIM, N, kv_rows, float(scale), _lib.ptr(out), _lib.ptr(workspace),
-        workspace.numel() * workspace.element_size(), _lib.stream_ptr()), "sdpa_decode_q8_0")
+        workspace.numel() * workspace.element_size()), "sdpa_decode_q8_0")
     return out
 
 
@@ -330,7 +333,7 @@ def sdpa_fa_prefill_q8(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, p
         raise ValueError("query heads per KV head must be 1, 2, 4 or 8")
     if L < 1:
         raise ValueError("the chunk must hold at least one token")
-    _lib.require_device(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, pv_biases, self_k, self_v)
+    dev = _lib.require_device(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, pv_biases, self_k, self_v)
     q, sk, sv = queries.contiguous(), self_k.contiguous(), self_v.contiguous()
     (kw, ks, kb, vw, vs, vb), past_rows = _cache_operands(
         (pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, pv_biases), P)
@@ -338,11 +341,12 @@ def sdpa_fa_prefill_q8(queries, pk_wq, pk_scales, pk_biases, pv_wq, pv_scales, p
     if workspace is None:
         nbytes = int(_lib.lib().mspr_sdpa_fa_prefill_q8_workspace_bytes(B, Hq, Hkv, L, P))
         workspace = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=q.device)
-    _lib.check(_lib.lib().mspr_sdpa_fa_prefill_q8(
+    _lib.check(_lib.launch(
+        dev, "mspr_sdpa_fa_prefill_q8",
         _lib.ptr(q), _lib.ptr(kw), _lib.ptr(ks), _lib.ptr(kb), _lib.ptr(vw), _lib.ptr(vs), _lib.ptr(vb),
         _lib.DTYPE_CODE[ks.dtype], _lib.ptr(sk), _lib.ptr(sv), _lib.DTYPE_CODE[sk.dtype], B, Hq, Hkv, _HEAD_DIM, L, P,
-        past_rows, float(scale), 64, 8, _lib.ptr(out), _lib.ptr(workspace), workspace.numel() * workspace.element_size(),
-        _lib.stream_ptr()), "sdpa_fa_prefill_q8")
+        past_rows, float(scale), 64, 8, _lib.ptr(out), _lib.ptr(workspace),
+        workspace.numel() * workspace.element_size()), "sdpa_fa_prefill_q8")
     return out
 
 
@@ -377,14 +381,14 @@ def flash_prefill(queries, keys, values, scale, *, past_len: int, workspace=None
     past_len = int(past_len)
     if L < 1 or past_len < 0 or past_len + L > rows:
         raise ValueError("need q_len >= 1, past_len >= 0 and past_len + q_len <= cache rows")
-    _lib.require_device(queries, keys, values)
+    dev = _lib.require_device(queries, keys, values)
     q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
     out = torch.empty_like(q)
     if workspace is None:
         nbytes = int(_lib.lib().mspr_flash_prefill_workspace_bytes(B, Hq, Hkv, L, past_len))
         workspace = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=q.device)
-    _lib.check(_lib.lib().mspr_flash_prefill(
+    _lib.check(_lib.launch(
+        dev, "mspr_flash_prefill",
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.DTYPE_CODE[q.dtype], B, Hq, Hkv, _HEAD_DIM, L, past_len, rows,
-        float(scale), _lib.ptr(out), _lib.ptr(workspace), workspace.numel() * workspace.element_size(),
-        _lib.stream_ptr()), "flash_prefill")
+        float(scale), _lib.ptr(out), _lib.ptr(workspace), workspace.numel() * workspace.element_size()), "flash_prefill")
     return out
