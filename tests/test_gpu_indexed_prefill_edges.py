@@ -55,5 +55,9 @@ def test_last_round_in_key_ranges(monkeypatch, batch, tokens, heads, top_k, pos0
     run = lambda: iak.indexed_mixed_attention_prefill_live_f32(q, raw, comp, ids, sinks, pos0=pos0, window=128, ratio=4)
     monkeypatch.delenv("MSPR_PREFILL_PERSISTENT", raising=False)
     got = run()
+    for b in range(batch):
+        want = ds4.indexed_mixed_attention_prefill(q[b].transpose(0, 1).cpu().numpy(), raw[b, 0].cpu().numpy(), comp[b].cpu().numpy(),
+                                                   ids[b].cpu().numpy(), sinks.cpu().numpy(), pos0=pos0, window=128, ratio=4)
+        np.testing.assert_allclose(got[b].transpose(0, 1).cpu().numpy(), want, rtol=2e-3, atol=2e-3)
     monkeypatch.setenv("MSPR_PREFILL_PERSISTENT", "1")
     torch.testing.assert_close(got, run(), rtol=2e-3, atol=2e-3)

@@ -39,6 +39,19 @@ def test_quantised_prefix_rows(tokens, past, dtype):
     assert np.abs(got.cpu().numpy() - want).max() < 2e-3
 
 
+# a prefix of more than 16384 rows is unpacked in the attention kernel for up to 256 tokens, a shorter one for up to 128
+@pytest.mark.parametrize("tokens,past", [(200, 16384), (200, 16385), (256, 16400), (257, 16400)])
+def test_quantised_prefix_at_the_line_between_unpacking_and_conversion(tokens, past):
+    gen = torch.Generator(device="cuda").manual_seed(past)
+    q, k, v = (torch.randn((1, h, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (4, 1, 1))
+    tk, tv = kquant.quantize(k), kquant.quantize(v)
+    dk, dv = kquant.dequantize(*tk), kquant.dequantize(*tv)
+    prefix = [t[:, :, :past] for t in (*tk, *tv)]
+    got = kquant.sdpa_fa_prefill_q8(q[:, :, past:], *prefix, dk[:, :, past:], dv[:, :, past:], 256 ** -0.5)
+    want = qwen.causal_prefill_attention(q[:, :, past:].cpu().numpy(), dk.cpu().numpy(), dv.cpu().numpy(), 256 ** -0.5, past=past)
+    assert np.abs(got.cpu().numpy() - want).max() < 2e-3
+
+
 # unpacked in the attention kernel; converted to float16; to bfloat16: one key range, several, and merges of two waves a row
 @pytest.mark.parametrize("tokens,past", [(17, 40), (17, 5000), (203, 301), (300, 9000), (1024, 70)])
 @pytest.mark.parametrize("side", ["key", "value"])
