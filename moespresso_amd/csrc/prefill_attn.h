@@ -26,5 +26,5 @@ struct IndexedPrefillArgs {
 // Whether the kernel takes the call: the ids of a token are staged in LDS next to the row tiles.
 bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx);
 // Room for the partials of a part-filled last round; without it every token is one workgroup's.
-size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int n_idx);
+size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int window_rows, int n_idx);
 int mspr_launch_indexed_prefill(const IndexedPrefillArgs& a, void* workspace, size_t workspace_bytes, hipStream_t st);

@@ -399,39 +399,69 @@ bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx) 
   return n_idx <= kMaxIds && (int64_t)batch * n_tokens * ((n_heads + 63) / 64) < ((int64_t)1 << 31);
 }
 
+static int tiles_of(int64_t rows) { return (int)((rows + kTile - 1) / kTile); }
+
 // Two workgroups on each of 256 CUs are a round; what is left of the last one runs one to a CU, and if it is few units the
-// chip is idle. Up to 80 of them are cut into key ranges, as many as keep the partials (128 KB each) under 24 MB, with at
-// least two id tiles in each. With the merge, 128 + 512 rows each: 1 token 29 -> 13 us, 20 29.5 -> 21, 64 30 -> 25, 513
-// 75 -> 62; 96 would gain nothing. (Partials under 16 MB: 64 tokens 28; under 32 MB: 544 tokens 73 instead of 68.)
-static void cut_last_round(IndexedPrefillArgs& a) {
+// chip is idle. They are cut into as many key ranges as keep the partials (128 KB each) under 24 MB, or, where those would be
+// one or two and no round is in front, as leave one workgroup to a CU; with at least two id tiles in each. Whether that pays is estimated: a tile
+// takes 1.13 us alone and about 1 us under the round in front, and the partials and their merge cost what was fitted to 1
+// to 96 units of 128 to 1024 ids and a window of 128, whole and in 2 to 8 ranges (float16 and float32 queries, pools of
+// 1200 to 6000 rows). Whole and cut, us: 512 ids 1 token 30 and 13, 16 tokens 31 and 21, 64 tokens 31 and 27, 80 tokens 31 and
+// 29 (in two ranges 32), 96 tokens 31 and 34 (left whole); 513 tokens 73 and 58, 576 tokens 75 and 71. 256 ids 24 tokens 21.5 and
+// 19.9, 48 tokens 21.5 and 23.2 (left whole). 128 ids 8 tokens 16.6 and 14.9, 24 tokens 16.9 and 18.0, 64 tokens 17 and 25 (left
+// whole), 520 tokens 40.7 and 40.2, 560 tokens 41.2 and 44.4 (left whole).
+// The kernel deals out the tiles of a window of `window_rows` and all of a token's ids; `tiles` of them hold rows at most.
+static void cut_last_round(IndexedPrefillArgs& a, int64_t window_rows, int tiles) {
   const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
   const int left = (int)(units % 512);
-  int ranges = left == 0 || left > 80 ? 1 : 192 / left;
+  const bool alone = units < 512;
+  int ranges = left == 0 ? 1 : (alone && left > 64 ? 256 : 192) / left;
   if (ranges > a.n_idx / (2 * kTile)) ranges = a.n_idx / (2 * kTile);
   if (ranges > kMaxRanges) ranges = kMaxRanges;
-  a.split_units = ranges > 1 ? left : 0;
-  a.ranges = ranges > 1 ? ranges : 1;
+  a.split_units = 0;
+  a.ranges = 1;
+  if (ranges < 2) return;
+  const float tile_us = alone ? 1.13f : 1.0f, parts = (float)(left * ranges);
+  // (many partials of long ranges, which are all written at once, cost 2 us more)
+  const float merge_us = alone ? 2.5f + (parts < 110.0f ? 0.065f * parts : 7.15f + 0.02f * (parts - 110.0f) +
+                                                                              (ranges == 2 ? 2.0f : 0.0f))
+                               : 3.0f + 0.035f * parts;
+  const int share = (tiles_of(window_rows) + tiles_of(a.n_idx) + ranges - 1) / ranges;
+  if (tile_us * (float)(share < tiles ? share : tiles) + merge_us >= tile_us * (float)tiles - 0.3f) return;
+  a.split_units = left;
+  a.ranges = ranges;
 }
 
 static size_t part_bytes(const IndexedPrefillArgs& a) {
   return (size_t)a.split_units * a.ranges * (64 * kD + 64 * 2) * sizeof(float);
 }
 
-size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int n_idx) {
+size_t mspr_indexed_prefill_workspace_bytes(int batch, int n_heads, int n_tokens, int window_rows, int n_idx) {
   IndexedPrefillArgs a = {};
   a.batch = batch;
   a.n_heads = n_heads;
   a.n_tokens = n_tokens;
   a.n_idx = n_idx;
-  cut_last_round(a);
+  cut_last_round(a, window_rows, tiles_of(window_rows) + tiles_of(n_idx));
   return part_bytes(a);
 }
 
 int mspr_launch_indexed_prefill(const IndexedPrefillArgs& call, void* workspace, size_t workspace_bytes, hipStream_t st) {
   IndexedPrefillArgs a = call;
-  cut_last_round(a);
+  // The units that may be cut are the first tokens' (of the first sequence): the rows that those see at most. (The workspace
+  // was sized without their position, for all rows; where it is too small for the ranges chosen here, there are fewer.)
+  const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
+  const int64_t last = units % 512 / ((a.n_heads + 63) / 64);
+  const int64_t seen = (int64_t)a.pos0 + (last < a.n_tokens ? last : a.n_tokens);
+  int64_t ids = a.ratio == 0u ? a.n_pool : seen / a.ratio;
+  if (ids > a.n_pool) ids = a.n_pool;
+  if (ids > a.n_idx) ids = a.n_idx;
+  cut_last_round(a, a.max_win, tiles_of(a.max_win < seen ? a.max_win : seen) + tiles_of(ids));
   a.parts = static_cast<float*>(workspace);
-  if (!workspace || workspace_bytes < part_bytes(a) || !mspr_aligned(workspace, 16)) a.split_units = 0;
+  if (!workspace || !mspr_aligned(workspace, 16)) a.split_units = 0;
+  while (a.ranges > 1 && workspace_bytes < part_bytes(a)) a.ranges--;
+  if (a.ranges == 1) a.split_units = 0;
+  if (a.split_units == 0) a.ranges = 1;
   if (a.split_units > 0) return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, true>(a, st) : launch<MSPR_F16, true>(a, st);
   return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, false>(a, st) : launch<MSPR_F16, false>(a, st);
 }

@@ -1679,7 +1679,7 @@ extern "C" size_t mspr_indexed_mixed_attention_prefill_workspace_bytes(int q_dty
   if (batch < 1 || n_heads < 1 || n_tokens < 1 || window_rows < 0 || top_k < 0) return 0;
   const PrefillForm form = prefill_form();
   if (form == kPrefillWaves && mspr_indexed_prefill_fits(batch, n_heads, n_tokens, top_k))
-    return mspr_indexed_prefill_workspace_bytes(batch, n_heads, n_tokens, top_k);
+    return mspr_indexed_prefill_workspace_bytes(batch, n_heads, n_tokens, window_rows, top_k);
   // the per-range partials of the split kernel (slot lists too long for the persistent consumer), or the
   // half-precision copy of float32 queries for the persistent consumer, whichever is larger
   size_t need = workspace_bytes(batch * n_tokens, n_heads, (int64_t)window_rows + top_k);

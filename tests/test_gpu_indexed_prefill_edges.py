@@ -40,7 +40,7 @@ def test_edges_match_the_oracle(monkeypatch, form, tokens, heads, top_k, window,
 
 
 # a part-filled last round of workgroups in key ranges: alone, behind a whole round, in two head blocks, ids that end early,
-# tokens whose last ranges hold nothing, the most tokens that are cut and one more
+# tokens whose last ranges hold nothing, more tokens than are worth cutting at a short list
 @pytest.mark.parametrize("batch,tokens,heads,top_k,pos0", [(1, 1, 64, 512, 3000), (1, 20, 64, 512, 0), (1, 515, 16, 130, 900),
                                                           (2, 7, 72, 300, 500), (1, 80, 32, 512, 2100), (1, 81, 32, 512, 2100)])
 def test_last_round_in_key_ranges(monkeypatch, batch, tokens, heads, top_k, pos0):
@@ -61,3 +61,27 @@ def test_last_round_in_key_ranges(monkeypatch, batch, tokens, heads, top_k, pos0
         np.testing.assert_allclose(got[b].transpose(0, 1).cpu().numpy(), want, rtol=2e-3, atol=2e-3)
     monkeypatch.setenv("MSPR_PREFILL_PERSISTENT", "1")
     torch.testing.assert_close(got, run(), rtol=2e-3, atol=2e-3)
+
+
+# cut rounds: three ranges (the most of them that leave one workgroup to a CU) and one token more, eight ranges, two sequences of
+# two head blocks, behind a whole round, a wide ring; each with ids of which most are not visible yet: ranges that end early or
+# hold nothing
+@pytest.mark.parametrize("batch,tokens,heads,top_k,pos0,window", [
+    (1, 85, 32, 512, 3000, 128), (1, 86, 32, 512, 3000, 128), (1, 5, 64, 1024, 3500, 128), (2, 7, 72, 300, 2000, 128),
+    (1, 560, 8, 400, 2400, 64), (1, 9, 40, 256, 3000, 600)])
+@pytest.mark.parametrize("first_id", [0, 500])
+def test_cut_rounds_match_the_oracle(batch, tokens, heads, top_k, pos0, window, first_id):
+    from moespresso_amd.runtime.deepseek_v4 import indexed_attention_kernel as iak
+
+    gen = torch.Generator(device="cuda").manual_seed(tokens + first_id)
+    q = torch.randn((batch, heads, tokens, 512), device="cuda", generator=gen).half()
+    raw = torch.randn((batch, 1, window - 1 + tokens, 512), device="cuda", generator=gen).half()
+    comp = torch.randn((batch, 1600, 512), device="cuda", generator=gen).half()
+    ids = first_id + torch.rand((batch, tokens, 1600 - first_id), device="cuda", generator=gen).topk(top_k, dim=2).indices.sort(dim=2).values
+    sinks = torch.randn(heads, device="cuda", generator=gen)
+    got = iak.indexed_mixed_attention_prefill_live_f16(q, raw, comp, ids.to(torch.int32), sinks, pos0=pos0, window=window, ratio=4)
+    for b in range(batch):
+        want = ds4.indexed_mixed_attention_prefill(q[b].transpose(0, 1).float().cpu().numpy(), raw[b, 0].cpu().numpy(),
+                                                   comp[b].cpu().numpy(), ids[b].cpu().numpy(), sinks.cpu().numpy(), pos0=pos0,
+                                                   window=window, ratio=4)
+        np.testing.assert_allclose(got[b].transpose(0, 1).cpu().numpy(), want, rtol=2e-3, atol=2e-3)

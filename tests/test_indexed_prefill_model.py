@@ -15,7 +15,7 @@ import shutil
 import numpy as np
 import pytest
 
-from moespresso_amd import build
+from moespresso_amd import _lib, build
 from test_prefill_row_table_model import host_n_win, unit_rows
 
 SOURCE = os.path.join(build.CSRC, "prefill_attn.hip")
@@ -95,6 +95,27 @@ def test_key_ranges_of_a_cut_unit_hold_every_tile_once():
             if begin < wt:                                  # its first copy is issued before the ids are known: it is awaited
                 assert end > begin
         assert seen == list(range(total))
+
+
+def test_a_last_round_is_cut_only_where_the_partials_pay():
+    """Scratch is asked for the partials of cut units alone: 64 heads, a window of 128."""
+    if not _lib.library_available():
+        pytest.skip("the library is not built")
+
+    def parts(tokens, n_idx, heads=64):
+        n = _lib.lib().mspr_indexed_mixed_attention_prefill_workspace_bytes(1, 1, heads, tokens, 128, n_idx)
+        assert n % (64 * 514 * 4) == 0
+        return n // (64 * 514 * 4)
+
+    for n_idx in (0, 64, 127):
+        assert all(parts(t, n_idx) == 0 for t in range(1, 600, 7))
+    assert parts(8, 128) == 16 and parts(24, 128) == 0 and parts(64, 128) == 0     # 24: 16.9 us whole, 18.0 in two ranges
+    assert parts(24, 256) == 96 and parts(48, 256) == 0
+    assert parts(1, 512) == 8 and parts(64, 512) == 192
+    assert parts(80, 512) == 240 and parts(85, 512) == 255 and parts(86, 512) == 0  # in two ranges 80 take longer than whole
+    assert parts(512, 512) == 0 and parts(512 + 64, 512) == 192 and parts(512 + 48, 128) == 0
+    assert all(parts(t, n) <= 256 for t in range(1, 1100, 3) for n in (128, 256, 512, 1024, 3000))
+    assert parts(3, 512, heads=72) == parts(6, 512)
 
 
 # ------------------------------------------------------------------------------------------------ schedule
