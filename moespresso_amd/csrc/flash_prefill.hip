@@ -820,13 +820,22 @@ extern "C" int mspr_flash_prefill(const void* q, const void* k, const void* v, i
   return prefill_launch<MSPR_F16, false, MSPR_F32>(a, st);
 }
 
+// Long chunks stage K/V and the queries as bfloat16 (the prefix is converted then, whatever it costs).
+static bool prefill_q8_bf16(int q_len) { return q_len >= 1024; }
+
 // Prefix tiles unpacked inside the attention kernel. Unpacking costs every workgroup that passes a tile 0.7 us next to
-// the 1.3 us of its attention; converting the prefix once (1 KB per key and KV head of scratch) costs a launch and
-// about 0.6 ns per row. From five 32-query blocks on, the prefix is therefore converted first and the attention
-// kernel runs on dense tiles only (at 128 queries both forms are within 5 % of each other from 2000 to 32000 keys;
-// 517 over 9000: 124 -> 114 us); behind a long prefix only from nine on (203 over 32768: 148 us unpacked, 150 converted).
-static int prefill_q8_tiles(int q_len, int64_t past_len) {
-  const bool converted = q_len > 256 || (q_len > 128 && past_len <= 16384);
+// the 1.3 us of its attention; converting the prefix once costs a launch and the rows' way through memory, which they leave
+// the L2s for beyond some 30 MB (1 KB per key and KV head). So it depends on how many workgroups pass each tile: from eight on
+// the prefix is converted, with fewer if it has at most 4096 rows, over all sequences and KV heads, for each of them. Unpacked
+// and converted, us, float32 scales: 16 / 2 heads, 203 queries (eight) over 9001 rows 66 and 64.5, over 32000 148 and 149; 160
+// queries (six) over 4000 47 and 45, 16000 79 and 79, 32000 121 and 124. 16 / 4 heads, 160 queries (three) over 2000 41 and
+// 39, 4000 47 and 48, 16000 79 and 87; 512 queries (eight) over 16000 167 and 166. 4 / 4 heads, 256 queries (one) over 2000 40
+// and 37, 4000 40 and 42, 16000 53 and 64. Up to 128 queries it is unpacked (16 / 2 heads, 128 over 4000 45 and 42.5, 16000
+// 69 and 71).
+static int prefill_q8_tiles(int batch, int n_q_heads, int n_kv_heads, int q_len, int64_t past_len) {
+  const int64_t passes = prefill_q_blocks(n_q_heads / n_kv_heads, q_len);
+  const bool converted = prefill_q8_bf16(q_len) ||
+                         (q_len > 128 && (passes >= 8 || (int64_t)batch * n_kv_heads * past_len <= 4096 * passes));
   return converted ? 0 : (int)(past_len / kTile);
 }
 
@@ -835,7 +844,7 @@ extern "C" size_t mspr_sdpa_fa_prefill_q8_workspace_bytes(int batch, int n_q_hea
   if (batch < 1 || n_kv_heads < 1 || n_q_heads < n_kv_heads || n_q_heads % n_kv_heads != 0 || q_len < 1 ||
       past_len < 0 || n_q_heads / n_kv_heads > 8)
     return 0;
-  const int64_t tail_rows = past_len - (int64_t)prefill_q8_tiles(q_len, past_len) * kTile + q_len;
+  const int64_t tail_rows = past_len - (int64_t)prefill_q8_tiles(batch, n_q_heads, n_kv_heads, q_len, past_len) * kTile + q_len;
   const size_t tail = ((size_t)batch * n_kv_heads * tail_rows * kRowBytes * 2 + 255) / 256 * 256;
   return tail + prefill_split_bytes(batch, n_q_heads, n_kv_heads, q_len, past_len) + 256;
 }
@@ -871,7 +880,7 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   MSPR_REQUIRE(workspace && workspace_bytes >= need && mspr_aligned(workspace, 16),
                "sdpa_fa_prefill_q8: workspace of %zu bytes (16-byte aligned) needed, %zu given", need, workspace_bytes);
   PrefillArgs a = {};
-  const int q8_tiles = prefill_q8_tiles(q_len, past_len);
+  const int q8_tiles = prefill_q8_tiles(batch, n_q_heads, n_kv_heads, q_len, past_len);
   const int tail_rows = (int)(past_len - (int64_t)q8_tiles * kTile) + q_len;
   uint16_t* tail_k = reinterpret_cast<uint16_t*>(workspace);
   uint16_t* tail_v = tail_k + (size_t)batch * n_kv_heads * tail_rows * kD;
@@ -903,10 +912,9 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   a.pv_s = pv_scales;
   a.pv_b = pv_biases;
   hipStream_t st = (hipStream_t)stream;
-  // Long chunks stage K/V and the queries as bfloat16 and run the bfloat16 matrix
-  // instructions: the device holds a higher clock under them than under the float16 ones, and the 8-bit codes
+  // bfloat16 staging runs the bfloat16 matrix instructions: the device holds a higher clock under them than under the float16 ones, and the 8-bit codes
   // leave the rounding of the staging type (2^-9 of a value) below their own step. Shorter chunks stay float16.
-  const bool bf16_staging = q_len >= 1024;
+  const bool bf16_staging = prefill_q8_bf16(q_len);
   dim3 rgrid((unsigned)((tail_rows + 15) / 16), (unsigned)n_kv_heads, (unsigned)batch);
 #define MSPR_ROWS_LAUNCH(SDT)                                                                                        \
   do {                                                                                                               \

@@ -39,11 +39,14 @@ def test_quantised_prefix_rows(tokens, past, dtype):
     assert np.abs(got.cpu().numpy() - want).max() < 2e-3
 
 
-# a prefix of more than 16384 rows is unpacked in the attention kernel for up to 256 tokens, a shorter one for up to 128
-@pytest.mark.parametrize("tokens,past", [(200, 16384), (200, 16385), (256, 16400), (257, 16400)])
-def test_quantised_prefix_at_the_line_between_unpacking_and_conversion(tokens, past):
+# Both sides of the line between unpacking in the attention kernel and converting beforehand, for four, five, one and six
+# workgroups to a tile; 1023 and 1024 tokens of one query head to a KV head (unpacked, and converted to bfloat16)
+@pytest.mark.parametrize("heads,kv_heads,tokens,past", [
+    (4, 1, 200, 16384), (4, 1, 200, 16385), (4, 1, 256, 16400), (4, 1, 257, 16400), (2, 2, 130, 2048), (2, 2, 130, 2049),
+    (16, 2, 150, 12288), (16, 2, 150, 12289), (3, 3, 1023, 6000), (3, 3, 1024, 6000)])
+def test_quantised_prefix_at_the_line_between_unpacking_and_conversion(heads, kv_heads, tokens, past):
     gen = torch.Generator(device="cuda").manual_seed(past)
-    q, k, v = (torch.randn((1, h, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (4, 1, 1))
+    q, k, v = (torch.randn((1, h, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (heads, kv_heads, kv_heads))
     tk, tv = kquant.quantize(k), kquant.quantize(v)
     dk, dv = kquant.dequantize(*tk), kquant.dequantize(*tv)
     prefix = [t[:, :, :past] for t in (*tk, *tv)]
