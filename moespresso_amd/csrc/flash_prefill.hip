@@ -713,7 +713,11 @@ int prefill_q_blocks(int rep, int q_len) {
 // few of them), and as many ranges as the partials are worth: tiles / ranges of about 1.3 us each against 1 KB per row
 // and range, written and read again at about 5 TB/s and partly under the tiles of other workgroups. The sum is
 // smallest near ranges^2 = 6000 * tiles / rows (3000 and 1500 measured up to 10 and 20 % slower). At least two or three tiles
-// per range: 33 queries of 16 heads over 9000 keys 39 -> 31 us (17 ranges before, 56 now), 203 over 2000 43 -> 33 us.
+// per range: 33 queries of 16 heads over 9000 keys 39 -> 31 us (17 ranges before, 56 now), 203 over 2000 43 -> 33 us. Two and
+// three, us: 33 queries over 256 keys 18.1 and 18.6, over 600 18.4 and 20.0, over 1000 23 and 20.6; 64 over 256 22.1 and 22.8,
+// over 600 25.5 and 24.0, over 1000 28.1 and 27.1; 97 over 300 24.9 and 24.0, 128 25.8 and 24.8 (8 heads 23.2 and 23.3). From 1500
+// keys on the first rule decides. Between 48 and 96 queries either is better by up to 3 us, by how the tiles divide: three from
+// 49 on gained 1 us over 400 to 1000 keys and lost 1 us over 256.
 int prefill_choose_splits(int batch, int n_q_heads, int n_kv_heads, int q_blocks, int64_t past_len, int q_len) {
   const int64_t wgs = (int64_t)batch * n_kv_heads * q_blocks;
   if (wgs >= 192) return 1;
@@ -754,8 +758,9 @@ int prefill_launch(const PrefillArgs& a, hipStream_t st) {
   MSPR_CHECK_LAUNCH("flash_prefill");
   if (a.n_splits > 1) {
     const int64_t n_rows = (int64_t)a.batch * a.n_q_heads * a.q_len;
-    // (16 ranges: 4096 rows 12.0 us with one wave each, 13.4 with two; 3248 rows equal. 20 of 2048: two waves 8.8, one 9.4,
-    // four 9.6)
+    // (16 ranges: 4096 rows 12.0 us with one wave each, 13.4 with two; between 3248 and 3584 rows equal, whole calls of 3568
+    // 54.6 and 54.5. 12 ranges of 4608 rows, whole calls: one wave 62.7, two 64.2. 20 of 2048: two waves 8.8, one 9.4, four 9.6;
+    // 18 of 3360, whole calls: two 114.7, one 114.0, four 113.9)
     const int share = a.n_splits <= 8 || (a.n_splits <= 16 && n_rows >= 3584) ? 1 : a.n_splits <= 32 ? 2 : 4;
     dim3 mgrid((unsigned)((n_rows * share + 3) / 4)), mblock(256);
     constexpr int ODT = IO32 ? (int)MSPR_F32 : KDT;
