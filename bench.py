@@ -496,8 +496,8 @@ def bench_ds4_prefill(dev, gen, reps=5):
     sc_deep = torch.randn((T, p_deep), device=dev, generator=gen)
     out["topk_512_deep_ms"] = timed(lambda: isk.topk_select(sc_deep, 512))
     out["tiled_scores_deep_TFLOPs"] = round(2.0 * T * p_deep * H * 128 / (out["tiled_scores_deep_ms"] * 1e-3) / 1e12, 1)
-    # the other two forms of the consumer at the same chunk: float32 queries (converted to half into the workspace,
-    # then the same kernel) and the banded route (band of 128 positions + every visible pool row at ratio 128)
+    # the other two forms of the consumer at the same chunk: float32 queries (rounded to half as the kernel loads them)
+    # and the banded route (band of 128 positions + every visible pool row at ratio 128)
     q32 = q.float()
     out["indexed_attention_f32_queries_ms"] = timed(lambda: iak.indexed_mixed_attention_prefill_live_f32(
         q32, raw, comp, ids, sinks, pos0=0, window=128, ratio=4))

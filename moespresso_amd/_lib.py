@@ -162,7 +162,8 @@ def sparse_attention_workspace(batch: int, n_heads: int, n_keys: int, device) ->
 
 def prefill_attention_workspace(q_dtype, batch: int, n_heads: int, n_tokens: int, window_rows: int, top_k: int,
                                 device) -> torch.Tensor:
-    """Scratch tensor for mspr_indexed_mixed_attention_prefill (split partials, or the half copy of float32 queries)."""
+    """Scratch tensor for mspr_indexed_mixed_attention_prefill (partials of units that are cut into key ranges; the half copy of
+    float32 queries only for the persistent form)."""
     nbytes = int(lib().mspr_indexed_mixed_attention_prefill_workspace_bytes(
         DTYPE_CODE[q_dtype], int(batch), int(n_heads), int(n_tokens), int(window_rows), int(top_k)))
     return torch.empty((max(nbytes, 16) + 3) // 4, dtype=torch.float32, device=device)

@@ -692,7 +692,8 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
 // can only tie with the lowest possible key and lose every tie to a real row. Emission order comes from ballots: the
 // hits of (chunk, wave) pairs are scanned and a wave stores its own side by side.
 // What is left is instructions per key and barriers. Four 8-bit digit passes with merged votes took, k = 512: 1 row of
-// 961 scores 7.0 us (now 4.1), 189 of 3974 20 (6.2), 517 of 2053 22 (6.7), 3844 of 961 24 (12), 3844 of 4000 78 (32).
+// 961 scores 7.0 us (now 4.1), 189 of 3974 20 (6.2), 517 of 2053 22 (6.7), 3844 of 961 24 (12), 3844 of 4000 78 (32): scores of
+// prompt chunks, a token's rows visible up to its position. (3844 of 961 with all rows visible 13.8, Gaussian scores 15.9.)
 constexpr uint32_t kRowBins = 1024;
 constexpr uint32_t kNegInfKey = 0x007FFFFFu;
 
