@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY. Nothing in the product package imports this. Only
 the test suite, the smoke check and the CPU-baseline leg of the benchmark may
-call it, and there only as the checker.
+call it, and there only to compare with.
 
 Every function restates, in NumPy, an algorithm of the reference and cites the
 reference file:line it follows. The reference cannot run outside Apple Metal

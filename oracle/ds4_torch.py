@@ -10,7 +10,7 @@ cores and tests/test_oracle_ds4.py pins it against the NumPy oracle (`oracle.ds4
     out[h]   = softmax(q[h] . kv[rows] * scale) . kv[rows, :512]                  (window rows, then 4 sel + 3)
 
 as dense tensor operations, so that the matrix products run on torch's threaded CPU kernels; `torch.set_num_threads`
-decides how many cores it uses. The NumPy oracle computes in float64 and is the checker; this one is float32 and is
+decides how many cores it uses. The NumPy oracle computes in float64 and is what results are compared with; this one is float32 and is
 a baseline to be timed, not a reference for parity.
 """
 

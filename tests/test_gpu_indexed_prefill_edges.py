@@ -85,3 +85,28 @@ def test_cut_rounds_match_the_oracle(batch, tokens, heads, top_k, pos0, window, 
                                                    comp[b].cpu().numpy(), ids[b].cpu().numpy(), sinks.cpu().numpy(), pos0=pos0,
                                                    window=window, ratio=4)
         np.testing.assert_allclose(got[b].transpose(0, 1).cpu().numpy(), want, rtol=2e-3, atol=2e-3)
+
+
+def test_scratch_for_fewer_ranges_cuts_into_fewer():
+    from moespresso_amd import _lib
+
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    tokens, n_ids, pool, pos0 = 16, 512, 900, 3600
+    q = torch.randn((1, 64, tokens, 512), device="cuda", generator=gen).half()
+    raw = torch.randn((1, 1, 127 + tokens, 512), device="cuda", generator=gen).half()
+    comp = torch.randn((1, pool, 512), device="cuda", generator=gen).half()
+    ids = torch.rand((1, tokens, pool), device="cuda", generator=gen).topk(n_ids, dim=2).indices.sort(dim=2).values.to(torch.int32)
+    sinks = torch.randn(64, device="cuda", generator=gen)
+    want = ds4.indexed_mixed_attention_prefill(q[0].transpose(0, 1).float().cpu().numpy(), raw[0, 0].cpu().numpy(), comp[0].cpu().numpy(),
+                                               ids[0].cpu().numpy(), sinks.cpu().numpy(), pos0=pos0, window=128, ratio=4)
+    part = 64 * 514 * 4
+    full = _lib.lib().mspr_indexed_mixed_attention_prefill_workspace_bytes(1, 1, 64, tokens, 128, n_ids)
+    assert full == 8 * tokens * part
+    for nbytes in (full, 3 * tokens * part + 16, 2 * tokens * part, 2 * tokens * part - 4, 0):
+        ws = torch.empty(max(nbytes, 4) // 4, device="cuda")
+        out = torch.full_like(q, float("nan"), dtype=torch.float32)
+        _lib.check(_lib.lib().mspr_indexed_mixed_attention_prefill(
+            _lib.ptr(q), 1, 1, 64, tokens, 64 * tokens * 512, tokens * 512, 512, _lib.ptr(raw), 127 + tokens, _lib.ptr(comp), pool,
+            _lib.ptr(ids), n_ids, _lib.ptr(sinks), pos0, 128, 4, 0, _lib.ptr(out), _lib.ptr(ws) if nbytes else None, nbytes,
+            _lib.stream_ptr()), "prefill")
+        np.testing.assert_allclose(out[0].transpose(0, 1).cpu().numpy(), want, rtol=2e-3, atol=2e-3)
