@@ -68,6 +68,12 @@ __device__ __forceinline__ h2_t sb_to_h2(uint32_t bits) {
   else h = (_Float16)__builtin_bit_cast(float, bits << 16);
   return h2_t{h, h};
 }
+template <int SDT>
+__device__ __forceinline__ float sb_to_f32(uint32_t bits) {
+  if constexpr (SDT == MSPR_F32) return __builtin_bit_cast(float, bits);
+  else if constexpr (SDT == MSPR_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+  else return __builtin_bit_cast(float, bits << 16);
+}
 // 16 unsigned 8-bit codes -> 16 float16 values code * scale + bias (two 16-byte pieces)
 __device__ __forceinline__ void dequant16(u32x4_t c, h2_t sc, h2_t bi, u32x4_t& p0, u32x4_t& p1) {
   const h2_t k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
@@ -84,6 +90,37 @@ __device__ __forceinline__ void dequant16(u32x4_t c, h2_t sc, h2_t bi, u32x4_t& 
       p1[2 * (w - 2) + 1] = h2_bits(hi);
     }
   }
+}
+
+// The same values as prefill_q8_rows_kernel makes: code * scale + bias in float32, one rounding, finite values saturate.
+__device__ __forceinline__ uint32_t h2_of(float a, float b) {
+  return h2_bits(__builtin_convertvector(f32x2_t{a, b}, h2_t));
+}
+__device__ __forceinline__ void dequant16_f32(u32x4_t c, float sc, float bi, u32x4_t& p0, u32x4_t& p1) {
+  uint32_t h[8];
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = __builtin_fmaf((float)((c[w] >> (8 * j)) & 0xFFu), sc, bi);
+    h[2 * w] = h2_of(v[0], v[1]);
+    h[2 * w + 1] = h2_of(v[2], v[3]);
+  }
+  // a wave with a group that can leave the float16 range does it again value by value
+  if (__any(!(__builtin_fabsf(bi) + 255.0f * __builtin_fabsf(sc) <= 65504.0f))) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      float v[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        v[j] = __builtin_fmaf((float)((c[i >> 1] >> (16 * (i & 1) + 8 * j)) & 0xFFu), sc, bi);
+        v[j] = __builtin_isfinite(v[j]) ? __builtin_amdgcn_fmed3f(v[j], -65504.0f, 65504.0f) : v[j];
+      }
+      h[i] = h2_of(v[0], v[1]);
+    }
+  }
+  p0 = u32x4_t{h[0], h[1], h[2], h[3]};
+  p1 = u32x4_t{h[4], h[5], h[6], h[7]};
 }
 
 template <int KDT>
@@ -135,7 +172,10 @@ __device__ __forceinline__ uint32_t lds_addr(const unsigned char* p) {
 __device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
 
 // Q8 = false: k / v are the whole 16-bit cache, q / out have its element type.
-// Q8 = true (KDT float16): float32 q / out, quantised prefix + float16 tail rows (see PrefillArgs).
+// Q8 = true (KDT float16): float32 q / out, quantised prefix + float16 tail rows (see PrefillArgs). SDT is the type of the
+// scales and biases, with kExactUnpack added to it where the prefix is unpacked to the values that a conversion beforehand
+// gives; without it in packed float16 arithmetic.
+constexpr int kExactUnpack = 4;
 template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
 __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(256))) unsigned char lds[];  // tile bases: zero low bits under the address XORs
@@ -382,7 +422,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     //      and a spill of a freshly loaded value waits for the whole memory latency once per tile).
     const int p_end = n_tiles < t1 ? n_tiles : t1;  // prefix tiles of this workgroup: [t_begin, p_end)
     if (t_begin < p_end) {
-      constexpr int kSB = SDT == MSPR_F32 ? 4 : 2;   // bytes per scale / bias
+      constexpr int kST = SDT % kExactUnpack;
+      constexpr int kSB = kST == MSPR_F32 ? 4 : 2;   // bytes per scale / bias
       constexpr int kCodeBytes = kTile * kD;         // 8 KB of codes per tile, K and V each
       constexpr int kScaleBytes = kTile * 4 * kSB;   // one tile of one scale or bias array: 256 or 512 B
       constexpr int kRawBytes = 2 * kCodeBytes + 4 * 512;
@@ -420,7 +461,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
         const unsigned char* sp = raw + 2 * kCodeBytes + (row * 4 + (pp >> 2)) * kSB;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          if constexpr (SDT == MSPR_F32) rs[i] = *reinterpret_cast<const uint32_t*>(sp + i * 512);
+          if constexpr (kST == MSPR_F32) rs[i] = *reinterpret_cast<const uint32_t*>(sp + i * 512);
           else rs[i] = *reinterpret_cast<const uint16_t*>(sp + i * 512);
         }
         const int f = swz(row);
@@ -428,10 +469,14 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
         const int w_off1 = row * kRowBytes + 16 * (((2 * pp + 1) & 16) | (((2 * pp + 1) ^ f) & 15));
         unsigned char* st = lds + slot * kStageBytes;
         u32x4_t p0, p1;
-        dequant16(rk, sb_to_h2<SDT>(rs[0]), sb_to_h2<SDT>(rs[1]), p0, p1);
+        auto dequant = [&](u32x4_t codes, uint32_t sc, uint32_t bi) {
+          if constexpr (SDT >= kExactUnpack) dequant16_f32(codes, sb_to_f32<kST>(sc), sb_to_f32<kST>(bi), p0, p1);
+          else dequant16(codes, sb_to_h2<kST>(sc), sb_to_h2<kST>(bi), p0, p1);
+        };
+        dequant(rk, rs[0], rs[1]);
         *reinterpret_cast<u32x4_t*>(st + w_off0) = p0;
         *reinterpret_cast<u32x4_t*>(st + w_off1) = p1;
-        dequant16(rv, sb_to_h2<SDT>(rs[2]), sb_to_h2<SDT>(rs[3]), p0, p1);
+        dequant(rv, rs[2], rs[3]);
         *reinterpret_cast<u32x4_t*>(st + kTileBytes + w_off0) = p0;
         *reinterpret_cast<u32x4_t*>(st + kTileBytes + w_off1) = p1;
       };
@@ -831,16 +876,21 @@ static bool prefill_q8_bf16(int q_len) { return q_len >= 1024; }
 // Prefix tiles unpacked inside the attention kernel. Unpacking costs every workgroup that passes a tile 0.7 us next to
 // the 1.3 us of its attention; converting the prefix once costs a launch and the rows' way through memory, which they leave
 // the L2s for beyond some 30 MB (1 KB per key and KV head). So it depends on how many workgroups pass each tile: from eight on
-// the prefix is converted, with fewer if it has at most 4096 rows, over all sequences and KV heads, for each of them. Unpacked
-// and converted, us, float32 scales: 16 / 2 heads, 203 queries (eight) over 9001 rows 66 and 64.5, over 32000 148 and 149; 160
-// queries (six) over 4000 47 and 45, 16000 79 and 79, 32000 121 and 124. 16 / 4 heads, 160 queries (three) over 2000 41 and
-// 39, 4000 47 and 48, 16000 79 and 87; 512 queries (eight) over 16000 167 and 166. 4 / 4 heads, 256 queries (one) over 2000 40
-// and 37, 4000 40 and 42, 16000 53 and 64. Up to 128 queries it is unpacked (16 / 2 heads, 128 over 4000 45 and 42.5, 16000
-// 69 and 71).
+// the prefix is converted, with fewer if it has at most 1536 rows, over all sequences and KV heads, times their square.
+// Unpacked and converted, us, float32 scales: 16 / 2 heads, 203 queries (eight) over 9001 rows 66 and 64.5, 256 over 32000 166
+// and 163; 160 (six) over 4000 47 and 45, 16000 81 and 80, 32000 125 and 125. 16 / 4 heads, 320 (five) over 8000 78 and 79,
+// 16000 120 and 122; 256 (four) over 4000 54 and 54, 8000 70 and 72; 160 (three) over 2000 41 and 39, 4000 47 and 48, 16000 82
+// and 88; 512 (eight) over 32000 295 and 298. 4 / 2 heads, 256 (two) over 4000 41 and 39, 8000 46 and 46, 16000 53 and 57. 4 / 4
+// heads, 256 (one) over 1000 37 and 36, 4000 40 and 42, 16000 53 and 65. Up to 128 queries it is unpacked, in packed float16
+// arithmetic (16 / 2 heads, 128 over 4000 45 and 42.5, 16000 69 and 71), and up to 256 behind more than 16384 rows. Elsewhere it
+// is unpacked to the values of the conversion, which takes 2 to 3 % longer (16 / 2 heads, 160 over 32000 121 and 124).
+static bool prefill_q8_packed(int q_len, int64_t past_len) { return q_len <= 128 || (q_len <= 256 && past_len > 16384); }
+
 static int prefill_q8_tiles(int batch, int n_q_heads, int n_kv_heads, int q_len, int64_t past_len) {
   const int64_t passes = prefill_q_blocks(n_q_heads / n_kv_heads, q_len);
   const bool converted = prefill_q8_bf16(q_len) ||
-                         (q_len > 128 && (passes >= 8 || (int64_t)batch * n_kv_heads * past_len <= 4096 * passes));
+                         (!prefill_q8_packed(q_len, past_len) &&
+                          (passes >= 8 || (int64_t)batch * n_kv_heads * past_len <= 1536 * passes * passes));
   return converted ? 0 : (int)(past_len / kTile);
 }
 
@@ -937,6 +987,11 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   if (q8_tiles == 0) {
     if (bf16_staging) return prefill_launch<MSPR_BF16, false, MSPR_F32, true>(a, st);
     return prefill_launch<MSPR_F16, false, MSPR_F32, true>(a, st);
+  }
+  if (!prefill_q8_packed(q_len, past_len)) {  // (converted on the other side of the line: the same values here)
+    if (sb_dtype == MSPR_F32) return prefill_launch<MSPR_F16, true, MSPR_F32 + kExactUnpack>(a, st);
+    if (sb_dtype == MSPR_F16) return prefill_launch<MSPR_F16, true, MSPR_F16 + kExactUnpack>(a, st);
+    return prefill_launch<MSPR_F16, true, MSPR_BF16 + kExactUnpack>(a, st);
   }
   if (sb_dtype == MSPR_F32) return prefill_launch<MSPR_F16, true, MSPR_F32>(a, st);
   if (sb_dtype == MSPR_F16) return prefill_launch<MSPR_F16, true, MSPR_F16>(a, st);

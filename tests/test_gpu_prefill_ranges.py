@@ -39,11 +39,12 @@ def test_quantised_prefix_rows(tokens, past, dtype):
     assert np.abs(got.cpu().numpy() - want).max() < 2e-3
 
 
-# Both sides of the line between unpacking in the attention kernel and converting beforehand, for four, five, one and six
-# workgroups to a tile; 1023 and 1024 tokens of one query head to a KV head (unpacked, and converted to bfloat16)
+# Both sides of the line between unpacking in the attention kernel and converting beforehand: for four, three, one and two
+# workgroups to a tile; behind 16384 rows (unpacked in packed arithmetic beyond); 1023 and 1024 tokens of one query head to a KV
+# head (unpacked, and converted to bfloat16)
 @pytest.mark.parametrize("heads,kv_heads,tokens,past", [
-    (4, 1, 200, 16384), (4, 1, 200, 16385), (4, 1, 256, 16400), (4, 1, 257, 16400), (2, 2, 130, 2048), (2, 2, 130, 2049),
-    (16, 2, 150, 12288), (16, 2, 150, 12289), (3, 3, 1023, 6000), (3, 3, 1024, 6000)])
+    (8, 2, 200, 12288), (8, 2, 200, 12289), (8, 4, 257, 3456), (8, 4, 257, 3457), (2, 2, 130, 768), (2, 2, 130, 769),
+    (4, 2, 150, 3072), (4, 2, 150, 3073), (4, 1, 200, 16384), (4, 1, 200, 16385), (3, 3, 1023, 6000), (3, 3, 1024, 6000)])
 def test_quantised_prefix_at_the_line_between_unpacking_and_conversion(heads, kv_heads, tokens, past):
     gen = torch.Generator(device="cuda").manual_seed(past)
     q, k, v = (torch.randn((1, h, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for h in (heads, kv_heads, kv_heads))
@@ -55,8 +56,46 @@ def test_quantised_prefix_at_the_line_between_unpacking_and_conversion(heads, kv
     assert np.abs(got.cpu().numpy() - want).max() < 2e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("offset", [0.0, 3.0])
+def test_unpacked_and_converted_prefixes_hold_the_same_values(dtype, offset):
+    """One sequence of 700 rows is converted, two are unpacked, with the same outputs. (Scales and biases of float32 do not go
+    through float16 on the way: with the offset that would move every value by up to 2^-10.)"""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    tokens, past = 130, 700
+    q = torch.randn((1, 2, tokens, 256), device="cuda", generator=gen)
+    k, v = (torch.randn((1, 2, past + tokens, 256), device="cuda", generator=gen).mul_(0.1).add_(offset).to(dtype) for _ in range(2))
+    tk, tv = kquant.quantize(k), kquant.quantize(v)
+    dk, dv = kquant.dequantize(*tk), kquant.dequantize(*tv)
+    outs = []
+    for batch in (1, 2):
+        wide = lambda t: t.expand(batch, *t.shape[1:]).contiguous()
+        prefix = [t[:, :, :past].view(torch.int32) if t.dtype == torch.uint32 else t[:, :, :past] for t in (*tk, *tv)]
+        prefix = [wide(t) for t in prefix]
+        outs.append(kquant.sdpa_fa_prefill_q8(wide(q), *prefix, wide(dk[:, :, past:]), wide(dv[:, :, past:]), 256 ** -0.5))
+    assert outs[1][0].equal(outs[1][1]) and outs[1][0].equal(outs[0][0])
+    want = qwen.causal_prefill_attention(q.cpu().numpy(), dk.float().cpu().numpy(), dv.float().cpu().numpy(), 256 ** -0.5, past=past)
+    assert np.abs(outs[1][:1].cpu().numpy() - want).max() < 2e-3
+
+
+# finite values beyond float16 saturate where the prefix is unpacked for a long chunk, as they do where it is converted
+def test_unpacked_values_beyond_float16_saturate():
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    tokens, past = 140, 2000
+    q, k, v = (torch.randn((1, 2, past + tokens, 256), device="cuda", generator=gen).mul_(0.1) for _ in range(3))
+    v[0, 1, 900, 70] = 3.0e5
+    prefix = [t[:, :, :past] for t in (*kquant.quantize(k), *kquant.quantize(v))]
+    dk, dv = (kquant.dequantize(*kquant.quantize(x)) for x in (k, v))
+    got = kquant.sdpa_fa_prefill_q8(q[:, :, past:], *prefix, dk[:, :, past:], dv[:, :, past:], 256 ** -0.5).cpu().numpy()
+    want = qwen.causal_prefill_attention(q[:, :, past:].cpu().numpy(), dk.cpu().numpy(), dv.clamp(-65504.0, 65504.0).cpu().numpy(),
+                                         256 ** -0.5, past=past)
+    assert np.isfinite(got).all()
+    # (the group's other values carry the bias's float32 rounding of 3e5 / 255 steps; 2^-10 of a value for the weights)
+    assert (np.abs(got - want) <= 2e-3 + 2.0 ** -9 * np.abs(want)).all()
+
+
 # unpacked in the attention kernel; converted to float16; to bfloat16: one key range, several, and merges of two waves a row
-@pytest.mark.parametrize("tokens,past", [(17, 40), (17, 5000), (203, 301), (300, 9000), (1024, 70)])
+@pytest.mark.parametrize("tokens,past", [(17, 40), (17, 5000), (203, 301), (203, 14000), (300, 9000), (1024, 70)])
 @pytest.mark.parametrize("side", ["key", "value"])
 @pytest.mark.parametrize("bad", ["infinite activation", "infinite bias", "NaN scale"])
 def test_infinities_and_nan_of_a_quantised_prefix_reach_the_output(tokens, past, side, bad):

@@ -18,12 +18,13 @@ def converted(heads, kv_heads, tokens, past, batch=1):
 
 
 def test_few_workgroups_to_a_tile_unpack_a_long_prefix():
-    # (us unpacked and converted: 4 / 4 heads, 256 over 16000 rows 53 and 64; 16 / 4, 160 over 16000 79 and 87)
+    # (us unpacked and converted: 4 / 4 heads, 256 over 16000 rows 53 and 65; 16 / 4, 160 over 16000 82 and 88)
     assert not converted(4, 4, 256, 16000) and not converted(4, 4, 512, 8000) and not converted(16, 4, 160, 16000)
     assert not converted(8, 2, 160, 12000) and not converted(16, 4, 257, 32000)
     assert converted(16, 4, 160, 2000) and converted(16, 4, 512, 16000)
-    assert converted(16, 2, 203, 9001) and converted(16, 2, 160, 12288) and not converted(16, 2, 160, 12289)
-    assert converted(16, 2, 160, 6144, batch=2) and not converted(16, 2, 160, 6145, batch=2)
+    assert converted(16, 2, 203, 9001) and converted(16, 2, 160, 16384) and not converted(16, 2, 160, 16385)
+    assert converted(16, 2, 160, 13824, batch=2) and not converted(16, 2, 160, 13825, batch=2)
+    assert converted(16, 2, 256, 16384) and not converted(16, 2, 256, 16385) and converted(16, 2, 257, 33333)
 
 
 def test_short_chunks_unpack_and_long_ones_convert():
