@@ -402,14 +402,15 @@ bool mspr_indexed_prefill_fits(int batch, int n_heads, int n_tokens, int n_idx) 
 static int tiles_of(int64_t rows) { return (int)((rows + kTile - 1) / kTile); }
 
 // Two workgroups on each of 256 CUs are a round; what is left of the last one runs one to a CU, and if it is few units the
-// chip is idle. They are cut into as many key ranges as keep the partials (128 KB each) under 24 MB, or, where those would be
-// one or two and no round is in front, as leave one workgroup to a CU; with at least two id tiles in each. Whether that pays is estimated: a tile
-// takes 1.13 us alone and about 1 us under the round in front, and the partials and their merge cost what was fitted to 1
-// to 96 units of 128 to 1024 ids and a window of 128, whole and in 2 to 8 ranges (float16 and float32 queries, pools of
-// 1200 to 6000 rows). Whole and cut, us: 512 ids 1 token 30 and 13, 16 tokens 31 and 21, 64 tokens 31 and 27, 80 tokens 31 and
-// 29 (in two ranges 32), 96 tokens 31 and 34 (left whole); 513 tokens 73 and 58, 576 tokens 75 and 71. 256 ids 24 tokens 21.5 and
-// 19.9, 48 tokens 21.5 and 23.2 (left whole). 128 ids 8 tokens 16.6 and 14.9, 24 tokens 16.9 and 18.0, 64 tokens 17 and 25 (left
-// whole), 520 tokens 40.7 and 40.2, 560 tokens 41.2 and 44.4 (left whole).
+// chip is idle. They are cut into as many key ranges as keep the partials (128 KB each) under 24 MB, or, where those would
+// be one or two and no round is in front, as leave one workgroup to a CU; with at least two id tiles in each. Whether that
+// pays is estimated: a tile takes 1.13 us alone and about 1 us under the round in front, and the partials and their merge
+// cost what was fitted to 1 to 96 units of 128 to 1024 ids and a window of 128, whole and in 2 to 8 ranges (float16 and
+// float32 queries, pools of 1200 to 6000 rows). Whole and cut, us: 512 ids 1 token 30 and 13, 16 tokens 31 and 21, 64
+// tokens 31 and 27, 80 tokens 31 and 29 (in two ranges 32), 96 tokens 31 and 34 (left whole); 513 tokens 73 and 58, 576
+// tokens 75 and 71. 256 ids 24 tokens 21.5 and 19.9, 48 tokens 21.5 and 23.2 (left whole). 128 ids 8 tokens 16.6 and 14.9,
+// 24 tokens 16.9 and 18.0, 64 tokens 17 and 25 (left whole), 520 tokens 40.7 and 40.2, 560 tokens 41.2 and 44.4 (left
+// whole).
 // The kernel deals out the tiles of a window of `window_rows` and all of a token's ids; `tiles` of them hold rows at most.
 static void cut_last_round(IndexedPrefillArgs& a, int64_t window_rows, int tiles) {
   const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
