@@ -888,6 +888,315 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
   }
 }
 
+// Rows of up to 4 P THREADS scores, one a workgroup, where k is a small part of them: what is done per key is one comparison
+// with a pivot that lies below the k-th key nearly always, and the rest is done on the keys at or above it.
+//  * Every wave takes 64 S keys spread over the row and finds the 16-bit prefix of the `rank`-th of them with ballots; the
+//    mean of the waves' prefixes is the pivot. One barrier, no histogram.
+//  * The rows at or above it go to a list in LDS, in any order; their keys are read from a copy of the row in LDS.
+//  * 256 bins over [pivot, highest sample] hold the k-th key; a bin of up to 64 keys (nearly always the first one) is ranked
+//    directly, otherwise it becomes the span.
+//  * Selected rows set their bit in a bitmap of the row. Bits come out in row order, so nothing before has to keep it.
+// Keys are compared as signed integers: the bits of a float32 themselves where the pivot is positive, all others after the
+// map that inverts the low bits of negative values. Whether the list contains the k-th key is checked exactly; if it does not
+// (or does not fit), the same binning runs over all keys, so the result never depends on the sample.
+// What bounds it: a CU takes 2000 cycles to fetch a row of 32768 scores, and an instruction per key is 500 cycles of its vector
+// units: the blocked kernel above maps and moves every key (two LDS passes) and takes five digit passes, 16 rows of 32768,
+// k = 2048, 10.0 us, now 8.6. For many rows it is instructions: 3844 rows of 7961, k = 512, 57 us, now 28. (Keys read again
+// from the L2 instead of from a copy of the row in LDS: 64 lines an instruction, 3 us more for 16 rows; neighbouring lanes on
+// neighbouring list entries: their bits meet in the same words, 1 us more.)
+constexpr int32_t kLowestKey = (int32_t)0x80000000u;
+
+__device__ __forceinline__ int32_t signed_key(int32_t bits) { return bits ^ (int32_t)((uint32_t)(bits >> 31) >> 1); }
+
+template <int P, int THREADS, int S>
+__global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __restrict__ scores_all, int64_t score_stride,
+                                                               int n_rows, int topk, int rank,
+                                                               int32_t* __restrict__ sel_all) {
+  constexpr int kW = THREADS / 64;
+  constexpr int kEach = 8;                 // list entries of a thread at most
+  constexpr int kCap = kEach * THREADS;
+  constexpr uint32_t kBits = 4 * P;        // of the bitmap, to a word: a word a thread
+  constexpr uint32_t kBins = 256;
+  static_assert(kBits <= 32 && S <= P && kBins <= THREADS && 16 % kW == 0, "a bin a thread, a piece a sample");
+  __shared__ __attribute__((aligned(16))) int32_t stage[4 * P * THREADS];
+  __shared__ uint16_t list[kCap];
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kBins];
+  __shared__ uint32_t bits_above[THREADS], bits_tie[THREADS];
+  __shared__ uint32_t wave_pivot[kW], wave_high[kW];
+  __shared__ uint32_t wave_tot[kW];
+  __shared__ __attribute__((aligned(16))) uint32_t near[64];
+  __shared__ uint32_t kth[2];
+  __shared__ Pick pick_box;
+  __shared__ uint32_t n_list, n_near;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float* scores = scores_all + (int64_t)blockIdx.x * score_stride;
+  int32_t* sel = sel_all + (int64_t)blockIdx.x * topk;
+
+  // ---- keys: element e of piece j of a thread is row 4 (j THREADS + tid) + e; past the end the lowest key, which loses every
+  //      tie to a real row. (Rows start at any multiple of 4 bytes.)
+  typedef __attribute__((ext_vector_type(4), aligned(4))) int i32x4_any_t;
+  typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+  i32x4_t key[P];
+  const int last_whole = (n_rows - 4) & ~3;  // (n_rows is at least 4)
+#pragma unroll
+  for (int j = 0; j < P; j++) {
+    const int r = 4 * (j * THREADS + tid);
+    key[j] = *reinterpret_cast<const i32x4_any_t*>(scores + (r < last_whole ? r : last_whole));
+  }
+  if (tid < (int)kBins) hist[tid] = 0u;
+  bits_above[tid] = 0u;
+  bits_tie[tid] = 0u;
+  if (tid == 0) {
+    n_list = 0u;
+    n_near = 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < P; j++) {
+    const int r = 4 * (j * THREADS + tid);
+    if (j == P - 1 || 4 * (j + 1) * THREADS > n_rows) {  // (uniform: pieces in front of the row's end are whole)
+      if (r + 3 >= n_rows) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) key[j][e] = r + e < n_rows ? __float_as_int(scores[r + e]) : -1;
+      }
+    }
+  }
+
+#pragma unroll
+  for (int j = 0; j < P; j++) *reinterpret_cast<i32x4_t*>(&stage[4 * (j * THREADS + tid)]) = key[j];
+
+  // ---- this wave's sample: lane l takes element l / P % 4 of pieces l + i of the P
+  uint32_t sample[S];
+  uint32_t high = 0u;
+#pragma unroll
+  for (int i = 0; i < S; i++) {
+    const int piece = (lane + i) % P, e = (lane / P) & 3;
+    int32_t v = 0;
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const int32_t x = e & 2 ? (e & 1 ? key[j].w : key[j].z) : (e & 1 ? key[j].y : key[j].x);
+      v = piece == j ? x : v;
+    }
+    sample[i] = (uint32_t)signed_key(v) ^ 0x80000000u;
+    high = umax(high, sample[i]);
+  }
+  high = wave_max(high);
+  uint32_t prefix = 0u;
+#pragma unroll
+  for (int bit = 31; bit >= 16; bit--) {
+    const uint32_t with = prefix | (1u << bit);
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < S; i++) n += (int)__popcll(__ballot(sample[i] >= with));
+    prefix = n >= rank ? with : prefix;
+  }
+  if (lane == 0) {
+    wave_pivot[wave] = prefix >> 16;
+    wave_high[wave] = high;
+  }
+  __syncthreads();
+  int32_t pivot, span_end;
+  {
+    uint32_t sum = wave_pivot[lane % kW], top = wave_high[lane % kW];  // (the same sixteen values in every row of lanes)
+    sum += dpp_u32<0x128>(sum);
+    sum += dpp_u32<0x124>(sum);
+    sum += dpp_u32<0x122>(sum);
+    sum += dpp_u32<0x121>(sum);
+    top = umax(top, dpp_u32<0x128>(top));
+    top = umax(top, dpp_u32<0x124>(top));
+    top = umax(top, dpp_u32<0x122>(top));
+    top = umax(top, dpp_u32<0x121>(top));
+    pivot = __builtin_amdgcn_readfirstlane((int)(((sum >> 4) << 16) ^ 0x80000000u));
+    span_end = __builtin_amdgcn_readfirstlane((int)(top ^ 0x80000000u));
+  }
+  const bool mapped = pivot <= 0;  // uniform
+  if (mapped) {
+#pragma unroll
+    for (int j = 0; j < P; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
+  }
+
+  // ---- rows at or above the pivot
+  uint32_t mask = 0u;
+#pragma unroll
+  for (int j = P - 1; j >= 0; j--)
+#pragma unroll
+    for (int e = 3; e >= 0; e--) mask = shift_in(mask, key[j][e] >= pivot);
+  const uint32_t cnt = (uint32_t)__popc(mask);
+  const uint32_t incl = wave_prefix_sum(cnt);
+  uint32_t base = 0u;
+  if (lane == 63) base = atomicAdd(&n_list, incl);
+  base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63);
+  if (base + (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) <= (uint32_t)kCap) {
+    uint16_t* at = list + base + incl - cnt;
+    while (mask) {
+      const int i = __builtin_ctz(mask);
+      mask &= mask - 1u;
+      *at++ = (uint16_t)(4 * ((i >> 2) * THREADS + tid) + (i & 3));
+    }
+  }
+  __syncthreads();
+  const uint32_t total = n_list;
+  const bool fits = total >= (uint32_t)topk && total <= (uint32_t)kCap && pivot != kLowestKey;  // uniform
+
+  // ---- the k-th key among the elements that `each` hands out (key in the signed order, row; keys below `lo` do not count),
+  //      then the selected rows
+  auto select = [&](auto each, int32_t lo, int32_t end) {
+    uint32_t need = (uint32_t)topk;
+    uint32_t span = end > lo ? (uint32_t)end - (uint32_t)lo : 0u;  // to a guess of the highest key; what is above is in the last bin
+    uint32_t limit = 0xFFFFFFFFu;  // distance from lo that the keys in question have at most
+    int32_t threshold;
+    while (true) {
+      const int shift = span >= kBins ? 24 - __builtin_clz(span) : 0;
+      each([&](int32_t k, int) {
+        const uint32_t d = (uint32_t)k - (uint32_t)lo;
+        if (k >= lo && d <= limit) atomicAdd(&hist[umin(d >> shift, kBins - 1u)], 1u);
+      });
+      __syncthreads();
+      if (wave == 0) {
+        const Pick pk = pick_bucket(hist, need, lane);
+        if (lane == 0) pick_box = pk;
+      }
+      __syncthreads();
+      const uint32_t bin = pick_box.digit, held = pick_box.live;
+      need = pick_box.need;
+      lo = (int32_t)((uint32_t)lo + (bin << shift));
+      const uint32_t rest = limit - (bin << shift), width = bin == kBins - 1u ? 0xFFFFFFFFu : (1u << shift) - 1u;
+      limit = rest < width ? rest : width;
+      if (limit == 0u) {
+        threshold = lo;
+        break;
+      }
+      if (held <= 64u) {
+        each([&](int32_t k, int) {
+          const bool in = k >= lo && (uint32_t)k - (uint32_t)lo <= limit;
+          if (__ballot(in) != 0ull) {  // (few waves hold any)
+            if (in) near[atomicAdd(&n_near, 1u)] = (uint32_t)k - (uint32_t)lo;
+          }
+        });
+        __syncthreads();
+        // sixteen lanes rank a candidate, each against four of them at a time
+        constexpr int kAtOnce = THREADS / 16;
+#pragma unroll
+        for (int c0 = 0; c0 < 64; c0 += kAtOnce) {
+          if (c0 > 0 && (uint32_t)c0 >= held) break;  // uniform
+          const int c = c0 + (tid >> 4);
+          const uint32_t mine = near[c];
+          const u32x4_t o = *reinterpret_cast<const u32x4_t*>(&near[4 * (lane & 15)]);
+          uint32_t n = 0u;  // higher ones, equal ones in the upper half
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const bool in = (uint32_t)(4 * (lane & 15) + j) < held;
+            n += in && o[j] > mine ? 1u : 0u;
+            n += in && o[j] == mine ? 1u << 16 : 0u;
+          }
+          n += dpp_u32<0x128>(n);
+          n += dpp_u32<0x124>(n);
+          n += dpp_u32<0x122>(n);
+          n += dpp_u32<0x121>(n);
+          const uint32_t above = n & 0xFFFFu;
+          if ((lane & 15) == 0 && (uint32_t)c < held && above < need && above + (n >> 16) >= need) {  // (all equal ones write the same)
+            kth[0] = mine;
+            kth[1] = need - above;
+          }
+        }
+        __syncthreads();
+        threshold = (int32_t)((uint32_t)lo + kth[0]);
+        need = kth[1];
+        break;
+      }
+      span = limit;
+      if (tid < (int)kBins) hist[tid] = 0u;
+      __syncthreads();
+    }
+    each([&](int32_t k, int row) {
+      const uint32_t word = (uint32_t)row / kBits, bit = 1u << ((uint32_t)row % kBits);
+      if (k > threshold) atomicOr(&bits_above[word], bit);
+      if (k == threshold) atomicOr(&bits_tie[word], bit);
+    });
+    __syncthreads();
+    uint32_t wa = bits_above[tid], wt = bits_tie[tid];
+    const uint32_t mine = (uint32_t)__popc(wa) | ((uint32_t)__popc(wt) << 16);
+    const uint32_t upto = wave_prefix_sum(mine);
+    if (lane == 63) wave_tot[wave] = upto;
+    __syncthreads();
+    const uint32_t tots = wave_prefix_sum(lane < kW ? wave_tot[lane < kW ? lane : 0] : 0u);
+    const uint32_t excl = upto - mine + (wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)tots, wave > 0 ? wave - 1 : 0) : 0u);
+    int32_t* out = sel + (excl & 0xFFFFu);
+    uint32_t order = excl >> 16;
+    while (wa) {
+      *out++ = (int)kBits * tid + (int)__builtin_ctz(wa);
+      wa &= wa - 1u;
+    }
+    out = sel + ((uint32_t)topk - need);
+    while (wt && order < need) {
+      out[order++] = (int)kBits * tid + (int)__builtin_ctz(wt);
+      wt &= wt - 1u;
+    }
+  };
+
+  if (fits) {
+    constexpr int kHalf = kEach / 2;
+    int32_t lk[kEach];
+    int lr[kEach];
+    const bool more = total > (uint32_t)(kHalf * THREADS);  // uniform
+    // (entry j of a thread: neighbouring lanes take entries a wave count apart, whose rows are in different bitmap words)
+    const uint32_t first = (uint32_t)(lane * kW + wave);
+    auto fetch = [&](int j0) {
+#pragma unroll
+      for (int j = j0; j < j0 + kHalf; j++) lr[j] = (int)list[j * THREADS + first];
+#pragma unroll
+      for (int j = j0; j < j0 + kHalf; j++) lr[j] = (uint32_t)(j * THREADS) + first < total ? lr[j] : 0;
+#pragma unroll
+      for (int j = j0; j < j0 + kHalf; j++) lk[j] = stage[lr[j]];
+#pragma unroll
+      for (int j = j0; j < j0 + kHalf; j++) {
+        if (mapped) lk[j] = signed_key(lk[j]);
+        lk[j] = (uint32_t)(j * THREADS) + first < total ? lk[j] : kLowestKey;
+      }
+    };
+    fetch(0);
+    if (more) fetch(kHalf);
+    select(
+        [&](auto f) {
+#pragma unroll
+          for (int j = 0; j < kHalf; j++) f(lk[j], lr[j]);
+          if (more) {
+#pragma unroll
+            for (int j = kHalf; j < kEach; j++) f(lk[j], lr[j]);
+          }
+        },
+        pivot, span_end);
+  } else {
+    if (!mapped) {
+#pragma unroll
+      for (int j = 0; j < P; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
+    }
+    select(
+        [&](auto f) {
+#pragma unroll
+          for (int j = 0; j < P; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) f(key[j][e], 4 * (j * THREADS + tid) + e);
+        },
+        kLowestKey, 0x7FFFFFFF);
+  }
+}
+
+// Rank of the pivot in a wave's 64 S keys: as many as are expected above the k-th key of the (padded) row, and 3 standard
+// deviations of the mean of the waves' ranks on top. 0 where the keys above such a pivot would not fit the list.
+int sample_rank(int keys, int waves, int s, int cap, int topk) {
+  const double share = (double)topk / keys, n = 64.0 * s, expect = share * n;
+  const double dev = std::sqrt((expect > 1.0 ? expect : 1.0) * (1.0 - share) / waves);
+  const double rank = std::ceil(expect + 3.0 * dev + 0.5);
+  if (rank > n || (rank + 4.0 * dev) / n * keys > (double)cap) return 0;
+  return (int)rank;
+}
+
 // Rank, inside the 1024-row sample, of the pivot of the pivot path; 0 switches the path off. With k of
 // the C*1024 (padded) rows wanted, k/C sample rows are expected above the k-th key; the rank adds 4.5
 // standard deviations so that the survivors almost always include it, and the path is used only where
@@ -907,11 +1216,54 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
                      hipStream_t st) {
   dim3 grid((unsigned)batch), block(kThreads);
   MsprProfScope prof(MSPR_K_TOPK, st);
-  // Up to 4096 scores a row: 256 threads a row keep the most rows in flight; a row of more than 2048 that has a CU for
-  // itself is better off with 512 (189 rows of 3974 scores: 6.2 against 7.4 us; 517 of 2053: 7.7 against 6.7). Up to 8192
-  // many rows take the row kernel too (3844 rows of 7961 scores, k = 512: 58 against 67 us, 517 11.4 against 15.2), few take
-  // the blocked form, whose sample bounds a large k better (1 row, k = 2048: 8.6 against 7.9; 20 rows are equal). Past
-  // that its work per key is less (16 rows of 32768: 10 against 17 us).
+  // Rows of more than 2048 scores of which at most three eighths (past 4096: less than a half) are wanted are selected from the
+  // keys above a sampled pivot, where those fit its list: 512 threads a row, 256 where many rows share the CUs, 1024 for what
+  // only they can hold. us, the other kernels and this one: 1 row of 4096 scores, k = 512, 5.3 and 4.7; of 8192, k = 2048, 7.2
+  // and 6.5; 5 of 19211, k = 1024, 9.3 and 7.2; 16 of 32768, k = 2048, 10.0 and 8.6; 517 of 7000, k = 512, 10.5 and 7.5; 3844 of
+  // 3000 24.5 and 18.4, of 7961 57 and 28; 600 of 16384 27 and 20. At the lines: 4096 scores 1 row, k = 1500, 5.7 and 5.4, k =
+  // 2048 5.5 and 6.3; 2100 scores, k = 700, 1 row 4.9 and 5.1, 517 7.0 and 6.6; 1500 scores, k = 512, 4.5 and 4.9, 3844 rows 16.2
+  // and 16.4; 8192 scores, k = 3000, 7.5 and 7.3, k = 4000 7.6 and 9.1. 384 rows of 4096, k = 512: 512 threads 6.4, 256 6.0; 256
+  // rows 5.4 and 5.6.
+  if (n_rows > 2048 && n_rows <= 32768 && (n_rows <= 4096 ? 8 * (int64_t)topk <= 3 * n_rows : 2 * (int64_t)topk < n_rows)) {
+    auto pieces = [&](int threads) { return (int)((n_rows + 4 * threads - 1) / (4 * threads)); };
+    int p = 0, threads = 0, rank = 0;
+    if (n_rows > 8192) {
+      p = pieces(threads = 1024) == 7 ? 8 : pieces(1024);
+      rank = sample_rank(4 * 1024 * p, 16, 1, 8 * 1024, topk);
+    } else {
+      if (batch > 384) {
+        p = pieces(threads = 256) == 7 ? 8 : pieces(256);
+        rank = sample_rank(4 * 256 * p, 4, 2, 8 * 256, topk);
+      }
+      if (rank == 0) {
+        p = pieces(threads = 512);
+        rank = sample_rank(4 * 512 * p, 8, 2, 8 * 512, topk);
+      }
+    }
+#define MSPR_TOPK_SAMPLED(P, THREADS, S)                                                                                      \
+  if (rank > 0 && p == P && threads == THREADS) {                                                                             \
+    topk_sampled_kernel<P, THREADS, S><<<grid, dim3(THREADS), 0, st>>>(scores, score_stride, (int)n_rows, topk, rank, sel);    \
+    MSPR_CHECK_LAUNCH("topk_select");                                                                                         \
+    return MSPR_OK;                                                                                                           \
+  }
+    MSPR_TOPK_SAMPLED(3, 256, 2)
+    MSPR_TOPK_SAMPLED(4, 256, 2)
+    MSPR_TOPK_SAMPLED(5, 256, 2)
+    MSPR_TOPK_SAMPLED(6, 256, 2)
+    MSPR_TOPK_SAMPLED(8, 256, 2)
+    MSPR_TOPK_SAMPLED(2, 512, 2)
+    MSPR_TOPK_SAMPLED(3, 512, 2)
+    MSPR_TOPK_SAMPLED(4, 512, 2)
+    MSPR_TOPK_SAMPLED(3, 1024, 1)
+    MSPR_TOPK_SAMPLED(4, 1024, 1)
+    MSPR_TOPK_SAMPLED(5, 1024, 1)
+    MSPR_TOPK_SAMPLED(6, 1024, 1)
+    MSPR_TOPK_SAMPLED(8, 1024, 1)
+#undef MSPR_TOPK_SAMPLED
+  }
+  // The others. Up to 4096 scores a row: 256 threads a row keep the most rows in flight; a row of more than 2048 that has a CU
+  // for itself is better off with 512. Up to 8192 many rows take the row kernel too, few take the blocked form, whose sample
+  // bounds a large k better; past that its work per key is less.
 #define MSPR_TOPK_ROW(C, THREADS) \
   topk_row_kernel<C, THREADS><<<grid, dim3(THREADS), 0, st>>>(scores, score_stride, (int)n_rows, topk, sel)
   if (n_rows <= 1024) MSPR_TOPK_ROW(4, 256);
