@@ -351,6 +351,60 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   const int64_t qoff = (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
                        (int64_t)(q_live ? head : 0) * a.q_head_stride + dh * G::kPart + 8 * g;
   u32x4_t qf[G::kSteps];
+  // 16-bit queries are requested in runs of a head's row (a wave's share is 32 heads x kPart columns) and change places through
+  // LDS, in two passes of kQLo and kQHi 16-byte pieces a head: asked for in operand order, 32 bytes of each of 32 heads an
+  // instruction, the block kept the address unit busy for 2300 cycles in front of the tiles. With the tile slots below counted
+  // up instead of divided out, the first tile is multiplied 600 to 1500 cycles earlier: 1 sequence of 2048 + 128 rows 22.9 ->
+  // 22.3 us, 5 of 1024 + 128 28.0 -> 27.85, a token over 961 pool rows 27.3 -> 27.2.
+  constexpr int kQLo = 2 * ((G::kSteps + 1) / 2), kQHi = G::kPart / 8 - kQLo;
+  const bool q_pieces = QDT == kQSame && a.q_head_stride >= 0 && a.q_head_stride < (1 << 24);  // 32-bit offsets
+  const int q_heads_left = a.n_heads - hb * 64 - hg * 32;                                       // the rest repeat the first
+  auto q_request = [&]() {
+    const unsigned char* q0 = reinterpret_cast<const unsigned char*>(
+        reinterpret_cast<const uint16_t*>(a.q) + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
+        (q_heads_left > 0 ? (int64_t)(hb * 64 + hg * 32) * a.q_head_stride : (int64_t)0) + dh * G::kPart);
+    const uint32_t head_bytes = (uint32_t)a.q_head_stride * 2u;
+    int head_of = lane / kQLo, piece = lane - head_of * kQLo;
+#pragma unroll
+    for (int i = 0; i < kQLo / 2; i++) {
+      const uint32_t off = (head_of < q_heads_left ? (uint32_t)head_of : 0u) * head_bytes + (uint32_t)piece * 16u;
+      qf[i] = *reinterpret_cast<const u32x4_t*>(q0 + off);
+      piece += 64 % kQLo;
+      head_of += 64 / kQLo + (piece >= kQLo ? 1 : 0);
+      piece -= piece >= kQLo ? kQLo : 0;
+    }
+    head_of = lane / kQHi;
+    piece = lane - head_of * kQHi;
+#pragma unroll
+    for (int i = 0; i < kQHi / 2; i++) {
+      const uint32_t off = (head_of < q_heads_left ? (uint32_t)head_of : 0u) * head_bytes + (uint32_t)(kQLo + piece) * 16u;
+      qf[kQLo / 2 + i] = *reinterpret_cast<const u32x4_t*>(q0 + off);
+      piece += 64 % kQHi;
+      head_of += 64 / kQHi + (piece >= kQHi ? 1 : 0);
+      piece -= piece >= kQHi ? kQHi : 0;
+    }
+  };
+  // (a staging area of the wave's own in the third tile buffer and the scores' exchange, neither in use yet; the head's pieces
+  // lie an odd number of 16-byte slots apart)
+  auto q_exchange = [&]() {
+    static_assert(kWaves * 32 * (kQLo + 1) * 16 <= G::kTileBytes + 2 * G::kSxBytes, "query staging area");
+    unsigned char* st = lds + 2 * G::kTileBytes + wave * (32 * (kQLo + 1) * 16);
+    auto pass = [&](int i0, int per, int n_i) {
+      const int pitch = (per + 1) * 16;
+      int head_of = lane / per, piece = lane - head_of * per;
+#pragma unroll
+      for (int i = 0; i < n_i; i++) {
+        *reinterpret_cast<u32x4_t*>(st + head_of * pitch + piece * 16) = qf[i0 + i];
+        piece += 64 % per;
+        head_of += 64 / per + (piece >= per ? 1 : 0);
+        piece -= piece >= per ? per : 0;
+      }
+#pragma unroll
+      for (int i = 0; i < n_i; i++) qf[i0 + i] = *reinterpret_cast<const u32x4_t*>(st + n * pitch + (2 * i + g) * 16);
+    };
+    pass(0, kQLo, kQLo / 2);
+    pass(kQLo / 2, kQHi, kQHi / 2);
+  };
   f32x4_t qraw32[QDT == MSPR_F32 ? G::kSteps : 1][2];
   // The gathered ids of this thread's slots are requested before anything else: ids -> row pointers ->
   // rows is the longest dependency chain of the prologue. Local slot ls = tid + 512 j of the range.
@@ -369,18 +423,27 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
       qraw32[ks][1] = *reinterpret_cast<const f32x4_t*>(qp + 16 * ks + 4);
     }
   } else {
-    const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + qoff;
+    if (q_pieces) {
+      q_request();
+    } else {
+      const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + qoff;
 #pragma unroll
-    for (int ks = 0; ks < G::kSteps; ks++) qf[ks] = *reinterpret_cast<const u32x4_t*>(qp + 16 * ks);
+      for (int ks = 0; ks < G::kSteps; ks++) qf[ks] = *reinterpret_cast<const u32x4_t*>(qp + 16 * ks);
+    }
   }
 
   // ---- static part of this thread's tile loads: LDS slot P = tid + 512 j holds (row P / kSlots, chunk P % kSlots)
   uint32_t pk[G::kPerThread];
+  {
+    int row = tid / G::kSlots, chunk = tid - row * G::kSlots;
 #pragma unroll
-  for (int j = 0; j < G::kPerThread; j++) {
-    const int P = tid + kThreads * j;
-    const int row = P / G::kSlots, chunk = P % G::kSlots;
-    pk[j] = (P < G::kTileSlots && chunk != G::kSlots - 1) ? ((uint32_t)row << 16) | (uint32_t)(chunk * 16) : 0xFFFFFFFFu;
+    for (int j = 0; j < G::kPerThread; j++) {
+      const bool in_tile = j < G::kPerThread - 1 || tid + kThreads * j < G::kTileSlots;
+      pk[j] = in_tile && chunk != G::kSlots - 1 ? ((uint32_t)row << 16) | (uint32_t)(chunk * 16) : 0xFFFFFFFFu;
+      chunk += kThreads % G::kSlots;
+      row += kThreads / G::kSlots + (chunk >= G::kSlots ? 1 : 0);
+      chunk -= chunk >= G::kSlots ? G::kSlots : 0;
+    }
   }
   const uint64_t zero_row = reinterpret_cast<uint64_t>(&g_zero_row[0]);
   // asynchronous loads of one tile straight into its LDS ring buffer: source addresses first (LDS
@@ -501,6 +564,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   } else {
 #pragma unroll
     for (int ks = 0; ks < G::kSteps; ks++) asm volatile("" : "+v"(qf[ks]));
+    if (q_pieces) q_exchange();
   }
   // two tiles are in flight when the tile loop starts
   if (wt < 1 && n_tiles > 0) issue_tile(0);
