@@ -158,8 +158,9 @@ __device__ __forceinline__ uint32_t score_key(float s) {
 // a float64 log decides it, which rounds to the same float32 value the table path assumes.
 // `tab` may be a copy of the table in LDS.
 __device__ __forceinline__ float pow2_group_scale(float amax, float denom, const float* tab = g_pow2_tab) {
-  float r = amax / denom;
-  uint32_t u = __float_as_uint(r);
+  // (the product with the reciprocal is off by two units of the quotient's last place at most, which changes neither the
+  // exponent nor the outcome of these bounds' use: closer to a power of two the quotient itself decides)
+  const uint32_t u = __float_as_uint(amax * (1.0f / denom));
   uint32_t ex = (u >> 23) & 0xFFu;
   uint32_t man = u & 0x7FFFFFu;
   bool fast = (u >> 31) == 0u && ex != 0u && ex != 0xFFu && man > 0x800u && man < 0x7FF800u;
@@ -167,6 +168,7 @@ __device__ __forceinline__ float pow2_group_scale(float amax, float denom, const
     int k = (int)ex - 127 + 1;
     return tab[k - MSPR_POW2_TAB_MIN];
   }
+  const float r = amax / denom;
   float l = (float)log((double)r);
   float l2 = l / MSPR_LN2F;
   float e = ceilf(l2) * MSPR_LN2F;

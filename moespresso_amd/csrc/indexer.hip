@@ -103,22 +103,25 @@ __device__ __forceinline__ float qat_scale(float amax, const float* tab = g_pow2
 // comparisons kept the vector units busy for 3.6 of the 12.6 us of a score row over 961 pool rows; the QAT of 3844
 // tokens' 64 heads took 49 us with them and 37 without.
 template <bool LIVE = false>
+__device__ __forceinline__ float qat_snap_pow2(float x, uint32_t scale_bits) {
+  const float inv = __uint_as_float(0x7F000000u - scale_bits);         // 1 / scale
+  const float half_scale = __uint_as_float(scale_bits - 0x00800000u);  // scale / 2
+  const float n = fminf(fabsf(x) * inv, 6.0f);
+  const uint32_t nbits = __float_as_uint(n);
+  const uint32_t p = (nbits > 0x3F800000u ? nbits : 0x3F800000u) & 0x7F800000u;  // twice the step: 1, 2 or 4
+  const float per_step = __uint_as_float(0x7F800000u - p);
+  const float t = LIVE ? rintf(n * per_step) : ceilf(__builtin_fmaf(n, per_step, -0.5f));
+  const float v = fabsf(t * (__uint_as_float(p) * half_scale));  // ceil leaves -0
+  return x < 0.0f ? -v : v;
+}
+
+template <bool LIVE = false>
 __device__ __forceinline__ f32x4_t qat_snap(f32x4_t x, float scale) {
   f32x4_t out;
   const uint32_t sbits = __float_as_uint(scale);
   if (__all((sbits & 0x807FFFFFu) == 0u && sbits - 0x20000000u < 0x40000000u)) {  // 2^-63 up to 2^64
-    const float inv = __uint_as_float(0x7F000000u - sbits);         // 1 / scale
-    const float half_scale = __uint_as_float(sbits - 0x00800000u);  // scale / 2
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float n = fminf(fabsf(x[j]) * inv, 6.0f);
-      const uint32_t nbits = __float_as_uint(n);
-      const uint32_t p = (nbits > 0x3F800000u ? nbits : 0x3F800000u) & 0x7F800000u;  // twice the step: 1, 2 or 4
-      const float per_step = __uint_as_float(0x7F800000u - p);
-      const float t = LIVE ? rintf(n * per_step) : ceilf(__builtin_fmaf(n, per_step, -0.5f));
-      const float v = fabsf(t * (__uint_as_float(p) * half_scale));  // ceil leaves -0
-      out[j] = x[j] < 0.0f ? -v : v;
-    }
+    for (int j = 0; j < 4; j++) out[j] = qat_snap_pow2<LIVE>(x[j], sbits);
     return out;
   }
 #pragma unroll
@@ -163,6 +166,70 @@ __device__ __forceinline__ f32x4_t load_row4(const void* base, int64_t row, int 
     }
   }
   return v;
+}
+
+// QAT of a 128-wide row held by eight lanes, sixteen consecutive elements each: the same operations in the same order as
+// qat128, four of the seven butterfly stages and the group maximum inside a lane. For a block that has to be prepared in a
+// hurry: with 32 lanes a row every lane exchanges in five stages and works out its group's scale with seven others.
+// (Maxima are taken on the bits of the magnitudes, where a NaN exceeds all numbers.)
+struct Qat16 {
+  float x[16];
+  float amax;
+};
+
+template <int M>
+__device__ __forceinline__ void butterfly_lanes(float (&x)[16], int lane) {
+  const float sgn = (lane & M) ? -1.0f : 1.0f;
+#pragma unroll
+  for (int j = 0; j < 16; j++) x[j] = __builtin_fmaf(x[j], sgn, lane_xor<M>(x[j]));
+}
+
+__device__ __forceinline__ void qat16_rotate(Qat16& r, int lane) {
+#pragma unroll
+  for (int m = 1; m < 16; m <<= 1)
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+      if ((j & m) == 0) {
+        const float a = r.x[j], b = r.x[j + m];
+        r.x[j] = a + b;
+        r.x[j + m] = a - b;
+      }
+  butterfly_lanes<1>(r.x, lane);
+  butterfly_lanes<2>(r.x, lane);
+  butterfly_lanes<4>(r.x, lane);
+  uint32_t top = 0u;
+#pragma unroll
+  for (int j = 0; j < 16; j++) {
+    r.x[j] *= kHadamardScale;
+    const uint32_t b = __float_as_uint(r.x[j]) & 0x7FFFFFFFu;
+    top = b > top ? b : top;
+  }
+  const uint32_t other = (uint32_t)__float_as_int(lane_xor<1>(__int_as_float((int)top)));
+  r.amax = mx_floor_max(__uint_as_float(other > top ? other : top), kAmaxFloor);
+}
+
+// sixteen consecutive elements, widened to float32
+template <int DT>
+__device__ __forceinline__ void load_row16(const void* base, int64_t row, int part, float (&v)[16]) {
+  if constexpr (DT == MSPR_F32) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f32x4_t t = load_row4<DT>(base, row, 4 * part + i);
+      v[4 * i] = t.x;
+      v[4 * i + 1] = t.y;
+      v[4 * i + 2] = t.z;
+      v[4 * i + 3] = t.w;
+    }
+  } else {
+    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(base) + row * 128 + 16 * part);
+    const u32x4_t w[2] = {p[0], p[1]};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t x = w[i >> 2][i & 3];
+      v[2 * i] = DT == MSPR_F16 ? f16_bits_to_f32((uint16_t)x) : bf16_bits_to_f32((uint16_t)x);
+      v[2 * i + 1] = DT == MSPR_F16 ? f16_bits_to_f32((uint16_t)(x >> 16)) : bf16_bits_to_f32((uint16_t)(x >> 16));
+    }
+  }
 }
 
 // ------------------------------------------------------------------ QAT rows
@@ -284,20 +351,20 @@ __device__ __forceinline__ void rope_pair_f16(float x0, float x1, float c, float
   *o1 = h_round(m2 + m3);
 }
 
-// Prepared KV row of the decode island, one job for the first wave of a workgroup (every thread of the
+// Prepared KV row of the decode island, one job for the first waves of a workgroup (every thread of the
 // workgroup calls this and reaches its one barrier). Lane l of the lower half-wave holds dims
 // [16l, 16l+16): dims < 448 take the E4M3FN round trip of the float16 values widened to float32, dims
-// >= 448 the partial rope at float16 op rounding. The upper half-wave works out the 32 cosine / sine
-// pairs, one frequency per lane, while the lower one loads the row; the four rope lanes then pick their
+// >= 448 the partial rope at float16 op rounding. Two more waves work out the 32 cosines and sines,
+// one frequency per lane, while the first loads the row; the four rope lanes then pick their
 // eight pairs up from LDS (cs, sn: 32 floats each).
 __device__ __forceinline__ void kv_row_job(int tid, float* cs, float* sn, const uint16_t* __restrict__ kv,
                                            const float* __restrict__ inv_freq, const int32_t* __restrict__ params,
                                            uint16_t* __restrict__ row_out) {
   const int lane32 = tid & 31;
-  if (tid >= 32 && tid < 64) {
+  if (tid >= 64 && tid < 192 && (tid & 63) < 32) {  // (a wave each, they take as long as the rest of the job)
     const float theta = (float)params[0] * inv_freq[lane32];
-    cs[lane32] = h_round((float)cos((double)theta));
-    sn[lane32] = h_round((float)sin((double)theta));
+    if (tid < 128) cs[lane32] = h_round((float)cos((double)theta));
+    else sn[lane32] = h_round((float)sin((double)theta));
   }
   float xv[16];
   if (tid < 32) {
@@ -355,6 +422,7 @@ constexpr int kScoreWaves = kScoreThreads / 64;
 // float32 row pitch of the QAT'd query block in LDS: 128 values plus 4, so that the 16-byte reads of
 // 16 lanes holding 16 different heads fall into different banks
 constexpr int kQPitch = 132;
+constexpr int kQBfPitch = 272;  // bytes; the same for the block as bf16
 
 template <int DT, bool STAGE_HALF>
 __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* __restrict__ q, int n_heads,
@@ -388,14 +456,13 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
   const int64_t wave_stride = (int64_t)score_blocks * kScoreWaves;
   int64_t tile = (int64_t)blockIdx.x + (int64_t)wave * score_blocks;
 
-  // The eight waves QAT the 64 query rows, one row per half-wave and four rows per lane; the rows of a
-  // lane are fetched together and the power-of-two table sits in LDS, so the pass waits for memory once.
-  f32x4_t raw[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int h = 16 * i + wave * 2 + half;
-    raw[i] = load_row4<DT>(q, h < n_heads ? h : n_heads - 1, lane32);
-  }
+  // The eight waves QAT the 64 query rows, eight lanes a row; the power-of-two table sits in LDS, so the pass waits for memory
+  // once. Every workgroup does the whole block, so it is instructions of one CU that bound it: 7900 cycles with 32 lanes a row
+  // and the lattice step in float32 arithmetic, now 4000 to 4700 of the workgroup's 12200 (961 pool rows: the launch 8.4 -> 6.3
+  // us, a decode token 27.3 -> 25.4).
+  const int q_head = tid >> 3, q_part = tid & 7;
+  Qat16 mine;
+  load_row16<DT>(q, q_head < n_heads ? q_head : n_heads - 1, q_part, mine.x);
   const float tab_a = g_pow2_tab[tid < kPow2TabLen ? tid : 0];
   const float w_mine = weights[tid < n_heads ? tid : 0];
   // The first pool tile of the wave is requested now and lands while the queries are prepared. Lane
@@ -419,21 +486,57 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
   if (tid < kPow2TabLen) ptab[tid] = tab_a;
   if (tid < 64) wbuf[tid] = tid < n_heads ? w_mine : 0.0f;
   __syncthreads();
-  QatRotated rot[4];
+  qat16_rotate(mine, lane);
+  const float q_scale = qat_scale(mine.amax, ptab);
+  // Lattice values times powers of two from 2^-13 to 2^13 are float16 and bf16 numbers as they are, and the fp4 conversion
+  // makes them: it rounds ties to the even code where the lower value is wanted, which differs where the upper code is the even
+  // one. Just below a tie it rounds down, and one unit above a tie with an even lower code the value itself rounds up: of the
+  // codes of x and of the number below x the odd one is right where they differ.
+  const uint32_t q_bits = __float_as_uint(q_scale);
+  const bool plain = __syncthreads_and((q_bits & 0x807FFFFFu) == 0u && q_bits - 0x39000000u <= 0x0D000000u);
+  unsigned char* qbf = reinterpret_cast<unsigned char*>(qbuf);  // [head][kQBfPitch], bf16
+  bool q_exact = true;
+  if (plain) {
 #pragma unroll
-  for (int i = 0; i < 4; i++) rot[i] = qat_rotate(raw[i], lane32);
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int h = 16 * i + wave * 2 + half;
-    f32x4_t y = qat_snap(rot[i].x, qat_scale(rot[i].amax, ptab));
-    if (STAGE_HALF) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) y[j] = f16_bits_to_f32(f32_to_f16_bits(y[j]));
+    for (int hf = 0; hf < 2; hf++) {
+      const float* x = mine.x + 8 * hf;
+      constexpr float kBelow = 0x1.fffffep-1f;
+      uint32_t c = 0u, d = 0u;
+      c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[0], x[1], q_scale, 0);
+      c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[2], x[3], q_scale, 1);
+      c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[4], x[5], q_scale, 2);
+      c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[6], x[7], q_scale, 3);
+      d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, x[0] * kBelow, x[1] * kBelow, q_scale, 0);
+      d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, x[2] * kBelow, x[3] * kBelow, q_scale, 1);
+      d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, x[4] * kBelow, x[5] * kBelow, q_scale, 2);
+      d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, x[6] * kBelow, x[7] * kBelow, q_scale, 3);
+      const uint32_t odd = c & 0x11111111u, take = (odd << 4) - odd;
+      c = q_head < n_heads ? (c & take) | (d & ~take) : 0u;
+      *reinterpret_cast<u32x4_t*>(qbf + q_head * kQBfPitch + 32 * q_part + 16 * hf) =
+          u32x4_t{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 0)),
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 1)),
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 2)),
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 3))};
     }
-    if (h >= n_heads) y = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    reinterpret_cast<f32x4_t*>(qbuf + h * kQPitch)[lane32] = y;
+    __syncthreads();
+  } else {
+    uint32_t q_low = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      f32x4_t y = qat_snap(f32x4_t{mine.x[4 * i], mine.x[4 * i + 1], mine.x[4 * i + 2], mine.x[4 * i + 3]}, q_scale);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (STAGE_HALF) y[j] = f16_bits_to_f32(f32_to_f16_bits(y[j]));
+        if (q_head >= n_heads) y[j] = 0.0f;
+        q_low |= __float_as_uint(y[j]);
+      }
+      *reinterpret_cast<f32x4_t*>(qbuf + q_head * kQPitch + 16 * q_part + 4 * i) = y;
+    }
+    // a QAT'd value is a bf16 number (zero low half) unless the input was out of range; then the whole
+    // workgroup takes the three-piece form (the pieces come from LDS again, they are not kept in registers)
+    q_exact = __syncthreads_and((q_low & 0xFFFFu) == 0u);
   }
-  __syncthreads();
+  if (tile >= n_tiles) return;  // (a wave without a tile was here for its rows)
 
   // A operand: lane (m -> head, g) holds q[head][64 g + 8 s .. + 7] as bf16 for k-step s. Piece 0 is the
   // truncated value itself (all of it for a bf16 number), pieces 1 and 2 the truncated remainders.
@@ -447,21 +550,20 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     return u32x4_t{pack_hi16(v[0], v[1]), pack_hi16(v[2], v[3]), pack_hi16(v[4], v[5]), pack_hi16(v[6], v[7])};
   };
   u32x4_t qa[2][8];
-  uint32_t q_low = 0u;
 #pragma unroll
   for (int mt = 0; mt < 2; mt++) {
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(qbuf + (mt * 32 + m) * kQPitch + 64 * g + 8 * s);
-      const u32x4_t t0 = src[0], t1 = src[1];
-      qa[mt][s] = u32x4_t{__builtin_amdgcn_perm(t0.y, t0.x, 0x07060302u), __builtin_amdgcn_perm(t0.w, t0.z, 0x07060302u),
-                          __builtin_amdgcn_perm(t1.y, t1.x, 0x07060302u), __builtin_amdgcn_perm(t1.w, t1.z, 0x07060302u)};
-      q_low |= t0.x | t0.y | t0.z | t0.w | t1.x | t1.y | t1.z | t1.w;
+      if (plain) {
+        qa[mt][s] = *reinterpret_cast<const u32x4_t*>(qbf + (mt * 32 + m) * kQBfPitch + 128 * g + 16 * s);
+      } else {
+        const u32x4_t* src = reinterpret_cast<const u32x4_t*>(qbuf + (mt * 32 + m) * kQPitch + 64 * g + 8 * s);
+        const u32x4_t t0 = src[0], t1 = src[1];
+        qa[mt][s] = u32x4_t{__builtin_amdgcn_perm(t0.y, t0.x, 0x07060302u), __builtin_amdgcn_perm(t0.w, t0.z, 0x07060302u),
+                            __builtin_amdgcn_perm(t1.y, t1.x, 0x07060302u), __builtin_amdgcn_perm(t1.w, t1.z, 0x07060302u)};
+      }
     }
   }
-  // a QAT'd value is a bf16 number (zero low half) unless the input was out of range; then the whole
-  // workgroup takes the three-piece form (the pieces come from LDS again, they are not kept in registers)
-  const bool q_exact = __syncthreads_and((q_low & 0xFFFFu) == 0u);
   // head weights for this lane's accumulator rows: head = 32mt + 8(i/4) + 4g + i%4
   float wl[2][16];
 #pragma unroll
@@ -522,7 +624,7 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     for (int i = 0; i < 16; i++) {
       sum += mul_rn(mul_rn(fmaxf(acc1[i], 0.0f), scale), wl[1][i]);
     }
-    sum += __shfl_xor(sum, 32, MSPR_WAVE);
+    sum = half_wave_sum(sum);
     // fixed-capacity form: the pool buffer holds n_rows rows of which the first *valid_rows are in use (a
     // count that lives on the device, so that a captured launch follows a growing pool); the rest score -inf
     if (g == 0 && row < n_rows) scores[row] = (valid_rows && row >= (int64_t)valid_rows[0]) ? -__builtin_inff() : sum;
