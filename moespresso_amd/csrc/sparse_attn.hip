@@ -190,9 +190,11 @@ __device__ __forceinline__ void async_load_16(uint64_t src, uint32_t lds_base) {
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Normalised output values of four consecutive columns -> output tensor, in the output element type
-// (the fused-decode form applies the inverse partial rope on the float16 values at float16 op rounding).
+// (the fused-decode form applies the inverse partial rope on the float16 values at float16 op rounding; `rope_cs` holds the
+// cosines of the columns' pairs and, eight further on, their negated sines, where they are known).
 template <int ODT>
-__device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float (&r)[4], int64_t ooff, int dim0) {
+__device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float (&r)[4], int64_t ooff, int dim0,
+                                            const float* rope_cs = nullptr) {
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = f32x4_t{r[0], r[1], r[2], r[3]};
   } else if constexpr (ODT == MSPR_BF16) {
@@ -207,9 +209,15 @@ __device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         int p = (dim0 - (kDV - 64)) / 2 + j;
-        float theta = (float)a.params[0] * a.inv_freq[p];
-        float cs = f16_bits_to_f32(f32_to_f16_bits((float)cos((double)theta)));
-        float sn = f16_bits_to_f32(f32_to_f16_bits(-(float)sin((double)theta)));
+        float cs, sn;
+        if (rope_cs) {
+          cs = rope_cs[j];
+          sn = rope_cs[8 + j];
+        } else {
+          float theta = (float)a.params[0] * a.inv_freq[p];
+          cs = f16_bits_to_f32(f32_to_f16_bits((float)cos((double)theta)));
+          sn = f16_bits_to_f32(f32_to_f16_bits(-(float)sin((double)theta)));
+        }
         float x0 = h[2 * j], x1 = h[2 * j + 1];
         float m0 = f16_bits_to_f32(f32_to_f16_bits(x0 * cs)), m1 = f16_bits_to_f32(f32_to_f16_bits(x1 * sn));
         float m2 = f16_bits_to_f32(f32_to_f16_bits(x0 * sn)), m3 = f16_bits_to_f32(f32_to_f16_bits(x1 * cs));
@@ -227,6 +235,17 @@ __device__ __forceinline__ float load_sink_log2(const SparseAttnArgs& a, int hea
   if (!a.sinks) return -__builtin_inff();
   return (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.sinks)[head])
                                     : reinterpret_cast<const float*>(a.sinks)[head]) * 1.4426950408889634f;
+}
+
+// A pair (x0, x1) of float16 rotated: (x0 c - x1 s, x0 s + x1 c), every operation rounded to float16 (cc and ss hold the cosine
+// and the sine twice). The same values as float32 operations rounded to float16 one by one: products of two float16 numbers
+// are exact in float32, and a sum rounded to 24 bits first rounds to 11 as the exact one does.
+__device__ __forceinline__ uint32_t rope_pair_h2(uint32_t x, uint32_t cc, uint32_t ss) {
+#pragma clang fp contract(off)
+  typedef __attribute__((ext_vector_type(2))) _Float16 h2_t;
+  const h2_t v = __builtin_bit_cast(h2_t, x), s = __builtin_bit_cast(h2_t, ss);
+  const h2_t a = v * __builtin_bit_cast(h2_t, cc), b = h2_t{v.y, v.x} * s;
+  return __builtin_bit_cast(uint32_t, a + h2_t{-b.x, b.y});
 }
 
 template <int DK>
@@ -267,8 +286,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   float* sx = reinterpret_cast<float*>(lds + G::kOffSx);                       // [8 waves][16*64]
   uint64_t* rowptr = reinterpret_cast<uint64_t*>(lds + G::kOffRowPtr);         // [kMaxIds]
   uint32_t* vmask = reinterpret_cast<uint32_t*>(lds + G::kOffVmask);           // [kMaxTiles]
-  float* rope_c = reinterpret_cast<float*>(lds + G::kOffRope);
-  float* rope_s = rope_c + 32;
+  uint32_t* rope_c = reinterpret_cast<uint32_t*>(lds + G::kOffRope);           // each value twice, as a float16 pair
+  uint32_t* rope_s = rope_c + 32;
   int* stop_shared = reinterpret_cast<int*>(lds + G::kOffStop);
   unsigned char* p_lds = lds + G::kOffP;
   float* stat = reinterpret_cast<float*>(lds + G::kOffStat);
@@ -507,10 +526,10 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   }
 
   // ---- stop position of the gathered walk, rope table
-  if (ROPE && tid < 32) {
-    float theta = (float)a.params[0] * a.inv_freq[tid];
-    rope_c[tid] = f16_bits_to_f32(f32_to_f16_bits((float)cos((double)theta)));
-    rope_s[tid] = f16_bits_to_f32(f32_to_f16_bits((float)sin((double)theta)));
+  if (ROPE && tid < 128 && (tid & 63) < 32) {  // (a wave each for the cosines and the sines)
+    const float theta = (float)a.params[0] * a.inv_freq[tid & 31];
+    const uint32_t h = f32_to_f16_bits((float)(tid < 64 ? cos((double)theta) : sin((double)theta)));
+    (tid < 64 ? rope_c : rope_s)[tid & 31] = h | (h << 16);
   }
   int stop_pos = a.n_idx;
   if (a.check_stop) {
@@ -571,7 +590,23 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   if (wt < 2 && n_tiles > 1) issue_tile(1);
 
   // ---- finish the query operand (type conversion, rope) while the first tiles are in flight
-  if constexpr (QDT == kQSame && !ROPE) {
+  static_assert(!ROPE || QDT == kQSame, "queries that are rotated have the row type");
+  if constexpr (QDT == kQSame) {
+    if constexpr (ROPE) {
+      // Partial rope of the last 64 columns, pair by pair, in float16 arithmetic: every product and every sum is rounded to
+      // float16. (All columns taken through float32 and back, six roundings a pair: the first tile waited 3600 cycles for it.)
+      static_assert(KDT == MSPR_F16, "rotated in float16 arithmetic");
+      if (dh == 3) {
+        constexpr int kFirst = (G::kPart - 64) / 16;
+#pragma unroll
+        for (int ks = kFirst; ks < G::kSteps; ks++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const int p = (dh * G::kPart + 16 * ks + 8 * g - (DK - 64)) / 2 + j;
+            qf[ks][j] = rope_pair_h2(qf[ks][j], rope_c[p], rope_s[p]);
+          }
+      }
+    }
     if (!q_live) {
 #pragma unroll
       for (int ks = 0; ks < G::kSteps; ks++) qf[ks] = u32x4_t{0u, 0u, 0u, 0u};
@@ -580,30 +615,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
 #pragma unroll
     for (int ks = 0; ks < G::kSteps; ks++) {
       float v[8];
-      if constexpr (QDT == MSPR_F32) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = round_to_kdt<KDT>(qraw32[ks][j >> 2][j & 3]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          v[2 * j] = unpack_lo<KDT>(qf[ks][j]);
-          v[2 * j + 1] = unpack_hi<KDT>(qf[ks][j]);
-        }
-      }
-      const int d0 = dh * G::kPart + 16 * ks + 8 * g;
-      if (ROPE && d0 >= DK - 64) {
-        // partial rope on interleaved pairs with every product and sum rounded to the element type
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          int p = (d0 - (DK - 64)) / 2 + j;
-          float c = rope_c[p], s = rope_s[p];
-          float x0 = v[2 * j], x1 = v[2 * j + 1];
-          float m0 = round_to_kdt<KDT>(x0 * c), m1 = round_to_kdt<KDT>(x1 * s);
-          float m2 = round_to_kdt<KDT>(x0 * s), m3 = round_to_kdt<KDT>(x1 * c);
-          v[2 * j] = round_to_kdt<KDT>(m0 - m1);
-          v[2 * j + 1] = round_to_kdt<KDT>(m2 + m3);
-        }
-      }
+      for (int j = 0; j < 8; j++) v[j] = round_to_kdt<KDT>(qraw32[ks][j >> 2][j & 3]);
       qf[ks] = q_live ? u32x4_t{pack2<KDT>(v[0], v[1]), pack2<KDT>(v[2], v[3]), pack2<KDT>(v[4], v[5]),
                                  pack2<KDT>(v[6], v[7])}
                       : u32x4_t{0u, 0u, 0u, 0u};
@@ -1447,6 +1460,7 @@ template <int ODT>
 __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a) {
   __shared__ float xm[4][64], xl[4][64];
   __shared__ __attribute__((aligned(16))) float xo[4][2][64][4];
+  __shared__ float rope_cs[16];  // of the workgroup's sixteen columns: eight cosines, eight negated sines
   const int lane = threadIdx.x & 63;
   const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // a sequence's partials are merged on the XCD whose workgroups wrote them (the split kernel's mapping), so
@@ -1473,6 +1487,16 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   const f32x2_t* ml0 = reinterpret_cast<const f32x2_t*>(a.ws_ml) + part0 * 64 + hg * 32 + n;
   const f16x8_t* wo0 = reinterpret_cast<const f16x8_t*>(a.ws_o) + (part0 * kWaves + wave) * (int64_t)(8 * 64) + piece * 64 + lane;
   constexpr int kChunk = 8;
+  // The inverse rope of the last 64 columns: waves 2 and 3 work out the workgroup's cosines and sines in float64 while the
+  // partials are on their way (left to the end, for each pair anew, they were the last thing the launch waited for).
+  const int col0 = dh * 128 + 32 * (piece >> 1) + 16 * (piece & 1);
+  const bool rope = ODT == MSPR_F16 && a.rope && col0 >= kDV - 64;  // the same in every wave
+  auto rope_columns = [&]() {
+    if (rope && w4 >= 2 && lane < 8) {
+      const double theta = (double)((float)a.params[0] * a.inv_freq[(col0 - (kDV - 64)) / 2 + lane]);
+      rope_cs[8 * (w4 - 2) + lane] = f16_bits_to_f32(f32_to_f16_bits(w4 == 2 ? (float)cos(theta) : -(float)sin(theta)));
+    }
+  };
   float m_run = -__builtin_inff(), l = 0.0f;
   float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int s0 = w4; s0 < a.n_splits; s0 += 4 * kChunk) {
@@ -1489,6 +1513,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
         ov[j] = f16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
       }
     }
+    if (s0 == w4) rope_columns();
     float m_new = m_run;
 #pragma unroll
     for (int j = 0; j < kChunk; j++) m_new = fmaxf(m_new, ml[j].x);
@@ -1506,6 +1531,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
     }
     m_run = m_new;
   }
+  if (w4 >= a.n_splits) rope_columns();  // (no range for this wave)
   const float sink = live ? load_sink_log2(a, head) : -__builtin_inff();
   xm[w4][lane] = m_run;
   xl[w4][lane] = l;
@@ -1534,7 +1560,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   const int dim0 = dh * 128 + 32 * (piece >> 1) + 16 * (piece & 1) + 8 * w4 + 4 * g;
   const int64_t ooff = (int64_t)b * a.out_batch_stride + (int64_t)t * a.out_token_stride +
                        (int64_t)head * a.out_head_stride + dim0;
-  emit_output<ODT>(a, r, ooff, dim0);
+  emit_output<ODT>(a, r, ooff, dim0, rope ? rope_cs + (8 * w4 + 4 * g) / 2 : nullptr);
 }
 
 // Key ranges of one sequence at most (unless its table forces more): at 40 a window of 128 and 2048 ids are 34 ranges of

@@ -42,3 +42,22 @@ def test_single_keys_outgrow_the_maximum(dtype, spike, heads, k_dim, batch, ids)
     mass = p[..., :-1] @ np.abs(kvr[:, rows[0], :512].astype(np.float64))
     assert np.isfinite(got).all()
     assert (np.abs(got[pick] - want) <= 2e-3 + 3 * eps * mass).all(), (np.abs(got[pick] - want) - 3 * eps * mass).max()
+
+
+@pytest.mark.parametrize("window,ids", [(16, 16), (32, 32), (32, 64), (64, 65), (128, 300)])  # one tile each, 2, 3, 5 and 14 ranges
+def test_rotated_decode_with_few_key_ranges(window, ids):
+    from moespresso_amd.runtime.deepseek_v4 import decode_attention_kernel as dak
+
+    rng = np.random.default_rng(window + ids)
+    q, ring = (rng.standard_normal(s).astype(np.float16) for s in ((64, 512), (window, 512)))
+    row, pooled = (rng.standard_normal(s).astype(np.float16) for s in (512, (400, 512)))
+    sel = np.sort(rng.choice(400, ids, replace=False)).astype(np.int32)
+    sinks = rng.standard_normal(64).astype(np.float16)
+    inv = ds4.rope_inverse_frequencies(64, ds4.DS4_COMPRESS_ROPE_BASE, ds4.DS4_YARN).astype(np.float32)
+    params = np.array([12345, 5], dtype=np.int32)
+    got = dak.fused_decode_sdpa(*(torch.from_numpy(x).cuda() for x in (q, ring, row, pooled, sel, sinks, inv, params)),
+                                scale=512 ** -0.5).float().cpu().numpy()
+    want = ds4.fused_decode_sdpa(q, ring, row, pooled, sel, sinks, inv, params, scale=512 ** -0.5).astype(np.float32)
+    # weights, partial, output and the three roundings of the rotation in float16, of values of at most max |V|
+    bound = 2e-3 + 6 * 2.0 ** -11 * max(np.abs(ring).max(), np.abs(row).max(), np.abs(pooled).max())
+    assert np.abs(got - want).max() <= bound
