@@ -251,36 +251,95 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     async_load_16(vt, o1, dst + kTileBytes + 8192);
   };
 
+  // ---- asynchronous copies of raw prefix tiles (quantised-prefix form, see its loop below)
+  const int p_end = n_tiles < t1 ? n_tiles : t1;  // prefix tiles of this workgroup: [t_begin, p_end)
+  constexpr int kST = SDT % kExactUnpack;
+  constexpr int kSB = kST == MSPR_F32 ? 4 : 2;   // bytes per scale / bias
+  constexpr int kCodeBytes = kTile * kD;         // 8 KB of codes per tile, K and V each
+  constexpr int kScaleBytes = kTile * 4 * kSB;   // one tile of one scale or bias array: 256 or 512 B
+  constexpr int kRawBytes = 2 * kCodeBytes + 4 * 512;
+  constexpr int kRawBase = 2 * kStageBytes;      // the unpacked stages use the lower 64 KB
+  static_assert(kRawBase + 3 * kRawBytes <= kLdsBytes, "raw ring does not fit");
+  const int64_t raw_row0 = ((int64_t)b * a.n_kv_heads + kvh) * a.past_rows;
+  const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.pk_wq) + raw_row0 * kD;
+  const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.pv_wq) + raw_row0 * kD;
+  // scale / bias copies: wave w moves array w & 3 (K scale, K bias, V scale, V bias), 4 bytes per lane; with
+  // float32 scales waves 4-7 move the second 256 bytes, with 16-bit ones they repeat the copy of waves 0-3
+  // (every wave then issues the same number of copies and the waits below are static counts)
+  const int arr = wave & 3;
+  const uint8_t* sb_base = reinterpret_cast<const uint8_t*>(arr == 0 ? a.pk_s : arr == 1 ? a.pk_b : arr == 2 ? a.pv_s : a.pv_b) +
+                           raw_row0 * 4 * kSB;
+  const int sb_half = kSB == 4 ? (wave >> 2) * 256 : 0;
+  const uint32_t code_off = (uint32_t)tid * 16;  // K / V codes: LDS slot tid of the tile's 512
+  const uint32_t sb_off = (uint32_t)(sb_half + lane * 4);
+  auto issue_raw = [&](int t, int rslot) {
+    if (t > p_end - 1) t = p_end - 1;  // past the end: a harmless re-read, so that the counts stay static
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0) + kRawBase + rslot * kRawBytes;
+    async_load_16((uint64_t)(kc + (int64_t)t * kCodeBytes), code_off, dst + wave * 1024);
+    async_load_16((uint64_t)(vc + (int64_t)t * kCodeBytes), code_off, dst + kCodeBytes + wave * 1024);
+    async_load_4((uint64_t)(sb_base + (int64_t)t * kScaleBytes), sb_off, dst + 2 * kCodeBytes + arr * 512 + sb_half);
+  };
+  const bool raw_first = Q8 && t_begin < p_end;
+#ifndef MSPR_FP_TILES_AHEAD
+#define MSPR_FP_TILES_AHEAD 2
+#endif
+  constexpr int kTilesAhead = MSPR_FP_TILES_AHEAD;  // tiles in flight behind the one being consumed (at most kBufs - 1)
+  static_assert(kTilesAhead >= 1 && kTilesAhead <= kBufs - 2, "ring too small (64 KB of it pass the queries on at first)");
+  const int r0 = t_begin > t1 ? t_begin : t1;  // first tile of this workgroup that is served from k / v
+  auto issue_first_tiles = [&]() {
+#pragma unroll
+    for (int j = 0; j < kTilesAhead; j++) issue_tile(r0 + j < n_tiles ? r0 + j : n_tiles - 1, j);
+  };
+
   // ---- Q^T operand: lane (n, g) holds q[q0 + n][16 s + 8 g .. +7] for k-step s
   u32x4_t qf[16];
   {
-    int qrow = q0 + n;
-    if (qrow > a.q_len - 1) qrow = a.q_len - 1;
-    if (qrow < 0) qrow = 0;
-    const int64_t qoff = (((int64_t)b * a.n_q_heads + head) * a.q_len + qrow) * kD + 8 * g;
-    if constexpr (!IO32) {
-      const u32x4_t* qp = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(a.q) + qoff);
+    // The first tiles are requested, then the wave's 32 rows in two halves of 128 columns, in whole runs of 512 (256) bytes an
+    // instruction; they change lanes in 8 KB of LDS that no tile uses yet (piece p of row r at slot p ^ (r & 15)). Loads
+    // straight into the operand's lanes touch 32 lines an instruction, which the address unit takes one a clock: 8192
+    // clocks for the eight waves' float32 rows, of the 13000 before the first tile. With the stores below, us: 203 float32
+    // queries over 9001 quantised keys 78.5 -> 74.0 (whole operator with its append), 30 queries 46.4 -> 42.2, 203 bfloat16
+    // ones over 9001 dense keys 56.5 -> 53. Tiles requested behind the queries 1 us more, behind their exchange the same.
+    const int64_t qbase = ((int64_t)b * a.n_q_heads + head) * a.q_len;
+    constexpr int kLanes = IO32 ? 32 : 16;  // lanes of a row
+    constexpr int kRows = 64 / kLanes;      // rows of an instruction
+    const int xr = lane / kLanes, xc = lane % kLanes;
+    if (raw_first) {
+      issue_raw(t_begin, 0);
+      issue_raw(t_begin + 1, 1);
+      issue_raw(t_begin + 2, 2);
+    } else if (r0 < n_tiles) {
+      issue_first_tiles();
+    }
+    u32x4_t raw[2][32 / kRows];
 #pragma unroll
-      for (int s = 0; s < 16; s++) qf[s] = qp[2 * s];
-    } else {
-      const f32x4_t* qp = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff);
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-      for (int s0 = 0; s0 < 16; s0 += 4) {
-        f32x4_t raw[8];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          raw[2 * j] = qp[4 * (s0 + j)];
-          raw[2 * j + 1] = qp[4 * (s0 + j) + 1];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          qf[s0 + j] = u32x4_t{pack2<KDT>(raw[2 * j][0], raw[2 * j][1]), pack2<KDT>(raw[2 * j][2], raw[2 * j][3]),
-                               pack2<KDT>(raw[2 * j + 1][0], raw[2 * j + 1][1]),
-                               pack2<KDT>(raw[2 * j + 1][2], raw[2 * j + 1][3])};
+      for (int i = 0; i < 32 / kRows; i++) {
+        int qrow = q0 + i * kRows + xr;
+        if (qrow > a.q_len - 1) qrow = a.q_len - 1;
+        raw[h][i] = reinterpret_cast<const u32x4_t*>(a.q)[(qbase + qrow) * (2 * kLanes) + h * kLanes + xc];
       }
+    unsigned char* xq = lds + (raw_first ? 0 : kTilesAhead * kStageBytes) + (wave << 13);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+      for (int i = 0; i < 32 / kRows; i++) {
+        const int r = i * kRows + xr;
+        if constexpr (IO32) {
+          const f32x4_t v = __builtin_bit_cast(f32x4_t, raw[h][i]);
+          *reinterpret_cast<u32x2_t*>(xq + r * 256 + 16 * ((xc >> 1) ^ (r & 15)) + 8 * (xc & 1)) =
+              u32x2_t{pack2<KDT>(v.x, v.y), pack2<KDT>(v.z, v.w)};
+        } else {
+          *reinterpret_cast<u32x4_t*>(xq + r * 256 + 16 * (xc ^ (r & 15))) = raw[h][i];
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 8; s++)
+        qf[8 * h + s] = *reinterpret_cast<const u32x4_t*>(xq + n * 256 + 16 * ((2 * s + g) ^ (n & 15)));
     }
 #pragma unroll
-    for (int s = 0; s < 16; s++) asm volatile("" : "+v"(qf[s]));  // complete before the first asynchronous copy
+    for (int s = 0; s < 16; s++) asm volatile("" : "+v"(qf[s]));
   }
 
   f32x16_t oacc[8];
@@ -420,34 +479,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     //      tile t+1 is unpacked from there into the other float16 stage at the top of step t. No register
     //      carries raw bytes across a step (twelve more live registers did not fit next to the accumulators,
     //      and a spill of a freshly loaded value waits for the whole memory latency once per tile).
-    const int p_end = n_tiles < t1 ? n_tiles : t1;  // prefix tiles of this workgroup: [t_begin, p_end)
-    if (t_begin < p_end) {
-      constexpr int kST = SDT % kExactUnpack;
-      constexpr int kSB = kST == MSPR_F32 ? 4 : 2;   // bytes per scale / bias
-      constexpr int kCodeBytes = kTile * kD;         // 8 KB of codes per tile, K and V each
-      constexpr int kScaleBytes = kTile * 4 * kSB;   // one tile of one scale or bias array: 256 or 512 B
-      constexpr int kRawBytes = 2 * kCodeBytes + 4 * 512;
-      constexpr int kRawBase = 2 * kStageBytes;      // the unpacked stages use the lower 64 KB
-      static_assert(kRawBase + 3 * kRawBytes <= kLdsBytes, "raw ring does not fit");
-      const int64_t row0 = ((int64_t)b * a.n_kv_heads + kvh) * a.past_rows;
-      const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.pk_wq) + row0 * kD;
-      const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.pv_wq) + row0 * kD;
-      // scale / bias copies: wave w moves array w & 3 (K scale, K bias, V scale, V bias), 4 bytes per lane; with
-      // float32 scales waves 4-7 move the second 256 bytes, with 16-bit ones they repeat the copy of waves 0-3
-      // (every wave then issues the same number of copies and the waits below are static counts)
-      const int arr = wave & 3;
-      const uint8_t* sb_base = reinterpret_cast<const uint8_t*>(arr == 0 ? a.pk_s : arr == 1 ? a.pk_b : arr == 2 ? a.pv_s : a.pv_b) +
-                               row0 * 4 * kSB;
-      const int sb_half = kSB == 4 ? (wave >> 2) * 256 : 0;
-      const uint32_t code_off = (uint32_t)tid * 16;  // K / V codes: LDS slot tid of the tile's 512
-      const uint32_t sb_off = (uint32_t)(sb_half + lane * 4);
-      auto issue_raw = [&](int t, int rslot) {
-        if (t > p_end - 1) t = p_end - 1;  // past the end: a harmless re-read, so that the counts stay static
-        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0) + kRawBase + rslot * kRawBytes;
-        async_load_16((uint64_t)(kc + (int64_t)t * kCodeBytes), code_off, dst + wave * 1024);
-        async_load_16((uint64_t)(vc + (int64_t)t * kCodeBytes), code_off, dst + kCodeBytes + wave * 1024);
-        async_load_4((uint64_t)(sb_base + (int64_t)t * kScaleBytes), sb_off, dst + 2 * kCodeBytes + arr * 512 + sb_half);
-      };
+    if (raw_first) {
       auto unpack = [&](int rslot, int slot) {
         // (the per-thread offsets are re-derived from the thread index at each use, which the empty asm
         // enforces: carried across the loop they end up in scratch, and a reload waits behind the copies)
@@ -480,9 +512,6 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
         *reinterpret_cast<u32x4_t*>(st + kTileBytes + w_off0) = p0;
         *reinterpret_cast<u32x4_t*>(st + kTileBytes + w_off1) = p1;
       };
-      issue_raw(t_begin, 0);
-      issue_raw(t_begin + 1, 1);
-      issue_raw(t_begin + 2, 2);
       wait_vm_and_barrier<6>();  // the raw bytes of the first tile are in LDS
       unpack(0, 0);
       for (int t = t_begin; t < p_end; t++) {
@@ -505,15 +534,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   //      iteration t. (Running the two waves of a SIMD half a tile apart, one of them with stage 2 of tile
   //      t-1 in front of stage 1 of tile t, paid while the tile loop still reloaded spilled registers; without
   //      those reloads it measured 1.7 % slower than this order, and both waves deferred 5 % slower.)
-#ifndef MSPR_FP_TILES_AHEAD
-#define MSPR_FP_TILES_AHEAD 2
-#endif
-  constexpr int kTilesAhead = MSPR_FP_TILES_AHEAD;  // tiles in flight behind the one being consumed (at most kBufs - 1)
-  static_assert(kTilesAhead >= 1 && kTilesAhead <= kBufs - 1, "ring too small");
-  const int r0 = t_begin > t1 ? t_begin : t1;  // first tile of this workgroup that is served from k / v
   if (r0 < n_tiles) {
-#pragma unroll
-    for (int j = 0; j < kTilesAhead; j++) issue_tile(r0 + j < n_tiles ? r0 + j : n_tiles - 1, j);
+    if (raw_first) issue_first_tiles();
     for (int t = r0; t < n_tiles; t++) {
       // tile t has landed once this wave's copies of it are done (those of the newer tiles may be in flight:
       // four per tile) and every wave got here; the ring slot of tile t-1 is free after the barrier
@@ -527,42 +549,57 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped trailing copies must not outlive the workgroup's LDS
 
-  // ---- normalise and store: lane (n, g) holds dims 32 mt + 8 (i/4) + 4 g + i%4 of query row q0 + n
+  // ---- normalise and store: lane (n, g) holds dims 32 mt + 8 (i/4) + 4 g + i%4 of query row q0 + n. The values change
+  //      lanes in the wave's 16 KB of the ring, so that an instruction stores whole 512-byte runs of two rows and not 32
+  //      bytes of each of 32 (3.7 -> 2.7 us for float32 values; 256 KB a CU are 4096 clocks of its way to the L2).
   const float l_tot = l_run + __shfl_xor(l_run, 32, MSPR_WAVE);
-  if (a.n_splits > 1) {
-    if (active && q0 + n < a.q_len) {
-      const int64_t row = (((int64_t)sp * a.batch + b) * a.n_q_heads + head) * a.q_len + q0 + n;
-      float* po = a.ws_o + row * kD;
+  __syncthreads();  // every wave has left the tiles
+  int tl = tid;
+  asm volatile("" : "+v"(tl));  // (the offsets below are made here, not carried through the tile loop)
+  const int en = tl & 31, eg = (tl >> 5) & 1;
+  unsigned char* xo = lds + (wave << 14);
+  const int64_t out_row = (((int64_t)(a.n_splits > 1 ? sp : 0) * a.batch + b) * a.n_q_heads + head) * a.q_len + q0;
+  const int n_rows = active ? a.q_len - q0 : 0;  // (of the wave's 32, those below it)
+  const float inv = a.n_splits > 1 ? 1.0f : l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
+  if (a.n_splits > 1 && en < n_rows && eg == 0) {
+    a.ws_ml[(out_row + en) * 2] = m_run;
+    a.ws_ml[(out_row + en) * 2 + 1] = l_tot;
+  }
+  if (IO32 || a.n_splits > 1) {
+    float* po = a.n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out);
 #pragma unroll
-      for (int mt = 0; mt < 8; mt++)
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-        for (int c = 0; c < 4; c++)
-          *reinterpret_cast<f32x4_t*>(po + 32 * mt + 8 * c + 4 * g) =
-              f32x4_t{oacc[mt][4 * c], oacc[mt][4 * c + 1], oacc[mt][4 * c + 2], oacc[mt][4 * c + 3]};
-      if (g == 0) {
-        a.ws_ml[row * 2] = m_run;
-        a.ws_ml[row * 2 + 1] = l_tot;
+      for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const f32x16_t& o = oacc[4 * h + mt];
+          *reinterpret_cast<f32x4_t*>(xo + en * 512 + 16 * ((8 * mt + 2 * c + eg) ^ (en & 15))) =
+              f32x4_t{o[4 * c] * inv, o[4 * c + 1] * inv, o[4 * c + 2] * inv, o[4 * c + 3] * inv};
+        }
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int r = 2 * i + eg;
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(xo + r * 512 + 16 * (en ^ (r & 15)));
+        if (r < n_rows) *reinterpret_cast<f32x4_t*>(po + (out_row + r) * kD + 128 * h + 4 * en) = v;
       }
     }
     return;
   }
-  const float inv = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
-  if (active && q0 + n < a.q_len) {
-    const int64_t ooff = (((int64_t)b * a.n_q_heads + head) * a.q_len + q0 + n) * kD;
+  if constexpr (!IO32) {
 #pragma unroll
     for (int mt = 0; mt < 8; mt++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        if constexpr (IO32) {
-          *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff + 32 * mt + 8 * c + 4 * g) =
-              f32x4_t{oacc[mt][4 * c] * inv, oacc[mt][4 * c + 1] * inv, oacc[mt][4 * c + 2] * inv,
-                      oacc[mt][4 * c + 3] * inv};
-        } else {
-          u32x2_t w = {pack2<KDT>(oacc[mt][4 * c] * inv, oacc[mt][4 * c + 1] * inv),
-                       pack2<KDT>(oacc[mt][4 * c + 2] * inv, oacc[mt][4 * c + 3] * inv)};
-          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(a.out) + ooff + 32 * mt + 8 * c + 4 * g) = w;
-        }
-      }
+      for (int c = 0; c < 4; c++)
+        *reinterpret_cast<u32x2_t*>(xo + en * 512 + 16 * ((4 * mt + c) ^ (en & 15)) + 8 * eg) =
+            u32x2_t{pack2<KDT>(oacc[mt][4 * c] * inv, oacc[mt][4 * c + 1] * inv),
+                    pack2<KDT>(oacc[mt][4 * c + 2] * inv, oacc[mt][4 * c + 3] * inv)};
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int r = 2 * i + eg;
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(xo + r * 512 + 16 * (en ^ (r & 15)));
+      if (r < n_rows) *reinterpret_cast<u32x4_t*>(reinterpret_cast<uint16_t*>(a.out) + (out_row + r) * kD + 8 * en) = v;
+    }
   }
 }
 

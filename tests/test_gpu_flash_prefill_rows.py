@@ -1,0 +1,63 @@
+"""GPU: query rows in and output rows out of the flash prefill kernel, element by element.
+
+Key j of the prefix is 64 times the unit vector of column j % 256 and a query is 64 times the unit vector of its own
+column, so with scale 1/16 one residue of keys scores 256 and every other key 0: the others' weights, exp(-256), are zero in
+float32 and the output is the mean of that residue's value rows. The value rows are equal within a residue and hold
+whole numbers from 0 to 255, which every 16-bit type, the 8-bit codes (scale 1, bias 0) and the sums over a residue hold
+exactly; float32 means are taken over powers of two. A row, column or head that went to another place therefore shows, and the comparison is exact.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(Hq, Hkv, L, past, seed):
+    g = torch.Generator().manual_seed(seed)
+    j = torch.arange(past) % 256
+    k = torch.zeros((1, Hkv, past, 256))
+    k[:, :, torch.arange(past), j] = 64.0
+    rows = torch.randint(0, 256, (1, Hkv, 256, 256), generator=g).float()
+    rows[..., ::64], rows[..., 1::64] = 0.0, 255.0  # every group of 64 spans the codes
+    v = rows[:, :, j]
+    col = torch.randint(0, 256, (1, Hq, L), generator=g)
+    q = torch.zeros((1, Hq, L, 256)).scatter_(3, col[..., None], 64.0)
+    want = torch.stack([rows[0, h // (Hq // Hkv), col[0, h]] for h in range(Hq)])[None]
+    return q, k, v, want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,L,past", [
+    (16, 2, 1, 256), (16, 2, 31, 512), (16, 2, 32, 2048), (16, 2, 97, 768), (16, 2, 203, 2048), (16, 2, 1600, 256),
+    (8, 2, 33, 512), (8, 2, 161, 768), (4, 2, 130, 512), (2, 2, 64, 256), (2, 2, 300, 1024), (2, 1, 1, 256),
+])
+def test_rows_of_dense_prefill(Hq, Hkv, L, past, dtype):
+    from moespresso_amd.runtime.qwen import kquant
+
+    q, k, v, want = _case(Hq, Hkv, L, past, seed=L + past)
+    tail = torch.zeros((1, Hkv, L, 256))
+    dev = torch.device("cuda:0")
+    got = kquant.flash_prefill(q.to(dev, dtype), torch.cat([k, tail], 2).to(dev, dtype),
+                               torch.cat([v, tail], 2).to(dev, dtype), 0.0625, past_len=past)
+    assert torch.equal(got.cpu().float(), want)
+
+
+@pytest.mark.parametrize("sb_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,L,past", [
+    (16, 2, 1, 256), (16, 2, 33, 2048), (16, 2, 97, 512), (16, 2, 160, 32768), (16, 2, 203, 2048), (16, 4, 320, 2048),
+    (8, 2, 129, 4096), (4, 2, 256, 8192), (2, 2, 48, 1024), (16, 2, 1025, 256),
+])
+def test_rows_of_quantised_prefill(Hq, Hkv, L, past, sb_dtype):
+    from moespresso_amd.runtime.qwen import kquant
+
+    q, k, v, want = _case(Hq, Hkv, L, past, seed=L + past)
+    dev = torch.device("cuda:0")
+
+    def codes(x):
+        return x.to(torch.uint8).contiguous().view(torch.int32).view(torch.uint32).to(dev)
+
+    one, zero = (torch.full((1, Hkv, past, 4), c, dtype=sb_dtype, device=dev) for c in (1.0, 0.0))
+    chunk = torch.zeros((1, Hkv, L, 256), device=dev)
+    got = kquant.sdpa_fa_prefill_q8(q.to(dev), codes(k), one, zero, codes(v), one, zero, chunk, chunk, 0.0625)
+    assert torch.equal(got.cpu(), want)
