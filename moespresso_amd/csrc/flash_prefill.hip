@@ -149,6 +149,18 @@ template <int N>
 __device__ __forceinline__ void wait_vm_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
+// Stores that go through the L2 to memory: what the next launch reads. Left in the L2, the data is written out when the
+// last workgroup has ended (4 MB an XCD 3 to 6 us); like this it leaves under the other workgroups' work. Launch and
+// merge of 150 queries over 2000 keys (33 MB of partials) 26.9 -> 25.9 us, of 203 over 300 23.4 -> 21.0, of 256 over 9000 59.3
+// -> 58.4; marked as streamed instead (nt) 26.2, 20.6 and 60.4. Stores at `bytes` and beyond are dropped by the hardware.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t through_window(float* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ void store_through(__amdgpu_buffer_rsrc_t w, int offset, f32x4_t v) {
+  constexpr int kSc1 = 16;  // device scope
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), w, offset, 0, kSc1);
+}
+
 // lane i's 16 bytes at `src` land at lds_base + 16 i (lds_base wave-uniform); issued through asm so
 // that the compiler's wait-count pass does not drain it in front of LDS transpose reads (s_nop: the copy needs
 // one instruction between it and the scalar write of M0, which the compiler does not add inside an asm statement)
@@ -176,7 +188,7 @@ __device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 
 // scales and biases, with kExactUnpack added to it where the prefix is unpacked to the values that a conversion beforehand
 // gives; without it in packed float16 arithmetic.
 constexpr int kExactUnpack = 4;
-template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
+template <int KDT, bool Q8, int SDT, bool IO32, bool RUNS>
 __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(256))) unsigned char lds[];  // tile bases: zero low bits under the address XORs
   const int tid = threadIdx.x;
@@ -196,12 +208,29 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   const int head_halves = 1 << (a.rep_shift - hpg_shift);
   const int n_blocks = (a.q_len + 31) / 32;
   const int n_pairs = a.q_blocks / head_halves;
+  // Where ranges are long, workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run of the list (batch, KV
+  // head, range, pair): an L2 then holds the keys of few ranges and one or two heads' queries, which all pairs of a range
+  // pass together. Elsewhere the ranges go round the XCDs. Us, round and in runs: 16 / 4 heads, 670 queries over 6000 keys
+  // (9 ranges of 23 tiles) 84.1 and 79.9, 350 over 3000 (10 of 11) 43.2 and 41.0; 16 / 2 heads, 500 quantised over 3000
+  // 72.0 and 68.5, 290 over 12000 (15 of 26) 74.2 and 71.6, 203 over 9001 (16 of 18) equal; but 150 over 2000 (13 of 6) 25.9 and 27.5, 33 over 9000 (50 of 6) 28.1 and
+  // 29.0: in runs the partials leave the L2s 2 us later.
   int work = blockIdx.x;
-  const int sp = work % a.n_splits;
-  work /= a.n_splits;
-  const int pair = (work % a.q_blocks) / head_halves;  // pair 0 (longest stream) first
-  const int head_half = work % head_halves;
-  work /= a.q_blocks;
+  int sp, q_block;
+  if constexpr (RUNS) {
+    const int wgs = a.batch * a.n_kv_heads * a.q_blocks * a.n_splits, xcd = work & 7;
+    work = xcd * (wgs >> 3) + (xcd < (wgs & 7) ? xcd : wgs & 7) + (work >> 3);
+    q_block = work % a.q_blocks;
+    work /= a.q_blocks;
+    sp = work % a.n_splits;
+    work /= a.n_splits;
+  } else {
+    sp = work % a.n_splits;
+    work /= a.n_splits;
+    q_block = work % a.q_blocks;
+    work /= a.q_blocks;
+  }
+  const int pair = q_block / head_halves;  // pair 0 (longest stream) first
+  const int head_half = q_block % head_halves;
   const int kvh = work % a.n_kv_heads;
   const int b = work / a.n_kv_heads;
   const int wi = wave & 3;
@@ -565,8 +594,12 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     a.ws_ml[(out_row + en) * 2] = m_run;
     a.ws_ml[(out_row + en) * 2 + 1] = l_tot;
   }
+  // (the merge leaves a range out whose denominator is zero: a wave without any other, under the causal rule or past the last
+  // range with tiles, has nothing to store)
+  if (a.n_splits > 1 && !__any(l_tot != 0.0f)) return;
   if (IO32 || a.n_splits > 1) {
-    float* po = a.n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out);
+    float* po = (a.n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out)) + out_row * kD;
+    const __amdgpu_buffer_rsrc_t win = through_window(po, (n_rows < 32 ? n_rows : 32) * kD * 4);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
 #pragma unroll
@@ -581,7 +614,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
       for (int i = 0; i < 16; i++) {
         const int r = 2 * i + eg;
         const f32x4_t v = *reinterpret_cast<const f32x4_t*>(xo + r * 512 + 16 * (en ^ (r & 15)));
-        if (r < n_rows) *reinterpret_cast<f32x4_t*>(po + (out_row + r) * kD + 128 * h + 4 * en) = v;
+        store_through(win, r * kD * 4 + 512 * h + 16 * en, v);
       }
     }
     return;
@@ -820,11 +853,11 @@ size_t prefill_split_bytes(int batch, int n_q_heads, int n_kv_heads, int q_len, 
   return (size_t)splits * batch * n_q_heads * q_len * (kD + 2) * sizeof(float);
 }
 
-template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
-int prefill_launch(const PrefillArgs& a, hipStream_t st) {
+template <int KDT, bool Q8, int SDT, bool IO32, bool RUNS>
+int prefill_launch_flash(const PrefillArgs& a, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_prefill_kernel<KDT, Q8, SDT, IO32>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_prefill_kernel<KDT, Q8, SDT, IO32, RUNS>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) {
       mspr_set_error("flash_prefill: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
@@ -835,9 +868,19 @@ int prefill_launch(const PrefillArgs& a, hipStream_t st) {
   dim3 grid((unsigned)(a.q_blocks * a.n_kv_heads * a.batch * a.n_splits)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_FLASH_PREFILL, st);
-    flash_prefill_kernel<KDT, Q8, SDT, IO32><<<grid, block, kLdsBytes, st>>>(a);
+    flash_prefill_kernel<KDT, Q8, SDT, IO32, RUNS><<<grid, block, kLdsBytes, st>>>(a);
   }
   MSPR_CHECK_LAUNCH("flash_prefill");
+  return MSPR_OK;
+}
+
+template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
+int prefill_launch(const PrefillArgs& a, hipStream_t st) {
+  // (the line of the kernel's mapping; a template parameter because as a run-time branch it cost long chunks 0.5 %)
+  const bool runs = a.n_splits > 1 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
+  const int rc = runs ? prefill_launch_flash<KDT, Q8, SDT, IO32, true>(a, st)
+                      : prefill_launch_flash<KDT, Q8, SDT, IO32, false>(a, st);
+  if (rc != MSPR_OK) return rc;
   if (a.n_splits > 1) {
     const int64_t n_rows = (int64_t)a.batch * a.n_q_heads * a.q_len;
     // (16 ranges: 4096 rows 12.0 us with one wave each, 13.4 with two; between 3248 and 3584 rows equal, whole calls of 3568

@@ -31,6 +31,7 @@ def _case(Hq, Hkv, L, past, seed):
 @pytest.mark.parametrize("Hq,Hkv,L,past", [
     (16, 2, 1, 256), (16, 2, 31, 512), (16, 2, 32, 2048), (16, 2, 97, 768), (16, 2, 203, 2048), (16, 2, 1600, 256),
     (8, 2, 33, 512), (8, 2, 161, 768), (4, 2, 130, 512), (2, 2, 64, 256), (2, 2, 300, 1024), (2, 1, 1, 256),
+    (16, 4, 350, 8192), (8, 2, 333, 16384), (16, 2, 290, 256), (6, 3, 450, 8192),  # long ranges; ranges without keys
 ])
 def test_rows_of_dense_prefill(Hq, Hkv, L, past, dtype):
     from moespresso_amd.runtime.qwen import kquant
@@ -47,6 +48,7 @@ def test_rows_of_dense_prefill(Hq, Hkv, L, past, dtype):
 @pytest.mark.parametrize("Hq,Hkv,L,past", [
     (16, 2, 1, 256), (16, 2, 33, 2048), (16, 2, 97, 512), (16, 2, 160, 32768), (16, 2, 203, 2048), (16, 4, 320, 2048),
     (8, 2, 129, 4096), (4, 2, 256, 8192), (2, 2, 48, 1024), (16, 2, 1025, 256),
+    (16, 2, 500, 8192), (16, 2, 128, 32768),
 ])
 def test_rows_of_quantised_prefill(Hq, Hkv, L, past, sb_dtype):
     from moespresso_amd.runtime.qwen import kquant
