@@ -52,6 +52,18 @@ static inline bool mspr_aligned(const void* p, size_t a) { return (reinterpret_c
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 
+// Stores through the L2 to memory, for what only later launches read. Data left in the L2s (4 MB an XCD) is written out
+// when the last workgroup has ended, 3 to 6 us in which nothing else runs; at device scope it leaves under the other
+// workgroups' work. The base is one per wave; stores at `bytes` and beyond are dropped by the hardware.
+constexpr int kStoreCached = 0, kStoreThrough = 16 /* sc1 */, kStoreThroughStreamed = 16 | 2 /* and nt: past the last-level cache too */;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t store_window(void* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
+}
+template <int POLICY>
+__device__ __forceinline__ void window_store(__amdgpu_buffer_rsrc_t w, int offset, u32x4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, w, offset, 0, POLICY);
+}
+
 // float32 -> bfloat16 bits, round to nearest even (NaN kept quiet).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   uint32_t u = __float_as_uint(f);

@@ -149,18 +149,6 @@ template <int N>
 __device__ __forceinline__ void wait_vm_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
-// Stores that go through the L2 to memory: what the next launch reads. Left in the L2, the data is written out when the
-// last workgroup has ended (4 MB an XCD 3 to 6 us); like this it leaves under the other workgroups' work. Launch and
-// merge of 150 queries over 2000 keys (33 MB of partials) 26.9 -> 25.9 us, of 203 over 300 23.4 -> 21.0, of 256 over 9000 59.3
-// -> 58.4; marked as streamed instead (nt) 26.2, 20.6 and 60.4. Stores at `bytes` and beyond are dropped by the hardware.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t through_window(float* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
-}
-__device__ __forceinline__ void store_through(__amdgpu_buffer_rsrc_t w, int offset, f32x4_t v) {
-  constexpr int kSc1 = 16;  // device scope
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), w, offset, 0, kSc1);
-}
-
 // lane i's 16 bytes at `src` land at lds_base + 16 i (lds_base wave-uniform); issued through asm so
 // that the compiler's wait-count pass does not drain it in front of LDS transpose reads (s_nop: the copy needs
 // one instruction between it and the scalar write of M0, which the compiler does not add inside an asm statement)
@@ -580,7 +568,9 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
 
   // ---- normalise and store: lane (n, g) holds dims 32 mt + 8 (i/4) + 4 g + i%4 of query row q0 + n. The values change
   //      lanes in the wave's 16 KB of the ring, so that an instruction stores whole 512-byte runs of two rows and not 32
-  //      bytes of each of 32 (3.7 -> 2.7 us for float32 values; 256 KB a CU are 4096 clocks of its way to the L2).
+  //      bytes of each of 32 (3.7 -> 2.7 us for float32 values; 256 KB a CU are 4096 clocks of its way to the L2). They go
+  //      through the L2, us with the merge: 150 queries over 2000 keys (33 MB of partials) 26.9 -> 25.9, 203 over 300 23.4
+  //      -> 21.0, 256 over 9000 59.3 -> 58.4; marked as streamed instead (nt alone) 26.2, 20.6 and 60.4.
   const float l_tot = l_run + __shfl_xor(l_run, 32, MSPR_WAVE);
   __syncthreads();  // every wave has left the tiles
   int tl = tid;
@@ -599,7 +589,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   if (a.n_splits > 1 && !__any(l_tot != 0.0f)) return;
   if (IO32 || a.n_splits > 1) {
     float* po = (a.n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out)) + out_row * kD;
-    const __amdgpu_buffer_rsrc_t win = through_window(po, (n_rows < 32 ? n_rows : 32) * kD * 4);
+    const __amdgpu_buffer_rsrc_t win = store_window(po, (n_rows < 32 ? n_rows : 32) * kD * 4);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
 #pragma unroll
@@ -614,7 +604,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
       for (int i = 0; i < 16; i++) {
         const int r = 2 * i + eg;
         const f32x4_t v = *reinterpret_cast<const f32x4_t*>(xo + r * 512 + 16 * (en ^ (r & 15)));
-        store_through(win, r * kD * 4 + 512 * h + 16 * en, v);
+        window_store<kStoreThrough>(win, r * kD * 4 + 512 * h + 16 * en, __builtin_bit_cast(u32x4_t, v));
       }
     }
     return;

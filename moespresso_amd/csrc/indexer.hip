@@ -242,7 +242,10 @@ __global__ __launch_bounds__(256) void qat_rows_kernel(const void* __restrict__ 
   int64_t src = row < n_rows ? row : n_rows - 1;
   f32x4_t v = load_row4<DT>(x, src, lane32);
   f32x4_t y = qat128<LIVE>(v, lane32);
-  if (row < n_rows) reinterpret_cast<f32x4_t*>(out + row * 128)[lane32] = y;
+  // (through the L2: 517 tokens of 64 rows, 17 MB, 9.2 -> 7.6 us; 126 MB the same)
+  const int64_t left = n_rows - (int64_t)blockIdx.x * 8;
+  window_store<kStoreThrough>(store_window(out + (int64_t)blockIdx.x * 8 * 128, (left < 8 ? (int)left : 8) * 512),
+                              threadIdx.x * 16, __builtin_bit_cast(u32x4_t, y));
 }
 
 // ------------------------------------------------------------------ score tail

@@ -115,10 +115,12 @@ __global__ __launch_bounds__(kThreads) void partial_rope_kernel(const void* __re
 // 32): the workgroup covers kThreads chunks = kThreads / chunks-per-row consecutive positions of one outer row at a time,
 // 4 KB of contiguous memory, and walks its slab of outer rows at the same positions. A thread keeps its place in the row
 // and its position, so its cosines and sines stay in registers and no index arithmetic is left in the loop.
-// STREAM: the rows are read past the caches, and 16-bit ones written past them. Bound by memory: 3844 tokens of 64 x 512,
-// 504 MB of float16 in and out 112 -> 86 us, 1008 MB of float32 162 -> 148 and 176 -> 173; 126 MB of float16 24.8 -> 23.6.
-// (Float32 rows written past the caches too: 163 and 163 us.)
-template <int DT, bool STREAM>
+// STREAM: the rows are read past the caches. STORE: how they are written (see store_window). Bound by memory: 3844 tokens
+// of 64 x 512 rows, fresh ones each call, 504 MB of float16 in and out 112 us cached, 85 read and written as streams, 77.5
+// read as a stream and written through; 1008 MB of float32 174 (read as a stream) and 169; 126 MB of float32 39.5 and 37.4;
+// 517 tokens of 64 x 512 in float32 22.6 and 21.4, in float16 12.0 and 12.2. (Written through and as a stream 1008 MB take
+// 162, but what reads them next more than that; 126 MB 41.7.)
+template <int DT, bool STREAM, int STORE>
 __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void* __restrict__ x, int n_outer, int seq_len,
                                                                     int chunks_log2, const float* __restrict__ inv_freq,
                                                                     const float* __restrict__ positions, int64_t offset,
@@ -157,7 +159,8 @@ __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void*
   int n = n_outer - o;
   if (n > rows_per_wg) n = rows_per_wg;
   const u32x4_t* src = reinterpret_cast<const u32x4_t*>(x) + o * row_step + ((int64_t)(l0 + lp) << chunks_log2) + chunk;
-  u32x4_t* dst = reinterpret_cast<u32x4_t*>(out) + (src - reinterpret_cast<const u32x4_t*>(x));
+  // (chunk tid of the workgroup's 4 KB in every outer row)
+  unsigned char* dst = reinterpret_cast<unsigned char*>(out) + 16 * (o * row_step + ((int64_t)l0 << chunks_log2));
   auto pair = [&](float x0, float x1, int p, float* y0, float* y1) {
     const float m0 = round_to<DT>(x0 * c[p]), m1 = round_to<DT>(x1 * s[p]);
     const float m2 = round_to<DT>(x0 * s[p]), m3 = round_to<DT>(x1 * c[p]);
@@ -186,10 +189,7 @@ __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void*
     if constexpr (STREAM) return __builtin_nontemporal_load(p);
     else return *p;
   };
-  auto put = [](u32x4_t v, u32x4_t* p) {
-    if constexpr (STREAM && DT != MSPR_F32) __builtin_nontemporal_store(v, p);
-    else *p = v;
-  };
+  auto put = [&](u32x4_t v, unsigned char* row) { window_store<STORE>(store_window(row, 16 * kThreads), 16 * tid, v); };
   constexpr int kAtOnce = 4;  // rows in flight per thread
   for (; n >= kAtOnce; n -= kAtOnce) {
     u32x4_t v[kAtOnce];
@@ -198,17 +198,17 @@ __global__ __launch_bounds__(kThreads) void partial_rope_wide_kernel(const void*
 #pragma unroll
     for (int j = 0; j < kAtOnce; j++) {
       if (tail) v[j] = rotate(v[j]);
-      put(v[j], dst + j * row_step);
+      put(v[j], dst + 16 * j * row_step);
     }
     src += kAtOnce * row_step;
-    dst += kAtOnce * row_step;
+    dst += 16 * kAtOnce * row_step;
   }
   for (; n > 0; n--) {
     u32x4_t v = get(src);
     if (tail) v = rotate(v);
     put(v, dst);
     src += row_step;
-    dst += row_step;
+    dst += 16 * row_step;
   }
 }
 
@@ -243,18 +243,19 @@ extern "C" int mspr_fused_partial_rope(const void* x, int dtype, int64_t n_outer
     if (slabs <= 65535) {
       dim3 grid((unsigned)pos_blocks, (unsigned)slabs), block(kThreads);
       const bool stream_rows = n_outer * seq_len * width >= ((int64_t)24 << 20);
-#define MSPR_ROPE_WIDE(DT)                                                                                               \
-  do {                                                                                                                   \
-    if (stream_rows)                                                                                                     \
-      partial_rope_wide_kernel<DT, true><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, \
-                                                                 offset, inverse, (int)rows, out);                       \
-    else                                                                                                                 \
-      partial_rope_wide_kernel<DT, false><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq, positions, \
-                                                                  offset, inverse, (int)rows, out);                      \
-  } while (0)
-      if (dtype == MSPR_F32) MSPR_ROPE_WIDE(MSPR_F32);
-      else if (dtype == MSPR_F16) MSPR_ROPE_WIDE(MSPR_F16);
-      else MSPR_ROPE_WIDE(MSPR_BF16);
+#define MSPR_ROPE_WIDE(DT, STREAM, STORE)                                                                                \
+  partial_rope_wide_kernel<DT, STREAM, STORE><<<grid, block, 0, st>>>(x, (int)n_outer, (int)seq_len, log2, inv_freq,       \
+                                                                      positions, offset, inverse, (int)rows, out)
+      if (dtype == MSPR_F32) {
+        if (stream_rows) MSPR_ROPE_WIDE(MSPR_F32, true, kStoreThrough);
+        else MSPR_ROPE_WIDE(MSPR_F32, false, kStoreThrough);
+      } else if (dtype == MSPR_F16) {
+        if (stream_rows) MSPR_ROPE_WIDE(MSPR_F16, true, kStoreThrough);
+        else MSPR_ROPE_WIDE(MSPR_F16, false, kStoreCached);
+      } else {
+        if (stream_rows) MSPR_ROPE_WIDE(MSPR_BF16, true, kStoreThrough);
+        else MSPR_ROPE_WIDE(MSPR_BF16, false, kStoreCached);
+      }
 #undef MSPR_ROPE_WIDE
       MSPR_CHECK_LAUNCH("fused_partial_rope");
       return MSPR_OK;
