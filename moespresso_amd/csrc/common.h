@@ -55,7 +55,7 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as
 // Stores through the L2 to memory, for what only later launches read. Data left in the L2s (4 MB an XCD) is written out
 // when the last workgroup has ended, 3 to 6 us in which nothing else runs; at device scope it leaves under the other
 // workgroups' work. The base is one per wave; stores at `bytes` and beyond are dropped by the hardware.
-constexpr int kStoreCached = 0, kStoreThrough = 16 /* sc1 */, kStoreThroughStreamed = 16 | 2 /* and nt: past the last-level cache too */;
+constexpr int kStoreCached = 0, kStoreThrough = 16;  // (16: sc1, device scope)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t store_window(void* base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
 }
