@@ -63,3 +63,27 @@ def test_rows_of_quantised_prefill(Hq, Hkv, L, past, sb_dtype):
     chunk = torch.zeros((1, Hkv, L, 256), device=dev)
     got = kquant.sdpa_fa_prefill_q8(q.to(dev), codes(k), one, zero, codes(v), one, zero, chunk, chunk, 0.0625)
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("L,past", [(1, 256), (97, 512), (203, 2048), (128, 32768), (1025, 256)])
+def test_quantised_prefill_may_overwrite_its_queries(L, past):
+    """Rounded queries lie in the output until the merge writes it, unless that is where the queries themselves are."""
+    from moespresso_amd import _lib
+
+    q, k, v, want = _case(16, 2, L, past, seed=L + past)
+    dev = torch.device("cuda:0")
+    kw, vw = (x.to(torch.uint8).contiguous().to(dev) for x in (k, v))
+    one, zero = (torch.full((1, 2, past, 4), c, device=dev) for c in (1.0, 0.0))
+    chunk = torch.zeros((1, 2, L, 256), device=dev)
+    ws = torch.empty(int(_lib.lib().mspr_sdpa_fa_prefill_q8_workspace_bytes(1, 16, 2, L, past)), dtype=torch.uint8, device=dev)
+    for shared in (False, True):
+        queries = q.to(dev)
+        out = queries if shared else torch.full_like(queries, float("nan"))
+        _lib.check(_lib.launch(
+            dev, "mspr_sdpa_fa_prefill_q8",
+            _lib.ptr(queries), _lib.ptr(kw), _lib.ptr(one), _lib.ptr(zero), _lib.ptr(vw), _lib.ptr(one), _lib.ptr(zero), 0,
+            _lib.ptr(chunk), _lib.ptr(chunk), 0, 1, 16, 2, 256, L, past, past, 0.0625, 64, 8, _lib.ptr(out), _lib.ptr(ws),
+            ws.numel()), "sdpa_fa_prefill_q8")
+        assert torch.equal(out.cpu(), want), shared
+        if not shared:
+            assert torch.equal(queries.cpu(), q)
