@@ -7,8 +7,8 @@
 // Work split: a workgroup owns (batch, 64-head block, slot range) and streams 32-slot tiles.
 // Each K row is read from HBM once and staged row-major in LDS (ring of three tiles, filled by
 // asynchronous global->LDS copies). The eight waves are (head group hg of 32 heads) x (quarter dh):
-// for S^T = K.Q^T a wave contracts its quarter of the row width and the four quarters are summed
-// through LDS; for O^T = V^T.P^T it owns 128 of the 512 output columns. Two waves share a SIMD and
+// for S^T = K.Q^T a wave contracts its quarter of the row width, the four quarters are summed
+// through LDS, a quarter of the keys by each wave, and the weights handed round the same way; for O^T = V^T.P^T it owns 128 of the 512 output columns. Two waves share a SIMD and
 // fill each other's waits (a wave has no matrix work while it stages or exchanges). V^T operands come
 // out of the same row-major tile through the LDS transpose read, so no second copy of the tile
 // exists.
@@ -305,8 +305,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   const int total = gridDim.x;
   int work = blockIdx.x;
   if ((total & 7) == 0) work = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
-  // (divisions by multiplication with floor(2^32 / n) and one correction step: a launch starts with an empty
-  // instruction cache, and a software division is a hundred instructions in front of the first memory request)
+  // (divisions by multiplication with floor(2^32 / n) and one correction step: a software division is a hundred
+  // instructions in front of the first memory request, four to five cycles each with two waves on a SIMD)
   auto div_by = [](uint32_t x, uint32_t n, uint32_t inv) -> uint32_t {
     if (n == 1u) return x;
     uint32_t q = __umulhi(x, inv);  // true quotient or one less
@@ -1566,7 +1566,8 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
 }
 
 // Key ranges of one sequence at most (unless its table forces more): at 40 a window of 128 and 2048 ids are 34 ranges of
-// two tiles. 72, one tile each, took 8.9 us + 4.8 us of merge for one sequence, 40 took 9.7 + 3.4, 32 (three tiles) 11.9 + 4.0.
+// two tiles. 72, one tile each, and 40, whole layers: one sequence 23.05 and 23.1 us, three 27.6 and 25.7; 32 (three tiles) were
+// 2 us slower for one.
 constexpr int kMaxRanges = 40;
 
 int choose_splits(int batch_hblk, int n_keys) {
