@@ -816,8 +816,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   // and fits float16 whenever V does; with bf16 V it saturates at the float16 range instead of
   // overflowing. Its rounding (2^-11 relative) stays below the rounding of the final output.
   const int64_t part = ((int64_t)(seq * a.n_hblk + hb) * a.n_splits + sp);
-  // Through the L2 (store_window): a layer of 16 sequences over 32768 keys 49.3 -> 47.9 us, of 8 36.6 -> 35.2; the merge still
-  // finds them in its XCD's L2. One token's few (the rotated form) are out sooner through the cache: 23.4 and 23.7 us.
+  // Through the L2 (store_window): a layer of 16 sequences over 32768 keys 49.3 -> 47.9 us, of 8 36.6 -> 35.2; the merge reads
+  // them from beyond the L2 either way (17 MB by the counters). One token's few (the rotated form) are out sooner through the cache: 23.4 and 23.7 us.
   const __amdgpu_buffer_rsrc_t win = store_window(a.ws_o + (part * kWaves + wave) * (int64_t)(4 * 16 * 64), 8192);
   const float inv_l = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
 #pragma unroll
@@ -1465,8 +1465,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   __shared__ float rope_cs[16];  // of the workgroup's sixteen columns: eight cosines, eight negated sines
   const int lane = threadIdx.x & 63;
   const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // a sequence's partials are merged on the XCD whose workgroups wrote them (the split kernel's mapping), so
-  // that they are read from that XCD's L2
+  // a sequence's partials are merged on the XCD whose workgroups wrote them (the split kernel's mapping)
   unsigned work = blockIdx.x;
   if ((gridDim.x & 7u) == 0u) work = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int piece = work & 7;        // registers 8 piece .. +7 of the wave's 64: columns tile piece / 2
