@@ -1049,11 +1049,20 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   }
   // Where key ranges pass the queries again and again (16 times for 203 of them), the launch that makes the rows rounds them
   // once, so that a workgroup of the attention fetches 128 KB of them in front of its first tile and not 256. They lie in the
-  // output, which is the merge's to write, unless the caller has output and queries overlap. Us: 203 queries over 9001 rows 73.6
+  // output, which is the merge's to write, unless it overlaps what is still to be read. Us: 203 queries over 9001 rows 73.6
   // -> 72.2, 128 over 20000 82.4 -> 80.1, 30 over 9001 the same.
   const size_t io_bytes = (size_t)batch * n_q_heads * q_len * kD * sizeof(float);
-  const bool apart = (uintptr_t)out + io_bytes <= (uintptr_t)queries || (uintptr_t)queries + io_bytes <= (uintptr_t)out;
-  uint16_t* q16 = a.n_splits > 1 && apart ? reinterpret_cast<uint16_t*>(out) : nullptr;
+  auto apart = [&](const void* p, size_t bytes) {
+    const uintptr_t o = (uintptr_t)out, i = (uintptr_t)p;
+    return o + io_bytes <= i || i + bytes <= o;
+  };
+  const size_t self_bytes = (size_t)batch * n_kv_heads * q_len * kD * (self_dtype == MSPR_F32 ? 4 : 2);
+  const size_t past_all = (size_t)batch * n_kv_heads * past_rows;  // rows, over all heads
+  const size_t sb_bytes = past_all * 4 * (sb_dtype == MSPR_F32 ? 4 : 2);
+  const bool free_out = apart(queries, io_bytes) && apart(self_k, self_bytes) && apart(self_v, self_bytes) &&
+                        apart(pk_wq, past_all * kD) && apart(pv_wq, past_all * kD) && apart(pk_scales, sb_bytes) &&
+                        apart(pk_biases, sb_bytes) && apart(pv_scales, sb_bytes) && apart(pv_biases, sb_bytes);
+  uint16_t* q16 = a.n_splits > 1 && free_out ? reinterpret_cast<uint16_t*>(out) : nullptr;
   if (q16) a.q = q16;
   a.pk_wq = pk_wq;
   a.pk_s = pk_scales;
