@@ -422,6 +422,7 @@ __device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
 
 constexpr int kScoreThreads = 512;
 constexpr int kScoreWaves = kScoreThreads / 64;
+static_assert(kScoreWaves == 8, "a byte of a word each");
 // float32 row pitch of the QAT'd query block in LDS: 128 values plus 4, so that the 16-byte reads of
 // 16 lanes holding 16 different heads fall into different banks
 constexpr int kQPitch = 132;
@@ -440,6 +441,7 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
   __shared__ float qbuf[64 * kQPitch];
   __shared__ float wbuf[64];
   __shared__ float ptab[kPow2TabLen];
+  __shared__ __attribute__((aligned(8))) uint8_t plain_waves[8];
   const int tid = threadIdx.x;
   // With a KV row to prepare (the fused decode prep), the launch carries one more workgroup, the last one,
   // whose first wave does that small job next to the score workgroups instead of in a launch of its own.
@@ -461,14 +463,17 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
 
   // The eight waves QAT the 64 query rows, eight lanes a row; the power-of-two table sits in LDS, so the pass waits for memory
   // once. Every workgroup does the whole block, so it is instructions of one CU that bound it: 7900 cycles with 32 lanes a row
-  // and the lattice step in float32 arithmetic, now 4000 to 4700 of the workgroup's 12200 (961 pool rows: the launch 8.4 -> 6.3
-  // us, a decode token 27.3 -> 25.4).
+  // and the lattice step in float32 arithmetic, then 4000 to 4700 of the workgroup's 12200 (961 pool rows: the launch 8.4 -> 6.3
+  // us, a decode token 27.3 -> 25.4). The butterflies wait for the query rows alone: behind the barrier of the table all waves
+  // waited for the ones with a pool tile to request it (sixteen loads of 64 lines). With that, one barrier for the waves'
+  // verdicts on their rows instead of three, and nothing spilled, us by pool rows, in a graph: 961 5.33 -> 4.31, 8000 5.93 ->
+  // 4.56, 32000 7.4 -> 5.9, 60000 10.6 -> 7.65; rows that need three pieces, 961, 11.3 -> 6.3.
   const int q_head = tid >> 3, q_part = tid & 7;
   Qat16 mine;
   load_row16<DT>(q, q_head < n_heads ? q_head : n_heads - 1, q_part, mine.x);
   const float tab_a = g_pow2_tab[tid < kPow2TabLen ? tid : 0];
   const float w_mine = weights[tid < n_heads ? tid : 0];
-  // The first pool tile of the wave is requested now and lands while the queries are prepared. Lane
+  // The first pool tile of the wave is requested behind the butterflies and lands under the rest. Lane
   // (m = row, g) owns the 64 consecutive float32 values [64 g, 64 g + 64) of its pool row.
   float kv[64];
   auto load_tile = [&](int64_t t) {
@@ -484,22 +489,21 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
       kv[4 * j + 3] = t4.w;
     }
   };
-  if (tile < n_tiles) load_tile(tile);
-
+  qat16_rotate(mine, lane);
   if (tid < kPow2TabLen) ptab[tid] = tab_a;
   if (tid < 64) wbuf[tid] = tid < n_heads ? w_mine : 0.0f;
+  if (tile < n_tiles) load_tile(tile);
   __syncthreads();
-  qat16_rotate(mine, lane);
   const float q_scale = qat_scale(mine.amax, ptab);
   // Lattice values times powers of two from 2^-13 to 2^13 are float16 and bf16 numbers as they are, and the fp4 conversion
   // makes them: it rounds ties to the even code where the lower value is wanted, which differs where the upper code is the even
   // one. Just below a tie it rounds down, and one unit above a tie with an even lower code the value itself rounds up: of the
   // codes of x and of the number below x the odd one is right where they differ.
   const uint32_t q_bits = __float_as_uint(q_scale);
-  const bool plain = __syncthreads_and((q_bits & 0x807FFFFFu) == 0u && q_bits - 0x39000000u <= 0x0D000000u);
+  const bool plain_wave = __all((q_bits & 0x807FFFFFu) == 0u && q_bits - 0x39000000u <= 0x0D000000u);
   unsigned char* qbf = reinterpret_cast<unsigned char*>(qbuf);  // [head][kQBfPitch], bf16
   bool q_exact = true;
-  if (plain) {
+  if (plain_wave) {
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
       const float* x = mine.x + 8 * hf;
@@ -521,8 +525,12 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
                   __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 2)),
                   __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c, q_scale, 3))};
     }
-    __syncthreads();
-  } else {
+  }
+  // (where another wave's rows are not plain, all of the block is written again below)
+  if (lane == 0) plain_waves[wave] = plain_wave ? 1 : 0;
+  __syncthreads();
+  const bool plain = *reinterpret_cast<const uint64_t*>(plain_waves) == 0x0101010101010101ull;
+  if (!plain) {
     uint32_t q_low = 0u;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -581,33 +589,36 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     for (int j = 0; j < 64; j++) low |= __float_as_uint(kv[j]);
     const bool k_exact = __all((low & 0xFFFFu) == 0u);  // wave-uniform
     f32x16_t acc0 = {0}, acc1 = {0};
-    auto k_operand = [&](const float (&kk)[64], int s) -> bf16x8_t {
-      const u32x4_t kf = {pack_hi16(kk[8 * s], kk[8 * s + 1]), pack_hi16(kk[8 * s + 2], kk[8 * s + 3]),
-                          pack_hi16(kk[8 * s + 4], kk[8 * s + 5]), pack_hi16(kk[8 * s + 6], kk[8 * s + 7])};
+    auto k_operand = [&](const float* kk) -> bf16x8_t {
+      const u32x4_t kf = {pack_hi16(kk[0], kk[1]), pack_hi16(kk[2], kk[3]), pack_hi16(kk[4], kk[5]), pack_hi16(kk[6], kk[7])};
       return __builtin_bit_cast(bf16x8_t, kf);
     };
     if (k_exact && q_exact) {
 #pragma unroll
       for (int s = 0; s < 8; s++) {
-        const bf16x8_t kfb = k_operand(kv, s);
+        const bf16x8_t kfb = k_operand(kv + 8 * s);
         acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, qa[0][s]), kfb, acc0, 0, 0, 0);
         acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, qa[1][s]), kfb, acc1, 0, 0, 0);
       }
     } else {
       // every piece of q meets every piece of k, smallest products first
       const int q_pieces = q_exact ? 1 : 3;
-      for (int kp_i = 2; kp_i >= 0; kp_i--) {
-        float kk[64];
 #pragma unroll
-        for (int j = 0; j < 64; j++) {
-          float v = kv[j];
-          for (int p = 0; p < kp_i; p++) v = v - __uint_as_float(__float_as_uint(v) & 0xFFFF0000u);
-          kk[j] = v;
-        }
+      for (int kp_i = 2; kp_i >= 0; kp_i--) {
+#pragma unroll 1
         for (int qp_i = q_pieces - 1; qp_i >= 0; qp_i--) {
 #pragma unroll
           for (int s = 0; s < 8; s++) {
-            const bf16x8_t kfb = k_operand(kk, s);
+            float kk[8];  // (a step at a time: sixty-four of them would push what the usual case needs out of the registers)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+              float v = kv[8 * s + j];
+              asm volatile("" : "+v"(v));  // (made here, not ahead of the loop over q's pieces)
+#pragma unroll
+              for (int p = 0; p < kp_i; p++) v = v - __uint_as_float(__float_as_uint(v) & 0xFFFF0000u);
+              kk[j] = v;
+            }
+            const bf16x8_t kfb = k_operand(kk);
             const u32x4_t q0 = qp_i == 0 ? qa[0][s] : q_piece(0, s, qp_i);
             const u32x4_t q1 = qp_i == 0 ? qa[1][s] : q_piece(1, s, qp_i);
             acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, q0), kfb, acc0, 0, 0, 0);

@@ -37,3 +37,20 @@ def test_prepared_queries_are_those_of_the_row_operator(heads, low, high):
         got = isk.fused_qat_indexer_scores(torch.from_numpy(q[None, :, None]).cuda(), torch.from_numpy(pooled[None]).cuda(),
                                            torch.from_numpy(w).cuda(), 1.0).cpu().numpy().reshape(256)
         np.testing.assert_array_equal(got[:128] - got[128:], want[h], err_msg=str(h))
+
+
+@pytest.mark.parametrize("outsider", [0, 9, 36, 63])
+def test_one_head_outside_the_direct_range(outsider):
+    """One wave's rows cannot be converted directly: all of the workgroup's are taken in float32 form, the ones already
+    written as bfloat16 numbers among them."""
+    rng = np.random.default_rng(outsider)
+    q = rng.standard_normal((64, 128)).astype(np.float32)
+    q[outsider] *= np.float32(2.0 ** 20)
+    pooled = np.concatenate([np.eye(128, dtype=np.float32), -np.eye(128, dtype=np.float32)])
+    want = ds4.indexer_qat(q)
+    for h in (0, 1, 7, 8, 9, 35, 36, 56, 63):
+        w = np.zeros((1, 1, 64), np.float32)
+        w[0, 0, h] = 1.0
+        got = isk.fused_qat_indexer_scores(torch.from_numpy(q[None, :, None]).cuda(), torch.from_numpy(pooled[None]).cuda(),
+                                           torch.from_numpy(w).cuda(), 1.0).cpu().numpy().reshape(256)
+        np.testing.assert_array_equal(got[:128] - got[128:], want[h], err_msg=str(h))
