@@ -196,12 +196,14 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   const int head_halves = 1 << (a.rep_shift - hpg_shift);
   const int n_blocks = (a.q_len + 31) / 32;
   const int n_pairs = a.q_blocks / head_halves;
-  // Where ranges are long, workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run of the list (batch, KV
+  // Where ranges are long and four or more, workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run of the list (batch, KV
   // head, range, pair): an L2 then holds the keys of few ranges and one or two heads' queries, which all pairs of a range
   // pass together. Elsewhere the ranges go round the XCDs. Us, round and in runs: 16 / 4 heads, 670 queries over 6000 keys
   // (9 ranges of 23 tiles) 84.1 and 79.9, 350 over 3000 (10 of 11) 43.2 and 41.0; 16 / 2 heads, 500 quantised over 3000
-  // 72.0 and 68.5, 290 over 12000 (15 of 26) 74.2 and 71.6, 203 over 9001 (16 of 18) equal; but 150 over 2000 (13 of 6) 25.9 and 27.5, 33 over 9000 (50 of 6) 28.1 and
-  // 29.0: in runs the partials leave the L2s 2 us later.
+  // 72.0 and 68.5, 290 over 12000 (15 of 26) 74.2 and 71.6, 203 over 9001 (16 of 18) equal; but 150 over 2000 (13 of 6) 25.9
+  // and 27.5, 33 over 9000 (50 of 6) 28.1 and
+  // 29.0: in runs the partials leave the L2s 2 us later. Two ranges (2048 quantised queries over 34952): 987 and, with the
+  // queries rounded ahead as below, 997.
   int work = blockIdx.x;
   int sp, q_block;
   if constexpr (RUNS) {
@@ -882,7 +884,7 @@ int prefill_launch_flash(const PrefillArgs& a, hipStream_t st) {
 template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
 int prefill_launch(const PrefillArgs& a, hipStream_t st, bool q32 = false) {
   // (the line of the kernel's mapping; a template parameter because as a run-time branch it cost long chunks 0.5 %)
-  const bool runs = a.n_splits > 1 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
+  const bool runs = a.n_splits >= 4 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
   int rc;
   if (IO32 && q32) rc = prefill_launch_flash<KDT, Q8, SDT, IO32, IO32, false>(a, st);
   else if (runs) rc = prefill_launch_flash<KDT, Q8, SDT, IO32, false, true>(a, st);
@@ -1047,7 +1049,7 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
     a.ws_o = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(workspace) + tail);
     a.ws_ml = a.ws_o + (size_t)a.n_splits * batch * n_q_heads * q_len * kD;
   }
-  // Where key ranges pass the queries again and again (16 times for 203 of them), the launch that makes the rows rounds them
+  // Where four key ranges or more pass the queries again and again (16 for 203 of them), the launch that makes the rows rounds them
   // once, so that a workgroup of the attention fetches 128 KB of them in front of its first tile and not 256. They lie in the
   // output, which is the merge's to write, unless it overlaps what is still to be read. Us: 203 queries over 9001 rows 73.6
   // -> 72.2, 128 over 20000 82.4 -> 80.1, 30 over 9001 the same.
@@ -1062,7 +1064,7 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   const bool free_out = apart(queries, io_bytes) && apart(self_k, self_bytes) && apart(self_v, self_bytes) &&
                         apart(pk_wq, past_all * kD) && apart(pv_wq, past_all * kD) && apart(pk_scales, sb_bytes) &&
                         apart(pk_biases, sb_bytes) && apart(pv_scales, sb_bytes) && apart(pv_biases, sb_bytes);
-  uint16_t* q16 = a.n_splits > 1 && free_out ? reinterpret_cast<uint16_t*>(out) : nullptr;
+  uint16_t* q16 = a.n_splits >= 4 && free_out ? reinterpret_cast<uint16_t*>(out) : nullptr;
   if (q16) a.q = q16;
   a.pk_wq = pk_wq;
   a.pk_s = pk_scales;
