@@ -402,8 +402,8 @@ __device__ __forceinline__ void kv_row_job(int tid, float* cs, float* sn, const 
 }
 
 // ------------------------------------------------------------------ score row, float32 pool rows
-// Block = 8 waves. The block QATs the (up to 64) query heads into LDS once (four rows per lane, while
-// the wave's first pool tile is already on its way), each wave then keeps them in registers as the
+// Block = 8 waves. The block QATs the (up to 64) query heads into LDS once (eight lanes a row, the wave's
+// first pool tile on its way under the second half of it), each wave then keeps them in registers as the
 // MFMA A operand and walks 32-row tiles of the pool.
 //
 // The contraction runs on the bf16 MFMA (32x32x16) without giving up exact products: a QAT'd query
