@@ -898,13 +898,18 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
 //  * Selected rows set their bit in a bitmap of the row. Bits come out in row order, so nothing before has to keep it.
 // Keys are compared as signed integers: the bits of a float32 themselves where the pivot is positive, all others after the
 // map that inverts the low bits of negative values. Whether the list contains the k-th key is checked exactly; if it does not
-// (or does not fit), the same binning runs over all keys, so the result never depends on the sample.
+// (or does not fit, or a second round of bins hardly splits it), the binning runs over all keys, so the result never depends
+// on the sample. There -inf is counted on the side and the span is that of the finite keys, and votes go to copies of the
+// counters: in one histogram the votes of a row that is mostly -inf, or of one value, follow each other on one counter in
+// every pass (1 row of 32768, k = 2048, with 400 finite 125 us, now 13; 3844 rows of 8192, k = 512, 100 finite 484, now 44; a
+// chunk of 8400 tokens from position 0, whose first quarter sees too few rows: scores selected in 100, now 37).
 // What bounds it: a CU takes 2000 cycles to fetch a row of 32768 scores, and an instruction per key is 500 cycles of its vector
 // units: the blocked kernel above maps and moves every key (two LDS passes) and takes five digit passes, 16 rows of 32768,
 // k = 2048, 10.0 us, now 8.6. For many rows it is instructions: 3844 rows of 7961, k = 512, 57 us, now 28. (Keys read again
 // from the L2 instead of from a copy of the row in LDS: 64 lines an instruction, 3 us more for 16 rows; neighbouring lanes on
 // neighbouring list entries: their bits meet in the same words, 1 us more.)
 constexpr int32_t kLowestKey = (int32_t)0x80000000u;
+constexpr int32_t kNegInfSigned = (int32_t)(kNegInfKey ^ 0x80000000u);
 
 __device__ __forceinline__ int32_t signed_key(int32_t bits) { return bits ^ (int32_t)((uint32_t)(bits >> 31) >> 1); }
 
@@ -919,7 +924,7 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   constexpr uint32_t kBins = 256;
   static_assert(kBits <= 32 && S <= P && kBins <= THREADS && 16 % kW == 0, "a bin a thread, a piece a sample");
   __shared__ __attribute__((aligned(16))) int32_t stage[4 * P * THREADS];
-  __shared__ uint16_t list[kCap];
+  __shared__ __attribute__((aligned(16))) uint16_t list[kCap];
   __shared__ __attribute__((aligned(16))) uint32_t hist[kBins];
   __shared__ uint32_t bits_above[THREADS], bits_tie[THREADS];
   __shared__ uint32_t wave_pivot[kW], wave_high[kW];
@@ -997,8 +1002,10 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   }
   __syncthreads();
   int32_t pivot, span_end;
+  bool masked;  // the wanted rank of some wave's sample is -inf (or below)
   {
     uint32_t sum = wave_pivot[lane % kW], top = wave_high[lane % kW];  // (the same sixteen values in every row of lanes)
+    masked = __ballot(sum <= kNegInfKey >> 16) != 0ull;
     sum += dpp_u32<0x128>(sum);
     sum += dpp_u32<0x124>(sum);
     sum += dpp_u32<0x122>(sum);
@@ -1018,123 +1025,91 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
       for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
   }
 
-  // ---- rows at or above the pivot
-  uint32_t mask = 0u;
+  auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+  // ---- rows at or above the pivot (one at or below -inf would list the rows a token does not see as well: those are counted
+  //      below, not binned)
+  uint32_t total = 0u;
+  if (pivot > kNegInfSigned) {  // uniform
+    uint32_t mask = 0u;
 #pragma unroll
-  for (int j = P - 1; j >= 0; j--)
+    for (int j = P - 1; j >= 0; j--)
 #pragma unroll
-    for (int e = 3; e >= 0; e--) mask = shift_in(mask, key[j][e] >= pivot);
-  const uint32_t cnt = (uint32_t)__popc(mask);
-  const uint32_t incl = wave_prefix_sum(cnt);
-  uint32_t base = 0u;
-  if (lane == 63) base = atomicAdd(&n_list, incl);
-  base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63);
-  if (base + (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) <= (uint32_t)kCap) {
-    uint16_t* at = list + base + incl - cnt;
-    while (mask) {
-      const int i = __builtin_ctz(mask);
-      mask &= mask - 1u;
-      *at++ = (uint16_t)(4 * ((i >> 2) * THREADS + tid) + (i & 3));
+      for (int e = 3; e >= 0; e--) mask = shift_in(mask, key[j][e] >= pivot);
+    const uint32_t cnt = (uint32_t)__popc(mask);
+    const uint32_t incl = wave_prefix_sum(cnt);
+    uint32_t base = 0u;
+    if (lane == 63) base = atomicAdd(&n_list, incl);
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63);
+    if (base + (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) <= (uint32_t)kCap) {
+      uint16_t* at = list + base + incl - cnt;
+      while (mask) {
+        const int i = __builtin_ctz(mask);
+        mask &= mask - 1u;
+        *at++ = (uint16_t)(4 * ((i >> 2) * THREADS + tid) + (i & 3));
+      }
     }
+    __syncthreads();
+    total = uniform(n_list);
   }
-  __syncthreads();
-  const uint32_t total = n_list;
-  const bool fits = total >= (uint32_t)topk && total <= (uint32_t)kCap && pivot != kLowestKey;  // uniform
+  const bool fits = total >= (uint32_t)topk && total <= (uint32_t)kCap;  // uniform
 
-  // ---- the k-th key among the elements that `each` hands out (key in the signed order, row; keys below `lo` do not count),
-  //      then the selected rows
-  auto select = [&](auto each, int32_t lo, int32_t end) {
-    uint32_t need = (uint32_t)topk;
-    uint32_t span = end > lo ? (uint32_t)end - (uint32_t)lo : 0u;  // to a guess of the highest key; what is above is in the last bin
-    uint32_t limit = 0xFFFFFFFFu;  // distance from lo that the keys in question have at most
-    int32_t threshold;
-    while (true) {
-      const int shift = span >= kBins ? 24 - __builtin_clz(span) : 0;
-      each([&](int32_t k, int) {
-        const uint32_t d = (uint32_t)k - (uint32_t)lo;
-        if (k >= lo && d <= limit) atomicAdd(&hist[umin(d >> shift, kBins - 1u)], 1u);
-      });
-      __syncthreads();
-      if (wave == 0) {
-        const Pick pk = pick_bucket(hist, need, lane);
-        if (lane == 0) pick_box = pk;
-      }
-      __syncthreads();
-      const uint32_t bin = pick_box.digit, held = pick_box.live;
-      need = pick_box.need;
-      lo = (int32_t)((uint32_t)lo + (bin << shift));
-      const uint32_t rest = limit - (bin << shift), width = bin == kBins - 1u ? 0xFFFFFFFFu : (1u << shift) - 1u;
-      limit = rest < width ? rest : width;
-      if (limit == 0u) {
-        threshold = lo;
-        break;
-      }
-      if (held <= 64u) {
-        each([&](int32_t k, int) {
-          const bool in = k >= lo && (uint32_t)k - (uint32_t)lo <= limit;
-          if (__ballot(in) != 0ull) {  // (few waves hold any)
-            if (in) near[atomicAdd(&n_near, 1u)] = (uint32_t)k - (uint32_t)lo;
-          }
-        });
-        __syncthreads();
-        // sixteen lanes rank a candidate, each against four of them at a time
-        constexpr int kAtOnce = THREADS / 16;
-#pragma unroll
-        for (int c0 = 0; c0 < 64; c0 += kAtOnce) {
-          if (c0 > 0 && (uint32_t)c0 >= held) break;  // uniform
-          const int c = c0 + (tid >> 4);
-          const uint32_t mine = near[c];
-          const u32x4_t o = *reinterpret_cast<const u32x4_t*>(&near[4 * (lane & 15)]);
-          uint32_t n = 0u;  // higher ones, equal ones in the upper half
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const bool in = (uint32_t)(4 * (lane & 15) + j) < held;
-            n += in && o[j] > mine ? 1u : 0u;
-            n += in && o[j] == mine ? 1u << 16 : 0u;
-          }
-          n += dpp_u32<0x128>(n);
-          n += dpp_u32<0x124>(n);
-          n += dpp_u32<0x122>(n);
-          n += dpp_u32<0x121>(n);
-          const uint32_t above = n & 0xFFFFu;
-          if ((lane & 15) == 0 && (uint32_t)c < held && above < need && above + (n >> 16) >= need) {  // (all equal ones write the same)
-            kth[0] = mine;
-            kth[1] = need - above;
-          }
-        }
-        __syncthreads();
-        threshold = (int32_t)((uint32_t)lo + kth[0]);
-        need = kth[1];
-        break;
-      }
-      span = limit;
-      if (tid < (int)kBins) hist[tid] = 0u;
-      __syncthreads();
-    }
-    each([&](int32_t k, int row) {
-      const uint32_t word = (uint32_t)row / kBits, bit = 1u << ((uint32_t)row % kBits);
-      if (k > threshold) atomicOr(&bits_above[word], bit);
-      if (k == threshold) atomicOr(&bits_tie[word], bit);
-    });
+  // ---- the k-th key, k = need, is one of those in [lo, lo + limit]; `span` is a guess of the distance from lo to the highest
+  //      one (what is above is in the last bin)
+  uint32_t need = (uint32_t)topk, limit = 0xFFFFFFFFu, span;
+  int32_t lo = pivot, threshold = 0;
+  bool found = fits;
+  // of the votes in `hist`, 1 << shift keys wide a bin: the bin with the k-th key, and how many keys it holds
+  auto narrow = [&](int shift) -> uint32_t {
     __syncthreads();
-    uint32_t wa = bits_above[tid], wt = bits_tie[tid];
-    const uint32_t mine = (uint32_t)__popc(wa) | ((uint32_t)__popc(wt) << 16);
-    const uint32_t upto = wave_prefix_sum(mine);
-    if (lane == 63) wave_tot[wave] = upto;
+    if (wave == 0) {
+      const Pick pk = pick_bucket(hist, need, lane);
+      if (lane == 0) pick_box = pk;
+    }
     __syncthreads();
-    const uint32_t tots = wave_prefix_sum(lane < kW ? wave_tot[lane < kW ? lane : 0] : 0u);
-    const uint32_t excl = upto - mine + (wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)tots, wave > 0 ? wave - 1 : 0) : 0u);
-    int32_t* out = sel + (excl & 0xFFFFu);
-    uint32_t order = excl >> 16;
-    while (wa) {
-      *out++ = (int)kBits * tid + (int)__builtin_ctz(wa);
-      wa &= wa - 1u;
+    const uint32_t bin = uniform(pick_box.digit);
+    need = uniform(pick_box.need);
+    lo = (int32_t)((uint32_t)lo + (bin << shift));
+    const uint32_t rest = limit - (bin << shift), width = bin == kBins - 1u ? 0xFFFFFFFFu : (1u << shift) - 1u;
+    limit = rest < width ? rest : width;
+    return uniform(pick_box.live);
+  };
+  auto candidate = [&](int32_t k) {
+    const bool in = k >= lo && (uint32_t)k - (uint32_t)lo <= limit;
+    if (__ballot(in) != 0ull) {  // (few waves hold any)
+      if (in) near[atomicAdd(&n_near, 1u)] = (uint32_t)k - (uint32_t)lo;
     }
-    out = sel + ((uint32_t)topk - need);
-    while (wt && order < need) {
-      out[order++] = (int)kBits * tid + (int)__builtin_ctz(wt);
-      wt &= wt - 1u;
+  };
+  // the k-th of up to 64 candidates: sixteen lanes rank one, each against four at a time
+  auto rank_candidates = [&](uint32_t held) {
+    __syncthreads();
+    constexpr int kAtOnce = THREADS / 16;
+#pragma unroll
+    for (int c0 = 0; c0 < 64; c0 += kAtOnce) {
+      if (c0 > 0 && (uint32_t)c0 >= held) break;  // uniform
+      const int c = c0 + (tid >> 4);
+      const uint32_t mine = near[c];
+      const u32x4_t o = *reinterpret_cast<const u32x4_t*>(&near[4 * (lane & 15)]);
+      uint32_t n = 0u;  // higher ones, equal ones in the upper half
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const bool in = (uint32_t)(4 * (lane & 15) + j) < held;
+        n += in && o[j] > mine ? 1u : 0u;
+        n += in && o[j] == mine ? 1u << 16 : 0u;
+      }
+      n += dpp_u32<0x128>(n);
+      n += dpp_u32<0x124>(n);
+      n += dpp_u32<0x122>(n);
+      n += dpp_u32<0x121>(n);
+      const uint32_t above = n & 0xFFFFu;
+      if ((lane & 15) == 0 && (uint32_t)c < held && above < need && above + (n >> 16) >= need) {  // (all equal ones write the same)
+        kth[0] = mine;
+        kth[1] = need - above;
+      }
     }
+    __syncthreads();
+    need = uniform(kth[1]);
+    lo = (int32_t)((uint32_t)lo + uniform(kth[0]));
+    limit = 0u;
   };
 
   if (fits) {
@@ -1159,31 +1134,171 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     };
     fetch(0);
     if (more) fetch(kHalf);
-    select(
-        [&](auto f) {
+    auto each = [&](auto f) {
 #pragma unroll
-          for (int j = 0; j < kHalf; j++) f(lk[j], lr[j]);
-          if (more) {
+      for (int j = 0; j < kHalf; j++) f(lk[j], lr[j]);
+      if (more) {
 #pragma unroll
-            for (int j = kHalf; j < kEach; j++) f(lk[j], lr[j]);
-          }
-        },
-        pivot, span_end);
-  } else {
-    if (!mapped) {
-#pragma unroll
-      for (int j = 0; j < P; j++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
+        for (int j = kHalf; j < kEach; j++) f(lk[j], lr[j]);
+      }
+    };
+    if (__builtin_expect(masked, 0)) {  // (uniform) a mean with -inf in it lies far below the listed keys: the lowest of them
+      uint32_t not_low = 0u;
+      each([&](int32_t k, int) { not_low = umax(not_low, k != kLowestKey ? ~((uint32_t)k ^ 0x80000000u) : 0u); });
+      not_low = wave_max(not_low);
+      if (lane == 0) wave_pivot[wave] = not_low;
+      __syncthreads();
+      lo = (int32_t)(uniform(~wave_max(wave_pivot[lane % kW])) ^ 0x80000000u);
     }
-    select(
-        [&](auto f) {
+    span = span_end > lo ? (uint32_t)span_end - (uint32_t)lo : 0u;
+    uint32_t half = 0xFFFFFFFFu;  // of the keys that the bin before held
+    while (true) {
+      const int shift = span >= kBins ? 24 - __builtin_clz(span) : 0;
+      each([&](int32_t k, int) {
+        const uint32_t d = (uint32_t)k - (uint32_t)lo;
+        if (k >= lo && d <= limit) atomicAdd(&hist[umin(d >> shift, kBins - 1u)], 1u);
+      });
+      const uint32_t held = narrow(shift);
+      if (limit == 0u) break;
+      if (held <= 64u) {
+        each([&](int32_t k, int) { candidate(k); });
+        rank_candidates(held);
+        break;
+      }
+      if (held > 512u && held > half) {
+        found = false;
+        break;
+      }
+      span = limit;
+  // (not found: keys that meet in one bin again and again)
+      half = held / 2u;
+      if (tid < (int)kBins) hist[tid] = 0u;
+      __syncthreads();
+    }
+    if (found) {
+      threshold = lo;
+      each([&](int32_t k, int row) {
+        const uint32_t word = (uint32_t)row / kBits, bit = 1u << ((uint32_t)row % kBits);
+        if (k > threshold) atomicOr(&bits_above[word], bit);
+        if (k == threshold) atomicOr(&bits_tie[word], bit);
+      });
+    }
+  }
+  if (__builtin_expect(!found, 0)) {
+    // All keys, from the copy of the row: rows with fewer finite scores than are wanted, rows of few values, and where the
+    // sample misled.
+    auto each = [&](auto f) {
+#pragma unroll 2
+      for (int j = 0; j < P; j++) {
+        i32x4_t k = *reinterpret_cast<const i32x4_t*>(&stage[4 * (j * THREADS + tid)]);
 #pragma unroll
-          for (int j = 0; j < P; j++)
+        for (int e = 0; e < 4; e++) k[e] = signed_key(k[e]);
+        f(k, 4u * (uint32_t)(j * THREADS + tid));
+      }
+    };
+    if (!fits) {
+      // Those of -inf are counted and not binned: rows a token does not see yet are most of a row at the start of a prompt,
+      // and the k-th key is -inf where fewer are seen than are wanted.
+      uint32_t not_low = 0u, top = 0u, counts = 0u;  // lowest finite key, highest key, finite keys and those of -inf
+      each([&](i32x4_t k, uint32_t) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) f(key[j][e], 4 * (j * THREADS + tid) + e);
-        },
-        kLowestKey, 0x7FFFFFFF);
+        for (int e = 0; e < 4; e++) {
+          const uint32_t u = (uint32_t)k[e] ^ 0x80000000u;
+          const bool fin = k[e] > kNegInfSigned;
+          top = umax(top, u);
+          not_low = umax(not_low, fin ? ~u : 0u);
+          counts += fin ? 1u : k[e] == kNegInfSigned ? 1u << 16 : 0u;
+        }
+      });
+      top = wave_max(top);
+      not_low = wave_max(not_low);
+      counts = wave_prefix_sum(counts);
+      __syncthreads();  // every wave has read the pivots
+      if (lane == 63) {
+        wave_pivot[wave] = not_low;
+        wave_high[wave] = top;
+        wave_tot[wave] = counts;
+      }
+      __syncthreads();
+      lo = (int32_t)(uniform(~wave_max(wave_pivot[lane % kW])) ^ 0x80000000u);
+      int32_t end = (int32_t)(uniform(wave_max(wave_high[lane % kW])) ^ 0x80000000u);
+      counts = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(lane < kW ? wave_tot[lane % kW] : 0u), 63);
+      const uint32_t n_fin = counts & 0xFFFFu, n_inf = counts >> 16;
+      if (need > n_fin) {  // -inf, or one of the negative NaNs below it
+        need -= n_fin;
+        lo = end = kNegInfSigned;
+        if (need > n_inf) {
+          need -= n_inf;
+          lo = kLowestKey;
+          end = kNegInfSigned - 1;
+        }
+      }
+      limit = (uint32_t)end - (uint32_t)lo;
+    }
+    while (limit != 0u) {
+      // votes go to kCopies copies of the counters, which take the list's place, so that few of a wave's meet
+      constexpr int kVoteCopies = kCap / 2 / (int)kBins, kPerBin = THREADS / (int)kBins;
+      static_assert(kVoteCopies == 4 * kPerBin, "a thread adds four copies");
+      uint32_t* counters = reinterpret_cast<uint32_t*>(list);
+      *reinterpret_cast<u32x4_t*>(&counters[4 * tid]) = u32x4_t{0u, 0u, 0u, 0u};
+      __syncthreads();
+      const int shift = limit >= kBins ? 24 - __builtin_clz(limit) : 0;
+      each([&](i32x4_t k, uint32_t) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t d = (uint32_t)k[e] - (uint32_t)lo;
+          if (k[e] >= lo && d <= limit)
+            atomicAdd(&counters[umin(d >> shift, kBins - 1u) * kVoteCopies + (uint32_t)(lane % kVoteCopies)], 1u);
+        }
+      });
+      __syncthreads();
+      const u32x4_t c = *reinterpret_cast<const u32x4_t*>(&counters[4 * tid]);  // kPerBin neighbouring lanes have a bin
+      uint32_t sum = c.x + c.y + c.z + c.w;
+#pragma unroll
+      for (int m = 1; m < kPerBin; m *= 2) sum += __shfl_xor(sum, m, MSPR_WAVE);
+      if (tid % kPerBin == 0) hist[tid / kPerBin] = sum;
+      const uint32_t held = narrow(shift);
+      if (limit != 0u && held <= 64u) {
+        each([&](i32x4_t k, uint32_t) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) candidate(k[e]);
+        });
+        rank_candidates(held);
+      }
+    }
+    threshold = lo;
+    // the four rows of a piece are in one word of the bitmap
+    each([&](i32x4_t k, uint32_t row) {
+      uint32_t above = 0u, tie = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        above |= k[e] > threshold ? 1u << e : 0u;
+        tie |= k[e] == threshold ? 1u << e : 0u;
+      }
+      if (above != 0u) atomicOr(&bits_above[row / kBits], above << (row % kBits));
+      if (tie != 0u) atomicOr(&bits_tie[row / kBits], tie << (row % kBits));
+    });
+  }
+  __syncthreads();
+
+  // ---- the selected rows
+  uint32_t wa = bits_above[tid], wt = bits_tie[tid];
+  const uint32_t mine = (uint32_t)__popc(wa) | ((uint32_t)__popc(wt) << 16);
+  const uint32_t upto = wave_prefix_sum(mine);
+  if (lane == 63) wave_tot[wave] = upto;
+  __syncthreads();
+  const uint32_t tots = wave_prefix_sum(lane < kW ? wave_tot[lane < kW ? lane : 0] : 0u);
+  const uint32_t excl = upto - mine + (wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)tots, wave > 0 ? wave - 1 : 0) : 0u);
+  int32_t* out = sel + (excl & 0xFFFFu);
+  uint32_t order = excl >> 16;
+  while (wa) {
+    *out++ = (int)kBits * tid + (int)__builtin_ctz(wa);
+    wa &= wa - 1u;
+  }
+  out = sel + ((uint32_t)topk - need);
+  while (wt && order < need) {
+    out[order++] = (int)kBits * tid + (int)__builtin_ctz(wt);
+    wt &= wt - 1u;
   }
 }
 
