@@ -98,8 +98,6 @@ __device__ __forceinline__ float load_as_f32(const void* p, int64_t i) {
   }
 }
 
-__device__ __forceinline__ float wave_xor_f32(float v, int mask) { return __shfl_xor(v, mask, MSPR_WAVE); }
-
 // The value lane (l ^ M) holds, for a single-bit M. Inside a row of 16 lanes the exchange is one or two
 // data-parallel-primitive moves (quad permutes give l^1, l^2, l^3; the half-row and row mirrors give
 // l^7 and l^15, and two of them compose to l^4 and l^8), which cost an ALU slot and no LDS round trip;

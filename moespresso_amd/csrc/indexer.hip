@@ -449,9 +449,7 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     return;
   }
   const int lane = tid & 63;
-  const int lane32 = tid & 31;
   const int wave = tid >> 6;
-  const int half = (tid >> 5) & 1;
   const int m = lane & 31;
   const int g = lane >> 5;
 

@@ -57,11 +57,6 @@ __device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
 __device__ __forceinline__ uint32_t h2_bits(h2_t v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ h2_t bits_h2(uint32_t v) { return __builtin_bit_cast(h2_t, v); }
 
-template <int SDT>
-__device__ __forceinline__ _Float16 load_scale(const void* p, int64_t i) {
-  return (_Float16)load_as_f32<SDT>(p, i);
-}
-
 // Four codes of one 32-bit word to four float16 values (two packed registers), exact integers:
 // byte b becomes the float16 with bits 0x6400 | b = 1024 + b, then the offset is taken off.
 template <int FMT>
@@ -98,7 +93,6 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
   const int64_t kv_row0 = ((int64_t)b * a.n_kv_heads + kvh) * a.kv_rows;  // first key row of this (b, kv head)
   const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.k_codes) + kv_row0 * kD;
   const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.v_codes) + kv_row0 * kD;
-  constexpr int kGroups = FMT == kFmtQ8_0 ? 8 : 4;  // scale groups per row
 
   f32x4_t oacc[16];
 #pragma unroll
@@ -133,7 +127,6 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
   const uint8_t* kbi = reinterpret_cast<const uint8_t*>(a.k_biases);
   const uint8_t* vsc = reinterpret_cast<const uint8_t*>(a.v_scales);
   const uint8_t* vbi = reinterpret_cast<const uint8_t*>(a.v_biases);
-  constexpr int kSB = SDT == MSPR_F32 ? 4 : 2;  // bytes per affine scale / bias
 
   auto load_k = [&](int64_t key0) {
 #pragma unroll

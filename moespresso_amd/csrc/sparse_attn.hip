@@ -131,17 +131,6 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 template <int KDT>
-__device__ __forceinline__ float unpack_lo(uint32_t w) {
-  if constexpr (KDT == MSPR_BF16) return bf16_bits_to_f32((uint16_t)(w & 0xFFFFu));
-  else return f16_bits_to_f32((uint16_t)(w & 0xFFFFu));
-}
-template <int KDT>
-__device__ __forceinline__ float unpack_hi(uint32_t w) {
-  if constexpr (KDT == MSPR_BF16) return bf16_bits_to_f32((uint16_t)(w >> 16));
-  else return f16_bits_to_f32((uint16_t)(w >> 16));
-}
-
-template <int KDT>
 __device__ __forceinline__ float round_to_kdt(float v) {
   if constexpr (KDT == MSPR_BF16) return bf16_bits_to_f32(f32_to_bf16_bits(v));
   else return f16_bits_to_f32(f32_to_f16_bits(v));
@@ -160,8 +149,6 @@ __device__ __attribute__((aligned(16))) const unsigned char g_zero_row[1280] = {
 // that the store instructions run with every lane active and the same count in every wave: 512 floats per lane
 // position, never read.
 __device__ __attribute__((aligned(16))) float g_store_sink[64 * 512];
-
-#define MSPR_GLB_PTR(T, p) ((__attribute__((address_space(1))) T*)(p))
 
 // Infinities of a packed float16 pair become the largest finite values. (IEEE 754-2019 minimum and maximum: a NaN stays one,
 // which v_med3 on the float32 values made the lowest finite value.)

@@ -75,7 +75,6 @@ __device__ __forceinline__ void choose_bucket(const uint32_t* totals, SelectStat
   }
 }
 
-template <int CACHE>
 __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __restrict__ scores_all,
                                                                 int64_t score_stride, int64_t n_rows, int topk,
                                                                 int32_t* __restrict__ sel_all) {
@@ -95,14 +94,6 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __re
   int32_t* sel = sel_all + (int64_t)blockIdx.x * topk;
   const int64_t n_chunks = (n_rows + kThreads - 1) / kThreads;
 
-  uint32_t kreg[CACHE > 0 ? CACHE : 1];
-  if constexpr (CACHE > 0) {
-#pragma unroll
-    for (int i = 0; i < CACHE; i++) {
-      int64_t r = (int64_t)i * kThreads + tid;
-      kreg[i] = r < n_rows ? score_key(scores[r]) : 0u;
-    }
-  }
   if (tid == 0) {
     st.prefix = 0u;
     st.need = (uint32_t)topk;
@@ -118,20 +109,11 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __re
     __syncthreads();
     const uint32_t prefix = st.prefix;
     const uint32_t mask_hi = pass == 0 ? 0u : (0xFFFFFFFFu << (shift + 8u));
-    if constexpr (CACHE > 0) {
-#pragma unroll
-      for (int i = 0; i < CACHE; i++) {
-        int64_t r = (int64_t)i * kThreads + tid;
-        uint32_t key = kreg[i];
-        if (r < n_rows && (key & mask_hi) == prefix) atomicAdd(&hist[((key >> shift) & 0xFFu) * kCopies + lane], 1u);
-      }
-    } else {
-      for (int64_t c = 0; c < n_chunks; c++) {
-        int64_t r = c * kThreads + tid;
-        if (r < n_rows) {
-          uint32_t key = score_key(scores[r]);
-          if ((key & mask_hi) == prefix) atomicAdd(&hist[((key >> shift) & 0xFFu) * kCopies + lane], 1u);
-        }
+    for (int64_t c = 0; c < n_chunks; c++) {
+      int64_t r = c * kThreads + tid;
+      if (r < n_rows) {
+        uint32_t key = score_key(scores[r]);
+        if ((key & mask_hi) == prefix) atomicAdd(&hist[((key >> shift) & 0xFFu) * kCopies + lane], 1u);
       }
     }
     __syncthreads();
@@ -156,20 +138,11 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __re
   if (st.live <= (uint32_t)kListCap) {
     // compact the keys that match the 16-bit prefix; their order does not matter here
     const uint32_t prefix = st.prefix;
-    if constexpr (CACHE > 0) {
-#pragma unroll
-      for (int i = 0; i < CACHE; i++) {
-        int64_t r = (int64_t)i * kThreads + tid;
-        uint32_t key = kreg[i];
-        if (r < n_rows && (key & 0xFFFF0000u) == prefix) list[atomicAdd(&st.list_n, 1u)] = key;
-      }
-    } else {
-      for (int64_t c = 0; c < n_chunks; c++) {
-        int64_t r = c * kThreads + tid;
-        if (r < n_rows) {
-          uint32_t key = score_key(scores[r]);
-          if ((key & 0xFFFF0000u) == prefix) list[atomicAdd(&st.list_n, 1u)] = key;
-        }
+    for (int64_t c = 0; c < n_chunks; c++) {
+      int64_t r = c * kThreads + tid;
+      if (r < n_rows) {
+        uint32_t key = score_key(scores[r]);
+        if ((key & 0xFFFF0000u) == prefix) list[atomicAdd(&st.list_n, 1u)] = key;
       }
     }
     __syncthreads();
@@ -227,20 +200,10 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __re
   };
   for (int64_t g0 = 0; g0 < n_chunks; g0 += 64) {
     const int gchunks = (int)((n_chunks - g0) < 64 ? (n_chunks - g0) : 64);
-    if constexpr (CACHE > 0) {
-#pragma unroll
-      for (int ci = 0; ci < CACHE; ci++) {
-        if (ci < gchunks) {
-          int64_t r = (int64_t)ci * kThreads + tid;
-          count_chunk(ci, r < n_rows, kreg[ci]);
-        }
-      }
-    } else {
-      for (int ci = 0; ci < gchunks; ci++) {
-        int64_t r = (g0 + ci) * kThreads + tid;
-        bool live = r < n_rows;
-        count_chunk(ci, live, live ? score_key(scores[r]) : 0u);
-      }
+    for (int ci = 0; ci < gchunks; ci++) {
+      int64_t r = (g0 + ci) * kThreads + tid;
+      bool live = r < n_rows;
+      count_chunk(ci, live, live ? score_key(scores[r]) : 0u);
     }
     for (int i = gchunks * kWaves + tid; i < kThreads; i += kThreads) {
       cnt_above[i] = 0u;
@@ -277,20 +240,10 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(const float* __re
       carry[1] = base_t + it;
     }
     __syncthreads();
-    if constexpr (CACHE > 0) {
-#pragma unroll
-      for (int ci = 0; ci < CACHE; ci++) {
-        if (ci < gchunks) {
-          int64_t r = (int64_t)ci * kThreads + tid;
-          emit_chunk(ci, r, r < n_rows, kreg[ci]);
-        }
-      }
-    } else {
-      for (int ci = 0; ci < gchunks; ci++) {
-        int64_t r = (g0 + ci) * kThreads + tid;
-        bool live = r < n_rows;
-        emit_chunk(ci, r, live, live ? score_key(scores[r]) : 0u);
-      }
+    for (int ci = 0; ci < gchunks; ci++) {
+      int64_t r = (g0 + ci) * kThreads + tid;
+      bool live = r < n_rows;
+      emit_chunk(ci, r, live, live ? score_key(scores[r]) : 0u);
     }
     __syncthreads();
   }
@@ -380,7 +333,10 @@ __device__ __forceinline__ Pick pick_bucket(const uint32_t* totals, uint32_t nee
 // from the same totals, which saves the broadcast barriers.
 // Rows past n_rows are given key 0: they can only tie with the lowest possible key and lose every
 // tie to a real row (ties go to the lower index), so no pass needs a bounds check.
-template <int C>
+// (The sampled kernel further down takes the rows of which a small part is wanted; the pivot path here is for those of up to
+// 8192 scores with more. Of longer rows, none that is left has a pivot whose keys would fit the list.)
+static_assert(kFastCap / 2 >= kListCap, "the list of the full passes fits the space of the pivot path's");
+template <int C, bool PIVOT>
 __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __restrict__ scores_all,
                                                                  int64_t score_stride, int n_rows, int topk,
                                                                  int sample_rank, int32_t* __restrict__ sel_all) {
@@ -394,7 +350,7 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
   __shared__ uint32_t totals[256];
   __shared__ uint32_t small_hist[2][256];   // digits 2 and 3 on the compacted list
   // survivor rows of the pivot path (16-bit row numbers), or the compacted keys of the full passes
-  __shared__ __attribute__((aligned(16))) uint32_t list_words[kFastCap / 2 > kListCap ? kFastCap / 2 : kListCap];
+  __shared__ __attribute__((aligned(16))) uint32_t list_words[PIVOT ? kFastCap / 2 : kListCap];
   uint32_t* list = list_words;
   uint16_t* fast_rows = reinterpret_cast<uint16_t*>(list_words);
   __shared__ uint32_t list_n;
@@ -407,7 +363,7 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
   const int wave = tid >> 6;
   const float* scores = scores_all + (int64_t)blockIdx.x * score_stride;
   int32_t* sel = sel_all + (int64_t)blockIdx.x * topk;
-  if (sample_rank > 0)
+  if (PIVOT && sample_rank > 0)
     for (int i = tid; i < 5 * 256; i += kThreads) (&fhist[0][0])[i] = 0u;  // ordered by the barriers of the load
 
   // Load with lane-contiguous 16-byte reads (a wave reads 1 KB at a time), then hand every thread its
@@ -472,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
     __syncthreads();
     return pick_box[slot];
   };
-  if (sample_rank > 0) {
+  if (PIVOT && sample_rank > 0) {
     const uint32_t skey = kreg[0];
     wave_hist_add(fhist[0], (int)(skey >> 24), lane);  // the top byte is shared by most rows: vote per wave
     __syncthreads();
@@ -1389,10 +1345,10 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
   else if (n_rows <= 8192 && batch > 32) MSPR_TOPK_ROW(16, 512);
 #undef MSPR_TOPK_ROW
   else if (n_rows <= 8 * 1024)
-    topk_blocked_kernel<8><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, pivot_sample_rank(8, topk), sel);
+    topk_blocked_kernel<8, true><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, pivot_sample_rank(8, topk), sel);
   else if (n_rows <= 32 * 1024)
-    topk_blocked_kernel<32><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, pivot_sample_rank(32, topk), sel);
-  else topk_select_kernel<0><<<grid, block, 0, st>>>(scores, score_stride, n_rows, topk, sel);
+    topk_blocked_kernel<32, false><<<grid, block, 0, st>>>(scores, score_stride, (int)n_rows, topk, 0, sel);
+  else topk_select_kernel<<<grid, block, 0, st>>>(scores, score_stride, n_rows, topk, sel);
   MSPR_CHECK_LAUNCH("topk_select");
   return MSPR_OK;
 }
