@@ -87,3 +87,37 @@ def test_quantised_prefill_may_overwrite_its_queries(L, past):
         assert torch.equal(out.cpu(), want), shared
         if not shared:
             assert torch.equal(queries.cpu(), q)
+
+
+@pytest.mark.parametrize("name", ["queries", "k_codes", "k_scales", "k_biases", "v_codes", "v_scales", "v_biases", "chunk_k", "chunk_v"])
+@pytest.mark.parametrize("L,past", [(97, 512), (97, 2048), (203, 2048)])  # prefix unpacked in the kernel, and converted
+def test_quantised_prefill_may_overwrite_any_operand(L, past, name):
+    """With four key ranges or more the output is written by the merge alone, when every operand has been read: it may overlap
+    any of them, the whole or an end of it. (Rounded queries must then not wait in it.)"""
+    from moespresso_amd import _lib
+
+    lib, dev = _lib.lib(), torch.device("cuda:0")
+    out_bytes = 16 * L * 256 * 4
+    # a range's partials: a row of float32 sums and two numbers for each query of a head
+    assert lib.mspr_flash_prefill_workspace_bytes(1, 16, 2, L, past) >= 4 * (out_bytes + 16 * L * 8)
+    q, k, v, want = _case(16, 2, L, past, seed=L + past)
+    one, zero, chunk = torch.ones((1, 2, past, 4)), torch.zeros((1, 2, past, 4)), torch.zeros((1, 2, L, 256))
+    host = dict(queries=q, k_codes=k.to(torch.uint8), k_scales=one, k_biases=zero, v_codes=v.to(torch.uint8), v_scales=one,
+                v_biases=zero, chunk_k=chunk, chunk_v=chunk)
+    ws = torch.empty(int(lib.mspr_sdpa_fa_prefill_q8_workspace_bytes(1, 16, 2, L, past)), dtype=torch.uint8, device=dev)
+    raw = host[name].contiguous().view(torch.uint8).reshape(-1)
+    half = raw.numel() // 32 * 16
+    for shift in (0, half, raw.numel() - 16, 16 - out_bytes, half - out_bytes):     # of the output against the operand
+        ops = {n: t.to(dev) for n, t in host.items()}
+        arena = torch.full((out_bytes * 2 + raw.numel() + 64,), 0xFF, dtype=torch.uint8, device=dev)
+        at = out_bytes + 16                              # (the arena starts at a multiple of 256, so both are multiples of 16)
+        arena[at:at + raw.numel()] = raw.to(dev)
+        ops[name] = arena[at:at + raw.numel()]
+        out = arena[at + shift:at + shift + out_bytes]
+        p = {n: _lib.ptr(t) for n, t in ops.items()}
+        _lib.check(_lib.launch(
+            dev, "mspr_sdpa_fa_prefill_q8",
+            p["queries"], p["k_codes"], p["k_scales"], p["k_biases"], p["v_codes"], p["v_scales"], p["v_biases"], 0,
+            p["chunk_k"], p["chunk_v"], 0, 1, 16, 2, 256, L, past, past, 0.0625, 64, 8, _lib.ptr(out), _lib.ptr(ws),
+            ws.numel()), "sdpa_fa_prefill_q8")
+        assert torch.equal(out.view(torch.float32).reshape(want.shape).cpu(), want), shift
