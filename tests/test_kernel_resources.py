@@ -88,3 +88,10 @@ def test_scalar_arguments_of_kernels_are_preloaded():
         text = build.device_assembly(os.path.join(build.CSRC, source))
         lengths = [int(l.split()[1]) for l in text.splitlines() if l.strip().startswith(".amdhsa_user_sgpr_kernarg_preload_length")]
         assert len(lengths) == kernels and all(n >= 7 for n in lengths), (source, lengths)
+
+
+@pytest.mark.parametrize("source,kernels", [("indexer.hip", 14), ("indexer_tiled.hip", 5)])
+def test_scalar_arguments_of_the_other_score_kernels_are_preloaded(source, kernels):
+    text = build.device_assembly(os.path.join(build.CSRC, source))
+    lengths = [int(l.split()[1]) for l in text.splitlines() if l.strip().startswith(".amdhsa_user_sgpr_kernarg_preload_length")]
+    assert len(lengths) == kernels and all(n >= 6 for n in lengths), lengths
