@@ -196,14 +196,11 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   const int head_halves = 1 << (a.rep_shift - hpg_shift);
   const int n_blocks = (a.q_len + 31) / 32;
   const int n_pairs = a.q_blocks / head_halves;
-  // Where ranges are long and four or more, workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run of the list (batch, KV
-  // head, range, pair): an L2 then holds the keys of few ranges and one or two heads' queries, which all pairs of a range
-  // pass together. Elsewhere the ranges go round the XCDs. Us, round and in runs: 16 / 4 heads, 670 queries over 6000 keys
-  // (9 ranges of 23 tiles) 84.1 and 79.9, 350 over 3000 (10 of 11) 43.2 and 41.0; 16 / 2 heads, 500 quantised over 3000
-  // 72.0 and 68.5, 290 over 12000 (15 of 26) 74.2 and 71.6, 203 over 9001 (16 of 18) equal; but 150 over 2000 (13 of 6) 25.9
-  // and 27.5, 33 over 9000 (50 of 6) 28.1 and
-  // 29.0: in runs the partials leave the L2s 2 us later. Two ranges (2048 quantised queries over 34952): 987 and, with the
-  // queries rounded ahead as below, 997.
+  // RUNS (four ranges or more, of ten tiles or more): workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run
+  // of the list (batch, KV head, range, pair). An L2 then holds the keys of few ranges and one or two heads' queries, which
+  // all pairs of a range pass together. Elsewhere the ranges go round the XCDs, as in runs the partials leave the L2s 2 us
+  // later. Us, round and in runs: 16 / 4 heads, 670 queries over 6000 keys (9 ranges of 23 tiles) 84.1 and 79.9, 350 over 3000
+  // (10 of 11) 43.2 and 41.0; 16 / 2 heads, 150 over 2000 (13 of 6) 25.9 and 27.5.
   int work = blockIdx.x;
   int sp, q_block;
   if constexpr (RUNS) {
@@ -1049,10 +1046,11 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
     a.ws_o = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(workspace) + tail);
     a.ws_ml = a.ws_o + (size_t)a.n_splits * batch * n_q_heads * q_len * kD;
   }
-  // Where four key ranges or more pass the queries again and again (16 for 203 of them), the launch that makes the rows rounds them
-  // once, so that a workgroup of the attention fetches 128 KB of them in front of its first tile and not 256. They lie in the
-  // output, which is the merge's to write, unless it overlaps what is still to be read. Us: 203 queries over 9001 rows 73.6
-  // -> 72.2, 128 over 20000 82.4 -> 80.1, 30 over 9001 the same.
+  // Where four key ranges or more pass the queries again and again (16 for 203 of them), the launch that makes the rows
+  // rounds them once, so that a workgroup of the attention fetches 128 KB of them in front of its first tile and not 256.
+  // They lie in the output, which is the merge's to write, unless it overlaps what is still to be read. Us: 203 queries over
+  // 9001 rows 73.6 -> 72.2, 128 over 20000 82.4 -> 80.1, 30 over 9001 the same; with two ranges (2048 over 34952) it would
+  // cost, 987 -> 997.
   const size_t io_bytes = (size_t)batch * n_q_heads * q_len * kD * sizeof(float);
   auto apart = [&](const void* p, size_t bytes) {
     const uintptr_t o = (uintptr_t)out, i = (uintptr_t)p;
@@ -1073,8 +1071,9 @@ extern "C" int mspr_sdpa_fa_prefill_q8(const void* queries, const void* pk_wq, c
   a.pv_s = pv_scales;
   a.pv_b = pv_biases;
   hipStream_t st = (hipStream_t)stream;
-  // bfloat16 staging runs the bfloat16 matrix instructions: the device holds a higher clock under them than under the float16 ones, and the 8-bit codes
-  // leave the rounding of the staging type (2^-9 of a value) below their own step. Shorter chunks stay float16.
+  // bfloat16 staging runs the bfloat16 matrix instructions: the device holds a higher clock under them than under the float16
+  // ones, and the 8-bit codes leave the rounding of the staging type (2^-9 of a value) below their own step. Shorter chunks
+  // stay float16.
   const bool bf16_staging = prefill_q8_bf16(q_len);
   const int q_rows = q16 ? rep * q_len : 0;
   dim3 rgrid((unsigned)((tail_rows + 15) / 16 + (q_rows + 15) / 16), (unsigned)n_kv_heads, (unsigned)batch);

@@ -459,11 +459,10 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
 
   // The eight waves QAT the 64 query rows, eight lanes a row; the power-of-two table sits in LDS, so the pass waits for memory
   // once. Every workgroup does the whole block, so it is instructions of one CU that bound it: 7900 cycles with 32 lanes a row
-  // and the lattice step in float32 arithmetic, then 4000 to 4700 of the workgroup's 12200 (961 pool rows: the launch 8.4 -> 6.3
-  // us, a decode token 27.3 -> 25.4). The butterflies wait for the query rows alone: behind the barrier of the table all waves
-  // waited for the ones with a pool tile to request it (sixteen loads of 64 lines). With that, one barrier for the waves'
-  // verdicts on their rows instead of three, and nothing spilled, us by pool rows, in a graph: 961 5.33 -> 4.31, 8000 5.93 ->
-  // 4.56, 32000 7.4 -> 5.9, 60000 10.6 -> 7.65; rows that need three pieces, 961, 11.3 -> 6.3.
+  // and the lattice step in float32 arithmetic, then 4000 to 4700 of the workgroup's 12200 (961 pool rows: 8.4 -> 6.3 us).
+  // The butterflies wait for the query rows alone: behind the barrier of the table all waves waited for the ones with a pool
+  // tile to request it (sixteen loads of 64 lines). With one barrier for the waves' verdicts on their rows, and nothing
+  // spilled: 961 pool rows 5.33 -> 4.31 us in a graph, 60000 10.6 -> 7.65.
   const int q_head = tid >> 3, q_part = tid & 7;
   Qat16 mine;
   load_row16<DT>(q, q_head < n_heads ? q_head : n_heads - 1, q_part, mine.x);

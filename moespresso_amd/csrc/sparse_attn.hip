@@ -8,10 +8,10 @@
 // Each K row is read from HBM once and staged row-major in LDS (ring of three tiles, filled by
 // asynchronous global->LDS copies). The eight waves are (head group hg of 32 heads) x (quarter dh):
 // for S^T = K.Q^T a wave contracts its quarter of the row width, the four quarters are summed
-// through LDS, a quarter of the keys by each wave, and the weights handed round the same way; for O^T = V^T.P^T it owns 128 of the 512 output columns. Two waves share a SIMD and
-// fill each other's waits (a wave has no matrix work while it stages or exchanges). V^T operands come
-// out of the same row-major tile through the LDS transpose read, so no second copy of the tile
-// exists.
+// through LDS, a quarter of the keys by each wave, and the weights handed round the same way; for
+// O^T = V^T.P^T it owns 128 of the 512 output columns. Two waves share a SIMD and fill each other's
+// waits (a wave has no matrix work while it stages or exchanges). V^T operands come out of the same
+// row-major tile through the LDS transpose read, so no second copy of the tile exists.
 //
 // Partial (m, l, O) per key range are merged by a second kernel (log-sum-exp), which also applies the
 // sink, the normalisation, the output cast and the optional inverse rope. (Merging inside the split
@@ -359,9 +359,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   u32x4_t qf[G::kSteps];
   // 16-bit queries are requested in runs of a head's row (a wave's share is 32 heads x kPart columns) and change places through
   // LDS, in two passes of kQLo and kQHi 16-byte pieces a head: asked for in operand order, 32 bytes of each of 32 heads an
-  // instruction, the block kept the address unit busy for 2300 cycles in front of the tiles. With the tile slots below counted
-  // up instead of divided out, the first tile is multiplied 600 to 1500 cycles earlier: 1 sequence of 2048 + 128 rows 22.9 ->
-  // 22.3 us, 5 of 1024 + 128 28.0 -> 27.85, a token over 961 pool rows 27.3 -> 27.2.
+  // instruction, the block kept the address unit busy for 2300 cycles in front of the tiles. (A decode layer of one sequence
+  // of 2048 + 128 rows 22.9 -> 22.3 us, with the tile slots below counted up instead of divided out.)
   constexpr int kQLo = 2 * ((G::kSteps + 1) / 2), kQHi = G::kPart / 8 - kQLo;
   const bool q_pieces = QDT == kQSame && a.q_head_stride >= 0 && a.q_head_stride < (1 << 24);  // 32-bit offsets
   const int q_heads_left = a.n_heads - hb * 64 - hg * 32;                                       // the rest repeat the first
@@ -804,7 +803,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   // overflowing. Its rounding (2^-11 relative) stays below the rounding of the final output.
   const int64_t part = ((int64_t)(seq * a.n_hblk + hb) * a.n_splits + sp);
   // Through the L2 (store_window): a layer of 16 sequences over 32768 keys 49.3 -> 47.9 us, of 8 36.6 -> 35.2; the merge reads
-  // them from beyond the L2 either way (17 MB by the counters). One token's few (the rotated form) are out sooner through the cache: 23.4 and 23.7 us.
+  // them from beyond the L2 either way (17 MB by the counters). One token's few (the rotated form) are out sooner through the
+  // cache: 23.4 and 23.7 us.
   const __amdgpu_buffer_rsrc_t win = store_window(a.ws_o + (part * kWaves + wave) * (int64_t)(4 * 16 * 64), 8192);
   const float inv_l = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
 #pragma unroll

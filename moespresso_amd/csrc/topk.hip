@@ -1,19 +1,19 @@
 // Deterministic top-k over float32 score rows: select on monotone uint32 keys, then ordered emission
 // (rows strictly above the k-th key in ascending row order, then the lowest-index rows tied with it).
 //
-// One 1024-thread workgroup per score row. Rows of up to 32768 scores are read once and kept in
-// registers, every thread owning a block of consecutive rows. Two ways to the k-th key:
-//  * pivot path: a 1024-row sample gives a 16-bit key prefix safely below the k-th key, the rows at
-//    or above it (a few thousand) are compacted in row order and three small digit passes plus the
-//    emission run on that list. The kernel checks exactly that the list contains the k-th key; the
-//    sample decides how long the call takes, never what it returns.
-//  * full passes (also the fallback of the pivot path): MSB radix select with four 8-bit digits over
-//    all keys. Histograms are 256 bins x 64 copies in LDS, copy = lane id, laid out [bin][copy], so
-//    every lane of an LDS atomic hits its own bank whatever the digit distribution is (scores of one
-//    row usually share their top byte, which would serialise a single shared counter 64-fold). After
-//    two digits the keys that still match the prefix are usually a handful; they are compacted into
-//    an LDS list and the last two digits run on that list only.
-// Longer rows use the striped kernel, which re-reads global memory each pass.
+// One workgroup per score row; which kernel depends on the row's length, k and the number of rows (mspr_launch_topk):
+//  * topk_sampled_kernel, rows of 2049 to 32768 scores of which a small part is wanted: the keys above a sampled pivot are
+//    listed, binned and ranked.
+//  * topk_row_kernel, rows of up to 8192: the keys stay in registers and are binned by value range.
+//  * topk_blocked_kernel, the others of up to 32768: a thread owns consecutive rows; a list above a pivot up to 8192 scores,
+//    else four 8-bit digits from the top over all keys.
+//  * topk_select_kernel, longer rows: the same digits, global memory re-read each pass.
+// Samples and pivots decide how long a call takes, never what it returns: that a list holds the k-th key is checked exactly.
+//
+// Digit histograms over all keys are 256 bins x 64 copies in LDS, copy = lane id, laid out [bin][copy], so every lane of an
+// LDS atomic hits its own bank whatever the digit distribution is (scores of one row usually share their top byte, which
+// would serialise a single shared counter 64-fold). After two digits the keys that still match the prefix are usually a
+// handful; they are compacted into an LDS list and the last two digits run on that list only.
 #include <cmath>
 
 #include "common.h"
