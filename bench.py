@@ -8,12 +8,12 @@ One step = one DeepSeek-V4-style sparse decode attention layer at 128K context o
       -> sparse multi-head-latent decode attention over the 2048 gathered rows plus the last
          128 rows of a 131072-token bf16 latent cache (576-wide K, 512-wide V, 64 heads)
 
-for a batch of 16 sequences (BASELINE configs 4 and 5 chained). Inputs are resident in HBM before
+for a batch of 16 sequences. Inputs are resident in HBM before
 the timed region; the step is captured in a HIP graph per buffer set and the timed loop replays
 the graphs round-robin over several buffer sets so that neither L2 nor the Infinity Cache can hold
 the streamed rows between steps.
 
-Prints ONE JSON line (see README of the driver contract): metric/value plus `roofline` for the
+Prints ONE JSON line : metric/value plus `roofline` for the
 dominant kernel (GPU-side duration from HIP events around that kernel on its launch stream) and
 `cpu_baseline` (a threaded torch restatement of the same layer, pinned against the NumPy oracle by the
 CPU tests, on a bounded sample on this host's cores; the float64 NumPy oracle itself is timed beside it).
@@ -107,10 +107,10 @@ def measured_traffic_bytes(kernel_prefix: str, workgroups: int):
         pass
     return None
 
-# workload constants (BASELINE configs 4 and 5)
+# workload constants of the sparse decode layer
 N_IDX_HEADS, IDX_DIM, N_KEYS, TOPK = 64, 128, 32768, 2048
 N_HEADS, K_DIM, V_DIM, N_TOKENS, WINDOW = 64, 576, 512, 131072, 128
-# algorithmic bytes per sequence: gathered rows + q + out + ids (config 5); keys + scales + q,w + ids (config 4)
+# algorithmic bytes per sequence: gathered rows + q + out + ids (attention); keys + scales + q,w + ids (indexer)
 MLA_BYTES_PER_SEQ = (TOPK + WINDOW) * K_DIM * 2 + N_HEADS * K_DIM * 2 + N_HEADS * V_DIM * 2 + TOPK * 4
 IDX_BYTES_PER_SEQ = N_KEYS * IDX_DIM + N_KEYS * 4 + N_IDX_HEADS * IDX_DIM * 2 + N_IDX_HEADS * 4 + TOPK * 4
 
@@ -219,8 +219,8 @@ def cpu_baseline(seconds_budget: float = 10.0, threads: int | None = None):
 
 
 def cpu_other_configs():
-    """BASELINE configs 2 and 3 on the host through the NumPy oracle, on bounded samples (a reported baseline):
-    config 3 whole at batch 1; config 2 on 128 of the 4096 query rows (the last ones: the deepest causal rows),
+    """The flash prefill and the Q8_0 decode on the host through the NumPy oracle, on bounded samples (a reported baseline):
+    the decode whole at batch 1; the prefill on 128 of the 4096 query rows (the last ones: the deepest causal rows),
     scaled by the ratio of causal FLOPs."""
     from oracle import qwen
 
@@ -272,7 +272,7 @@ def cpu_other_configs():
 
 
 def cpu_config1():
-    """BASELINE config 1 (dense GQA decode, 8 q heads / 1 KV head, D=128, 4096 keys, fp16) on the host: the NumPy
+    """Dense GQA decode (8 q heads / 1 KV head, D=128, 4096 keys, fp16) on the host: the NumPy
     restatement of softmax attention, warm-up 3, 20 repeats."""
     from oracle import qwen
 
@@ -286,11 +286,11 @@ def cpu_config1():
     for _ in range(20):
         qwen.gqa_decode_attention(q, k, v, 128 ** -0.5).astype(np.float16)
     return {"us": round((time.perf_counter() - t0) / 20 * 1e6, 1), "kind": "port", "cores": 1,
-            "workload": "dense GQA decode, 8q/1kv heads, D=128, 4096 fp16 keys (BASELINE config 1), NumPy float64"}
+            "workload": "dense GQA decode, 8q/1kv heads, D=128, 4096 fp16 keys, NumPy float64"}
 
 
 def bench_prefill(dev, gen, reps=10, warmup=20):
-    """4096-token bf16 chunk over a 32768-token prefix, 16 q / 2 KV heads, D=256.
+    """Flash prefill: 4096-token bf16 chunk over a 32768-token prefix, 16 q / 2 KV heads, D=256.
 
     The launches run back to back; the first ones after lighter work are about a tenth slower than the
     sustained rate, hence the warm-up."""
@@ -314,7 +314,7 @@ def bench_prefill(dev, gen, reps=10, warmup=20):
     tf = flops / (ms * 1e-3) / 1e12
     return {"ms": round(ms, 4), "TFLOPs": round(tf, 1), "peak_TFLOPs": 2500.0, "frac": round(tf / 2500.0, 4),
             "tokens_per_s": round(L / (ms * 1e-3), 1), "bound": "mfma",
-            "workload": "causal prefill, 4096 new x 32768 prefix, 16q/2kv heads, D=256, bf16 (BASELINE config 2)"}
+            "workload": "causal prefill, 4096 new x 32768 prefix, 16q/2kv heads, D=256, bf16"}
 
 
 def bench_prefill_q8(dev, gen, reps=6, warmup=10):
@@ -356,7 +356,7 @@ def bench_prefill_q8(dev, gen, reps=6, warmup=10):
 
 
 def bench_q8_decode(dev, gen, reps=40):
-    """BASELINE config 3: GQA decode over a Q8_0 cache of 37000 tokens, batch 1 and 8."""
+    """GQA decode over a Q8_0 cache of 37000 tokens, batch 1 and 8."""
     from moespresso_amd import _lib
     from moespresso_amd.runtime.qwen import kquant
 
@@ -386,7 +386,7 @@ def bench_q8_decode(dev, gen, reps=40):
                         "GBps": round(nbytes / ((split + merge) * 1e-6) / 1e9, 1),
                         "frac_of_8TBps": round(nbytes / ((split + merge) * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)}
         del sets
-    out["workload"] = "GQA decode, 16q/2kv heads, D=256, 37000-token int8+f16/32 cache (BASELINE config 3)"
+    out["workload"] = "GQA decode, 16q/2kv heads, D=256, 37000-token int8+f16/32 cache"
     # the reference's own decode callable at the same depth: affine 8-bit cache (group 64, bfloat16 scales and
     # biases as served), float32 queries, batch 1 (runtime/qwen/full_attention.py:323-335 call site)
     sets = []

@@ -14,8 +14,8 @@
  *     reported a launch error. mspr_last_error() gives the reason as text.
  *
  * Each entry point cites the reference interface it stands in for (paths under
- * the reference tree). Entry points marked "extension" have the BASELINE
- * configuration shapes (batch > 1, fp8 keys, 576/512 MLA, bf16, g32 Q8) that
+ * the reference tree). Entry points marked "extension" have served
+ * shapes (batch > 1, fp8 keys, 576/512 MLA, bf16, g32 Q8) that
  * the reference's own callables reject.
  */
 #ifndef MOESPRESSO_AMD_H
@@ -105,7 +105,7 @@ int mspr_fused_decode_prep_fixed(const void* q_idx, int q_dtype, int n_heads, co
                                  const float* inv_freq, const int32_t* params, float scale, int topk,
                                  int32_t* sel, void* row_out, float* scores, void* stream);
 
-/* Extension: batched lightning-indexer scores with FP8 keys.
+/* Extension (64 heads x 128, 32768 keys): batched lightning-indexer scores with FP8 keys.
  *   scores[b,r] = sum_h w[b,h] * relu(q[b,h] . e4m3(keys[b,r])) * key_scales[b,r]
  * q: bf16 [batch,n_heads,128] (n_heads <= 64); keys: E4M3FN bytes [batch,n_rows,128];
  * key_scales: f32 [batch,n_rows] (> 0); weights: f32 [batch,n_heads]; scores: f32 [batch,n_rows]. */
@@ -211,7 +211,7 @@ int mspr_fused_decode_sdpa_fixed(const void* q, int n_heads, const void* window,
                                  float scale, void* out, void* workspace, size_t workspace_bytes,
                                  void* stream);
 
-/* Extension: batched sparse multi-head latent decode attention.
+/* Extension (64 heads, 576 / 512 wide, 131072 rows): batched sparse multi-head latent decode attention.
  * Every head of batch b attends rows kv[b, rows[b, :]] of a shared latent cache; K is the whole
  * k_dim-wide row and V its first v_dim columns.
  * q: [batch,n_heads,k_dim] of dtype (f16|bf16); kv: [batch,n_pool,k_dim] same dtype;
@@ -289,7 +289,7 @@ int mspr_sdpa_decode_q8(const void* queries, int q_dtype, const void* k_wq, cons
                         int head_dim, int64_t n_keys, int64_t kv_rows, float scale, int group_size, int bits,
                         void* out, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Extension: the same decode over a Q8_0 cache — int8 codes
+/* Extension (37000 keys, 16 / 2 heads): the same decode over a Q8_0 cache — int8 codes
  * [batch,n_kv_heads,kv_rows,256] with one float16 scale per 32 elements
  * [batch,n_kv_heads,kv_rows,8], value = code*scale (the first n_keys rows of every head are attended).
  * queries/out: [batch,n_q_heads,256] of q_dtype (f32|f16|bf16). */
@@ -301,7 +301,7 @@ int mspr_sdpa_decode_q8_0(const void* queries, int q_dtype, const void* k_codes,
 /* Causal chunked-prefill GQA attention over a dense 16-bit KV cache that already holds the chunk:
  * query row i (position past_len + i) attends keys [0, past_len + i].
  * Stands in for mx.fast.scaled_dot_product_attention(mask="causal") over the fetched cache, the
- * composed prefill route of runtime/qwen/full_attention.py:399-409, at BASELINE config 2.
+ * composed prefill route of runtime/qwen/full_attention.py:399-409 (4096 new over 32768 cached tokens).
  * q/out: [batch,n_q_heads,q_len,256] of dtype (f16|bf16); k, v: [batch,n_kv_heads,kv_rows,256]
  * same dtype, rows [0, past_len+q_len) valid; n_q_heads/n_kv_heads in {1,2,4,8}. */
 int mspr_flash_prefill(const void* q, const void* k, const void* v, int dtype, int batch, int n_q_heads,

@@ -2,8 +2,8 @@
 
 Mirror of the reference module
 ``src/moespresso/runtime/deepseek_v4/indexed_attention_kernel.py`` for the
-one-token decode consumer, plus the batched multi-head-latent form of the
-BASELINE configuration (576-wide K, 512-wide V, bf16, batch > 1).
+one-token decode consumer, plus a batched multi-head-latent form
+(576-wide K, 512-wide V, bf16, batch > 1).
 
 Visit rules of the decode consumer (reference kernel source, :120-173): ring
 rows for positions ``[max(first_raw, pos0+1-window), pos0]`` at
@@ -120,7 +120,7 @@ def indexed_mixed_attention_decode(q, raw_kv, comp_kv, topk, sinks, *, pos0: int
 
 def sparse_mla_decode(q, kv, rows, *, scale: float, v_dim: int = 512, window_start: int | None = None,
                       window_rows: int = 0, sinks=None, workspace=None, row_mul: int = 1, row_add: int = 0):
-    """Batched sparse multi-head-latent decode attention (BASELINE config 5 shape).
+    """Batched sparse multi-head-latent decode attention (as served: 64 heads, 576 / 512 wide).
 
     Every head of batch entry ``b`` attends ``kv[b, rows[b, i]]`` for each
     gathered id plus the contiguous window ``kv[b, window_start : window_start

@@ -230,7 +230,7 @@ def fused_score_tail(scores, weights_raw, params, *, scale) -> torch.Tensor:
 
 
 # ----------------------------------------------------------------------------
-# Extensions beyond the reference module (BASELINE config 4 shapes).
+# Extensions beyond the reference module (batches, FP8 keys).
 # ----------------------------------------------------------------------------
 
 def topk_select(scores: torch.Tensor, topk: int) -> torch.Tensor:
@@ -270,7 +270,7 @@ def topk_select(scores: torch.Tensor, topk: int) -> torch.Tensor:
 
 
 def indexer_scores_fp8(q, keys, key_scales, weights) -> torch.Tensor:
-    """Batched lightning-indexer score rows with FP8 keys (BASELINE config 4 shape).
+    """Batched lightning-indexer score rows with FP8 keys (as served: 64 heads x 128, 32768 keys).
 
     ``scores[b, r] = sum_h weights[b, h] * relu(q[b, h] . e4m3(keys[b, r])) * key_scales[b, r]``.
     The batched, fp8-key extension of ``fused_qat_indexer_scores`` (whose

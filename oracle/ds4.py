@@ -813,7 +813,7 @@ def fused_decode_sdpa(q, window, row, pooled, sel, sinks, inv_freq, params, *, s
 
 
 # --------------------------------------------------------------------------
-# BASELINE config 4/5 shapes (batched extensions of a3/a6/a8)
+# FP8 keys and the latent cache (batched extensions of a3/a6/a8)
 # --------------------------------------------------------------------------
 
 def e4m3_decode(codes: np.ndarray) -> np.ndarray:
@@ -844,7 +844,7 @@ def indexer_scores_fp8(q: np.ndarray, key_codes: np.ndarray, key_scales: np.ndar
     """Lightning-indexer score row with FP8 keys, float64.
 
     ``score[b,r] = sum_h w[b,h] * relu(q[b,h] . (e4m3(codes[b,r]) * kscale[b,r]))``;
-    the batched, fp8-key form of a3 named by BASELINE config 4.
+    the batched, fp8-key form of a3.
     q ``[B,H,128]`` (bf16 values as float32), key_codes uint8 ``[B,N,128]``,
     key_scales f32 ``[B,N]``, weights f32 ``[B,H]`` -> ``[B,N]``.
     """

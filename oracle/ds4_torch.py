@@ -3,7 +3,7 @@ the benchmark.
 
 TEST INFRASTRUCTURE ONLY, like the rest of this package: the benchmark's `cpu_baseline` times it on the host's
 cores and tests/test_oracle_ds4.py pins it against the NumPy oracle (`oracle.ds4`: `indexer_scores_fp8`,
-`radix_select_topk`, `sparse_mla_decode`). It states the same three steps as BASELINE configs 4 and 5 chained
+`radix_select_topk`, `sparse_mla_decode`). It states the three steps of the sparse decode layer
 
     score[r] = sum_h w[h] * relu(q_idx[h] . e4m3(codes[r])) * key_scale[r]        (lightning indexer, fp8 keys)
     sel      = the top-k rows by score, ties to the lower row, in ascending row order

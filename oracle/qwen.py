@@ -77,7 +77,7 @@ def affine_q8_dequantize(packed: np.ndarray, scales: np.ndarray, biases: np.ndar
 
 
 def q8_0_quantize(x: np.ndarray, block: int = 32):
-    """Symmetric int8 blocks with one float16 scale (BASELINE config 3 format).
+    """Symmetric int8 blocks with one float16 scale (the Q8_0 format).
 
     ``d = amax/127`` (float32), ``code = clip(round(x/d), -127, 127)``, scale
     stored as float16. Returns ``(int8 [..., D], float16 [..., D/block])``.
@@ -108,8 +108,7 @@ def gqa_decode_attention(q: np.ndarray, k: np.ndarray, v: np.ndarray, scale: flo
     """One-token GQA attention, float64.
 
     q ``[B,Hq,1,D]``, k/v ``[B,Hkv,N,D]`` -> ``[B,Hq,1,D]``; head ``h`` reads KV
-    head ``h // (Hq/Hkv)`` (full_attention.py:323-335 call site; BASELINE
-    configs 1 and 3).
+    head ``h // (Hq/Hkv)`` (full_attention.py:323-335 call site).
     """
     q = np.asarray(q, dtype=np.float64)
     k = np.asarray(k, dtype=np.float64)
@@ -134,7 +133,7 @@ def causal_prefill_attention(q: np.ndarray, k: np.ndarray, v: np.ndarray, scale:
     """Causal GQA prefill with a ``past``-token prefix, float64.
 
     q ``[1,Hq,Tq,D]``; k/v ``[1,Hkv,past+Tq,D]``: query ``t`` sees keys
-    ``[0, past+t]`` (full_attention.py:372-382 call site; BASELINE config 2).
+    ``[0, past+t]`` (full_attention.py:372-382 call site).
     """
     q = np.asarray(q, dtype=np.float64)
     k = np.asarray(k, dtype=np.float64)

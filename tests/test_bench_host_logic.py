@@ -56,7 +56,7 @@ def test_committed_summaries_if_current_agree_with_the_algorithmic_bytes():
 
 
 def test_algorithmic_bytes_follow_the_configuration():
-    # config 5: 2176 rows x 1152 B + q + out + ids; config 4: fp8 keys + scales + q, w + ids
+    # attention: 2176 rows x 1152 B + q + out + ids; indexer: fp8 keys + scales + q, w + ids
     assert bench.MLA_BYTES_PER_SEQ == 2176 * 1152 + 64 * 576 * 2 + 64 * 512 * 2 + 2048 * 4 == 2654208
     assert bench.IDX_BYTES_PER_SEQ == 32768 * 128 + 32768 * 4 + 64 * 128 * 2 + 64 * 4 + 2048 * 4
 

@@ -58,7 +58,7 @@ def test_flash_prefill_matches_oracle(B, Hq, Hkv, L, past, dtype, extra):
 
 
 def test_flash_prefill_full_size_sampled_rows():
-    """BASELINE config 2 at full size (4096 new tokens over a 32768-token prefix, 16 query / 2 KV heads):
+    """The served chunk at full size (4096 new tokens over a 32768-token prefix, 16 query / 2 KV heads):
     sampled query rows (block boundaries, first, last) against the oracle run on that one row, 2e-3."""
     from moespresso_amd.runtime.qwen import kquant
 

@@ -44,7 +44,7 @@ def _affine_cache(rng, B, Hkv, N, sb_dtype):
     (2, 8, 4, 1000, torch.float16),
     (1, 16, 2, 4099, torch.bfloat16),
     (1, 16, 2, 8192, torch.bfloat16),      # the depth from which the reference engages this operator
-    (1, 16, 2, 37000, torch.bfloat16),     # BASELINE config 3 depth, scales as served (bfloat16)
+    (1, 16, 2, 37000, torch.bfloat16),     # the served depth, scales as served (bfloat16)
     (1, 4, 4, 300, torch.float32),
     (1, 32, 2, 129, torch.float32),
 ])
@@ -72,7 +72,7 @@ def test_sdpa_decode_q8_affine(B, Hq, Hkv, N, sb_dtype):
     (5, 9000, torch.float16),
 ])
 def test_sdpa_decode_q8_0(B, N, qdt):
-    """int8 codes + one float16 scale per 32, bf16 queries, batch 1 and 8."""
+    """The served cache: int8 codes + one float16 scale per 32, bf16 queries, batch 1 and 8."""
     from moespresso_amd.runtime.qwen import kquant
 
     Hq, Hkv = 16, 2

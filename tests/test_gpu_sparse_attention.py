@@ -150,7 +150,7 @@ def test_sparse_mla_decode_matches_oracle(cfg):
 
 
 def test_sparse_mla_decode_full_config_batch16_with_sinks():
-    # 64 heads, 576/512, bf16, 131072-token cache, 2048 gathered + 128 window
+    # as served: 64 heads, 576/512, bf16, 131072-token cache, 2048 gathered + 128 window
     B, H, DK, N, R, W = 16, 64, 576, 131072, 2048, 128
     gen = torch.Generator(device=dev()).manual_seed(0)
     kv = torch.randn((B, N, DK), device=dev(), generator=gen, dtype=torch.float32).to(torch.bfloat16)
@@ -197,7 +197,7 @@ def _mla_oracle(q, kv, ids, snk, W):
 
 
 def test_sparse_mla_decode_full_config_batch4():
-    # BASELINE config 5, batch 4 leg at full size (32 key ranges per sequence)
+    # the same at batch 4, full size (32 key ranges per sequence)
     q, kv, ids, snk = _mla_case(4, 64, 576, 131072, 2048, 128, seed=4)
     got = iak.sparse_mla_decode(q, kv, to_dev(ids), scale=576 ** -0.5, window_start=131072 - 128, window_rows=128,
                                 row_mul=4, row_add=3)
