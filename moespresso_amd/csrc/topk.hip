@@ -888,7 +888,7 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   __shared__ __attribute__((aligned(16))) uint32_t near[64];
   __shared__ uint32_t kth[2];
   __shared__ Pick pick_box;
-  __shared__ uint32_t n_list, n_near;
+  __shared__ uint32_t n_list[2], n_near;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -910,7 +910,8 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   bits_above[tid] = 0u;
   bits_tie[tid] = 0u;
   if (tid == 0) {
-    n_list = 0u;
+    n_list[0] = 0u;
+    n_list[1] = 0u;
     n_near = 0u;
   }
 #pragma unroll
@@ -973,19 +974,18 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     pivot = __builtin_amdgcn_readfirstlane((int)(((sum >> 4) << 16) ^ 0x80000000u));
     span_end = __builtin_amdgcn_readfirstlane((int)(top ^ 0x80000000u));
   }
-  const bool mapped = pivot <= 0;  // uniform
-  if (mapped) {
-#pragma unroll
-    for (int j = 0; j < P; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
-  }
-
   auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
-  // ---- rows at or above the pivot (one at or below -inf would list the rows a token does not see as well: those are counted
-  //      below, not binned)
-  uint32_t total = 0u;
-  if (pivot > kNegInfSigned) {  // uniform
+
+  // ---- rows at or above the pivot
+  bool mapped = false;
+  auto listed = [&](uint32_t* counter) -> uint32_t {
+    if (!mapped && pivot <= 0) {  // uniform
+      mapped = true;
+#pragma unroll
+      for (int j = 0; j < P; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) key[j][e] = signed_key(key[j][e]);
+    }
     uint32_t mask = 0u;
 #pragma unroll
     for (int j = P - 1; j >= 0; j--)
@@ -994,7 +994,7 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     const uint32_t cnt = (uint32_t)__popc(mask);
     const uint32_t incl = wave_prefix_sum(cnt);
     uint32_t base = 0u;
-    if (lane == 63) base = atomicAdd(&n_list, incl);
+    if (lane == 63) base = atomicAdd(counter, incl);
     base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63);
     if (base + (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) <= (uint32_t)kCap) {
       uint16_t* at = list + base + incl - cnt;
@@ -1005,7 +1005,17 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
       }
     }
     __syncthreads();
-    total = uniform(n_list);
+    return uniform(*counter);
+  };
+  // (One at or below -inf would list the rows a token does not see as well: those are counted below, not binned. Where the
+  // waves' parts of the row differ, the mean of their pivots may lie above the k-th key: the lowest of them is taken then.)
+  uint32_t total = 0u;
+  if (pivot > kNegInfSigned) {  // uniform
+    total = listed(&n_list[0]);
+    if (__builtin_expect(total < (uint32_t)topk && !masked, 0)) {
+      pivot = (int32_t)((uniform(~wave_max(~wave_pivot[lane % kW])) << 16) ^ 0x80000000u);
+      total = listed(&n_list[1]);
+    }
   }
   const bool fits = total >= (uint32_t)topk && total <= (uint32_t)kCap;  // uniform
 
@@ -1152,18 +1162,21 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
         f(k, 4u * (uint32_t)(j * THREADS + tid));
       }
     };
+    limit = umin(limit, 0x7FFFFFFFu - (uint32_t)lo);
     if (!fits) {
-      // Those of -inf are counted and not binned: rows a token does not see yet are most of a row at the start of a prompt,
-      // and the k-th key is -inf where fewer are seen than are wanted.
-      uint32_t not_low = 0u, top = 0u, counts = 0u;  // lowest finite key, highest key, finite keys and those of -inf
+      // The bins are those of the keys above -inf, or at the pivot and above where the list overflowed. Those of -inf are counted:
+      // rows a token does not see yet are most of a row at the start of a prompt, and the k-th key is -inf where fewer are seen
+      // than are wanted.
+      const int32_t low = total > (uint32_t)kCap ? pivot : kNegInfSigned + 1;
+      uint32_t not_low = 0u, top = 0u, counts = 0u;  // lowest of them, highest key, how many and how many of -inf
       each([&](i32x4_t k, uint32_t) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const uint32_t u = (uint32_t)k[e] ^ 0x80000000u;
-          const bool fin = k[e] > kNegInfSigned;
+          const bool in = k[e] >= low;
           top = umax(top, u);
-          not_low = umax(not_low, fin ? ~u : 0u);
-          counts += fin ? 1u : k[e] == kNegInfSigned ? 1u << 16 : 0u;
+          not_low = umax(not_low, in ? ~u : 0u);
+          counts += in ? 1u : k[e] == kNegInfSigned ? 1u << 16 : 0u;
         }
       });
       top = wave_max(top);
@@ -1179,9 +1192,9 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
       lo = (int32_t)(uniform(~wave_max(wave_pivot[lane % kW])) ^ 0x80000000u);
       int32_t end = (int32_t)(uniform(wave_max(wave_high[lane % kW])) ^ 0x80000000u);
       counts = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(lane < kW ? wave_tot[lane % kW] : 0u), 63);
-      const uint32_t n_fin = counts & 0xFFFFu, n_inf = counts >> 16;
-      if (need > n_fin) {  // -inf, or one of the negative NaNs below it
-        need -= n_fin;
+      const uint32_t n_in = counts & 0xFFFFu, n_inf = counts >> 16;
+      if (need > n_in) {  // -inf, or one of the negative NaNs below it
+        need -= n_in;
         lo = end = kNegInfSigned;
         if (need > n_inf) {
           need -= n_inf;
@@ -1203,8 +1216,8 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const uint32_t d = (uint32_t)k[e] - (uint32_t)lo;
-          if (k[e] >= lo && d <= limit)
-            atomicAdd(&counters[umin(d >> shift, kBins - 1u) * kVoteCopies + (uint32_t)(lane % kVoteCopies)], 1u);
+          if (d <= limit)  // (keys below lo are further off than any above it)
+            atomicAdd(&counters[(d >> shift) * kVoteCopies + (uint32_t)(lane % kVoteCopies)], 1u);
         }
       });
       __syncthreads();

@@ -107,3 +107,44 @@ def test_crowded_rows_take_no_longer_than_passes_over_them(rows, n, k):
         assert best_us(lambda: isk.topk_select(part, k), 20) < 3 * usual, seen
     full.fill_(0.25)
     assert best_us(lambda: isk.topk_select(full, k), 20) < 3 * usual
+
+
+def uneven(n, k, rng):
+    """Rows whose scores change along them, so that the parts which the waves sample say different things."""
+    s = np.abs(rng.standard_normal((7, n))).astype(np.float32) * 3 + 20
+    few = min(max(int(k * 0.97), 1), n)
+    s[0, :few] += 1000                                   # nearly all of the wanted ones at the row's start,
+    s[1, n - few:] *= 1.6                                # at its end,
+    s[2, n // 2:n // 2 + few] -= 40                      # and the same below zero in its middle
+    s[2] = -s[2]
+    s[3] += np.linspace(0, 60, n, dtype=np.float32)
+    s[4, n // 2:] *= 1e-3
+    s[5, :few] = np.float32(3e38)
+    s[5, few:] *= -1                                     # the k-th key negative, the listed ones not
+    s[6, few:] = np.float32(1.5)                         # and one value in the rest
+    return s
+
+
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("n,k", [(2049, 1), (2051, 768), (3072, 512), (4096, 512), (4097, 512), (5121, 2000), (6145, 3000),
+                                 (8192, 2048), (8193, 512), (12289, 1024), (20481, 4000), (28673, 2048), (32768, 2048)])
+def test_uneven_rows(n, k, many):
+    s = uneven(n, k, np.random.default_rng(n * 5 + k))
+    data = torch.from_numpy(s).cuda()
+    if many:
+        data = data.repeat(56, 1)                        # 392 rows
+    got = isk.topk_select(data, k).cpu().numpy()
+    for b in range(7):
+        want = ds4.radix_select_topk(s[b], k)
+        np.testing.assert_array_equal(got[b], want)
+        np.testing.assert_array_equal(got[-7 + b], want)
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 32768, 2048), (16, 16384, 1024), (387, 8192, 512), (3844, 8192, 512)])
+def test_uneven_rows_take_no_longer_than_passes_over_them(rows, n, k):
+    """Three times a row whose parts are alike, as above (1.2 to 1.9 times on the shapes below; 3.4 to 5 times where a first pivot
+    above the k-th key meant all keys in one histogram)."""
+    s = torch.randn((rows, n), device="cuda").abs() * 3 + 20
+    usual = best_us(lambda: isk.topk_select(s, k), 20)
+    s[:, :int(k * 0.97)] += 1000
+    assert best_us(lambda: isk.topk_select(s, k), 20) < 3 * usual
