@@ -848,16 +848,20 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
 // with a pivot that lies below the k-th key nearly always, and the rest is done on the keys at or above it.
 //  * Every wave takes 64 S keys spread over the row and finds the 16-bit prefix of the `rank`-th of them with ballots; the
 //    mean of the waves' prefixes is the pivot. One barrier, no histogram.
-//  * The rows at or above it go to a list in LDS, in any order; their keys are read from a copy of the row in LDS.
+//  * The rows at or above it go to a list in LDS, in any order; their keys are read from a copy of the row in LDS. Where they are
+//    fewer than k, the list is made again from the lowest of the waves' prefixes: a wave samples stretches of the row, and of
+//    a row whose scores change along it the mean may say nothing (97 % of the wanted scores in one stretch: 1 row of 32768, k =
+//    2048, 42 us through the binning of all keys, now 13.7; 3844 of 8192, k = 512, 144 and 45). Where all parts are alike it is
+//    one row in some hundreds, which the launch then waits for: 3844 rows of 7961 Gaussian scores 33.5 us, now 29.
 //  * 256 bins over [pivot, highest sample] hold the k-th key; a bin of up to 64 keys (nearly always the first one) is ranked
 //    directly, otherwise it becomes the span.
 //  * Selected rows set their bit in a bitmap of the row. Bits come out in row order, so nothing before has to keep it.
 // Keys are compared as signed integers: the bits of a float32 themselves where the pivot is positive, all others after the
 // map that inverts the low bits of negative values. Whether the list contains the k-th key is checked exactly; if it does not
 // (or does not fit, or a second round of bins hardly splits it), the binning runs over all keys, so the result never depends
-// on the sample. There -inf is counted on the side and the span is that of the finite keys, and votes go to copies of the
+// on the sample. There -inf is counted on the side, the span is that of the keys in question, and votes go to copies of the
 // counters: in one histogram the votes of a row that is mostly -inf, or of one value, follow each other on one counter in
-// every pass (1 row of 32768, k = 2048, with 400 finite 125 us, now 13; 3844 rows of 8192, k = 512, 100 finite 484, now 44; a
+// every pass (1 row of 32768, k = 2048, 400 finite: 125 us, now 13; 3844 rows of 8192, k = 512, 100 finite: 484, now 44; a
 // chunk of 8400 tokens from position 0, whose first quarter sees too few rows: scores selected in 100, now 37).
 // What bounds it: a CU takes 2000 cycles to fetch a row of 32768 scores, and an instruction per key is 500 cycles of its vector
 // units: the blocked kernel above maps and moves every key (two LDS passes) and takes five digit passes, 16 rows of 32768,
