@@ -23,11 +23,12 @@
 //    the four waves drift apart and one wave's sums run under another's products.
 //    3844 tokens x 7961 rows from position 28000: 24 us packing + 157 us (float16 form 633), vector units busy three
 //    quarters of it; x 961 rows from position 0: 24 + 21 us (75); 517 tokens x 2053 rows: 7 + 14 us (46).
-//  * Where a value is outside that lattice (a pool row, or a query of the workgroup's tokens) the float16 form does the
-//    work, with pool tiles staged in LDS. It is a launch of its own behind the first, whose workgroups leave at once where
-//    nothing is left to do: in one kernel the two forms' registers held it to two waves per SIMD. What the first launch costs
-//    such operands: 3844 float32 tokens x 961 rows 68 us in the float16 form alone, 78 with it (97 when every row was
-//    packed before a block was found not exact); x 7961 rows 557 and 574 (602); 517 x 2053 rows 45 and 54 (58).
+//  * Where a value is outside that lattice (a pool row, or a query of the workgroup's tokens) the same workgroup goes through
+//    its rows in the float16 form, with pool tiles staged in LDS. (Three waves fit a SIMD with both forms in the kernel since
+//    queries are rounded 32 heads at a time as they arrive; before, the float16 form was a launch of its own, 2 to 3 us of
+//    every call: 517 x 2053 rows 22.0 -> 19.4, 255 x 1988 14.5 -> 12.1.) What the look at them costs operands that are not of
+//    the format: 3844 float32 tokens x 961 rows 65 us in the float16 form alone, 74 with it; x 7961 rows 549 and 558; 517 x
+//    2053 rows 45 and 48.
 #include "common.h"
 #include "profile.h"
 
@@ -274,11 +275,113 @@ struct ScoreJob {
   }
 };
 
-// fp4 form. grid: (row blocks, token blocks, batch); a wave walks its rows in pairs of tiles, one packed block at a time.
+// A workgroup = 4 waves = 4 consecutive tokens walks `rows_per_block` pool rows (a multiple of 64) in tiles of 32. Float16
+// form:
+// A tile is fetched once per workgroup (every thread 32 bytes of it, rounded to float16) into one of two LDS buffers,
+// a tile ahead of its use, and the four waves read their B operands from there: fetched by each wave for itself, the
+// 16-byte pieces of 32 rows keep a CU's address path busier than its matrix pipes. Rows past a token's visible
+// prefix score -inf whatever the products are, so a wave multiplies only the tiles that hold a row it sees.
+constexpr int kTilePitch = 272;  // bytes between rows of a tile in LDS: 256 + 16, operand reads of 32 rows x 2 pieces
+                                 // and the 16-byte writes of two rows at a time both without bank conflicts
+
+template <int DT>
+__device__ __forceinline__ void scores_f16(const ScoreJob& j, const void* __restrict__ q, const float* __restrict__ w,
+                                           const void* __restrict__ comp, int n_heads, int n_tokens, int64_t n_comp,
+                                           unsigned char (&tile_lds)[2][32 * kTilePitch]) {
+  const int tid = threadIdx.x, n = j.n, g = j.g, b = j.b, t = j.t;
+  const int n_live = j.n_live, n_fetch = j.n_fetch;
+  const int64_t row_begin = j.row_begin;
+
+  if (n_fetch > 0) {  // (the same in every wave of the workgroup: the barriers below are met by all)
+    const void* comp_b =
+        DT == MSPR_F16 ? static_cast<const void*>(reinterpret_cast<const uint16_t*>(comp) + (int64_t)b * n_comp * 128)
+                       : static_cast<const void*>(reinterpret_cast<const float*>(comp) + (int64_t)b * n_comp * 128);
+    // this thread's share of a tile: row tid / 8, columns [16 (tid % 8), +16)
+    const int f_row = tid >> 3, f_col = (tid & 7) * 16;
+    auto fetch = [&](int64_t r0, u32x4_t (&st)[2]) {
+      int64_t row = r0 + f_row;
+      if (row >= n_comp) row = n_comp - 1;
+      st[0] = load8_as_f16<DT>(comp_b, row * 128 + f_col);
+      st[1] = load8_as_f16<DT>(comp_b, row * 128 + f_col + 8);
+    };
+    auto stash = [&](int buf, const u32x4_t (&st)[2]) {
+      unsigned char* p = tile_lds[buf] + f_row * kTilePitch + f_col * 2;
+      *reinterpret_cast<u32x4_t*>(p) = st[0];
+      *reinterpret_cast<u32x4_t*>(p + 16) = st[1];
+    };
+    u32x4_t st[2];
+    fetch(row_begin, st);  // (in flight while the query block and the weights arrive)
+
+    // A operand: q[b, head, t, 16 s + 8 g .. +7] for head = n (+32), zero rows past n_heads
+    u32x4_t qa[2][8];
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++) {
+      const int head = 32 * hb + n;
+      const bool live = head < n_heads;
+      const int64_t off = (((int64_t)b * n_heads + (live ? head : 0)) * n_tokens + t) * 128 + 8 * g;
+#pragma unroll
+      for (int s = 0; s < 8; s++) {
+        u32x4_t v = load8_as_f16<DT>(q, off + 16 * s);
+        qa[hb][s] = live ? v : u32x4_t{0, 0, 0, 0};
+      }
+      // (rounded here: the rest of the block does not fit the registers in float32)
+#pragma unroll
+      for (int s = 0; s < 8; s++) asm volatile("" : "+v"(qa[hb][s]));
+    }
+    float wv[2][16];
+    j.head_weights(w, n_tokens, n_heads, wv);
+    stash(0, st);
+    __syncthreads();
+
+    for (int i = 0; i < n_fetch; i++) {
+      if (i + 1 < n_fetch) fetch(row_begin + 32 * (int64_t)(i + 1), st);
+      if (i < n_live) {
+        // B operand: lane (n, g) holds comp[row r0 + n][16 s + 8 g .. +7] for k-step s
+        const unsigned char* kt = tile_lds[i & 1] + n * kTilePitch + 16 * g;
+        f32x16_t acc0 = {0}, acc1 = {0};
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+          const u32x4_t kb = *reinterpret_cast<const u32x4_t*>(kt + 32 * s);
+          acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, qa[0][s]),
+                                                        __builtin_bit_cast(f16x8_t, kb), acc0, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, qa[1][s]),
+                                                        __builtin_bit_cast(f16x8_t, kb), acc1, 0, 0, 0);
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+          sum += fmaxf(acc0[k], 0.0f) * wv[0][k];
+          sum += fmaxf(acc1[k], 0.0f) * wv[1][k];
+        }
+        sum += __shfl_xor(sum, 32, MSPR_WAVE);
+        const int64_t c = row_begin + 32 * (int64_t)i + n;
+        if (j.t_live && g == 0 && c < j.row_end) j.out_row[c] = c < j.visible ? sum : -__builtin_inff();
+      }
+      if (i + 1 < n_fetch) stash((i + 1) & 1, st);
+      __syncthreads();  // tile i+1 written by every thread; tile i read by every wave
+    }
+  }
+  j.mask_rest(n_live);
+}
+
+template <int DT>
+__global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __restrict__ q, const float* __restrict__ w,
+                                                           const void* __restrict__ comp, int n_heads, int n_tokens,
+                                                           int64_t n_comp, uint32_t pos0, uint32_t ratio,
+                                                           int rows_per_block, float* __restrict__ scores) {
+  __shared__ __attribute__((aligned(16))) unsigned char tile_lds[2][32 * kTilePitch];
+  scores_f16<DT>(ScoreJob(n_tokens, n_comp, pos0, ratio, rows_per_block, scores), q, w, comp, n_heads, n_tokens, n_comp,
+                 tile_lds);
+}
+
+// fp4 form, or the float16 form where the operands are not of the format. grid: (row blocks, token blocks, batch); a wave
+// walks its rows in pairs of tiles, one packed block at a time.
 __global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restrict__ w, int n_heads, int n_tokens,
                                                             int64_t n_comp, uint32_t pos0, uint32_t ratio,
-                                                            int rows_per_block, PackedOperands ops,
-                                                            float* __restrict__ scores) {
+                                                            int rows_per_block, float* __restrict__ scores,
+                                                            PackedOperands ops, const void* __restrict__ q,
+                                                            const void* __restrict__ comp, int dtype) {
+  __shared__ __attribute__((aligned(16))) unsigned char tile_lds[2][32 * kTilePitch];
   const ScoreJob j(n_tokens, n_comp, pos0, ratio, rows_per_block, scores);
   if (j.n_fetch == 0) {  // no row of the block is visible to any of the four tokens, whatever the operands are
     j.mask_rest(0);
@@ -312,7 +415,11 @@ __global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restr
   const uint32_t qs = reinterpret_cast<const uint32_t*>(ops.q_scales + token * kBlockScaleBytes)[j.lane];
   float wv[2][16];
   j.head_weights(w, n_tokens, n_heads, wv);
-  if (!exact.all()) return;
+  if (!exact.all()) {
+    if (dtype == MSPR_F16) scores_f16<MSPR_F16>(j, q, w, comp, n_heads, n_tokens, n_comp, tile_lds);
+    else scores_f16<MSPR_F32>(j, q, w, comp, n_heads, n_tokens, n_comp, tile_lds);
+    return;
+  }
 
   float* out = j.out_row + j.row_begin + j.lane;
   int left = (int)(j.row_end - j.row_begin) - j.lane, seen = (int)(j.visible - j.row_begin) - j.lane;
@@ -359,97 +466,6 @@ __global__ __launch_bounds__(256, 3) void scores_fp4_kernel(const float* __restr
   j.mask_rest(2 * n_pairs);
 }
 
-// A workgroup = 4 waves = 4 consecutive tokens walks `rows_per_block` pool rows (a multiple of 64) in tiles of 32. Float16
-// form:
-// A tile is fetched once per workgroup (every thread 32 bytes of it, rounded to float16) into one of two LDS buffers,
-// a tile ahead of its use, and the four waves read their B operands from there: fetched by each wave for itself, the
-// 16-byte pieces of 32 rows keep a CU's address path busier than its matrix pipes. Rows past a token's visible
-// prefix score -inf whatever the products are, so a wave multiplies only the tiles that hold a row it sees.
-constexpr int kTilePitch = 272;  // bytes between rows of a tile in LDS: 256 + 16, operand reads of 32 rows x 2 pieces
-                                 // and the 16-byte writes of two rows at a time both without bank conflicts
-
-template <int DT>
-__global__ __launch_bounds__(256, 2) void scores_tiled_kernel(const void* __restrict__ q, const float* __restrict__ w,
-                                                           const void* __restrict__ comp, int n_heads, int n_tokens,
-                                                           int64_t n_comp, uint32_t pos0, uint32_t ratio,
-                                                           int rows_per_block, PackedOperands packed,
-                                                           float* __restrict__ scores) {
-  __shared__ __attribute__((aligned(16))) unsigned char tile_lds[2][32 * kTilePitch];
-  if (packed.pool_codes && OperandsExact(packed, n_tokens, n_comp).all()) return;  // the fp4 form has done the work
-  const ScoreJob j(n_tokens, n_comp, pos0, ratio, rows_per_block, scores);
-  const int tid = threadIdx.x, n = j.n, g = j.g, b = j.b, t = j.t;
-  const int n_live = j.n_live, n_fetch = j.n_fetch;
-  const int64_t row_begin = j.row_begin;
-
-  if (n_fetch > 0) {  // (the same in every wave of the workgroup: the barriers below are met by all)
-    const void* comp_b =
-        DT == MSPR_F16 ? static_cast<const void*>(reinterpret_cast<const uint16_t*>(comp) + (int64_t)b * n_comp * 128)
-                       : static_cast<const void*>(reinterpret_cast<const float*>(comp) + (int64_t)b * n_comp * 128);
-    // this thread's share of a tile: row tid / 8, columns [16 (tid % 8), +16)
-    const int f_row = tid >> 3, f_col = (tid & 7) * 16;
-    auto fetch = [&](int64_t r0, u32x4_t (&st)[2]) {
-      int64_t row = r0 + f_row;
-      if (row >= n_comp) row = n_comp - 1;
-      st[0] = load8_as_f16<DT>(comp_b, row * 128 + f_col);
-      st[1] = load8_as_f16<DT>(comp_b, row * 128 + f_col + 8);
-    };
-    auto stash = [&](int buf, const u32x4_t (&st)[2]) {
-      unsigned char* p = tile_lds[buf] + f_row * kTilePitch + f_col * 2;
-      *reinterpret_cast<u32x4_t*>(p) = st[0];
-      *reinterpret_cast<u32x4_t*>(p + 16) = st[1];
-    };
-    u32x4_t st[2];
-    fetch(row_begin, st);  // (in flight while the query block and the weights arrive)
-
-    // A operand: q[b, head, t, 16 s + 8 g .. +7] for head = n (+32), zero rows past n_heads
-    u32x4_t qa[2][8];
-#pragma unroll
-    for (int hb = 0; hb < 2; hb++) {
-      const int head = 32 * hb + n;
-      const bool live = head < n_heads;
-      const int64_t off = (((int64_t)b * n_heads + (live ? head : 0)) * n_tokens + t) * 128 + 8 * g;
-#pragma unroll
-      for (int s = 0; s < 8; s++) {
-        u32x4_t v = load8_as_f16<DT>(q, off + 16 * s);
-        qa[hb][s] = live ? v : u32x4_t{0, 0, 0, 0};
-      }
-    }
-    float wv[2][16];
-    j.head_weights(w, n_tokens, n_heads, wv);
-    stash(0, st);
-    __syncthreads();
-
-    for (int i = 0; i < n_fetch; i++) {
-      if (i + 1 < n_fetch) fetch(row_begin + 32 * (int64_t)(i + 1), st);
-      if (i < n_live) {
-        // B operand: lane (n, g) holds comp[row r0 + n][16 s + 8 g .. +7] for k-step s
-        const unsigned char* kt = tile_lds[i & 1] + n * kTilePitch + 16 * g;
-        f32x16_t acc0 = {0}, acc1 = {0};
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-          const u32x4_t kb = *reinterpret_cast<const u32x4_t*>(kt + 32 * s);
-          acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, qa[0][s]),
-                                                        __builtin_bit_cast(f16x8_t, kb), acc0, 0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, qa[1][s]),
-                                                        __builtin_bit_cast(f16x8_t, kb), acc1, 0, 0, 0);
-        }
-        float sum = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-          sum += fmaxf(acc0[k], 0.0f) * wv[0][k];
-          sum += fmaxf(acc1[k], 0.0f) * wv[1][k];
-        }
-        sum += __shfl_xor(sum, 32, MSPR_WAVE);
-        const int64_t c = row_begin + 32 * (int64_t)i + n;
-        if (j.t_live && g == 0 && c < j.row_end) j.out_row[c] = c < j.visible ? sum : -__builtin_inff();
-      }
-      if (i + 1 < n_fetch) stash((i + 1) & 1, st);
-      __syncthreads();  // tile i+1 written by every thread; tile i read by every wave
-    }
-  }
-  j.mask_rest(n_live);
-}
-
 }  // namespace
 
 extern "C" size_t mspr_indexer_scores_tiled_live_workspace_bytes(int batch, int n_heads, int n_tokens, int64_t n_comp) {
@@ -487,10 +503,11 @@ extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* wei
   hipStream_t st = (hipStream_t)stream;
   dim3 block(256);
   PackedOperands packed = {};
-  // The fp4 form is two launches more, some 5 us, which cheaper products have to earn. It does so from 2^17 scores on with
-  // float32 operands, which the float16 form rounds as it loads them (us without and with it: 64 tokens x 2000 rows 12.1 and
-  // 12.9, 128 x 1000 12.4 and 13.0, 96 x 2000 17.5 and 13.6, 17 x 8000 16.7 and 14.1, 517 x 500 22.6 and 15.1), and from 450
-  // thousand with float16 ones (384 x 1000 14.2 and 14.8, 128 x 4000 15.1 and 15.1, 517 x 1000 19.0 and 17.5).
+  // The fp4 form is a launch more, some 3 us, which cheaper products have to earn. It does so from 2^17 scores on with
+  // float32 operands, which the float16 form rounds as it loads them (us without and with it: 32 tokens x 2000 rows 7.4 and
+  // 10.5, 64 x 2000 12.0 and 10.6, 96 x 2000 16.2 and 9.3, 17 x 8000 16.7 and 11.5, 517 x 500 22.6 and 12), and from 450
+  // thousand with float16 ones (128 x 2000 9.9 and 11.6, 400 x 1000 17.9 and 12.9). Both lines lie a little high for operands
+  // of the format; what is not of it pays for being looked at and is left alone below them.
   if (workspace && (int64_t)batch * n_tokens * n_comp >= (dtype == MSPR_F32 ? 1 << 17 : 450000)) {
     packed = packed_operands(workspace, batch, n_tokens, n_comp);
     const int64_t blocks = pool_blocks(n_comp) + n_tokens;
@@ -502,28 +519,35 @@ extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* wei
     else
       pack_operands_kernel<MSPR_F32><<<pgrid, block, 0, st>>>(q, index_comp, n_heads, n_tokens, n_comp, packed);
     // A workgroup's start (operands, flags: some 3 us) has to be carried by its tiles: at least 16 pairs of them, or 8 where
-    // the chip is not full otherwise. Three rounds of workgroups level the last one: 3844 tokens x 7961 rows took 164, 160,
-    // 157, 168 us with 1, 2, 3, 4 row blocks, x 961 rows from position 0 took 21, 25, 31 us with 1, 2, 4; 517 tokens x
-    // 2053 rows 15.5 us with 2 and 13.7 us with 4.
+    // the chip is not full otherwise, or 4 where there are not two workgroups to a CU even so. Three rounds of workgroups level
+    // the last one: 3844 tokens x 7961 rows took 164, 160, 157, 168 us with 1, 2, 3, 4 row blocks, x 961 rows from position 0
+    // took 21, 25, 31 us with 1, 2, 4; 517 tokens x 2053 rows 15.5 us with 2 and 13.7 us with 4. At least 8 and 4 pairs, whole
+    // calls: 96 x 2000 10.9 and 9.3 (random operands 23.7 and 16.9), 64 x 4000 11.4 and 9.7, 300 x 600 12.2 and 10.3, 517 x
+    // 1000 14.8 and 14.4, 1000 x 500 14.8 and 15.1, 517 x 2053 19.4 and 20.2.
     int64_t rows = rows_per_workgroup(2304, 16);
-    if ((n_comp + rows - 1) / rows * tok_blocks * batch < 768) rows = rows_per_workgroup(768, 8);
+    auto workgroups = [&]() -> int64_t { return (n_comp + rows - 1) / rows * tok_blocks * batch; };
+    if (workgroups() < 768) rows = rows_per_workgroup(768, 8);
+    if (workgroups() < 512) rows = rows_per_workgroup(768, 4);
     dim3 grid((unsigned)((n_comp + rows - 1) / rows), (unsigned)tok_blocks, (unsigned)batch);
     scores_fp4_kernel<<<grid, block, 0, st>>>(weights, n_heads, n_tokens, n_comp, (uint32_t)pos0, (uint32_t)ratio,
-                                              (int)rows, packed, scores);
+                                              (int)rows, scores, packed, q, index_comp, dtype);
     MSPR_CHECK_LAUNCH("indexer_scores_tiled_live (fp4)");
+    return MSPR_OK;
   }
-  // float16 form: about three workgroups for each of the 256 CUs (every workgroup fetches its tokens' query blocks anew)
-  const int64_t rows = rows_per_workgroup(768, 1);
+  // float16 form: three rounds of workgroups where each has sixteen pairs of tiles, else about one (every workgroup fetches
+  // its tokens' query blocks anew). 3844 tokens x 7961 rows one round 619 us, three 559.
+  int64_t rows = rows_per_workgroup(2304, 16);
+  if ((n_comp + rows - 1) / rows * tok_blocks * batch < 768) rows = rows_per_workgroup(768, 1);
   const int64_t row_blocks = (n_comp + rows - 1) / rows;
   MSPR_REQUIRE(row_blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && rows < ((int64_t)1 << 31),
                "indexer_scores_tiled_live: grid too large");
   dim3 grid((unsigned)row_blocks, (unsigned)tok_blocks, (unsigned)batch);
   if (dtype == MSPR_F16)
     scores_tiled_kernel<MSPR_F16><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp, (uint32_t)pos0,
-                                                          (uint32_t)ratio, (int)rows, packed, scores);
+                                                          (uint32_t)ratio, (int)rows, scores);
   else
     scores_tiled_kernel<MSPR_F32><<<grid, block, 0, st>>>(q, weights, index_comp, n_heads, n_tokens, n_comp, (uint32_t)pos0,
-                                                          (uint32_t)ratio, (int)rows, packed, scores);
+                                                          (uint32_t)ratio, (int)rows, scores);
   MSPR_CHECK_LAUNCH("indexer_scores_tiled_live");
   return MSPR_OK;
 }
