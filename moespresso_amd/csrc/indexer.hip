@@ -426,11 +426,14 @@ static_assert(kScoreWaves == 8, "a byte of a word each");
 constexpr int kQPitch = 132;
 constexpr int kQBfPitch = 272;  // bytes; the same for the block as bf16
 
+// (Arguments in the order they are asked for: the first 14 words come in registers with the wave, and score workgroups need
+// no others. counted: *valid_rows holds the number of rows in use.)
 template <int DT, bool STAGE_HALF>
-__global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* __restrict__ q, int n_heads,
-                                                                   const float* __restrict__ pooled, int64_t n_rows,
-                                                                   const float* __restrict__ weights, float scale,
-                                                                   float* __restrict__ scores,
+__global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* __restrict__ q,
+                                                                   const float* __restrict__ pooled,
+                                                                   const float* __restrict__ weights,
+                                                                   float* __restrict__ scores, int64_t n_rows,
+                                                                   int n_heads, float scale, int score_blocks, int counted,
                                                                    const uint16_t* __restrict__ kv_row,
                                                                    const float* __restrict__ inv_freq,
                                                                    const int32_t* __restrict__ params,
@@ -438,12 +441,13 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
                                                                    const int32_t* __restrict__ valid_rows) {
   __shared__ float qbuf[64 * kQPitch];
   __shared__ float wbuf[64];
-  __shared__ float ptab[kPow2TabLen];
+  // (filled by all threads: what they fetch for it and for wbuf goes out with the queries; under a condition the fetch was made
+  // where the condition stands, behind the butterflies)
+  __shared__ float ptab[kScoreThreads];
   __shared__ __attribute__((aligned(8))) uint8_t plain_waves[8];
   const int tid = threadIdx.x;
   // With a KV row to prepare (the fused decode prep), the launch carries one more workgroup, the last one,
   // whose first wave does that small job next to the score workgroups instead of in a launch of its own.
-  const int score_blocks = (int)gridDim.x - (kv_row ? 1 : 0);
   if ((int)blockIdx.x == score_blocks) {
     kv_row_job(tid, qbuf, qbuf + 32, kv_row, inv_freq, params, row_out);
     return;
@@ -466,8 +470,10 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
   const int q_head = tid >> 3, q_part = tid & 7;
   Qat16 mine;
   load_row16<DT>(q, q_head < n_heads ? q_head : n_heads - 1, q_part, mine.x);
+  static_assert(kPow2TabLen <= kScoreThreads, "a table entry per thread");
   const float tab_a = g_pow2_tab[tid < kPow2TabLen ? tid : 0];
-  const float w_mine = weights[tid < n_heads ? tid : 0];
+  const int w_head = tid & 63;  // (the same from each wave)
+  const float w_mine = weights[w_head < n_heads ? w_head : 0];
   // The first pool tile of the wave is requested behind the butterflies and lands under the rest. Lane
   // (m = row, g) owns the 64 consecutive float32 values [64 g, 64 g + 64) of its pool row.
   float kv[64];
@@ -485,8 +491,8 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     }
   };
   qat16_rotate(mine, lane);
-  if (tid < kPow2TabLen) ptab[tid] = tab_a;
-  if (tid < 64) wbuf[tid] = tid < n_heads ? w_mine : 0.0f;
+  ptab[tid] = tab_a;
+  wbuf[w_head] = w_head < n_heads ? w_mine : 0.0f;
   if (tile < n_tiles) load_tile(tile);
   __syncthreads();
   const float q_scale = qat_scale(mine.amax, ptab);
@@ -636,7 +642,7 @@ __global__ __launch_bounds__(kScoreThreads) void scores_f32_kernel(const void* _
     sum = half_wave_sum(sum);
     // fixed-capacity form: the pool buffer holds n_rows rows of which the first *valid_rows are in use (a
     // count that lives on the device, so that a captured launch follows a growing pool); the rest score -inf
-    if (g == 0 && row < n_rows) scores[row] = (valid_rows && row >= (int64_t)valid_rows[0]) ? -__builtin_inff() : sum;
+    if (g == 0 && row < n_rows) scores[row] = (counted && row >= (int64_t)valid_rows[0]) ? -__builtin_inff() : sum;
   }
 }
 
@@ -684,15 +690,10 @@ int mspr_launch_scores_f32(const void* q, int q_dtype, int n_heads, const float*
   const uint16_t* kvp = reinterpret_cast<const uint16_t*>(kv_row);
   uint16_t* rop = reinterpret_cast<uint16_t*>(row_out);
   MsprProfScope prof(MSPR_K_SCORES_F32, st);
-#define MSPR_SCORES_LAUNCH(DT)                                                                          \
-  do {                                                                                                  \
-    if (stage_half)                                                                                     \
-      scores_f32_kernel<DT, true><<<grid, block, 0, st>>>(q, n_heads, pooled, n_rows, weights, scale, scores, kvp, \
-                                                          inv_freq, params, rop, valid_rows);            \
-    else                                                                                                \
-      scores_f32_kernel<DT, false><<<grid, block, 0, st>>>(q, n_heads, pooled, n_rows, weights, scale, scores, kvp, \
-                                                           inv_freq, params, rop, valid_rows);            \
-  } while (0)
+#define MSPR_SCORES_LAUNCH(DT)                                                                                            \
+  (stage_half ? &scores_f32_kernel<DT, true> : &scores_f32_kernel<DT, false>)<<<grid, block, 0, st>>>(                     \
+      q, pooled, weights, scores, n_rows, n_heads, scale, (int)blocks, valid_rows ? 1 : 0, kvp, inv_freq, params, rop,     \
+      valid_rows)
   if (q_dtype == MSPR_F32) MSPR_SCORES_LAUNCH(MSPR_F32);
   else if (q_dtype == MSPR_F16) MSPR_SCORES_LAUNCH(MSPR_F16);
   else MSPR_SCORES_LAUNCH(MSPR_BF16);

@@ -132,11 +132,14 @@ __global__ __launch_bounds__(256) void pack_operands_kernel(const void* __restri
   const int n_rows = left < kBlockRows ? (int)left : kBlockRows;
   const int col = (tid & 31) * 4;  // 32 lanes a row: eight rows per pass of the workgroup
   auto load = [&](int i) -> f32x4_t {
+    // (Past the block the last row again: under a condition a load is waited for before the next, 28.4 us and 26.9 for 3844
+    // tokens.)
     const int r = 8 * i + (tid >> 5);
-    return r < n_rows ? load4_as_f32<DT>(src, (row0 + r * row_step) * 128 + col) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    return load4_as_f32<DT>(src, (row0 + (r < n_rows ? r : n_rows - 1) * row_step) * 128 + col);
   };
-  auto pack = [&](int i, const f32x4_t& v) -> bool {
+  auto pack = [&](int i, f32x4_t v) -> bool {
     const int r = 8 * i + (tid >> 5);
+    if (r >= n_rows) v = f32x4_t{0.f, 0.f, 0.f, 0.f};
     uint32_t top = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {

@@ -394,9 +394,14 @@ __global__ __launch_bounds__(kThreads) void topk_blocked_kernel(const float* __r
       u32x4_t keys;
       if (vec_ok && r + 3 < n_rows) {
         keys = u32x4_t{score_key(v[k].x), score_key(v[k].y), score_key(v[k].z), score_key(v[k].w)};
-      } else {
+      } else if (r < n_rows) {
+        float t[4];  // (requested together)
 #pragma unroll
-        for (int e = 0; e < 4; e++) keys[e] = r + e < n_rows ? score_key(scores[r + e]) : 0u;
+        for (int e = 0; e < 4; e++) t[e] = scores[r + e < n_rows ? r + e : n_rows - 1];
+#pragma unroll
+        for (int e = 0; e < 4; e++) keys[e] = r + e < n_rows ? score_key(t[e]) : 0u;
+      } else {
+        keys = u32x4_t{0u, 0u, 0u, 0u};
       }
       const int owner = piece / kPieces, j = piece % kPieces;
       *reinterpret_cast<u32x4_t*>(&stage[owner * C + 4 * (j ^ (owner & (kPieces - 1)))]) = keys;
@@ -687,12 +692,17 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
   const float* scores = scores_all + (int64_t)blockIdx.x * score_stride;
   int32_t* sel = sel_all + (int64_t)blockIdx.x * topk;
 
-  uint32_t key[C];
+  // (All requested at once, past the end the last score again: under a condition each load is waited for before the next. One row
+  // of 961 scores 4.16 -> 3.56 us, 15 rows of 2015 5.9 -> 4.2, 3844 rows of 961 12.2 -> 11.3.)
+  float score[C];
 #pragma unroll
   for (int j = 0; j < C; j++) {
     const int e = j * THREADS + tid;
-    key[j] = e < n_rows ? score_key(scores[e]) : 0u;
+    score[j] = scores[e < n_rows ? e : n_rows - 1];
   }
+  uint32_t key[C];
+#pragma unroll
+  for (int j = 0; j < C; j++) key[j] = j * THREADS + tid < n_rows ? score_key(score[j]) : 0u;
 #pragma unroll
   for (int i = 0; i < (int)kRowBins / THREADS; i++) hist[i * THREADS + tid] = 0u;
   if (tid == 0) list_n = 0u;
