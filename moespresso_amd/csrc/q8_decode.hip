@@ -440,33 +440,34 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Arg
   float m_run = -__builtin_inff(), l = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = sg; s0 < a.n_splits; s0 += kMergeWaves * kChunk) {
-    float mv[kChunk], lv[kChunk];
+    // The statistics of range j by lane j, in one load, whose weight is then taken once: with scalar loads of them each range's
+    // were waited for in front of the next range's row, and every lane took all sixteen exponentials.
+    const int mine = s0 + kMergeWaves * (lane % kChunk);
+    f32x2_t stat = {-__builtin_inff(), 0.0f};
+    if (mine < a.n_splits) stat = *reinterpret_cast<const f32x2_t*>(ml + (int64_t)mine * 32);
     f32x4_t ov[kChunk];
 #pragma unroll
-    for (int j = 0; j < kChunk; j++) {
-      const int sj = s0 + kMergeWaves * j;  // wave-uniform: ranges past the end cost no load
-      mv[j] = -__builtin_inff();
-      lv[j] = 0.0f;
-      ov[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (sj < a.n_splits) {
-        mv[j] = ml[(int64_t)sj * 32];
-        lv[j] = ml[(int64_t)sj * 32 + 1];
-        ov[j] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)sj * (16 * kD));
-      }
-    }
-    float m_new = m_run;
-#pragma unroll
-    for (int j = 0; j < kChunk; j++) m_new = fmaxf(m_new, mv[j]);
+    for (int j = 0; j < kChunk; j++)  // (wave-uniform: ranges past the end cost no load)
+      if (s0 + kMergeWaves * j < a.n_splits)
+        ov[j] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)(s0 + kMergeWaves * j) * (16 * kD));
+    static_assert(kChunk == 16, "reduced over rows of sixteen lanes");
+    float m_new = stat.x;
+    m_new = fmaxf(m_new, lane_xor<1>(m_new));
+    m_new = fmaxf(m_new, lane_xor<2>(m_new));
+    m_new = fmaxf(m_new, lane_xor<4>(m_new));
+    m_new = fmaxf(m_run, fmaxf(m_new, lane_xor<8>(m_new)));
     const float m_safe = m_new == -__builtin_inff() ? 0.0f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);  // 0 while m_run is -inf
-    l *= alpha;
+    const float w = __builtin_amdgcn_exp2f(stat.x - m_safe);
+    float lw = stat.y * w;
+    lw += lane_xor<1>(lw);
+    lw += lane_xor<2>(lw);
+    lw += lane_xor<4>(lw);
+    l = l * alpha + (lw + lane_xor<8>(lw));
     o = o * alpha;
 #pragma unroll
-    for (int j = 0; j < kChunk; j++) {
-      const float w = __builtin_amdgcn_exp2f(mv[j] - m_safe);
-      l += lv[j] * w;
-      o += ov[j] * w;
-    }
+    for (int j = 0; j < kChunk; j++)
+      if (s0 + kMergeWaves * j < a.n_splits) o += ov[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
     m_run = m_new;
   }
   if (lane == 0) {
