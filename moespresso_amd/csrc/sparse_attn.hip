@@ -55,16 +55,17 @@ struct SparseAttnArgs {
   // prefill form: window range and visible pool prefix follow from the token's position pos0 + t
   int prefill;
   uint32_t pos0, window, ratio;
-  // window segment
+  // window segment (the split kernel reads win_first .. subst_slot, and check_stop .. scale_log2 below, with one load of four
+  // words each; a word of such a load that it had no use for would be given away, and its next owner wait for the load)
   const void* win;
   int64_t win_batch_stride;
   int n_win;
   int win_first;  // logical index of the first visited ring row
   int raw_start;
   int raw_cap;
-  const void* subst_row;
   int subst_slot;          // window slot replaced by subst_row (-1: none)
   int subst_from_params;   // take the slot from params[1] on the device instead
+  const void* subst_row;
   // gathered segment
   const void* pool;
   int64_t pool_batch_stride;
@@ -78,9 +79,9 @@ struct SparseAttnArgs {
   int row_mul;  // pool row = id * row_mul + row_add
   int row_add;
   // softmax
+  float scale_log2;
   const void* sinks;
   int sinks_dtype;
-  float scale_log2;
   // rope
   const float* inv_freq;
   const int32_t* params;
@@ -179,8 +180,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Normalised output values of four consecutive columns -> output tensor, in the output element type
 // (the fused-decode form applies the inverse partial rope on the float16 values at float16 op rounding; `rope_cs` holds the
 // cosines of the columns' pairs and, eight further on, their negated sines, where they are known).
-template <int ODT>
-__device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float (&r)[4], int64_t ooff, int dim0,
+template <int ODT, class Args>
+__device__ __forceinline__ void emit_output(Args& a, const float (&r)[4], int64_t ooff, int dim0,
                                             const float* rope_cs = nullptr) {
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = f32x4_t{r[0], r[1], r[2], r[3]};
@@ -218,7 +219,8 @@ __device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float
   }
 }
 
-__device__ __forceinline__ float load_sink_log2(const SparseAttnArgs& a, int head) {
+template <class Args>
+__device__ __forceinline__ float load_sink_log2(Args& a, int head) {
   if (!a.sinks) return -__builtin_inff();
   return (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.sinks)[head])
                                     : reinterpret_cast<const float*>(a.sinks)[head]) * 1.4426950408889634f;
@@ -265,8 +267,17 @@ struct Geometry {
   static_assert(kLastWaves >= 1 && kLastWaves <= kWaves, "the last round of tile loads is issued by the first waves");
 };
 
+// What the ids' addresses take comes as plain arguments, in registers with the wave; the struct behind them is loaded while
+// the ids are on their way. plain_stride: idx_batch_stride of calls with one token and one head block a sequence that are not
+// of the prefill form; -1 otherwise. Every launch began with 0.35 us of waiting for arguments, the grid's size among them; with
+// the merge's, whose sink waits for nothing any more, a layer of one sequence of 8192 keys 22.26 -> 21.95 us, of 16 of 32768
+// 49.1 -> 48.7.
 template <int KDT, int DK, int QDT, bool ROPE>
-__global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAttnArgs a) {
+__global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(const int32_t* idx, const void* q, int total,
+                                                                        int n_splits, uint32_t inv_splits,
+                                                                        int tiles_per_split, int win_per_split,
+                                                                        int idx_per_split, int n_win, int n_idx,
+                                                                        int plain_stride, SparseAttnArgs a) {
   using G = Geometry<DK>;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   unsigned char* kbuf = lds;                                                   // [kBufs][kTileBytes]
@@ -289,7 +300,6 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   const int g = lane >> 5;
 
   // ---- workgroup -> (batch, head block, split); consecutive splits of one batch share an XCD
-  const int total = gridDim.x;
   int work = blockIdx.x;
   if ((total & 7) == 0) work = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
   // (divisions by multiplication with floor(2^32 / n) and one correction step: a software division is a hundred
@@ -300,55 +310,73 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
     if (x - q * n >= n) q++;
     return q;
   };
-  const int bh = (int)div_by((uint32_t)work, (uint32_t)a.n_splits, a.inv_splits);
-  const int sp = work - bh * a.n_splits;
-  const int seq = (int)div_by((uint32_t)bh, (uint32_t)a.n_hblk, a.inv_hblk);
-  const int hb = bh - seq * a.n_hblk;
-  const int b = (int)div_by((uint32_t)seq, (uint32_t)a.n_tokens, a.inv_tokens);
-  const int t = seq - b * a.n_tokens;
-
-  // window rows and visible pool prefix of this sequence; the prefill form derives them from the
-  // token's position in the unsigned 32-bit arithmetic of the reference kernel
-  int seq_n_win = a.n_win, seq_win_first = a.win_first;
-  int64_t seq_visible = a.visible;
-  if (a.prefill) {
-    const uint32_t qpos = a.pos0 + (uint32_t)t, n_raw = (uint32_t)a.raw_cap;
-    const uint32_t last_pos = a.pos0 + (uint32_t)a.n_tokens - 1u;
-    const uint32_t first_raw_pos = last_pos + 1u - n_raw;
-    const uint32_t window_first = (a.window != 0u && qpos + 1u > a.window) ? qpos + 1u - a.window : 0u;
-    const uint32_t first = first_raw_pos > window_first ? first_raw_pos : window_first;
-    const uint32_t last = qpos < last_pos ? qpos : last_pos;
-    seq_n_win = first <= last ? (int)(last - first + 1u) : 0;
-    if (seq_n_win > a.n_win) seq_n_win = a.n_win;  // the host sized the slot space for n_win window rows
-    seq_win_first = first <= last ? (int)(first - first_raw_pos) : 0;
-    const int64_t vis = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
-    seq_visible = vis < a.n_pool ? vis : a.n_pool;
-  }
+  const int bh = (int)div_by((uint32_t)work, (uint32_t)n_splits, inv_splits);
+  const int sp = work - bh * n_splits;
 
   // range sp: its share of the window slots, then its share of the gathered ids. Window tiles come
   // first in the tile order: their rows need no ids, so their copies leave before the id round trip.
-  int w0 = sp * a.win_per_split;
-  int w1 = w0 + a.win_per_split;
-  int g0 = sp * a.idx_per_split;
-  int g1 = g0 + a.idx_per_split;
-  if (a.tiles_per_split > 0) {
-    const int win_tiles = (a.n_win + kTile - 1) / kTile;
-    const int t0 = sp * a.tiles_per_split, t1 = t0 + a.tiles_per_split;
-    w0 = t0 < win_tiles ? t0 * kTile : a.n_win;
-    w1 = t1 < win_tiles ? t1 * kTile : a.n_win;
+  int w0 = sp * win_per_split;
+  int w1 = w0 + win_per_split;
+  int g0 = sp * idx_per_split;
+  int g1 = g0 + idx_per_split;
+  if (tiles_per_split > 0) {
+    const int win_tiles = (n_win + kTile - 1) / kTile;
+    const int t0 = sp * tiles_per_split, t1 = t0 + tiles_per_split;
+    w0 = t0 < win_tiles ? t0 * kTile : n_win;
+    w1 = t1 < win_tiles ? t1 * kTile : n_win;
     g0 = t0 > win_tiles ? (t0 - win_tiles) * kTile : 0;
     g1 = t1 > win_tiles ? (t1 - win_tiles) * kTile : 0;
   }
-  if (w1 > seq_n_win) w1 = seq_n_win;
-  const int wt = w1 > w0 ? (w1 - w0 + kTile - 1) / kTile : 0;
-  if (g1 > a.n_idx) g1 = a.n_idx;
+  if (g1 > n_idx) g1 = n_idx;
+  // The gathered ids of this thread's slots are requested before anything else: ids -> row pointers ->
+  // rows is the longest dependency chain of the prologue. Local slot ls = tid + 512 j of the range.
+  int wt = 0;  // window tiles
+  int my_id[G::kMaxIds / kThreads];
+  const int32_t* idx_b = idx;
+  auto request_ids = [&](int seq_n_win, int64_t first) {
+    if (w1 > seq_n_win) w1 = seq_n_win;
+    wt = w1 > w0 ? (w1 - w0 + kTile - 1) / kTile : 0;
+    idx_b = idx + first;
+#pragma unroll
+    for (int j = 0; j < G::kMaxIds / kThreads; j++) {
+      const int ls = tid + kThreads * j;
+      const int gi = g0 + ls - wt * kTile;
+      my_id[j] = (ls >= wt * kTile && gi < g1) ? idx_b[gi] : -1;
+    }
+  };
+  if (plain_stride >= 0) request_ids(n_win, (int64_t)bh * plain_stride);
+
+  int seq = bh, hb = 0, b = bh, t = 0;
+  // window rows and visible pool prefix of this sequence; the prefill form derives them from the
+  // token's position in the unsigned 32-bit arithmetic of the reference kernel
+  int seq_n_win = n_win, seq_win_first = a.win_first;
+  int64_t seq_visible = a.visible;
+  if (plain_stride < 0) {
+    seq = (int)div_by((uint32_t)bh, (uint32_t)a.n_hblk, a.inv_hblk);
+    hb = bh - seq * a.n_hblk;
+    b = (int)div_by((uint32_t)seq, (uint32_t)a.n_tokens, a.inv_tokens);
+    t = seq - b * a.n_tokens;
+    if (a.prefill) {
+      const uint32_t qpos = a.pos0 + (uint32_t)t, n_raw = (uint32_t)a.raw_cap;
+      const uint32_t last_pos = a.pos0 + (uint32_t)a.n_tokens - 1u;
+      const uint32_t first_raw_pos = last_pos + 1u - n_raw;
+      const uint32_t window_first = (a.window != 0u && qpos + 1u > a.window) ? qpos + 1u - a.window : 0u;
+      const uint32_t first = first_raw_pos > window_first ? first_raw_pos : window_first;
+      const uint32_t last = qpos < last_pos ? qpos : last_pos;
+      seq_n_win = first <= last ? (int)(last - first + 1u) : 0;
+      if (seq_n_win > n_win) seq_n_win = n_win;  // the host sized the slot space for n_win window rows
+      seq_win_first = first <= last ? (int)(first - first_raw_pos) : 0;
+      const int64_t vis = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
+      seq_visible = vis < a.n_pool ? vis : a.n_pool;
+    }
+    request_ids(seq_n_win, (int64_t)seq * a.idx_batch_stride);
+  }
   const int gt = g1 > g0 ? (g1 - g0 + kTile - 1) / kTile : 0;
   const int n_tiles = wt + gt;
   const int g_ls0 = wt * kTile;  // first local slot of the gathered part
 
   const uint16_t* win_b = reinterpret_cast<const uint16_t*>(a.win) + (int64_t)b * a.win_batch_stride;
   const uint16_t* pool_b = reinterpret_cast<const uint16_t*>(a.pool) + (int64_t)b * a.pool_batch_stride;
-  const int32_t* idx_b = a.idx + (int64_t)seq * a.idx_batch_stride;
 
   // ---- query operand: lane (n = head, g) holds q[head][dh*kPart + 16ks + 8g .. +7]; its loads go out
   //      right behind the id loads below and are back by the time the row pointer table is built
@@ -366,7 +394,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   const int q_heads_left = a.n_heads - hb * 64 - hg * 32;                                       // the rest repeat the first
   auto q_request = [&]() {
     const unsigned char* q0 = reinterpret_cast<const unsigned char*>(
-        reinterpret_cast<const uint16_t*>(a.q) + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
+        reinterpret_cast<const uint16_t*>(q) + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
         (q_heads_left > 0 ? (int64_t)(hb * 64 + hg * 32) * a.q_head_stride : (int64_t)0) + dh * G::kPart);
     const uint32_t head_bytes = (uint32_t)a.q_head_stride * 2u;
     int head_of = lane / kQLo, piece = lane - head_of * kQLo;
@@ -411,17 +439,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
     pass(kQLo / 2, kQHi, kQHi / 2);
   };
   f32x4_t qraw32[QDT == MSPR_F32 ? G::kSteps : 1][2];
-  // The gathered ids of this thread's slots are requested before anything else: ids -> row pointers ->
-  // rows is the longest dependency chain of the prologue. Local slot ls = tid + 512 j of the range.
-  int my_id[G::kMaxIds / kThreads];
-#pragma unroll
-  for (int j = 0; j < G::kMaxIds / kThreads; j++) {
-    const int ls = tid + kThreads * j;
-    const int gi = g0 + ls - g_ls0;
-    my_id[j] = (ls >= g_ls0 && gi < g1) ? idx_b[gi] : -1;
-  }
   if constexpr (QDT == MSPR_F32) {
-    const float* qp = reinterpret_cast<const float*>(a.q) + qoff;
+    const float* qp = reinterpret_cast<const float*>(q) + qoff;
 #pragma unroll
     for (int ks = 0; ks < G::kSteps; ks++) {
       qraw32[ks][0] = *reinterpret_cast<const f32x4_t*>(qp + 16 * ks);
@@ -431,7 +450,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
     if (q_pieces) {
       q_request();
     } else {
-      const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + qoff;
+      const uint16_t* qp = reinterpret_cast<const uint16_t*>(q) + qoff;
 #pragma unroll
       for (int ks = 0; ks < G::kSteps; ks++) qf[ks] = *reinterpret_cast<const u32x4_t*>(qp + 16 * ks);
     }
@@ -517,16 +536,16 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
     const uint32_t h = f32_to_f16_bits((float)(tid < 64 ? cos((double)theta) : sin((double)theta)));
     (tid < 64 ? rope_c : rope_s)[tid & 31] = h | (h << 16);
   }
-  int stop_pos = a.n_idx;
+  int stop_pos = n_idx;
   if (a.check_stop) {
-    if (tid == 0) *stop_shared = a.n_idx;
+    if (tid == 0) *stop_shared = n_idx;
     __syncthreads();
-    int first = a.n_idx;
-    for (int i = tid; i < a.n_idx; i += kThreads) {
+    int first = n_idx;
+    for (int i = tid; i < n_idx; i += kThreads) {
       int id = idx_b[i];
       if (id >= 0 && (int64_t)id >= seq_visible && i < first) first = i;
     }
-    if (first < a.n_idx) atomicMin(stop_shared, first);
+    if (first < n_idx) atomicMin(stop_shared, first);
     __syncthreads();
     stop_pos = *stop_shared;
   }
@@ -801,7 +820,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(SparseAt
   // partial row is stored normalised by its own denominator, so it is a convex combination of V rows
   // and fits float16 whenever V does; with bf16 V it saturates at the float16 range instead of
   // overflowing. Its rounding (2^-11 relative) stays below the rounding of the final output.
-  const int64_t part = ((int64_t)(seq * a.n_hblk + hb) * a.n_splits + sp);
+  const int64_t part = ((int64_t)(seq * a.n_hblk + hb) * n_splits + sp);
   // Through the L2 (store_window): a layer of 16 sequences over 32768 keys 49.3 -> 47.9 us, of 8 36.6 -> 35.2; the merge reads
   // them from beyond the L2 either way (17 MB by the counters). One token's few (the rotated form) are out sooner through the
   // cache: 23.4 and 23.7 us.
@@ -1445,8 +1464,19 @@ __global__ __launch_bounds__(256) void prefill_q_to_half_kernel(const float* q, 
 // each, up to eight at once (one trip to memory for up to 32 ranges), and meet in LDS. The kernel is bound by that trip, 2 us
 // to partials that other dies' L2s have written back: with every range in each wave, in rounds of sixteen with two loads for
 // the statistics, it took 6.2 us at 16 ranges (16 sequences; now 5.1) and 6.3 at 32 (one sequence; now 3.9).
+// (Plain arguments first: they come in registers with the wave.)
 template <int ODT>
-__global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a) {
+__global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, float* ws_ml, const void* sinks,
+                                                                int sinks_dtype, unsigned total, int n_splits, int n_hblk,
+                                                                uint32_t inv_hblk, int n_heads, SparseAttnArgs a) {
+  a.ws_o = ws_o;
+  a.ws_ml = ws_ml;
+  a.sinks = sinks;
+  a.sinks_dtype = sinks_dtype;
+  a.n_splits = n_splits;
+  a.n_hblk = n_hblk;
+  a.inv_hblk = inv_hblk;
+  a.n_heads = n_heads;
   __shared__ float xm[4][64], xl[4][64];
   __shared__ __attribute__((aligned(16))) float xo[4][2][64][4];
   __shared__ float rope_cs[16];  // of the workgroup's sixteen columns: eight cosines, eight negated sines
@@ -1454,7 +1484,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // a sequence's partials are merged on the XCD whose workgroups wrote them (the split kernel's mapping)
   unsigned work = blockIdx.x;
-  if ((gridDim.x & 7u) == 0u) work = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if ((total & 7u) == 0u) work = (blockIdx.x & 7u) * (total >> 3) + (blockIdx.x >> 3);
   const int piece = work & 7;        // registers 8 piece .. +7 of the wave's 64: columns tile piece / 2
   const int wave = (work >> 3) & 7;  // wave of the split kernel whose registers this workgroup merges
   const int bh = work >> 6;
@@ -1474,6 +1504,12 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   const int64_t part0 = (int64_t)bh * a.n_splits;
   const f32x2_t* ml0 = reinterpret_cast<const f32x2_t*>(a.ws_ml) + part0 * 64 + hg * 32 + n;
   const f16x8_t* wo0 = reinterpret_cast<const f16x8_t*>(a.ws_o) + (part0 * kWaves + wave) * (int64_t)(8 * 64) + piece * 64 + lane;
+  uint32_t sink_bits = 0;  // (on its way with the partials; made a number of behind them)
+  if (a.sinks) {
+    const int h = live ? head : 0;
+    sink_bits = a.sinks_dtype == MSPR_F16 ? reinterpret_cast<const uint16_t*>(a.sinks)[h]
+                                          : reinterpret_cast<const uint32_t*>(a.sinks)[h];
+  }
   constexpr int kChunk = 8;
   // The inverse rope of the last 64 columns: waves 2 and 3 work out the workgroup's cosines and sines in float64 while the
   // partials are on their way (left to the end, for each pair anew, they were the last thing the launch waited for).
@@ -1520,7 +1556,6 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
     m_run = m_new;
   }
   if (w4 >= a.n_splits) rope_columns();  // (no range for this wave)
-  const float sink = live ? load_sink_log2(a, head) : -__builtin_inff();
   xm[w4][lane] = m_run;
   xl[w4][lane] = l;
 #pragma unroll
@@ -1529,6 +1564,9 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(SparseAttnArgs a
   __syncthreads();
   // waves 0 and 1 finish four of the eight columns each; the sink joins the maximum and the denominator once
   if (w4 >= 2 || !live) return;
+  const float sink = !a.sinks ? -__builtin_inff()
+                              : (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32((uint16_t)sink_bits)
+                                                           : __uint_as_float(sink_bits)) * 1.4426950408889634f;
   float m_all = sink;
 #pragma unroll
   for (int w = 0; w < 4; w++) m_all = fmaxf(m_all, xm[w][lane]);
@@ -1626,7 +1664,11 @@ int launch_split(const SparseAttnArgs& a, hipStream_t st) {
   dim3 grid((unsigned)(a.batch * a.n_hblk * a.n_splits)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
-    sparse_attn_split_kernel<KDT, DK, QDT, ROPE><<<grid, block, G::kLdsBytes, st>>>(a);
+    const bool plain = a.n_hblk == 1 && a.n_tokens == 1 && !a.prefill && a.idx_batch_stride >= 0 &&
+                       a.idx_batch_stride < ((int64_t)1 << 31);
+    sparse_attn_split_kernel<KDT, DK, QDT, ROPE><<<grid, block, G::kLdsBytes, st>>>(
+        a.idx, a.q, (int)grid.x, a.n_splits, a.inv_splits, a.tiles_per_split, a.win_per_split, a.idx_per_split, a.n_win, a.n_idx,
+        plain ? (int)a.idx_batch_stride : -1, a);
   }
   MSPR_CHECK_LAUNCH("sparse attention (split)");
   return MSPR_OK;
@@ -1754,9 +1796,10 @@ int run_sparse_attention(SparseAttnArgs a, int kv_dtype, int k_dim, void* worksp
   dim3 grid((unsigned)(a.batch * a.n_hblk * 64)), block(256);
   {
     MsprProfScope prof(MSPR_K_SPARSE_MERGE, st);
-    if (a.out_dtype == MSPR_F32) sparse_attn_merge_kernel<MSPR_F32><<<grid, block, 0, st>>>(a);
-    else if (a.out_dtype == MSPR_BF16) sparse_attn_merge_kernel<MSPR_BF16><<<grid, block, 0, st>>>(a);
-    else sparse_attn_merge_kernel<MSPR_F16><<<grid, block, 0, st>>>(a);
+    const auto merge = a.out_dtype == MSPR_F32 ? &sparse_attn_merge_kernel<MSPR_F32>
+                       : a.out_dtype == MSPR_BF16 ? &sparse_attn_merge_kernel<MSPR_BF16>
+                                                  : &sparse_attn_merge_kernel<MSPR_F16>;
+    merge<<<grid, block, 0, st>>>(a.ws_o, a.ws_ml, a.sinks, a.sinks_dtype, grid.x, a.n_splits, a.n_hblk, a.inv_hblk, a.n_heads, a);
   }
   MSPR_CHECK_LAUNCH("sparse attention (merge)");
   return MSPR_OK;
