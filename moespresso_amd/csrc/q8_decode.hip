@@ -39,6 +39,7 @@ struct Q8Args {
   const void* v_scales;
   const void* v_biases;
   int batch, n_q_heads, n_kv_heads;
+  int rep;  // query heads per KV head
   int64_t n_keys;
   int64_t kv_rows;  // rows allocated per (batch, kv head); >= n_keys
   float scale_log2;
@@ -71,8 +72,17 @@ __device__ __forceinline__ void codes4_to_h(uint32_t w, h2_t& lo, h2_t& hi) {
   }
 }
 
+// (What the first loads' addresses take comes first: fourteen words of plain arguments are in registers when a wave starts, the
+// rest is loaded under those requests. With one struct for both kernels, and the merge's head taken apart by a division: one
+// sequence of 8192 keys, appended and attended, 16.0 us of device time, now 15.0; eight of 37000 keys 64.9, now 63.7.)
 template <int FMT, int QDT, int SDT>
-__global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Args a) {
+__global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const uint8_t* k_codes, const uint8_t* v_codes,
+                                                                          const uint8_t* ksc, const uint8_t* vsc,
+                                                                          int64_t kv_rows, int n_keys, int keys_per_split,
+                                                                          int n_kv_heads, const void* q,
+                                                                          const uint8_t* kbi, const uint8_t* vbi,
+                                                                          float* ws_o, float* ws_ml, float scale_log2,
+                                                                          int n_splits, int rep) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -84,15 +94,14 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
   const int sp = blockIdx.x;
   const int kvh = blockIdx.y;
   const int b = blockIdx.z;
-  const int rep = a.n_q_heads / a.n_kv_heads;
-  const int64_t N = a.n_keys;
-  const int64_t k0 = (int64_t)sp * a.keys_per_split;
-  int64_t k1 = k0 + a.keys_per_split;
+  const int64_t N = n_keys;
+  const int64_t k0 = (int64_t)sp * keys_per_split;
+  int64_t k1 = k0 + keys_per_split;
   if (k1 > N) k1 = N;
 
-  const int64_t kv_row0 = ((int64_t)b * a.n_kv_heads + kvh) * a.kv_rows;  // first key row of this (b, kv head)
-  const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.k_codes) + kv_row0 * kD;
-  const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.v_codes) + kv_row0 * kD;
+  const int64_t kv_row0 = ((int64_t)b * n_kv_heads + kvh) * kv_rows;  // first key row of this (b, kv head)
+  const uint8_t* kc = k_codes + kv_row0 * kD;
+  const uint8_t* vc = v_codes + kv_row0 * kD;
 
   f32x4_t oacc[16];
 #pragma unroll
@@ -123,10 +132,6 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
     u32x4_t c[8];
     uint32_t s[4], bz[4];  // affine: raw bits per row; Q8_0: s[0], s[1] hold the half row's four float16 scales
   } vr;
-  const uint8_t* ksc = reinterpret_cast<const uint8_t*>(a.k_scales);
-  const uint8_t* kbi = reinterpret_cast<const uint8_t*>(a.k_biases);
-  const uint8_t* vsc = reinterpret_cast<const uint8_t*>(a.v_scales);
-  const uint8_t* vbi = reinterpret_cast<const uint8_t*>(a.v_biases);
 
   auto load_k = [&](int64_t key0) {
 #pragma unroll
@@ -196,10 +201,10 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
   u32x4_t qf[8];
   {
     const bool live = n < rep;
-    const int64_t qoff = ((int64_t)b * a.n_q_heads + kvh * rep + (live ? n : 0)) * kD + 64 * g;
+    const int64_t qoff = (((int64_t)b * n_kv_heads + kvh) * rep + (live ? n : 0)) * kD + 64 * g;
     float v[8][8];
     if constexpr (QDT == MSPR_F32) {
-      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff);
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(q) + qoff);
       f32x4_t raw[16];
 #pragma unroll
       for (int j = 0; j < 16; j++) raw[j] = p[j];
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
 #pragma unroll
         for (int j = 0; j < 8; j++) v[s][j] = raw[2 * s + (j >> 2)][j & 3];
     } else {
-      const u32x4_t* p = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(a.q) + qoff);
+      const u32x4_t* p = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(q) + qoff);
       u32x4_t raw[8];
 #pragma unroll
       for (int s = 0; s < 8; s++) raw[s] = p[s];
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
       u32x4_t f;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        h2_t h = {(_Float16)(live ? v[s][2 * j] * a.scale_log2 : 0.0f), (_Float16)(live ? v[s][2 * j + 1] * a.scale_log2 : 0.0f)};
+        h2_t h = {(_Float16)(live ? v[s][2 * j] * scale_log2 : 0.0f), (_Float16)(live ? v[s][2 * j + 1] * scale_log2 : 0.0f)};
         f[j] = h2_bits(h);
       }
       qf[s] = f;
@@ -398,8 +403,8 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
     mw[w] = __builtin_amdgcn_exp2f(mw[w] - m_safe);
     l_all += lw[w] * mw[w];
   }
-  const int64_t part = (((int64_t)b * a.n_kv_heads + kvh) * a.n_splits + sp);
-  float* po = a.ws_o + part * (16 * kD);
+  const int64_t part = (((int64_t)b * n_kv_heads + kvh) * n_splits + sp);
+  float* po = ws_o + part * (16 * kD);
   // every wave reduces its share of the 16 M-tiles: dims 16mt + 4g + i of head n
 #pragma unroll
   for (int q4 = 0; q4 < 16 / kQ8Waves; q4++) {
@@ -413,7 +418,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
     if (n < rep) *reinterpret_cast<f32x4_t*>(po + n * kD + 16 * mt + 4 * g) = acc;  // (columns past the real heads are padding)
   }
   if (wave == 0 && g == 0) {
-    float* pml = a.ws_ml + part * 32;
+    float* pml = ws_ml + part * 32;
     pml[n * 2] = m_all;
     pml[n * 2 + 1] = l_all;
   }
@@ -424,31 +429,30 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(Q8Arg
 // (one memory round trip for up to 256 ranges), the wave results are combined in LDS.
 constexpr int kMergeWaves = 16;
 template <int ODT>
-__global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Args a) {
+__global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(const float* ws_o, const float* ws_ml, void* out,
+                                                                          int n_splits, int rep) {
   __shared__ float xm[kMergeWaves], xl[kMergeWaves];
   __shared__ __attribute__((aligned(16))) float xo[kMergeWaves][kD];
   const int lane = threadIdx.x & 63;
   const int sg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int qh = blockIdx.x;
-  const int b = blockIdx.y;
-  const int rep = a.n_q_heads / a.n_kv_heads;
-  const int kvh = qh / rep, hn = qh % rep;
-  const int64_t part0 = ((int64_t)b * a.n_kv_heads + kvh) * a.n_splits;
-  const float* ml = a.ws_ml + part0 * 32 + hn * 2;
-  const float* po = a.ws_o + part0 * (16 * kD) + hn * kD + 4 * lane;
+  const int64_t bh = blockIdx.x;  // KV head of a sequence
+  const int hn = blockIdx.y;      // query head of its group
+  const int64_t part0 = bh * n_splits;
+  const float* ml = ws_ml + part0 * 32 + hn * 2;
+  const float* po = ws_o + part0 * (16 * kD) + hn * kD + 4 * lane;
   constexpr int kChunk = 16;
   float m_run = -__builtin_inff(), l = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = sg; s0 < a.n_splits; s0 += kMergeWaves * kChunk) {
+  for (int s0 = sg; s0 < n_splits; s0 += kMergeWaves * kChunk) {
     // The statistics of range j by lane j, in one load, whose weight is then taken once: with scalar loads of them each range's
     // were waited for in front of the next range's row, and every lane took all sixteen exponentials.
     const int mine = s0 + kMergeWaves * (lane % kChunk);
     f32x2_t stat = {-__builtin_inff(), 0.0f};
-    if (mine < a.n_splits) stat = *reinterpret_cast<const f32x2_t*>(ml + (int64_t)mine * 32);
+    if (mine < n_splits) stat = *reinterpret_cast<const f32x2_t*>(ml + (int64_t)mine * 32);
     f32x4_t ov[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; j++)  // (wave-uniform: ranges past the end cost no load)
-      if (s0 + kMergeWaves * j < a.n_splits)
+      if (s0 + kMergeWaves * j < n_splits)
         ov[j] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)(s0 + kMergeWaves * j) * (16 * kD));
     static_assert(kChunk == 16, "reduced over rows of sixteen lanes");
     float m_new = stat.x;
@@ -467,7 +471,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Arg
     o = o * alpha;
 #pragma unroll
     for (int j = 0; j < kChunk; j++)
-      if (s0 + kMergeWaves * j < a.n_splits) o += ov[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+      if (s0 + kMergeWaves * j < n_splits) o += ov[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
     m_run = m_new;
   }
   if (lane == 0) {
@@ -490,16 +494,16 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Arg
     o_all += *reinterpret_cast<const f32x4_t*>(&xo[w][4 * lane]) * wt;
   }
   const float inv = l_all == 0.0f ? 0.0f : 1.0f / l_all;
-  const int64_t ooff = ((int64_t)b * a.n_q_heads + qh) * kD + 4 * lane;
+  const int64_t ooff = (bh * rep + hn) * kD + 4 * lane;
   if constexpr (ODT == MSPR_F32) {
-    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = o_all * inv;
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + ooff) = o_all * inv;
   } else {
     uint16_t h[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
       h[i] = ODT == MSPR_BF16 ? f32_to_bf16_bits(o_all[i] * inv) : f32_to_f16_bits(o_all[i] * inv);
     u32x2_t pk = {(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(a.out) + ooff) = pk;
+    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(out) + ooff) = pk;
   }
 }
 
@@ -545,16 +549,17 @@ int q8_launch(Q8Args a, hipStream_t st) {
   dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv_heads, (unsigned)a.batch), block(64 * kQ8Waves);
   {
     MsprProfScope prof(MSPR_K_Q8_DECODE, st);
-    q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(a);
+    q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(
+        reinterpret_cast<const uint8_t*>(a.k_codes), reinterpret_cast<const uint8_t*>(a.v_codes),
+        reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales), a.kv_rows, (int)a.n_keys,
+        a.keys_per_split, a.n_kv_heads, a.q, reinterpret_cast<const uint8_t*>(a.k_biases),
+        reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml, a.scale_log2, a.n_splits, a.rep);
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (split)");
-  dim3 mgrid((unsigned)a.n_q_heads, (unsigned)a.batch);
   {
     MsprProfScope prof(MSPR_K_Q8_MERGE, st);
-    dim3 mblock(64 * kMergeWaves);
-    if (QDT == MSPR_F32) q8_decode_merge_kernel<MSPR_F32><<<mgrid, mblock, 0, st>>>(a);
-    else if (QDT == MSPR_BF16) q8_decode_merge_kernel<MSPR_BF16><<<mgrid, mblock, 0, st>>>(a);
-    else q8_decode_merge_kernel<MSPR_F16><<<mgrid, mblock, 0, st>>>(a);
+    q8_decode_merge_kernel<QDT><<<dim3((unsigned)(a.batch * a.n_kv_heads), (unsigned)a.rep), dim3(64 * kMergeWaves), 0, st>>>(
+        a.ws_o, a.ws_ml, a.out, a.n_splits, a.rep);
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (merge)");
   return MSPR_OK;
@@ -583,6 +588,7 @@ void q8_fill_args(Q8Args& a, int batch, int n_q_heads, int n_kv_heads, int64_t n
   a.batch = batch;
   a.n_q_heads = n_q_heads;
   a.n_kv_heads = n_kv_heads;
+  a.rep = n_q_heads / n_kv_heads;
   a.n_keys = n_keys;
   a.scale_log2 = (float)((double)scale * 1.4426950408889634);
   int64_t kps;
