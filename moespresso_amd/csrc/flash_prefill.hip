@@ -39,6 +39,7 @@ struct PrefillArgs {
   float scale_log2;
   int rep_shift;    // log2(query heads per KV head), 0..3
   int q_blocks;     // workgroups along the query axis
+  uint32_t inv_splits, inv_q_blocks, inv_kv_heads;  // floor(2^32 / n), for divisions by n_splits, q_blocks, n_kv_heads
   // key-range splits (short chunks over deep prefixes do not fill the device otherwise): split sp of a
   // query block takes every n_splits-th share of that block's tiles; partials are merged afterwards
   int n_splits;
@@ -176,8 +177,23 @@ __device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 
 // scales and biases, with kExactUnpack added to it where the prefix is unpacked to the values that a conversion beforehand
 // gives; without it in packed float16 arithmetic.
 constexpr int kExactUnpack = 4;
+
+// x / n with inv = floor(2^32 / n): a software division is some thirty instructions, four of them stood in front of the first
+// memory request
+__device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
+  if (n == 1) return x;
+  int q = (int)__umulhi((uint32_t)x, inv);  // the quotient or one less
+  if (x - q * n >= n) q++;
+  return q;
+}
+
+// (Plain arguments first: what the first tiles' addresses take comes in registers with the wave, and the struct is loaded
+// meanwhile. heads: n_kv_heads, and rep_shift from bit 28 on.)
 template <int KDT, bool Q8, int SDT, bool IO32, bool Q32, bool RUNS>
-__global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsigned char* k, const unsigned char* v,
+                                                                   const void* q, int q_len, int past, int kv_rows,
+                                                                   int n_splits, uint32_t inv_splits, int q_blocks,
+                                                                   uint32_t inv_q_blocks, uint32_t heads, PrefillArgs a) {
   extern __shared__ __attribute__((aligned(256))) unsigned char lds[];  // tile bases: zero low bits under the address XORs
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -190,12 +206,13 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   // the early end, so every workgroup carries the same matrix work although the causal key count grows with the
   // query position; the tile stream runs to the late block's last key and the early waves leave it when their
   // last key has passed. Four heads per group; with fewer heads per KV head a group takes 2 or 4 adjacent blocks.
-  const int rep = 1 << a.rep_shift;
-  const int hpg_shift = a.rep_shift < 2 ? a.rep_shift : 2;  // log2(heads per group)
+  const int n_kv_heads = (int)(heads & 0x0FFFFFFFu), rep_shift = (int)(heads >> 28);
+  const int rep = 1 << rep_shift;
+  const int hpg_shift = rep_shift < 2 ? rep_shift : 2;  // log2(heads per group)
   const int blocks_per_group = 4 >> hpg_shift;
-  const int head_halves = 1 << (a.rep_shift - hpg_shift);
-  const int n_blocks = (a.q_len + 31) / 32;
-  const int n_pairs = a.q_blocks / head_halves;
+  const int halves_shift = rep_shift - hpg_shift;
+  const int n_blocks = (q_len + 31) >> 5;
+  const int n_pairs = q_blocks >> halves_shift;
   // RUNS (four ranges or more, of ten tiles or more): workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run
   // of the list (batch, KV head, range, pair). An L2 then holds the keys of few ranges and one or two heads' queries, which
   // all pairs of a range pass together. Elsewhere the ranges go round the XCDs, as in runs the partials leave the L2s 2 us
@@ -204,22 +221,25 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   int work = blockIdx.x;
   int sp, q_block;
   if constexpr (RUNS) {
-    const int wgs = a.batch * a.n_kv_heads * a.q_blocks * a.n_splits, xcd = work & 7;
+    const int wgs = a.batch * n_kv_heads * q_blocks * n_splits, xcd = work & 7;
     work = xcd * (wgs >> 3) + (xcd < (wgs & 7) ? xcd : wgs & 7) + (work >> 3);
-    q_block = work % a.q_blocks;
-    work /= a.q_blocks;
-    sp = work % a.n_splits;
-    work /= a.n_splits;
+    const int rest = div_by(work, q_blocks, inv_q_blocks);
+    q_block = work - rest * q_blocks;
+    work = div_by(rest, n_splits, inv_splits);
+    sp = rest - work * n_splits;
   } else {
-    sp = work % a.n_splits;
-    work /= a.n_splits;
-    q_block = work % a.q_blocks;
-    work /= a.q_blocks;
+    const int rest = div_by(work, n_splits, inv_splits);
+    sp = work - rest * n_splits;
+    work = div_by(rest, q_blocks, inv_q_blocks);
+    q_block = rest - work * q_blocks;
   }
-  const int pair = q_block / head_halves;  // pair 0 (longest stream) first
-  const int head_half = q_block % head_halves;
-  const int kvh = work % a.n_kv_heads;
-  const int b = work / a.n_kv_heads;
+  const int pair = q_block >> halves_shift;  // pair 0 (longest stream) first
+  const int head_half = q_block & ((1 << halves_shift) - 1);
+  int kvh = work, b = 0;
+  if (work >= n_kv_heads) {
+    b = div_by(work, n_kv_heads, a.inv_kv_heads);
+    kvh = work - b * n_kv_heads;
+  }
   const int wi = wave & 3;
   const int head = kvh * rep + (head_half << hpg_shift) + (wi & ((1 << hpg_shift) - 1));
   // late group: blocks [n_blocks - bpg (pair + 1), n_blocks - bpg pair); early group: blocks [bpg pair, bpg (pair + 1))
@@ -228,19 +248,16 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
                            : blocks_per_group * pair + (wi >> hpg_shift);
   const bool active = wave < 4 ? blk >= 0 : blk < n_blocks - blocks_per_group * n_pairs;  // wave-uniform
   const int q0 = active ? 32 * blk : 0;  // first query row of this wave
-  const int past = (int)a.past_len;
 
-  const unsigned char* kbase =
-      reinterpret_cast<const unsigned char*>(a.k) + ((int64_t)b * a.n_kv_heads + kvh) * a.kv_rows * kRowBytes;
-  const unsigned char* vbase =
-      reinterpret_cast<const unsigned char*>(a.v) + ((int64_t)b * a.n_kv_heads + kvh) * a.kv_rows * kRowBytes;
+  const unsigned char* kbase = k + ((int64_t)b * n_kv_heads + kvh) * kv_rows * kRowBytes;
+  const unsigned char* vbase = v + ((int64_t)b * n_kv_heads + kvh) * kv_rows * kRowBytes;
 
   // keys needed by the workgroup: [0, past + last query row]
   int q_last = 32 * (n_blocks - blocks_per_group * pair) - 1;  // last row of the late group
-  if (q_last > a.q_len - 1) q_last = a.q_len - 1;
-  const int all_tiles = (int)((past + q_last) / kTile) + 1;
+  if (q_last > q_len - 1) q_last = q_len - 1;
+  const int all_tiles = (int)((uint32_t)(past + q_last) / kTile) + 1;
   // this workgroup's share of the block's tiles: [t_begin, n_tiles)
-  const int tiles_per_split = (all_tiles + a.n_splits - 1) / a.n_splits;
+  const int tiles_per_split = div_by(all_tiles + n_splits - 1, n_splits, inv_splits);
   const int t_begin = sp * tiles_per_split < all_tiles ? sp * tiles_per_split : all_tiles;
   const int n_tiles = t_begin + tiles_per_split < all_tiles ? t_begin + tiles_per_split : all_tiles;
 
@@ -250,7 +267,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   const int c_piece = (tid & 16) | ((tid ^ swz(c_row)) & 15);  // global 16-byte piece that lands in the slot
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSPR_LDS_PTR(unsigned char, lds);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds0) + wave * 1024;
-  const int n_keys = (int)(past + a.q_len);  // keys that exist
+  const int n_keys = past + q_len;  // keys that exist
   const int t1 = Q8 ? a.q8_tiles : 0;        // first tile served from k / v; their row 0 is key 32 t1
   auto issue_tile = [&](int t_abs, int slot) {
     // rows past the last key (only in the last tile) are masked by the causal rule; read the last key instead
@@ -276,7 +293,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   constexpr int kRawBytes = 2 * kCodeBytes + 4 * 512;
   constexpr int kRawBase = 2 * kStageBytes;      // the unpacked stages use the lower 64 KB
   static_assert(kRawBase + 3 * kRawBytes <= kLdsBytes, "raw ring does not fit");
-  const int64_t raw_row0 = ((int64_t)b * a.n_kv_heads + kvh) * a.past_rows;
+  const int64_t raw_row0 = ((int64_t)b * n_kv_heads + kvh) * a.past_rows;
   const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.pk_wq) + raw_row0 * kD;
   const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.pv_wq) + raw_row0 * kD;
   // scale / bias copies: wave w moves array w & 3 (K scale, K bias, V scale, V bias), 4 bytes per lane; with
@@ -316,7 +333,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
     // clocks for the eight waves' float32 rows, of the 13000 before the first tile. With the stores below, us: 203 float32
     // queries over 9001 quantised keys 78.5 -> 74.0 (whole operator with its append), 30 queries 46.4 -> 42.2, 203 bfloat16
     // ones over 9001 dense keys 56.5 -> 53. Tiles requested behind the queries 1 us more, behind their exchange the same.
-    const int64_t qbase = ((int64_t)b * a.n_q_heads + head) * a.q_len;
+    const int64_t qbase = ((int64_t)b * a.n_q_heads + head) * q_len;
     constexpr int kLanes = Q32 ? 32 : 16;  // lanes of a row
     constexpr int kRows = 64 / kLanes;      // rows of an instruction
     const int xr = lane / kLanes, xc = lane % kLanes;
@@ -333,8 +350,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
 #pragma unroll
       for (int i = 0; i < 32 / kRows; i++) {
         int qrow = q0 + i * kRows + xr;
-        if (qrow > a.q_len - 1) qrow = a.q_len - 1;
-        raw[h][i] = reinterpret_cast<const u32x4_t*>(a.q)[(qbase + qrow) * (2 * kLanes) + h * kLanes + xc];
+        if (qrow > q_len - 1) qrow = q_len - 1;
+        raw[h][i] = reinterpret_cast<const u32x4_t*>(q)[(qbase + qrow) * (2 * kLanes) + h * kLanes + xc];
       }
     unsigned char* xq = lds + (raw_first ? 0 : kTilesAhead * kStageBytes) + (wave << 13);
 #pragma unroll
@@ -576,18 +593,18 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(PrefillArgs 
   asm volatile("" : "+v"(tl));  // (the offsets below are made here, not carried through the tile loop)
   const int en = tl & 31, eg = (tl >> 5) & 1;
   unsigned char* xo = lds + (wave << 14);
-  const int64_t out_row = (((int64_t)(a.n_splits > 1 ? sp : 0) * a.batch + b) * a.n_q_heads + head) * a.q_len + q0;
-  const int n_rows = active ? a.q_len - q0 : 0;  // (of the wave's 32, those below it)
-  const float inv = a.n_splits > 1 ? 1.0f : l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
-  if (a.n_splits > 1 && en < n_rows && eg == 0) {
+  const int64_t out_row = (((int64_t)(n_splits > 1 ? sp : 0) * a.batch + b) * a.n_q_heads + head) * q_len + q0;
+  const int n_rows = active ? q_len - q0 : 0;  // (of the wave's 32, those below it)
+  const float inv = n_splits > 1 ? 1.0f : l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
+  if (n_splits > 1 && en < n_rows && eg == 0) {
     a.ws_ml[(out_row + en) * 2] = m_run;
     a.ws_ml[(out_row + en) * 2 + 1] = l_tot;
   }
   // (the merge leaves a range out whose denominator is zero: a wave without any other, under the causal rule or past the last
   // range with tiles, has nothing to store)
-  if (a.n_splits > 1 && !__any(l_tot != 0.0f)) return;
-  if (IO32 || a.n_splits > 1) {
-    float* po = (a.n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out)) + out_row * kD;
+  if (n_splits > 1 && !__any(l_tot != 0.0f)) return;
+  if (IO32 || n_splits > 1) {
+    float* po = (n_splits > 1 ? a.ws_o : reinterpret_cast<float*>(a.out)) + out_row * kD;
     const __amdgpu_buffer_rsrc_t win = store_window(po, (n_rows < 32 ? n_rows : 32) * kD * 4);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -742,30 +759,30 @@ __global__ __launch_bounds__(256) void prefill_q8_rows_kernel(PrefillArgs a, con
 // rows 4.2 us, with one wave a row 7.1); with few ranges a wave per row keeps more loads in flight (4 ranges of 14400
 // rows: four waves a row took 13 us more).
 template <int ODT, int SHARE>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const float* ws_o, const float* ws_ml, void* out,
+                                                            int64_t n_rows, int n_splits) {
   __shared__ float xm[4], xl[4];
   __shared__ f32x4_t xo[4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // row and range are scalar then
-  const int64_t n_rows = (int64_t)a.batch * a.n_q_heads * a.q_len;
   const int64_t row = (int64_t)blockIdx.x * (4 / SHARE) + wave / SHARE;
   const bool live = row < n_rows;
   float m_run = -__builtin_inff(), l = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
   constexpr int kChunk = 8;
-  for (int s0 = live ? wave % SHARE : a.n_splits; s0 < a.n_splits; s0 += SHARE * kChunk) {
+  for (int s0 = live ? wave % SHARE : n_splits; s0 < n_splits; s0 += SHARE * kChunk) {
     float mv[kChunk], lv[kChunk];
     f32x4_t ov[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; j++) {
-      const int sj = s0 + SHARE * j < a.n_splits ? s0 + SHARE * j : s0;
+      const int sj = s0 + SHARE * j < n_splits ? s0 + SHARE * j : s0;
       const int64_t r = (int64_t)sj * n_rows + row;
-      mv[j] = a.ws_ml[r * 2];
-      lv[j] = a.ws_ml[r * 2 + 1];
-      ov[j] = *reinterpret_cast<const f32x4_t*>(a.ws_o + r * kD + 4 * lane);
+      mv[j] = ws_ml[r * 2];
+      lv[j] = ws_ml[r * 2 + 1];
+      ov[j] = *reinterpret_cast<const f32x4_t*>(ws_o + r * kD + 4 * lane);
       // a range that saw no key of this row contributes nothing (its O may be zero times a value that is not finite); one
       // whose denominator is NaN makes the row NaN
-      if (s0 + SHARE * j >= a.n_splits || lv[j] == 0.0f) {
+      if (s0 + SHARE * j >= n_splits || lv[j] == 0.0f) {
         mv[j] = -__builtin_inff();
         lv[j] = 0.0f;
         ov[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -811,10 +828,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   if (!live) return;
   const float inv = l == 0.0f ? 0.0f : 1.0f / l;
   if constexpr (ODT == MSPR_F32) {
-    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + row * kD + 4 * lane) = o * inv;
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + row * kD + 4 * lane) = o * inv;
   } else {
     u32x2_t w = {pack2<ODT>(o.x * inv, o.y * inv), pack2<ODT>(o.z * inv, o.w * inv)};
-    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(a.out) + row * kD + 4 * lane) = w;
+    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(out) + row * kD + 4 * lane) = w;
   }
 }
 
@@ -872,14 +889,22 @@ int prefill_launch_flash(const PrefillArgs& a, hipStream_t st) {
   dim3 grid((unsigned)(a.q_blocks * a.n_kv_heads * a.batch * a.n_splits)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_FLASH_PREFILL, st);
-    flash_prefill_kernel<KDT, Q8, SDT, IO32, Q32, RUNS><<<grid, block, kLdsBytes, st>>>(a);
+    flash_prefill_kernel<KDT, Q8, SDT, IO32, Q32, RUNS><<<grid, block, kLdsBytes, st>>>(
+        reinterpret_cast<const unsigned char*>(a.k), reinterpret_cast<const unsigned char*>(a.v), a.q, a.q_len,
+        (int)a.past_len, (int)a.kv_rows, a.n_splits, a.inv_splits, a.q_blocks, a.inv_q_blocks,
+        (uint32_t)a.n_kv_heads | (uint32_t)a.rep_shift << 28, a);
   }
   MSPR_CHECK_LAUNCH("flash_prefill");
   return MSPR_OK;
 }
 
 template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
-int prefill_launch(const PrefillArgs& a, hipStream_t st, bool q32 = false) {
+int prefill_launch(const PrefillArgs& call, hipStream_t st, bool q32 = false) {
+  PrefillArgs a = call;
+  auto inverse = [](int n) -> uint32_t { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); };
+  a.inv_splits = inverse(a.n_splits);
+  a.inv_q_blocks = inverse(a.q_blocks);
+  a.inv_kv_heads = inverse(a.n_kv_heads);
   // (the line of the kernel's mapping; a template parameter because as a run-time branch it cost long chunks 0.5 %)
   const bool runs = a.n_splits >= 4 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
   int rc;
@@ -895,9 +920,9 @@ int prefill_launch(const PrefillArgs& a, hipStream_t st, bool q32 = false) {
     const int share = a.n_splits <= 8 || (a.n_splits <= 16 && n_rows >= 3584) ? 1 : a.n_splits <= 32 ? 2 : 4;
     dim3 mgrid((unsigned)((n_rows * share + 3) / 4)), mblock(256);
     constexpr int ODT = IO32 ? (int)MSPR_F32 : KDT;
-    if (share == 1) prefill_merge_kernel<ODT, 1><<<mgrid, mblock, 0, st>>>(a);
-    else if (share == 2) prefill_merge_kernel<ODT, 2><<<mgrid, mblock, 0, st>>>(a);
-    else prefill_merge_kernel<ODT, 4><<<mgrid, mblock, 0, st>>>(a);
+    const auto merge = share == 1 ? &prefill_merge_kernel<ODT, 1> : share == 2 ? &prefill_merge_kernel<ODT, 2>
+                                                                               : &prefill_merge_kernel<ODT, 4>;
+    merge<<<mgrid, mblock, 0, st>>>(a.ws_o, a.ws_ml, a.out, n_rows, a.n_splits);
     MSPR_CHECK_LAUNCH("flash_prefill (merge)");
   }
   return MSPR_OK;
