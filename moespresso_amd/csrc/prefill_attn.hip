@@ -27,6 +27,8 @@
 #include "prefill_attn.h"
 #include "profile.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kTile = 32;
@@ -65,9 +67,27 @@ __device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint3
                : "memory", "m0");
 }
 
+// x / n with inv = floor(2^32 / n), x below 2^31: a software division is some thirty instructions
+__device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
+  if (n == 1) return x;
+  int q = (int)__umulhi((uint32_t)x, inv);  // the quotient or one less
+  if (x - q * n >= n) q++;
+  return q;
+}
+
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
-template <int QDT, bool CUT>
-__global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPrefillArgs a) {
+// EAGER: the queries are requested before the ids are looked at, not behind. That takes a trip to memory off a workgroup's
+// start, and pays where all start at once and none follows (60 tokens behind 28000: 34.9 us, and 34.2 with the requests
+// ahead; 255 tokens 46.1 and 45.2); with more than a round of 512 units they crowd out the other workgroup's rows (1536 tokens
+// 166.6 and 169.6).
+// (Plain arguments first: what the first copies and the ids take comes in registers with the wave, and the struct is loaded
+// meanwhile.)
+template <int QDT, bool CUT, bool EAGER>
+__global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void* win, const int32_t* idx, int units,
+                                                                      int n_tokens, uint32_t inv_tokens, int n_hblk,
+                                                                      uint32_t pos0, uint32_t window, uint32_t n_raw,
+                                                                      int raw_start, int max_win, int n_idx,
+                                                                      IndexedPrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int* ids = reinterpret_cast<int*>(lds + kOffIds);
   int* stop_sh = reinterpret_cast<int*>(lds + kOffStop);
@@ -78,43 +98,39 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   const int kg = lane >> 4;
 
   // The tokens with the most rows (the last ones, at the start of a context) are started first.
-  const int n_hblk = (a.n_heads + 63) / 64;
   // The first a.split_units units, a part-filled last round, are cut into a.ranges key ranges each and come last.
-  int unit = (int)(gridDim.x - 1u - blockIdx.x), range = 0;
+  int unit = units - 1 - (int)blockIdx.x, range = 0;
   bool split = false;
   if constexpr (CUT) {
-    const int whole = a.batch * a.n_tokens * n_hblk - a.split_units;
+    const int whole = units - a.split_units;
     split = (int)blockIdx.x >= whole;
     const int i = (int)blockIdx.x - whole;
-    unit = split ? i / a.ranges : a.split_units - 1 - i;
+    unit = split ? div_by(i, a.ranges, a.inv_ranges) : a.split_units - 1 - i;
     range = split ? i - unit * a.ranges : 0;
   }
-  const int hb = unit % n_hblk;
-  const int seq = unit / n_hblk;
-  const int b = seq / a.n_tokens;
-  const int t = seq - b * a.n_tokens;
+  const int seq = n_hblk == 1 ? unit : div_by(unit, n_hblk, a.inv_hblk);
+  const int hb = unit - seq * n_hblk;
+  const int b = div_by(seq, n_tokens, inv_tokens);
+  const int t = seq - b * n_tokens;
 
   // window rows and visible pool prefix, in the unsigned 32-bit arithmetic of the reference kernel
-  const uint32_t qpos = a.pos0 + (uint32_t)t, n_raw = (uint32_t)a.raw_cap;
-  const uint32_t last_pos = a.pos0 + (uint32_t)a.n_tokens - 1u;
+  const uint32_t qpos = pos0 + (uint32_t)t;
+  const uint32_t last_pos = pos0 + (uint32_t)n_tokens - 1u;
   const uint32_t first_raw_pos = last_pos + 1u - n_raw;
-  const uint32_t window_first = (a.window != 0u && qpos + 1u > a.window) ? qpos + 1u - a.window : 0u;
+  const uint32_t window_first = (window != 0u && qpos + 1u > window) ? qpos + 1u - window : 0u;
   const uint32_t first = first_raw_pos > window_first ? first_raw_pos : window_first;
   const uint32_t last = qpos < last_pos ? qpos : last_pos;
   int n_win = first <= last ? (int)(last - first + 1u) : 0;
-  if (n_win > a.max_win) n_win = a.max_win;
+  if (n_win > max_win) n_win = max_win;
   const int win_first = first <= last ? (int)(first - first_raw_pos) : 0;
-  int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
-  if (visible > a.n_pool) visible = a.n_pool;
   const int wt = (n_win + kTile - 1) / kTile;
   // this workgroup's tiles: all of them, or its share of what the token has at most
   int t_begin = 0, t_share = 0x7FFFFFFF;
   if (CUT && split) {
-    t_share = (wt + (a.n_idx + kTile - 1) / kTile + a.ranges - 1) / a.ranges;
+    t_share = div_by(wt + (n_idx + kTile - 1) / kTile + a.ranges - 1, a.ranges, a.inv_ranges);
     t_begin = range * t_share;
   }
-  const uint64_t win_base = reinterpret_cast<uint64_t>(a.win) + (uint64_t)b * (uint64_t)a.raw_cap * (kD * 2);
-  const uint64_t pool_base = reinterpret_cast<uint64_t>(a.pool) + (uint64_t)b * (uint64_t)a.n_pool * (kD * 2);
+  const uint64_t win_base = reinterpret_cast<uint64_t>(win) + (uint64_t)b * (uint64_t)n_raw * (kD * 2);
 
   // Copies of a tile: this wave's eight rows. `row` holds, per lane l < 32, the row of slot l (-1: no row, zeros).
   const uint32_t lane_off = (uint32_t)lane * 16u;
@@ -131,7 +147,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   };
   auto window_row = [&](int tile) -> int {
     const int ls = tile * kTile + (lane & 31);
-    uint32_t r = (uint32_t)a.raw_start + (uint32_t)win_first + (uint32_t)ls;
+    uint32_t r = (uint32_t)raw_start + (uint32_t)win_first + (uint32_t)ls;
     if (r >= n_raw) r -= n_raw;
     return ls < n_win ? (int)r : -1;
   };
@@ -139,25 +155,43 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
   // ---- the first window tile needs no ids: on its way before anything else
   if (t_begin < wt) copy_rows(t_begin, win_base, window_row(t_begin));
 
-  // ---- ids to LDS, position of the first one that ends the walk
-  if (tid == 0) *stop_sh = a.n_idx;
+  // ---- the first ids of a thread, which go to LDS below
+  constexpr int kEager = EAGER ? 2 : 0;
+  const int32_t* src = idx + (int64_t)seq * n_idx;
+  int eager[EAGER ? kEager : 1] = {};
+  if (EAGER && n_idx > 0) {
+#pragma unroll
+    for (int j = 0; j < kEager; j++) {
+      const int i = tid + j * kThreads;
+      eager[j] = src[i < n_idx ? i : 0];
+    }
+  }
+  if (tid == 0) *stop_sh = n_idx;
   __syncthreads();
-  {
-    const int32_t* src = a.idx + ((int64_t)b * a.n_tokens + t) * a.n_idx;
-    int found = a.n_idx;
-    for (int i = tid; i < a.n_idx; i += kThreads) {
-      const int id = src[i];
+
+  // ---- ids to LDS, position of the first one that ends the walk
+  auto stage_ids = [&]() {
+    int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
+    if (visible > a.n_pool) visible = a.n_pool;
+    int found = n_idx;
+    auto look = [&](int i, int id) {
       ids[i] = id;
       if (id >= 0 && (int64_t)id >= visible && i < found) found = i;
-    }
-    if (found < a.n_idx) atomicMin(stop_sh, found);
-  }
+    };
+#pragma unroll
+    for (int j = 0; j < kEager; j++)
+      if (tid + j * kThreads < n_idx) look(tid + j * kThreads, eager[j]);
+    for (int i = tid + kEager * kThreads; i < n_idx; i += kThreads) look(i, src[i]);
+    if (found < n_idx) atomicMin(stop_sh, found);
+  };
+  if constexpr (!EAGER) stage_ids();
 
   // ---- query operand: lane (head c16, kg) holds q[head][32 ks + 8 kg .. +7], zero rows past n_heads
   const int head = hb * 64 + 16 * wave + c16;
   const bool live = head < a.n_heads;
   const int64_t qoff = (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
                        (int64_t)(live ? head : 0) * a.q_head_stride + 8 * kg;
+  f32x4_t raw[QDT == MSPR_F16 ? 1 : 2 * kQSteps];
   u32x4_t qf[kQSteps];
 #pragma unroll
   for (int ks = 0; ks < kQSteps; ks++) {
@@ -165,7 +199,15 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
       qf[ks] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(a.q) + qoff + 32 * ks);
     } else {
       const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff + 32 * ks);
-      const f32x4_t lo = p[0], hi = p[1];
+      raw[2 * ks] = p[0];
+      raw[2 * ks + 1] = p[1];
+    }
+  }
+  if constexpr (EAGER) stage_ids();
+#pragma unroll
+  for (int ks = 0; ks < kQSteps; ks++) {
+    if constexpr (QDT != MSPR_F16) {
+      const f32x4_t lo = raw[2 * ks], hi = raw[2 * ks + 1];
       qf[ks] = u32x4_t{pack_h2(lo.x, lo.y), pack_h2(lo.z, lo.w), pack_h2(hi.x, hi.y), pack_h2(hi.z, hi.w)};
     }
     if (!live) qf[ks] = u32x4_t{0u, 0u, 0u, 0u};
@@ -181,6 +223,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
     const int id = ids[gi < kMaxIds ? gi : 0];
     return gi < stop ? (id >= 0 ? id : -1) : -1;  // (an id in front of the stop is inside the visible prefix)
   };
+  const uint64_t pool_base = reinterpret_cast<uint64_t>(a.pool) + (uint64_t)b * (uint64_t)a.n_pool * (kD * 2);
   // rows and validity word of a tile
   auto rows_of = [&](int tile) -> int { return tile < wt ? window_row(tile) : pool_row(tile); };
   int row = rows_of(t_begin);
@@ -326,28 +369,31 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(IndexedPre
 
 // The ranges of the cut units and the sink, normalised. A wave takes one accumulator register quad (16 heads, 16 columns) of
 // a unit: every range's is 1 KB, and all are requested at once.
-__global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(IndexedPrefillArgs a) {
+__global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(const float* parts, const float* sinks, int split_units,
+                                                                    int ranges, int n_heads, int n_hblk, uint32_t inv_hblk,
+                                                                    int n_tokens, uint32_t inv_tokens, float* out,
+                                                                    int64_t batch_stride, int64_t token_stride,
+                                                                    int64_t head_stride) {
   const int lane = threadIdx.x & 63;
   const int c16 = lane & 15, kg = lane >> 4;
   const int piece = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
   const int unit = piece >> 7, wave = (piece >> 5) & 3, mt = piece & 31;
-  const int n_hblk = (a.n_heads + 63) / 64;
-  const int hb = unit % n_hblk, seq = unit / n_hblk;
-  const int b = seq / a.n_tokens, t = seq - b * a.n_tokens;
+  const int seq = div_by(unit, n_hblk, inv_hblk), hb = unit - seq * n_hblk;
+  const int b = div_by(seq, n_tokens, inv_tokens), t = seq - b * n_tokens;
   const int head = hb * 64 + 16 * wave + c16;
-  const float* po = a.parts + (int64_t)unit * a.ranges * (64 * kD) + ((wave * 32 + mt) * 64 + lane) * 4;
-  const float* ml = a.parts + (int64_t)a.split_units * a.ranges * (64 * kD) + ((int64_t)unit * a.ranges * 64 + 16 * wave + c16) * 2;
+  const float* po = parts + (int64_t)unit * ranges * (64 * kD) + ((wave * 32 + mt) * 64 + lane) * 4;
+  const float* ml = parts + (int64_t)split_units * ranges * (64 * kD) + ((int64_t)unit * ranges * 64 + 16 * wave + c16) * 2;
   float m[kMaxRanges], l[kMaxRanges];
   f32x4_t o[kMaxRanges];
 #pragma unroll
   for (int r = 0; r < kMaxRanges; r++) {
-    const int rr = r < a.ranges ? r : 0;
+    const int rr = r < ranges ? r : 0;
     m[r] = ml[rr * 128];
     l[r] = ml[rr * 128 + 1];
     o[r] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)rr * (64 * kD));
-    if (r >= a.ranges) m[r] = -__builtin_inff();
+    if (r >= ranges) m[r] = -__builtin_inff();
   }
-  const float sink = head < a.n_heads && a.sinks ? a.sinks[head] * 1.4426950408889634f : -__builtin_inff();
+  const float sink = head < n_heads && sinks ? sinks[head] * 1.4426950408889634f : -__builtin_inff();
   float m_all = sink;
 #pragma unroll
   for (int r = 0; r < kMaxRanges; r++) m_all = fmaxf(m_all, m[r]);
@@ -361,16 +407,16 @@ __global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(IndexedPrefi
     acc += o[r] * w;
   }
   const float f = den == 0.0f ? 0.0f : 1.0f / den;
-  if (head < a.n_heads)
-    *reinterpret_cast<f32x4_t*>(a.out + (int64_t)b * a.q_batch_stride + (int64_t)t * a.q_token_stride +
-                                (int64_t)head * a.q_head_stride + 16 * mt + 4 * kg) = acc * f;
+  if (head < n_heads)
+    *reinterpret_cast<f32x4_t*>(out + (int64_t)b * batch_stride + (int64_t)t * token_stride + (int64_t)head * head_stride +
+                                16 * mt + 4 * kg) = acc * f;
 }
 
-template <int QDT, bool CUT>
-int launch(const IndexedPrefillArgs& a, hipStream_t st) {
+template <int QDT, bool CUT, bool EAGER>
+int launch(const IndexedPrefillArgs& call, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT, EAGER>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) {
       mspr_set_error("indexed prefill attention: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
@@ -378,16 +424,26 @@ int launch(const IndexedPrefillArgs& a, hipStream_t st) {
     }
     attr_set = true;
   }
-  const int64_t units = (int64_t)a.batch * a.n_tokens * ((a.n_heads + 63) / 64);
+  IndexedPrefillArgs a = call;
+  const int n_hblk = (a.n_heads + 63) / 64;
+  const int64_t units = (int64_t)a.batch * a.n_tokens * n_hblk;
+  auto inverse = [](int n) -> uint32_t { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); };
+  a.inv_hblk = inverse(n_hblk);
+  a.inv_ranges = inverse(a.ranges);
+  const uint32_t inv_tokens = inverse(a.n_tokens);
   dim3 grid((unsigned)(units - a.split_units + a.split_units * a.ranges)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
-    indexed_prefill_kernel<QDT, CUT><<<grid, block, kLdsBytes, st>>>(a);
+    indexed_prefill_kernel<QDT, CUT, EAGER><<<grid, block, kLdsBytes, st>>>(a.win, a.idx, (int)units, a.n_tokens, inv_tokens, n_hblk, a.pos0,
+                                                                     a.window, (uint32_t)a.raw_cap, a.raw_start, a.max_win,
+                                                                     a.n_idx, a);
   }
   MSPR_CHECK_LAUNCH("indexed prefill attention");
   if constexpr (CUT) {
     MsprProfScope prof(MSPR_K_SPARSE_MERGE, st);
-    indexed_prefill_merge_kernel<<<dim3((unsigned)(a.split_units * 32)), block, 0, st>>>(a);
+    indexed_prefill_merge_kernel<<<dim3((unsigned)(a.split_units * 32)), block, 0, st>>>(
+        a.parts, a.sinks, a.split_units, a.ranges, a.n_heads, n_hblk, a.inv_hblk, a.n_tokens, inv_tokens, a.out,
+        a.q_batch_stride, a.q_token_stride, a.q_head_stride);
     MSPR_CHECK_LAUNCH("indexed prefill attention (merge)");
   }
   return MSPR_OK;
@@ -463,6 +519,11 @@ int mspr_launch_indexed_prefill(const IndexedPrefillArgs& call, void* workspace,
   while (a.ranges > 1 && workspace_bytes < part_bytes(a)) a.ranges--;
   if (a.ranges == 1) a.split_units = 0;
   if (a.split_units == 0) a.ranges = 1;
-  if (a.split_units > 0) return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, true>(a, st) : launch<MSPR_F16, true>(a, st);
-  return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, false>(a, st) : launch<MSPR_F16, false>(a, st);
+  const bool one_round = units <= 512;
+  auto pick = [&](auto cut, auto eager) {
+    constexpr bool kCut = decltype(cut)::value, kEager = decltype(eager)::value;
+    return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, kCut, kEager>(a, st) : launch<MSPR_F16, kCut, kEager>(a, st);
+  };
+  if (a.split_units > 0) return one_round ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{});
+  return one_round ? pick(std::false_type{}, std::true_type{}) : pick(std::false_type{}, std::false_type{});
 }
