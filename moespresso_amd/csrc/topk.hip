@@ -862,7 +862,7 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
 //    fewer than k, the list is made again from the lowest of the waves' prefixes: a wave samples stretches of the row, and of
 //    a row whose scores change along it the mean may say nothing (97 % of the wanted scores in one stretch: 1 row of 32768, k =
 //    2048, 42 us through the binning of all keys, now 13.7; 3844 of 8192, k = 512, 144 and 45). Where all parts are alike it is
-//    one row in some hundreds, which the launch then waits for: 3844 rows of 7961 Gaussian scores 33.5 us, now 29.
+//    one row in some hundreds, which the launch then waits for: 3844 rows of 7961 Gaussian scores 33.5 us, now 26.
 //  * 256 bins over [pivot, highest sample] hold the k-th key; a bin of up to 64 keys (nearly always the first one) is ranked
 //    directly, otherwise it becomes the span.
 //  * Selected rows set their bit in a bitmap of the row. Bits come out in row order, so nothing before has to keep it.
@@ -875,13 +875,30 @@ __global__ __launch_bounds__(THREADS) void topk_row_kernel(const float* __restri
 // chunk of 8400 tokens from position 0, whose first quarter sees too few rows: scores selected in 100, now 37).
 // What bounds it: a CU takes 2000 cycles to fetch a row of 32768 scores, and an instruction per key is 500 cycles of its vector
 // units: the blocked kernel above maps and moves every key (two LDS passes) and takes five digit passes, 16 rows of 32768,
-// k = 2048, 10.0 us, now 8.6. For many rows it is instructions: 3844 rows of 7961, k = 512, 57 us, now 28. (Keys read again
+// k = 2048, 10.0 us, now 7.7. For many rows it is instructions: 3844 rows of 7961, k = 512, 57 us, now 26. (Keys read again
 // from the L2 instead of from a copy of the row in LDS: 64 lines an instruction, 3 us more for 16 rows; neighbouring lanes on
 // neighbouring list entries: their bits meet in the same words, 1 us more.)
 constexpr int32_t kLowestKey = (int32_t)0x80000000u;
 constexpr int32_t kNegInfSigned = (int32_t)(kNegInfKey ^ 0x80000000u);
 
 __device__ __forceinline__ int32_t signed_key(int32_t bits) { return bits ^ (int32_t)((uint32_t)(bits >> 31) >> 1); }
+
+// mask = 16 mask + (bits k.w, k.z, k.y, k.x at or above the pivot): a comparison and an addition with carry a key. (From the
+// compiler it is four instructions and two wait states: a comparison's result may not be read by the next two. With the list
+// written two rows at a time, the sample read from the copy of the row, its end shifted instead of loaded again and only the
+// waves with a candidate ranking one: 16 rows of 32768 scores, k = 2048, 8.4 -> 7.7 us; 3844 of 7961, k = 512, 29.4 -> 26.2; 5 of
+// 19211, k = 1024, 7.2 -> 6.8; 1 of 4096, k = 512, 4.6 and 4.6.)
+__device__ __forceinline__ uint32_t shift_in_four(uint32_t mask, __attribute__((ext_vector_type(4))) int k, int32_t pivot) {
+  uint64_t c0, c1, c2, c3;
+  asm("v_cmp_le_i32_e64 %1, %9, %5\n\tv_cmp_le_i32_e64 %2, %9, %6\n\tv_cmp_le_i32_e64 %3, %9, %7\n\t"
+      "v_cmp_le_i32_e64 %4, %9, %8\n\t"
+      "v_addc_co_u32_e64 %0, vcc, %0, %0, %1\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %2\n\t"
+      "v_addc_co_u32_e64 %0, vcc, %0, %0, %3\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %4"
+      : "+v"(mask), "=&s"(c0), "=&s"(c1), "=&s"(c2), "=&s"(c3)
+      : "v"(k.w), "v"(k.z), "v"(k.y), "v"(k.x), "s"(pivot)
+      : "vcc");
+  return mask;
+}
 
 template <int P, int THREADS, int S>
 __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __restrict__ scores_all, int64_t score_stride,
@@ -913,12 +930,13 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   //      tie to a real row. (Rows start at any multiple of 4 bytes.)
   typedef __attribute__((ext_vector_type(4), aligned(4))) int i32x4_any_t;
   typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+  auto row_of = [&](int j, int e) { return 4 * (j * THREADS + tid) + e; };
   i32x4_t key[P];
-  const int last_whole = (n_rows - 4) & ~3;  // (n_rows is at least 4)
+  const int last_four = n_rows - 4;  // (n_rows is at least 4)
 #pragma unroll
   for (int j = 0; j < P; j++) {
-    const int r = 4 * (j * THREADS + tid);
-    key[j] = *reinterpret_cast<const i32x4_any_t*>(scores + (r < last_whole ? r : last_whole));
+    const int r = row_of(j, 0);
+    key[j] = *reinterpret_cast<const i32x4_any_t*>(scores + (r < last_four ? r : last_four));
   }
   if (tid < (int)kBins) hist[tid] = 0u;
   bits_above[tid] = 0u;
@@ -930,17 +948,18 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   }
 #pragma unroll
   for (int j = 0; j < P; j++) {
-    const int r = 4 * (j * THREADS + tid);
-    if (j == P - 1 || 4 * (j + 1) * THREADS > n_rows) {  // (uniform: pieces in front of the row's end are whole)
-      if (r + 3 >= n_rows) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) key[j][e] = r + e < n_rows ? __float_as_int(scores[r + e]) : -1;
-      }
+    const int r = row_of(j, 0);
+    if (4 * (j + 1) * THREADS > n_rows) {  // (uniform: pieces in front of the row's end are whole)
+      // the row's last four scores, shifted (loaded one by one, they held up everything behind them)
+      const int by = r - last_four;
+      i32x4_t k = key[j];
+      if (by > 0 && (by & 1)) k = i32x4_t{k.y, k.z, k.w, -1};
+      if (by > 0 && (by & 2)) k = i32x4_t{k.z, k.w, -1, -1};
+      if (by > 3) k = i32x4_t{-1, -1, -1, -1};
+      key[j] = k;
     }
+    *reinterpret_cast<i32x4_t*>(&stage[r]) = key[j];
   }
-
-#pragma unroll
-  for (int j = 0; j < P; j++) *reinterpret_cast<i32x4_t*>(&stage[4 * (j * THREADS + tid)]) = key[j];
 
   // ---- this wave's sample: lane l takes element l / P % 4 of pieces l + i of the P
   uint32_t sample[S];
@@ -949,10 +968,15 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   for (int i = 0; i < S; i++) {
     const int piece = (lane + i) % P, e = (lane / P) & 3;
     int32_t v = 0;
+    if constexpr (P > 2) {
+      v = stage[row_of(piece, e)];  // (its own copy: picked by comparison it is five instructions a piece)
+    } else {
 #pragma unroll
-    for (int j = 0; j < P; j++) {
-      const int32_t x = e & 2 ? (e & 1 ? key[j].w : key[j].z) : (e & 1 ? key[j].y : key[j].x);
-      v = piece == j ? x : v;
+      for (int j = 0; j < P; j++) {
+        const i32x4_t k = key[j];
+        const int32_t x = e & 2 ? (e & 1 ? k.w : k.z) : (e & 1 ? k.y : k.x);
+        v = piece == j ? x : v;
+      }
     }
     sample[i] = (uint32_t)signed_key(v) ^ 0x80000000u;
     high = umax(high, sample[i]);
@@ -1002,9 +1026,7 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     }
     uint32_t mask = 0u;
 #pragma unroll
-    for (int j = P - 1; j >= 0; j--)
-#pragma unroll
-      for (int e = 3; e >= 0; e--) mask = shift_in(mask, key[j][e] >= pivot);
+    for (int j = P - 1; j >= 0; j--) mask = shift_in_four(mask, key[j], pivot);
     const uint32_t cnt = (uint32_t)__popc(mask);
     const uint32_t incl = wave_prefix_sum(cnt);
     uint32_t base = 0u;
@@ -1012,10 +1034,20 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63);
     if (base + (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) <= (uint32_t)kCap) {
       uint16_t* at = list + base + incl - cnt;
-      while (mask) {
+      auto row_of_bit = [&](int i) { return (uint16_t)row_of(i >> 2, i & 3); };
+      while (mask) {  // (two at a time, where a thread has many; a last odd one is written twice)
         const int i = __builtin_ctz(mask);
         mask &= mask - 1u;
-        *at++ = (uint16_t)(4 * ((i >> 2) * THREADS + tid) + (i & 3));
+        if constexpr (P < 4) {
+          *at++ = row_of_bit(i);
+          continue;
+        }
+        const uint32_t another = mask != 0u ? 1u : 0u;
+        const int i2 = another ? __builtin_ctz(mask) : i;
+        at[0] = row_of_bit(i);
+        at[another] = row_of_bit(i2);
+        at += 2;
+        mask &= mask - 1u;
       }
     }
     __syncthreads();
@@ -1041,17 +1073,23 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
   // of the votes in `hist`, 1 << shift keys wide a bin: the bin with the k-th key, and how many keys it holds
   auto narrow = [&](int shift) -> uint32_t {
     __syncthreads();
-    if (wave == 0) {
-      const Pick pk = pick_bucket(hist, need, lane);
-      if (lane == 0) pick_box = pk;
+    Pick pk;
+    if constexpr (kW <= 4) {
+      pk = pick_bucket(hist, need, lane);  // (every wave for itself: handed on by one, it was a barrier and a read more)
+    } else {  // (four waves a SIMD wait for each other's instructions longer than that)
+      if (wave == 0) {
+        pk = pick_bucket(hist, need, lane);
+        if (lane == 0) pick_box = pk;
+      }
+      __syncthreads();
+      pk = Pick{uniform(pick_box.digit), uniform(pick_box.need), uniform(pick_box.live)};
     }
-    __syncthreads();
-    const uint32_t bin = uniform(pick_box.digit);
-    need = uniform(pick_box.need);
+    const uint32_t bin = pk.digit;
+    need = pk.need;
     lo = (int32_t)((uint32_t)lo + (bin << shift));
     const uint32_t rest = limit - (bin << shift), width = bin == kBins - 1u ? 0xFFFFFFFFu : (1u << shift) - 1u;
     limit = rest < width ? rest : width;
-    return uniform(pick_box.live);
+    return pk.live;
   };
   auto candidate = [&](int32_t k) {
     const bool in = k >= lo && (uint32_t)k - (uint32_t)lo <= limit;
@@ -1065,7 +1103,7 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
     constexpr int kAtOnce = THREADS / 16;
 #pragma unroll
     for (int c0 = 0; c0 < 64; c0 += kAtOnce) {
-      if (c0 > 0 && (uint32_t)c0 >= held) break;  // uniform
+      if ((uint32_t)(c0 + 4 * wave) >= held) break;  // (the wave's four)
       const int c = c0 + (tid >> 4);
       const uint32_t mine = near[c];
       const u32x4_t o = *reinterpret_cast<const u32x4_t*>(&near[4 * (lane & 15)]);
@@ -1145,13 +1183,13 @@ __global__ __launch_bounds__(THREADS) void topk_sampled_kernel(const float* __re
         rank_candidates(held);
         break;
       }
-      if (held > 512u && held > half) {
+      if (held > 512u && held > half) {  // keys that meet in one bin again and again
         found = false;
         break;
       }
       span = limit;
-  // (not found: keys that meet in one bin again and again)
       half = held / 2u;
+      __syncthreads();  // every wave has read the counters
       if (tid < (int)kBins) hist[tid] = 0u;
       __syncthreads();
     }
@@ -1316,9 +1354,9 @@ int mspr_launch_topk(const float* scores, int64_t score_stride, int batch, int64
   MsprProfScope prof(MSPR_K_TOPK, st);
   // Rows of more than 2048 scores of which at most three eighths (past 4096: less than a half) are wanted are selected from the
   // keys above a sampled pivot, where those fit its list: 512 threads a row, 256 where many rows share the CUs, 1024 for what
-  // only they can hold. us, the other kernels and this one: 1 row of 4096 scores, k = 512, 5.3 and 4.7; of 8192, k = 2048, 7.2
-  // and 6.5; 5 of 19211, k = 1024, 9.3 and 7.2; 16 of 32768, k = 2048, 10.0 and 8.6; 517 of 7000, k = 512, 10.5 and 7.5; 3844 of
-  // 3000 24.5 and 18.4, of 7961 57 and 28; 600 of 16384 27 and 20. At the lines: 4096 scores 1 row, k = 1500, 5.7 and 5.4, k =
+  // only they can hold. us, the other kernels and this one: 1 row of 4096 scores, k = 512, 5.3 and 4.6; of 8192, k = 2048, 7.2
+  // and 6.1; 5 of 19211, k = 1024, 9.3 and 6.8; 16 of 32768, k = 2048, 10.0 and 7.7; 517 of 7000, k = 512, 10.5 and 7.0; 3844 of
+  // 3000 24.5 and 18.2, of 7961 57 and 26; 600 of 16384 27 and 19. At the lines: 4096 scores 1 row, k = 1500, 5.7 and 5.4, k =
   // 2048 5.5 and 6.3; 2100 scores, k = 700, 1 row 4.9 and 5.1, 517 7.0 and 6.6; 1500 scores, k = 512, 4.5 and 4.9, 3844 rows 16.2
   // and 16.4; 8192 scores, k = 3000, 7.5 and 7.3, k = 4000 7.6 and 9.1. 384 rows of 4096, k = 512: 512 threads 6.4, 256 6.0; 256
   // rows 5.4 and 5.6.
