@@ -72,18 +72,27 @@ __device__ __forceinline__ void codes4_to_h(uint32_t w, h2_t& lo, h2_t& hi) {
   }
 }
 
+// What the split kernel needs behind its first loads.
+struct Q8Rest {
+  const void* q;
+  const uint8_t* kbi;
+  const uint8_t* vbi;
+  float* ws_o;
+  float* ws_ml;
+  float scale_log2;
+  int n_splits, rep;
+};
+
 // (What the first loads' addresses take comes first: fourteen words of plain arguments are in registers when a wave starts, the
-// rest is loaded under those requests. With one struct for both kernels, and the merge's head taken apart by a division: one
-// sequence of 8192 keys, appended and attended, 16.0 us of device time, now 15.0; eight of 37000 keys 64.9, now 63.7.)
+// rest is loaded under those requests. heads_rows: rows allocated per (batch, kv head), KV heads from bit 48 on; keys: n_keys,
+// keys per range from bit 32 on.)
 template <int FMT, int QDT, int SDT>
 __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const uint8_t* k_codes, const uint8_t* v_codes,
                                                                           const uint8_t* ksc, const uint8_t* vsc,
-                                                                          int64_t kv_rows, int n_keys, int keys_per_split,
-                                                                          int n_kv_heads, const void* q,
-                                                                          const uint8_t* kbi, const uint8_t* vbi,
-                                                                          float* ws_o, float* ws_ml, float scale_log2,
-                                                                          int n_splits, int rep) {
+                                                                          uint64_t heads_rows, uint64_t keys, Q8Rest a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int64_t kv_rows = (int64_t)(heads_rows & 0xFFFFFFFFFFFFull);
+  const int n_kv_heads = (int)(heads_rows >> 48), n_keys = (int)(uint32_t)keys, keys_per_split = (int)(keys >> 32);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -145,10 +154,10 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
         kr.s[u] = *reinterpret_cast<const uint32_t*>(ksc + ((kv_row0 + key) * 8 + 2 * g) * 2);
       } else if constexpr (SDT == MSPR_F32) {
         kr.s[u] = *reinterpret_cast<const uint32_t*>(ksc + ((kv_row0 + key) * 4 + g) * 4);
-        kr.bz[u] = *reinterpret_cast<const uint32_t*>(kbi + ((kv_row0 + key) * 4 + g) * 4);
+        kr.bz[u] = *reinterpret_cast<const uint32_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 4);
       } else {
         kr.s[u] = *reinterpret_cast<const uint16_t*>(ksc + ((kv_row0 + key) * 4 + g) * 2);
-        kr.bz[u] = *reinterpret_cast<const uint16_t*>(kbi + ((kv_row0 + key) * 4 + g) * 2);
+        kr.bz[u] = *reinterpret_cast<const uint16_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 2);
       }
     }
   };
@@ -166,10 +175,10 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
         vr.s[1] = sv.y;
       } else if constexpr (SDT == MSPR_F32) {
         vr.s[i] = *reinterpret_cast<const uint32_t*>(vsc + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
-        vr.bz[i] = *reinterpret_cast<const uint32_t*>(vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
+        vr.bz[i] = *reinterpret_cast<const uint32_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
       } else {
         vr.s[i] = *reinterpret_cast<const uint16_t*>(vsc + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
-        vr.bz[i] = *reinterpret_cast<const uint16_t*>(vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
+        vr.bz[i] = *reinterpret_cast<const uint16_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
       }
     }
   };
@@ -200,11 +209,11 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
   //      scale * log2(e) and rounded to float16
   u32x4_t qf[8];
   {
-    const bool live = n < rep;
-    const int64_t qoff = (((int64_t)b * n_kv_heads + kvh) * rep + (live ? n : 0)) * kD + 64 * g;
+    const bool live = n < a.rep;
+    const int64_t qoff = (((int64_t)b * n_kv_heads + kvh) * a.rep + (live ? n : 0)) * kD + 64 * g;
     float v[8][8];
     if constexpr (QDT == MSPR_F32) {
-      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(q) + qoff);
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff);
       f32x4_t raw[16];
 #pragma unroll
       for (int j = 0; j < 16; j++) raw[j] = p[j];
@@ -213,7 +222,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
 #pragma unroll
         for (int j = 0; j < 8; j++) v[s][j] = raw[2 * s + (j >> 2)][j & 3];
     } else {
-      const u32x4_t* p = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(q) + qoff);
+      const u32x4_t* p = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(a.q) + qoff);
       u32x4_t raw[8];
 #pragma unroll
       for (int s = 0; s < 8; s++) raw[s] = p[s];
@@ -235,7 +244,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
       u32x4_t f;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        h2_t h = {(_Float16)(live ? v[s][2 * j] * scale_log2 : 0.0f), (_Float16)(live ? v[s][2 * j + 1] * scale_log2 : 0.0f)};
+        h2_t h = {(_Float16)(live ? v[s][2 * j] * a.scale_log2 : 0.0f), (_Float16)(live ? v[s][2 * j + 1] * a.scale_log2 : 0.0f)};
         f[j] = h2_bits(h);
       }
       qf[s] = f;
@@ -403,8 +412,8 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
     mw[w] = __builtin_amdgcn_exp2f(mw[w] - m_safe);
     l_all += lw[w] * mw[w];
   }
-  const int64_t part = (((int64_t)b * n_kv_heads + kvh) * n_splits + sp);
-  float* po = ws_o + part * (16 * kD);
+  const int64_t part = (((int64_t)b * n_kv_heads + kvh) * a.n_splits + sp);
+  float* po = a.ws_o + part * (16 * kD);
   // every wave reduces its share of the 16 M-tiles: dims 16mt + 4g + i of head n
 #pragma unroll
   for (int q4 = 0; q4 < 16 / kQ8Waves; q4++) {
@@ -415,10 +424,10 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
       f32x4_t v = *reinterpret_cast<const f32x4_t*>(xo + ((w * 16 + mt) * 64 + lane) * 4);
       acc += v * mw[w];
     }
-    if (n < rep) *reinterpret_cast<f32x4_t*>(po + n * kD + 16 * mt + 4 * g) = acc;  // (columns past the real heads are padding)
+    if (n < a.rep) *reinterpret_cast<f32x4_t*>(po + n * kD + 16 * mt + 4 * g) = acc;  // (columns past the real heads are padding)
   }
   if (wave == 0 && g == 0) {
-    float* pml = ws_ml + part * 32;
+    float* pml = a.ws_ml + part * 32;
     pml[n * 2] = m_all;
     pml[n * 2 + 1] = l_all;
   }
@@ -427,32 +436,35 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
 // Merge of the per-range partials: one workgroup per (batch, query head); 64 lanes cover the 256
 // dims four at a time, the 16 waves each take every 16th range and fetch up to 16 of them in one go
 // (one memory round trip for up to 256 ranges), the wave results are combined in LDS.
+// (Its arguments come in the struct: as plain ones, in registers, they take 0.6 us off the device's time, but 32 bytes of arguments
+// for the call's last launch leave the host 0.3 to 0.6 us behind, and one sequence's step is the host's: appended and attended
+// with 8192 keys 17.3 and 17.9 us, where the host keeps up 15.6 and 15.0. With both kernels on the struct and the merge's head
+// taken apart by a division, 16.0.)
 constexpr int kMergeWaves = 16;
 template <int ODT>
-__global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(const float* ws_o, const float* ws_ml, void* out,
-                                                                          int n_splits, int rep) {
+__global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Args a) {
   __shared__ float xm[kMergeWaves], xl[kMergeWaves];
   __shared__ __attribute__((aligned(16))) float xo[kMergeWaves][kD];
   const int lane = threadIdx.x & 63;
   const int sg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t bh = blockIdx.x;  // KV head of a sequence
   const int hn = blockIdx.y;      // query head of its group
-  const int64_t part0 = bh * n_splits;
-  const float* ml = ws_ml + part0 * 32 + hn * 2;
-  const float* po = ws_o + part0 * (16 * kD) + hn * kD + 4 * lane;
+  const int64_t part0 = bh * a.n_splits;
+  const float* ml = a.ws_ml + part0 * 32 + hn * 2;
+  const float* po = a.ws_o + part0 * (16 * kD) + hn * kD + 4 * lane;
   constexpr int kChunk = 16;
   float m_run = -__builtin_inff(), l = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = sg; s0 < n_splits; s0 += kMergeWaves * kChunk) {
+  for (int s0 = sg; s0 < a.n_splits; s0 += kMergeWaves * kChunk) {
     // The statistics of range j by lane j, in one load, whose weight is then taken once: with scalar loads of them each range's
     // were waited for in front of the next range's row, and every lane took all sixteen exponentials.
     const int mine = s0 + kMergeWaves * (lane % kChunk);
     f32x2_t stat = {-__builtin_inff(), 0.0f};
-    if (mine < n_splits) stat = *reinterpret_cast<const f32x2_t*>(ml + (int64_t)mine * 32);
+    if (mine < a.n_splits) stat = *reinterpret_cast<const f32x2_t*>(ml + (int64_t)mine * 32);
     f32x4_t ov[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; j++)  // (wave-uniform: ranges past the end cost no load)
-      if (s0 + kMergeWaves * j < n_splits)
+      if (s0 + kMergeWaves * j < a.n_splits)
         ov[j] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)(s0 + kMergeWaves * j) * (16 * kD));
     static_assert(kChunk == 16, "reduced over rows of sixteen lanes");
     float m_new = stat.x;
@@ -471,7 +483,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(const
     o = o * alpha;
 #pragma unroll
     for (int j = 0; j < kChunk; j++)
-      if (s0 + kMergeWaves * j < n_splits) o += ov[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+      if (s0 + kMergeWaves * j < a.n_splits) o += ov[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
     m_run = m_new;
   }
   if (lane == 0) {
@@ -494,16 +506,16 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(const
     o_all += *reinterpret_cast<const f32x4_t*>(&xo[w][4 * lane]) * wt;
   }
   const float inv = l_all == 0.0f ? 0.0f : 1.0f / l_all;
-  const int64_t ooff = (bh * rep + hn) * kD + 4 * lane;
+  const int64_t ooff = (bh * a.rep + hn) * kD + 4 * lane;
   if constexpr (ODT == MSPR_F32) {
-    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + ooff) = o_all * inv;
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = o_all * inv;
   } else {
     uint16_t h[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
       h[i] = ODT == MSPR_BF16 ? f32_to_bf16_bits(o_all[i] * inv) : f32_to_f16_bits(o_all[i] * inv);
     u32x2_t pk = {(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(out) + ooff) = pk;
+    *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(a.out) + ooff) = pk;
   }
 }
 
@@ -551,15 +563,16 @@ int q8_launch(Q8Args a, hipStream_t st) {
     MsprProfScope prof(MSPR_K_Q8_DECODE, st);
     q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(
         reinterpret_cast<const uint8_t*>(a.k_codes), reinterpret_cast<const uint8_t*>(a.v_codes),
-        reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales), a.kv_rows, (int)a.n_keys,
-        a.keys_per_split, a.n_kv_heads, a.q, reinterpret_cast<const uint8_t*>(a.k_biases),
-        reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml, a.scale_log2, a.n_splits, a.rep);
+        reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales),
+        (uint64_t)a.n_kv_heads << 48 | (uint64_t)a.kv_rows, (uint64_t)a.keys_per_split << 32 | (uint64_t)a.n_keys,
+        Q8Rest{a.q, reinterpret_cast<const uint8_t*>(a.k_biases), reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml,
+               a.scale_log2, a.n_splits, a.rep});
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (split)");
   {
     MsprProfScope prof(MSPR_K_Q8_MERGE, st);
     q8_decode_merge_kernel<QDT><<<dim3((unsigned)(a.batch * a.n_kv_heads), (unsigned)a.rep), dim3(64 * kMergeWaves), 0, st>>>(
-        a.ws_o, a.ws_ml, a.out, a.n_splits, a.rep);
+        a);
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (merge)");
   return MSPR_OK;
