@@ -27,8 +27,6 @@
 #include "prefill_attn.h"
 #include "profile.h"
 
-#include <type_traits>
-
 namespace {
 
 constexpr int kTile = 32;
@@ -45,6 +43,7 @@ constexpr int kQSteps = kD / 32;
 constexpr int kOutPitch = 256 + 4;  // floats between rows of the output staging: 16 heads' stores fall on 16 bank groups
 static_assert(4 * 16 * kOutPitch * 4 <= 2 * kTileBytes, "output staging lies in the tile buffers");
 constexpr int kMaxRanges = 8;
+constexpr int kRound = 512;  // units at work at once: two to a CU
 constexpr int kAheadK = 8, kAheadV = 6;  // operand reads in flight (6/4 measures the same, 10/8 9 % slower)
 
 __device__ __attribute__((aligned(16))) const unsigned char g_prefill_zero_row[kD * 2] = {0};
@@ -76,13 +75,9 @@ __device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
 }
 
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
-// EAGER: the queries are requested before the ids are looked at, not behind. That takes a trip to memory off a workgroup's
-// start, and pays where all start at once and none follows (60 tokens behind 28000: 34.9 us, and 34.2 with the requests
-// ahead; 255 tokens 46.1 and 45.2); with more than a round of 512 units they crowd out the other workgroup's rows (1536 tokens
-// 166.6 and 169.6).
 // (Plain arguments first: what the first copies and the ids take comes in registers with the wave, and the struct is loaded
 // meanwhile.)
-template <int QDT, bool CUT, bool EAGER>
+template <int QDT, bool CUT>
 __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void* win, const int32_t* idx, int units,
                                                                       int n_tokens, uint32_t inv_tokens, int n_hblk,
                                                                       uint32_t pos0, uint32_t window, uint32_t n_raw,
@@ -156,10 +151,15 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   if (t_begin < wt) copy_rows(t_begin, win_base, window_row(t_begin));
 
   // ---- the first ids of a thread, which go to LDS below
-  constexpr int kEager = EAGER ? 2 : 0;
+  // In a single round of units, cut into ranges, the queries are requested before the ids are looked at, not behind. That takes a
+  // trip to memory off a workgroup's start, and pays where all start at once and none follows (60 tokens behind 28000: 34.9 us, and
+  // 34.2 with the requests ahead); with more than a round they crowd out the other workgroup's rows (1536 tokens 166.6 and 169.6),
+  // and the choice itself costs whole units 0.5 %.
+  constexpr int kEager = 2;
+  const bool ahead = CUT && units <= kRound;  // uniform
   const int32_t* src = idx + (int64_t)seq * n_idx;
-  int eager[EAGER ? kEager : 1] = {};
-  if (EAGER && n_idx > 0) {
+  int eager[kEager] = {};
+  if (ahead && n_idx > 0) {
 #pragma unroll
     for (int j = 0; j < kEager; j++) {
       const int i = tid + j * kThreads;
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   __syncthreads();
 
   // ---- ids to LDS, position of the first one that ends the walk
-  auto stage_ids = [&]() {
+  auto stage_ids = [&](int done) {
     int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
     if (visible > a.n_pool) visible = a.n_pool;
     int found = n_idx;
@@ -180,11 +180,11 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
     };
 #pragma unroll
     for (int j = 0; j < kEager; j++)
-      if (tid + j * kThreads < n_idx) look(tid + j * kThreads, eager[j]);
-    for (int i = tid + kEager * kThreads; i < n_idx; i += kThreads) look(i, src[i]);
+      if (j < done && tid + j * kThreads < n_idx) look(tid + j * kThreads, eager[j]);
+    for (int i = tid + done * kThreads; i < n_idx; i += kThreads) look(i, src[i]);
     if (found < n_idx) atomicMin(stop_sh, found);
   };
-  if constexpr (!EAGER) stage_ids();
+  if (!ahead) stage_ids(0);
 
   // ---- query operand: lane (head c16, kg) holds q[head][32 ks + 8 kg .. +7], zero rows past n_heads
   const int head = hb * 64 + 16 * wave + c16;
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
       raw[2 * ks + 1] = p[1];
     }
   }
-  if constexpr (EAGER) stage_ids();
+  if (ahead) stage_ids(kEager);
 #pragma unroll
   for (int ks = 0; ks < kQSteps; ks++) {
     if constexpr (QDT != MSPR_F16) {
@@ -412,11 +412,11 @@ __global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(const float*
                                 16 * mt + 4 * kg) = acc * f;
 }
 
-template <int QDT, bool CUT, bool EAGER>
+template <int QDT, bool CUT>
 int launch(const IndexedPrefillArgs& call, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT, EAGER>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) {
       mspr_set_error("indexed prefill attention: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
@@ -434,7 +434,7 @@ int launch(const IndexedPrefillArgs& call, hipStream_t st) {
   dim3 grid((unsigned)(units - a.split_units + a.split_units * a.ranges)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
-    indexed_prefill_kernel<QDT, CUT, EAGER><<<grid, block, kLdsBytes, st>>>(a.win, a.idx, (int)units, a.n_tokens, inv_tokens, n_hblk, a.pos0,
+    indexed_prefill_kernel<QDT, CUT><<<grid, block, kLdsBytes, st>>>(a.win, a.idx, (int)units, a.n_tokens, inv_tokens, n_hblk, a.pos0,
                                                                      a.window, (uint32_t)a.raw_cap, a.raw_start, a.max_win,
                                                                      a.n_idx, a);
   }
@@ -519,11 +519,6 @@ int mspr_launch_indexed_prefill(const IndexedPrefillArgs& call, void* workspace,
   while (a.ranges > 1 && workspace_bytes < part_bytes(a)) a.ranges--;
   if (a.ranges == 1) a.split_units = 0;
   if (a.split_units == 0) a.ranges = 1;
-  const bool one_round = units <= 512;
-  auto pick = [&](auto cut, auto eager) {
-    constexpr bool kCut = decltype(cut)::value, kEager = decltype(eager)::value;
-    return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, kCut, kEager>(a, st) : launch<MSPR_F16, kCut, kEager>(a, st);
-  };
-  if (a.split_units > 0) return one_round ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{});
-  return one_round ? pick(std::false_type{}, std::true_type{}) : pick(std::false_type{}, std::false_type{});
+  if (a.split_units > 0) return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, true>(a, st) : launch<MSPR_F16, true>(a, st);
+  return a.q_dtype == MSPR_F32 ? launch<MSPR_F32, false>(a, st) : launch<MSPR_F16, false>(a, st);
 }

@@ -1,5 +1,5 @@
-"""The prefill attention kernel's id staging: two rounds of 256 ids are requested ahead of the queries in calls of up to 512
-units, none in longer ones."""
+"""The prefill attention kernel's id staging: two rounds of 256 ids are requested ahead of the queries where a single
+round of units is cut into ranges, none elsewhere."""
 
 import numpy as np
 import pytest
