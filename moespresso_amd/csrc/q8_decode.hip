@@ -559,12 +559,14 @@ int q8_launch(Q8Args a, hipStream_t st) {
     attr_set = true;
   }
   dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv_heads, (unsigned)a.batch), block(64 * kQ8Waves);
+  // (the distance of heads means nothing for a single one, whose tensor may name any)
+  const uint64_t head_rows = a.batch == 1 && a.n_kv_heads == 1 ? (uint64_t)a.n_keys : (uint64_t)a.kv_rows;
   {
     MsprProfScope prof(MSPR_K_Q8_DECODE, st);
     q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(
         reinterpret_cast<const uint8_t*>(a.k_codes), reinterpret_cast<const uint8_t*>(a.v_codes),
         reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales),
-        (uint64_t)a.n_kv_heads << 48 | (uint64_t)a.kv_rows, (uint64_t)a.keys_per_split << 32 | (uint64_t)a.n_keys,
+        (uint64_t)a.n_kv_heads << 48 | head_rows, (uint64_t)a.keys_per_split << 32 | (uint64_t)a.n_keys,
         Q8Rest{a.q, reinterpret_cast<const uint8_t*>(a.k_biases), reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml,
                a.scale_log2, a.n_splits, a.rep});
   }
