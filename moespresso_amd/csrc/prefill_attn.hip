@@ -76,7 +76,8 @@ __device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
 
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
 // (Plain arguments first: what the first copies and the ids take comes in registers with the wave, and the struct is loaded
-// meanwhile.)
+// meanwhile: it was loaded in three dependent steps with three software divisions between. One token behind 28000 rows 22.1 ->
+// 21.6 us with its merge, 255 tokens 43.8 -> 43.5; full rounds, which power bounds, are as they were.)
 template <int QDT, bool CUT>
 __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void* win, const int32_t* idx, int units,
                                                                       int n_tokens, uint32_t inv_tokens, int n_hblk,
