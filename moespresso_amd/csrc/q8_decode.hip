@@ -84,15 +84,14 @@ struct Q8Rest {
 };
 
 // (What the first loads' addresses take comes first: fourteen words of plain arguments are in registers when a wave starts, the
-// rest is loaded under those requests. heads_rows: rows allocated per (batch, kv head), KV heads from bit 48 on; keys: n_keys,
-// keys per range from bit 32 on.)
+// rest is loaded under those requests. Each is a word or two of its own: KV heads above the bits of kv_rows lost all but sixteen of
+// theirs, and 65536 heads of two sequences read one another's rows.)
 template <int FMT, int QDT, int SDT>
 __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const uint8_t* k_codes, const uint8_t* v_codes,
                                                                           const uint8_t* ksc, const uint8_t* vsc,
-                                                                          uint64_t heads_rows, uint64_t keys, Q8Rest a) {
+                                                                          int64_t kv_rows, int n_kv_heads, int n_keys,
+                                                                          int keys_per_split, Q8Rest a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int64_t kv_rows = (int64_t)(heads_rows & 0xFFFFFFFFFFFFull);
-  const int n_kv_heads = (int)(heads_rows >> 48), n_keys = (int)(uint32_t)keys, keys_per_split = (int)(keys >> 32);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -559,14 +558,12 @@ int q8_launch(Q8Args a, hipStream_t st) {
     attr_set = true;
   }
   dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv_heads, (unsigned)a.batch), block(64 * kQ8Waves);
-  // (the distance of heads means nothing for a single one, whose tensor may name any)
-  const uint64_t head_rows = a.batch == 1 && a.n_kv_heads == 1 ? (uint64_t)a.n_keys : (uint64_t)a.kv_rows;
   {
     MsprProfScope prof(MSPR_K_Q8_DECODE, st);
     q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(
         reinterpret_cast<const uint8_t*>(a.k_codes), reinterpret_cast<const uint8_t*>(a.v_codes),
         reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales),
-        (uint64_t)a.n_kv_heads << 48 | head_rows, (uint64_t)a.keys_per_split << 32 | (uint64_t)a.n_keys,
+        a.kv_rows, a.n_kv_heads, (int)a.n_keys, a.keys_per_split,
         Q8Rest{a.q, reinterpret_cast<const uint8_t*>(a.k_biases), reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml,
                a.scale_log2, a.n_splits, a.rep});
   }

@@ -1,4 +1,4 @@
-"""The 8-bit decode's distance between heads: many of it past the cache's rows, and any at all for a single head."""
+"""The 8-bit decode's KV heads: how far apart they lie (any distance at all for a single one), and as many as a grid takes."""
 
 import pytest
 import torch
@@ -28,3 +28,23 @@ def test_rows_between_heads(batch, heads, n_keys, kv_rows):
     got = run(codes[0], scales[0], codes[1], scales[1], kv_rows)
     dense = [t[:, :, :n_keys].contiguous() for t in (codes[0], scales[0], codes[1], scales[1])]
     assert torch.equal(got, run(*dense, n_keys))
+
+
+def test_as_many_heads_as_a_grid_takes():
+    """65536 KV heads of two sequences: the number is a word of its own among the kernel's arguments. With one key the softmax
+    is 1, so the output is that key's value row in the cache's format."""
+    from moespresso_amd import _lib
+
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    batch, heads = 2, 65536
+    codes = [torch.randint(-127, 128, (batch, heads, 1, 256), device="cuda", generator=gen).to(torch.int8) for _ in range(2)]
+    scales = [(torch.rand((batch, heads, 1, 8), device="cuda", generator=gen) / 50).half() for _ in range(2)]
+    q = torch.randn((batch, heads, 256), device="cuda", generator=gen)
+    need = _lib.lib().mspr_sdpa_decode_q8_workspace_bytes(batch, heads, 1)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(q)
+    _lib.check(_lib.lib().mspr_sdpa_decode_q8_0(
+        _lib.ptr(q), _lib.DTYPE_CODE[q.dtype], _lib.ptr(codes[0]), _lib.ptr(scales[0]), _lib.ptr(codes[1]), _lib.ptr(scales[1]), batch,
+        heads, heads, 256, 1, 1, 256 ** -0.5, _lib.ptr(out), _lib.ptr(ws), need, _lib.stream_ptr()), "q8_0")
+    want = (codes[1].half().reshape(batch, heads, 8, 32) * scales[1].reshape(batch, heads, 8, 1)).reshape(batch, heads, 256)
+    assert torch.equal(out, want.float())
