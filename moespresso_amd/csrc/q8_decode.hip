@@ -446,8 +446,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Arg
   __shared__ __attribute__((aligned(16))) float xo[kMergeWaves][kD];
   const int lane = threadIdx.x & 63;
   const int sg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t bh = blockIdx.x;  // KV head of a sequence
-  const int hn = blockIdx.y;      // query head of its group
+  const int64_t bh = (int64_t)blockIdx.z * a.n_kv_heads + blockIdx.x;  // KV head of a sequence
+  const int hn = blockIdx.y;                                           // query head of its group
   const int64_t part0 = bh * a.n_splits;
   const float* ml = a.ws_ml + part0 * 32 + hn * 2;
   const float* po = a.ws_o + part0 * (16 * kD) + hn * kD + 4 * lane;
@@ -570,8 +570,9 @@ int q8_launch(Q8Args a, hipStream_t st) {
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (split)");
   {
     MsprProfScope prof(MSPR_K_Q8_MERGE, st);
-    q8_decode_merge_kernel<QDT><<<dim3((unsigned)(a.batch * a.n_kv_heads), (unsigned)a.rep), dim3(64 * kMergeWaves), 0, st>>>(
-        a);
+    // (sequences and heads apart, as in the split's grid: 4 million of them are more threads than one grid dimension takes)
+    const dim3 mgrid((unsigned)a.n_kv_heads, (unsigned)a.rep, (unsigned)a.batch);
+    q8_decode_merge_kernel<QDT><<<mgrid, dim3(64 * kMergeWaves), 0, st>>>(a);
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (merge)");
   return MSPR_OK;
