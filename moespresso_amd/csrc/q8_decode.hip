@@ -80,17 +80,20 @@ struct Q8Rest {
   float* ws_o;
   float* ws_ml;
   float scale_log2;
-  int n_splits, rep;
+  int n_splits;
 };
 
 // (What the first loads' addresses take comes first: fourteen words of plain arguments are in registers when a wave starts, the
-// rest is loaded under those requests. Each is a word or two of its own: KV heads above the bits of kv_rows lost all but sixteen of
-// theirs, and 65536 heads of two sequences read one another's rows.)
+// rest is loaded under those requests. Each is a word or two of its own: KV heads above the bits of kv_rows lost all but sixteen
+// of theirs, and 65536 heads of two sequences read one another's rows. Q8Rest has no words to spare behind its last: three
+// words are loaded as four, and the register of the fourth, given to an address at once, made that address wait for the load.
+// Without it, and with the affine form's biases behind the codes and scales, both of the split and merge: one sequence of 8191
+// affine keys with its append 15.4 -> 15.0 us of the device's time, eight of 37000 Q8_0 keys 63.3 -> 63.0.)
 template <int FMT, int QDT, int SDT>
 __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const uint8_t* k_codes, const uint8_t* v_codes,
                                                                           const uint8_t* ksc, const uint8_t* vsc,
                                                                           int64_t kv_rows, int n_kv_heads, int n_keys,
-                                                                          int keys_per_split, Q8Rest a) {
+                                                                          int keys_per_split, int rep, Q8Rest a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -153,10 +156,19 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
         kr.s[u] = *reinterpret_cast<const uint32_t*>(ksc + ((kv_row0 + key) * 8 + 2 * g) * 2);
       } else if constexpr (SDT == MSPR_F32) {
         kr.s[u] = *reinterpret_cast<const uint32_t*>(ksc + ((kv_row0 + key) * 4 + g) * 4);
-        kr.bz[u] = *reinterpret_cast<const uint32_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 4);
       } else {
         kr.s[u] = *reinterpret_cast<const uint16_t*>(ksc + ((kv_row0 + key) * 4 + g) * 2);
-        kr.bz[u] = *reinterpret_cast<const uint16_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 2);
+      }
+    }
+  };
+  auto load_k_biases = [&](int64_t key0) {
+    if constexpr (FMT == kFmtAffine) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        int64_t key = key0 + 16 * u + n;
+        if (key >= N) key = N - 1;
+        if constexpr (SDT == MSPR_F32) kr.bz[u] = *reinterpret_cast<const uint32_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 4);
+        else kr.bz[u] = *reinterpret_cast<const uint16_t*>(a.kbi + ((kv_row0 + key) * 4 + g) * 2);
       }
     }
   };
@@ -174,10 +186,19 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
         vr.s[1] = sv.y;
       } else if constexpr (SDT == MSPR_F32) {
         vr.s[i] = *reinterpret_cast<const uint32_t*>(vsc + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
-        vr.bz[i] = *reinterpret_cast<const uint32_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
       } else {
         vr.s[i] = *reinterpret_cast<const uint16_t*>(vsc + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
-        vr.bz[i] = *reinterpret_cast<const uint16_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
+      }
+    }
+  };
+  auto load_v_biases = [&](int64_t key0) {
+    if constexpr (FMT == kFmtAffine) {
+#pragma unroll
+      for (int i = 0; i < kVRows; i++) {
+        int64_t key = key0 + 64 / kVLanes * i + vrow;
+        if (key >= N) key = N - 1;
+        if constexpr (SDT == MSPR_F32) vr.bz[i] = *reinterpret_cast<const uint32_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 4);
+        else vr.bz[i] = *reinterpret_cast<const uint16_t*>(a.vbi + ((kv_row0 + key) * 4 + (vpc >> 1)) * 2);
       }
     }
   };
@@ -200,6 +221,9 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
   if (wave < n_tiles) {
     load_k(k0 + (int64_t)wave * kTileKeys);
     load_v(k0 + (int64_t)wave * kTileKeys);
+    __builtin_amdgcn_sched_barrier(0);  // (the biases' addresses are in the struct, which is still on its way)
+    load_k_biases(k0 + (int64_t)wave * kTileKeys);
+    load_v_biases(k0 + (int64_t)wave * kTileKeys);
   }
   __builtin_amdgcn_sched_barrier(0);  // the first tile is on its way before the query is fetched: one memory
                                       // round trip in front of the first MFMA instead of two
@@ -208,8 +232,8 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
   //      scale * log2(e) and rounded to float16
   u32x4_t qf[8];
   {
-    const bool live = n < a.rep;
-    const int64_t qoff = (((int64_t)b * n_kv_heads + kvh) * a.rep + (live ? n : 0)) * kD + 64 * g;
+    const bool live = n < rep;
+    const int64_t qoff = (((int64_t)b * n_kv_heads + kvh) * rep + (live ? n : 0)) * kD + 64 * g;
     float v[8][8];
     if constexpr (QDT == MSPR_F32) {
       const f32x4_t* p = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.q) + qoff);
@@ -293,6 +317,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
       sacc[u] = acc;
     }
     load_k(next_key0);
+    load_k_biases(next_key0);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- online softmax (log2 domain); lane (n, g) holds keys 16u + 4g + i of the tile
@@ -365,6 +390,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
     }
 
     load_v(next_key0);
+    load_v_biases(next_key0);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- O^T += V^T . P^T (the V tile was written by this wave only: LDS operations of one wave
@@ -423,7 +449,7 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
       f32x4_t v = *reinterpret_cast<const f32x4_t*>(xo + ((w * 16 + mt) * 64 + lane) * 4);
       acc += v * mw[w];
     }
-    if (n < a.rep) *reinterpret_cast<f32x4_t*>(po + n * kD + 16 * mt + 4 * g) = acc;  // (columns past the real heads are padding)
+    if (n < rep) *reinterpret_cast<f32x4_t*>(po + n * kD + 16 * mt + 4 * g) = acc;  // (columns past the real heads are padding)
   }
   if (wave == 0 && g == 0) {
     float* pml = a.ws_ml + part * 32;
@@ -563,9 +589,9 @@ int q8_launch(Q8Args a, hipStream_t st) {
     q8_decode_split_kernel<FMT, QDT, SDT><<<grid, block, kLds, st>>>(
         reinterpret_cast<const uint8_t*>(a.k_codes), reinterpret_cast<const uint8_t*>(a.v_codes),
         reinterpret_cast<const uint8_t*>(a.k_scales), reinterpret_cast<const uint8_t*>(a.v_scales),
-        a.kv_rows, a.n_kv_heads, (int)a.n_keys, a.keys_per_split,
+        a.kv_rows, a.n_kv_heads, (int)a.n_keys, a.keys_per_split, a.rep,
         Q8Rest{a.q, reinterpret_cast<const uint8_t*>(a.k_biases), reinterpret_cast<const uint8_t*>(a.v_biases), a.ws_o, a.ws_ml,
-               a.scale_log2, a.n_splits, a.rep});
+               a.scale_log2, a.n_splits});
   }
   MSPR_CHECK_LAUNCH("sdpa_decode_q8 (split)");
   {

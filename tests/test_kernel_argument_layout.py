@@ -1,5 +1,5 @@
-"""Arguments that sparse attention's split and merge kernels need at their start come in scalar registers with the wave (CPU:
-hipcc compiles the source to assembly for gfx950, nothing runs)."""
+"""Arguments that the attention kernels need at their start come in scalar registers with the wave, and their first requests to
+memory wait for no others (CPU: hipcc compiles the source to assembly for gfx950, nothing runs)."""
 import os
 import re
 import shutil
@@ -15,8 +15,8 @@ def _first_lines(lines, until):
     code = [l.split(";")[0].strip() for l in lines]
     code = [l for l in code if l and not l.startswith(".")]
     start = next(i for i, l in enumerate(code) if l.startswith("s_branch"))  # (in front: the form for firmware that preloads nothing)
-    end = next(i for i, l in enumerate(code) if re.match(until, l))
-    return code[start + 1:end]
+    code = code[start + 1:]
+    return code[:next(i for i, l in enumerate(code) if re.match(until, l))]
 
 
 def test_the_split_kernel_requests_its_ids_before_it_waits_for_an_argument():
@@ -28,3 +28,14 @@ def test_the_split_kernel_requests_its_ids_before_it_waits_for_an_argument():
         assert not any(l.startswith("s_waitcnt") for l in head), name
     preload = dict(re.findall(r"\.amdhsa_kernel (\S+).*?kernarg_preload_length (\d+)", text, flags=re.S))
     assert all(int(n) >= 11 for k, n in preload.items() if "split_kernel" in k or "merge_kernel" in k)
+
+
+def test_the_8_bit_split_requests_its_first_tiles_before_it_waits_for_an_argument():
+    """A tile is eight 16-byte loads a lane of K codes and eight of V codes. (The first of them, and what they wait for, is one
+    basic block: a wave without a tile branches around it.)"""
+    text = build.device_assembly(os.path.join(build.CSRC, "q8_decode.hip"))
+    bodies = {k: v for k, v in build.kernel_bodies(text).items() if "q8_decode_split_kernel" in k}
+    assert len(bodies) == 6
+    for name, lines in bodies.items():
+        head = _first_lines(lines, r"s_waitcnt")
+        assert sum(l.startswith("global_load_dwordx4 ") for l in head) >= 16, name
