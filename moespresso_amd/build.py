@@ -9,6 +9,7 @@ cross-compiles without a GPU.
 from __future__ import annotations
 
 import concurrent.futures
+import functools
 import os
 import subprocess
 import sys
@@ -106,8 +107,9 @@ def build(verbose: bool = True) -> str:
     return LIB_PATH
 
 
+@functools.lru_cache(maxsize=None)
 def device_assembly(src: str) -> str:
-    """gfx950 assembly of one HIP source (device-only compile, nothing runs)."""
+    """gfx950 assembly of one HIP source (device-only compile, nothing runs), made once a process."""
     import tempfile
 
     with tempfile.TemporaryDirectory() as tmp:
@@ -188,6 +190,39 @@ def m0_hazards(lines: list[str]) -> list[str]:
         if "_load_lds_" in text and re.match(r"s_\w+ m0\b", previous):
             found.append(f"{previous} / {text}")
         previous = text
+    return found
+
+
+def scalar_register_hazards(lines: list[str]) -> list[str]:
+    """Instructions of inline asm statements that read a scalar register too soon after a vector instruction wrote it: two wait
+    states have to lie between for another vector instruction, five for a memory instruction. The compiler keeps to that in its
+    own code but does not look inside an asm statement."""
+    import re
+
+    def scalars(operand: str) -> set[str]:
+        if operand == "vcc":
+            return {"vcc"}
+        m = re.fullmatch(r"s(?:(\d+)|\[(\d+):(\d+)\])", operand)
+        return {f"s{i}" for i in range(int(m[1] or m[2]), int(m[1] or m[3]) + 1)} if m else set()
+
+    found, inside, written = [], False, []  # `written`: per wait state, the scalar registers that a vector instruction wrote
+    for line in lines:
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            inside = "#ASMSTART" in line
+        text = line.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        name, _, rest = text.partition(" ")
+        operands = [o.split()[0] if o.split() else "" for o in rest.split(",")]
+        vector = name.startswith("v_")
+        n_out = 2 if vector and "_co_" in name else 1 if vector else 0
+        states = 0 if not inside else 2 if vector else 5 if name.startswith(("global_", "buffer_", "flat_", "scratch_")) else 0
+        read = set().union(*map(scalars, operands[n_out:])) if operands[n_out:] else set()
+        if states and any(read & w for w in written[-states:]):
+            found.append(text)
+        written.append(set().union(*map(scalars, operands[:n_out])) if n_out else set())
+        if name == "s_nop":
+            written += [set()] * int(operands[0], 0)
     return found
 
 

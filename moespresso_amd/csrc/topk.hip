@@ -887,7 +887,9 @@ __device__ __forceinline__ int32_t signed_key(int32_t bits) { return bits ^ (int
 // compiler it is four instructions and two wait states: a comparison's result may not be read by the next two. With the list
 // written two rows at a time, the sample read from the copy of the row, its end shifted instead of loaded again and only the
 // waves with a candidate ranking one: 16 rows of 32768 scores, k = 2048, 8.4 -> 7.7 us; 3844 of 7961, k = 512, 29.4 -> 26.2; 5 of
-// 19211, k = 1024, 7.2 -> 6.8; 1 of 4096, k = 512, 4.6 and 4.6.)
+// 19211, k = 1024, 7.2 -> 6.8; 1 of 4096, k = 512, 4.6 and 4.6. The pivot is taken from a vector register: in a scalar one that a
+// vector instruction has just written, the first comparison would be one of those two, and the compiler puts no wait states in
+// front of inline assembly. Within it, three instructions lie between a comparison and the addition that reads it.)
 __device__ __forceinline__ uint32_t shift_in_four(uint32_t mask, __attribute__((ext_vector_type(4))) int k, int32_t pivot) {
   uint64_t c0, c1, c2, c3;
   asm("v_cmp_le_i32_e64 %1, %9, %5\n\tv_cmp_le_i32_e64 %2, %9, %6\n\tv_cmp_le_i32_e64 %3, %9, %7\n\t"
@@ -895,7 +897,7 @@ __device__ __forceinline__ uint32_t shift_in_four(uint32_t mask, __attribute__((
       "v_addc_co_u32_e64 %0, vcc, %0, %0, %1\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %2\n\t"
       "v_addc_co_u32_e64 %0, vcc, %0, %0, %3\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %4"
       : "+v"(mask), "=&s"(c0), "=&s"(c1), "=&s"(c2), "=&s"(c3)
-      : "v"(k.w), "v"(k.z), "v"(k.y), "v"(k.x), "s"(pivot)
+      : "v"(k.w), "v"(k.z), "v"(k.y), "v"(k.x), "v"(pivot)
       : "vcc");
   return mask;
 }

@@ -82,6 +82,36 @@ def test_no_copy_into_lds_directly_follows_the_write_of_its_address_register(sou
     assert build.m0_hazards(["\ts_mov_b32 m0, s8", "\ts_nop 0", copy, copy]) == []
 
 
+@pytest.mark.parametrize("source", ["sparse_attn.hip", "prefill_attn.hip", "flash_prefill.hip", "topk.hip", "indexer.hip", "indexer_tiled.hip"])
+def test_inline_asm_reads_no_scalar_register_too_soon(source):
+    bodies = build.kernel_bodies(build.device_assembly(os.path.join(build.CSRC, source)))
+    assert any("#ASMSTART" in l for lines in bodies.values() for l in lines)
+    for name, lines in bodies.items():
+        assert build.scalar_register_hazards(lines) == [], name
+        # (the comparisons of the sampled top-k take no scalar operand at all, whatever the compiler puts in front of them)
+        assert not any("v_cmp_le_i32_e64" in l and " s" in l.split(",", 1)[1] for l in _asm_lines(lines)), name
+    compare = "\tv_cmp_le_i32_e64 s[2:3], s8, v1"
+    for between, hazard in (([], 1), (["\ts_nop 0"], 1), (["\ts_nop 1"], 0), (["\tv_mov_b32_e32 v2, v3", "\ts_nop 0"], 0)):
+        lines = ["\tv_readfirstlane_b32 s8, v0", *between, "\t;;#ASMSTART", compare, "\t;;#ASMEND"]
+        assert len(build.scalar_register_hazards(lines)) == hazard
+    copy = ["\t;;#ASMSTART", "\ts_mov_b32 m0, s4", "\ts_nop 0", "\tglobal_load_lds_dwordx4 v2, s[8:9]", "\t;;#ASMEND"]
+    assert len(build.scalar_register_hazards(["\tv_readlane_b32 s9, v0, 3", "\ts_nop 1", *copy])) == 1
+    assert build.scalar_register_hazards(["\tv_readlane_b32 s9, v0, 3", "\ts_nop 2", *copy]) == []
+    assert build.scalar_register_hazards(["\tv_readlane_b32 s9, v0, 3", copy[3]]) == []  # (the compiler's own)
+    carry = ["\t;;#ASMSTART", "\tv_addc_co_u32_e64 v1, vcc, v1, v1, s[2:3]", "\tv_addc_co_u32_e64 v1, vcc, v1, v1, s[4:5]"]
+    assert build.scalar_register_hazards(carry) == []
+
+
+def _asm_lines(lines):
+    inside, out = False, []
+    for line in lines:
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            inside = "#ASMSTART" in line
+        elif inside:
+            out.append(line)
+    return out
+
+
 def test_scalar_arguments_of_kernels_are_preloaded():
     """The score, selection and rope kernels take plain arguments, which arrive in scalar registers with the wave."""
     for source, kernels in (("indexer_fp8.hip", 2), ("topk.hip", 22), ("rope_seam.hip", 9)):
