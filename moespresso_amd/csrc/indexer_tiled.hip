@@ -506,12 +506,20 @@ extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* wei
   hipStream_t st = (hipStream_t)stream;
   dim3 block(256);
   PackedOperands packed = {};
-  // The fp4 form is a launch more, some 3 us, which cheaper products have to earn. It does so from 2^17 scores on with
-  // float32 operands, which the float16 form rounds as it loads them (us without and with it: 32 tokens x 2000 rows 7.4 and
-  // 10.5, 64 x 2000 12.0 and 10.6, 96 x 2000 16.2 and 9.3, 17 x 8000 16.7 and 11.5, 517 x 500 22.6 and 12), and from 450
-  // thousand with float16 ones (128 x 2000 9.9 and 11.6, 400 x 1000 17.9 and 12.9). Both lines lie a little high for operands
-  // of the format; what is not of it pays for being looked at and is left alone below them.
-  if (workspace && (int64_t)batch * n_tokens * n_comp >= (dtype == MSPR_F32 ? 1 << 17 : 450000)) {
+  // The fp4 form is a launch more, some 3 us and what packing takes, which cheaper products have to earn. The float16 form runs
+  // in rounds of 256 pieces (64 rows for four tokens, one to a CU) of 4.3 us with float32 operands, which it rounds as it loads
+  // them, and of 2.4 us with float16 ones. float32: from the second round on, unless a token's 64 queries are packed for no more
+  // than 64 rows. float16: from the fifth full round on, and behind it where the packed blocks are many. us without and with it,
+  // float32: 64 tokens x 1000 rows (256 pieces) 7.2 and 8.5, 66 x 1000 11.4 and 8.6, 400 x 1000 25.5 and 11.5, 530 x 128 13.2 and
+  // 9.3, 3844 x 100 26.2 and 29.7, 1 x 20000 11.5 and 9.9, 2000 x 33 13.2 and 17.2, 4097 x 33 24.8 and 30.8. float16: 256 x 1000
+  // (1024) 9.9 and 10.0, 270 x 1000 12.4 and 10.9, 400 x 1000 17.8 and 11.6, 520 x 500 12.4 and 12.1, 1300 x 256 13.5 and 15.4,
+  // 1562 x 256 17.1 and 15.8, 3844 x 128 19.7 and 25.0, 3844 x 256 26.3 and 27.4, 1 x 120000 15.0 and 18.4. Operands that are not
+  // of the format, and that the caller does not name as such, pay for being looked at: 90 x 1000 float32 11.4 and 16.3, 131 x
+  // 1000 15.9 and 16.6; 330 x 1000 float16 13.9 and 17.2, 400 x 1000 18.0 and 17.6.
+  const int64_t packed_blocks = (row_pairs + n_tokens) * batch, token_pairs = row_pairs * n_tokens * batch;
+  const bool fp4_pays = dtype == MSPR_F32 ? row_pairs * tok_blocks * batch > 256 && row_pairs > 1
+                                          : token_pairs > 4 * 1024 && token_pairs > 3072 + 2 * packed_blocks;
+  if (workspace && fp4_pays) {
     packed = packed_operands(workspace, batch, n_tokens, n_comp);
     const int64_t blocks = pool_blocks(n_comp) + n_tokens;
     MSPR_REQUIRE(blocks < ((int64_t)1 << 31) && tok_blocks <= 65535 && n_comp < ((int64_t)1 << 31),
@@ -525,8 +533,9 @@ extern "C" int mspr_indexer_scores_tiled_live_ws(const void* q, const float* wei
     // the chip is not full otherwise, or 4 where there are not two workgroups to a CU even so. Three rounds of workgroups level
     // the last one: 3844 tokens x 7961 rows took 164, 160, 157, 168 us with 1, 2, 3, 4 row blocks, x 961 rows from position 0
     // took 21, 25, 31 us with 1, 2, 4; 517 tokens x 2053 rows 15.5 us with 2 and 13.7 us with 4. At least 8 and 4 pairs, whole
-    // calls: 96 x 2000 10.9 and 9.3 (random operands 23.7 and 16.9), 64 x 4000 11.4 and 9.7, 300 x 600 12.2 and 10.3, 517 x
-    // 1000 14.8 and 14.4, 1000 x 500 14.8 and 15.1, 517 x 2053 19.4 and 20.2.
+    // calls: 96 x 2000 10.9 and 9.3 (random operands 23.7 and 16.9), 64 x 4000 11.4 and 9.7, 300 x 600 12.2 and 10.3, 1200 x 500
+    // 17.9 and 17.0, 528 x 1000 14.6 and 13.7. Where 8 leave just under a workgroup to a CU, either: 928 x 500 float32 13.7 and
+    // 14.4, 928 x 600 float16 15.4 and 14.8. From 512 on 8: 517 x 2053 19.4 and 20.2.
     int64_t rows = rows_per_workgroup(2304, 16);
     auto workgroups = [&]() -> int64_t { return (n_comp + rows - 1) / rows * tok_blocks * batch; };
     if (workgroups() < 768) rows = rows_per_workgroup(768, 8);

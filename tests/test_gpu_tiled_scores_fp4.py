@@ -42,15 +42,21 @@ def test_qat_operands_give_the_float16_form_bit_for_bit(dtype, batch, heads, tok
     assert ratio != 0 or bool(torch.isfinite(got).all())
 
 
-# Enough scores for the fp4 form (2^17 of float32 operands, 450 thousand of float16 ones), and the last numbers below them:
-# ragged blocks of rows, tokens and heads, several sequences, the whole pool visible.
+# On both sides of the lines from which the fp4 form is taken (float32: more than 256 pieces of four tokens by 64 rows, and more
+# than 64 rows; float16: 4096 pairs of a token and 64 rows, and 3072 and twice the packed blocks): ragged blocks of rows, tokens
+# and heads, several sequences, the whole pool visible.
 @pytest.mark.parametrize("dtype,batch,heads,tokens,rows,pos0,ratio", [
     (torch.float32, 1, 64, 4097, 33, 0, 4), (torch.float32, 2, 64, 1025, 64, 60, 4), (torch.float32, 1, 40, 1031, 130, 512, 4),
     (torch.float32, 3, 64, 46, 1000, 3800, 4), (torch.float32, 1, 1, 45, 3001, 11980, 4), (torch.float32, 1, 64, 6, 22011, 0, 0),
     (torch.float32, 1, 64, 2, 65535, 0, 0), (torch.float32, 1, 64, 2, 65536, 0, 0),
     (torch.float16, 1, 64, 4097, 129, 0, 4), (torch.float16, 2, 64, 1001, 255, 60, 4), (torch.float16, 1, 40, 3511, 130, 512, 4),
     (torch.float16, 3, 64, 150, 1024, 3800, 4), (torch.float16, 1, 1, 151, 2999, 11900, 4), (torch.float16, 1, 64, 22, 22011, 0, 0),
-    (torch.float16, 1, 64, 18, 24999, 0, 0), (torch.float16, 1, 64, 18, 25000, 0, 0)])
+    (torch.float16, 1, 64, 18, 24999, 0, 0), (torch.float16, 1, 64, 18, 25000, 0, 0),
+    (torch.float32, 1, 64, 64, 1024, 0, 0), (torch.float32, 1, 64, 65, 1024, 0, 0), (torch.float32, 1, 64, 64, 1025, 0, 0),
+    (torch.float32, 1, 64, 1, 16384, 0, 0), (torch.float32, 1, 64, 1, 16385, 0, 0), (torch.float32, 2, 64, 515, 64, 0, 0),
+    (torch.float32, 2, 64, 515, 65, 0, 0), (torch.float16, 1, 64, 256, 1024, 0, 0), (torch.float16, 1, 64, 257, 1024, 0, 0),
+    (torch.float16, 1, 64, 256, 1025, 0, 0), (torch.float16, 2, 64, 130, 1024, 0, 0), (torch.float16, 1, 64, 1537, 200, 0, 0),
+    (torch.float16, 1, 64, 1544, 200, 0, 0)])
 def test_both_forms_agree_where_the_fp4_form_is_taken(dtype, batch, heads, tokens, rows, pos0, ratio):
     got, want = _both(*_operands(batch, heads, tokens, rows, dtype), pos0, ratio)
     assert got.equal(want)
@@ -134,3 +140,15 @@ def test_group_exponents_far_apart_round_in_float32():
     errors = [(x[0].cpu().double() - exact).abs() for x in (got, f16)]
     assert all(bool((e <= 8 * 2.0 ** -23 * size).all()) for e in errors)
     assert errors[0].norm() <= errors[1].norm()      # no less precise than the form it takes the place of
+
+
+# The last sizes of the float16 form and the first of the fp4 form, told apart by how such sums round.
+@pytest.mark.parametrize("dtype,tokens,rows,fp4", [
+    (torch.float32, 64, 1024, False), (torch.float32, 65, 1024, True), (torch.float32, 64, 1025, True), (torch.float32, 2060, 64, False),
+    (torch.float32, 2060, 65, True), (torch.float16, 256, 1024, False), (torch.float16, 257, 1024, True),
+    (torch.float16, 1537, 200, False), (torch.float16, 1544, 200, True)])
+def test_which_form_is_taken_on_either_side_of_its_line(dtype, tokens, rows, fp4):
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q, comp = _lattice_rows(tokens, -12, 12, gen).to(dtype), _lattice_rows(rows, -12, 12, gen).to(dtype)
+    got, f16 = _both(q.reshape(1, 1, tokens, 128), torch.ones((1, tokens, 1), device="cuda"), comp.reshape(1, rows, 128), 0, 0)
+    assert got.equal(f16) != fp4
