@@ -64,6 +64,16 @@ __device__ __forceinline__ void window_store(__amdgpu_buffer_rsrc_t w, int offse
   __builtin_amdgcn_raw_buffer_store_b128(v, w, offset, 0, POLICY);
 }
 
+// x / n for x below 2^31 with inv = mspr_inverse(n): a software division is thirty instructions and more, in front of a kernel's
+// first memory request four to five cycles each with two waves on a SIMD.
+inline uint32_t mspr_inverse(int n) { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); }  // floor(2^32 / n)
+__device__ __forceinline__ int mspr_div(int x, int n, uint32_t inv) {
+  if (n == 1) return x;
+  int q = (int)__umulhi((uint32_t)x, inv);  // the quotient or one less
+  if (x - q * n >= n) q++;
+  return q;
+}
+
 // float32 -> bfloat16 bits, round to nearest even (NaN kept quiet).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   uint32_t u = __float_as_uint(f);

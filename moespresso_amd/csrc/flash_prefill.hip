@@ -39,7 +39,7 @@ struct PrefillArgs {
   float scale_log2;
   int rep_shift;    // log2(query heads per KV head), 0..3
   int q_blocks;     // workgroups along the query axis
-  uint32_t inv_splits, inv_q_blocks, inv_kv_heads;  // floor(2^32 / n), for divisions by n_splits, q_blocks, n_kv_heads
+  uint32_t inv_splits, inv_q_blocks, inv_kv_heads;  // mspr_inverse() of n_splits, q_blocks, n_kv_heads
   // key-range splits (short chunks over deep prefixes do not fill the device otherwise): split sp of a
   // query block takes every n_splits-th share of that block's tiles; partials are merged afterwards
   int n_splits;
@@ -178,15 +178,6 @@ __device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 
 // gives; without it in packed float16 arithmetic.
 constexpr int kExactUnpack = 4;
 
-// x / n with inv = floor(2^32 / n): a software division is some thirty instructions, four of them stood in front of the first
-// memory request
-__device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
-  if (n == 1) return x;
-  int q = (int)__umulhi((uint32_t)x, inv);  // the quotient or one less
-  if (x - q * n >= n) q++;
-  return q;
-}
-
 // (Plain arguments first: what the first tiles' addresses take comes in registers with the wave, and the struct is loaded
 // meanwhile. With that and without software divisions, 100 queries behind 1000 rows 18.5 -> 18.0 us, 203 behind 9001 42.7 -> 42.2,
 // and their merges 5.3 -> 5.1 and 9.3 -> 9.2. heads: n_kv_heads, and rep_shift from bit 28 on.)
@@ -224,21 +215,21 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   if constexpr (RUNS) {
     const int wgs = a.batch * n_kv_heads * q_blocks * n_splits, xcd = work & 7;
     work = xcd * (wgs >> 3) + (xcd < (wgs & 7) ? xcd : wgs & 7) + (work >> 3);
-    const int rest = div_by(work, q_blocks, inv_q_blocks);
+    const int rest = mspr_div(work, q_blocks, inv_q_blocks);
     q_block = work - rest * q_blocks;
-    work = div_by(rest, n_splits, inv_splits);
+    work = mspr_div(rest, n_splits, inv_splits);
     sp = rest - work * n_splits;
   } else {
-    const int rest = div_by(work, n_splits, inv_splits);
+    const int rest = mspr_div(work, n_splits, inv_splits);
     sp = work - rest * n_splits;
-    work = div_by(rest, q_blocks, inv_q_blocks);
+    work = mspr_div(rest, q_blocks, inv_q_blocks);
     q_block = rest - work * q_blocks;
   }
   const int pair = q_block >> halves_shift;  // pair 0 (longest stream) first
   const int head_half = q_block & ((1 << halves_shift) - 1);
   int kvh = work, b = 0;
   if (work >= n_kv_heads) {
-    b = div_by(work, n_kv_heads, a.inv_kv_heads);
+    b = mspr_div(work, n_kv_heads, a.inv_kv_heads);
     kvh = work - b * n_kv_heads;
   }
   const int wi = wave & 3;
@@ -258,7 +249,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   if (q_last > q_len - 1) q_last = q_len - 1;
   const int all_tiles = (int)((uint32_t)(past + q_last) / kTile) + 1;
   // this workgroup's share of the block's tiles: [t_begin, n_tiles)
-  const int tiles_per_split = div_by(all_tiles + n_splits - 1, n_splits, inv_splits);
+  const int tiles_per_split = mspr_div(all_tiles + n_splits - 1, n_splits, inv_splits);
   const int t_begin = sp * tiles_per_split < all_tiles ? sp * tiles_per_split : all_tiles;
   const int n_tiles = t_begin + tiles_per_split < all_tiles ? t_begin + tiles_per_split : all_tiles;
 
@@ -902,10 +893,9 @@ int prefill_launch_flash(const PrefillArgs& a, hipStream_t st) {
 template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
 int prefill_launch(const PrefillArgs& call, hipStream_t st, bool q32 = false) {
   PrefillArgs a = call;
-  auto inverse = [](int n) -> uint32_t { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); };
-  a.inv_splits = inverse(a.n_splits);
-  a.inv_q_blocks = inverse(a.q_blocks);
-  a.inv_kv_heads = inverse(a.n_kv_heads);
+  a.inv_splits = mspr_inverse(a.n_splits);
+  a.inv_q_blocks = mspr_inverse(a.q_blocks);
+  a.inv_kv_heads = mspr_inverse(a.n_kv_heads);
   // (the line of the kernel's mapping; a template parameter because as a run-time branch it cost long chunks 0.5 %)
   const bool runs = a.n_splits >= 4 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
   int rc;

@@ -20,7 +20,7 @@ struct IndexedPrefillArgs {
   float* out;  // strides as q
   // filled in by the launch: units (token and block of 64 heads) that are cut into key ranges, and their partials
   int split_units, ranges;
-  uint32_t inv_hblk, inv_ranges;  // floor(2^32 / n), for divisions by the blocks of 64 heads and by ranges
+  uint32_t inv_hblk, inv_ranges;  // mspr_inverse() of the blocks of 64 heads and of ranges
   float* parts;
 };
 

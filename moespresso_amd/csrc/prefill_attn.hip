@@ -66,14 +66,6 @@ __device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint3
                : "memory", "m0");
 }
 
-// x / n with inv = floor(2^32 / n), x below 2^31: a software division is some thirty instructions
-__device__ __forceinline__ int div_by(int x, int n, uint32_t inv) {
-  if (n == 1) return x;
-  int q = (int)__umulhi((uint32_t)x, inv);  // the quotient or one less
-  if (x - q * n >= n) q++;
-  return q;
-}
-
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
 // (Plain arguments first: what the first copies and the ids take comes in registers with the wave, and the struct is loaded
 // meanwhile: it was loaded in three dependent steps with three software divisions between. One token behind 28000 rows 22.1 ->
@@ -101,12 +93,12 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
     const int whole = units - a.split_units;
     split = (int)blockIdx.x >= whole;
     const int i = (int)blockIdx.x - whole;
-    unit = split ? div_by(i, a.ranges, a.inv_ranges) : a.split_units - 1 - i;
+    unit = split ? mspr_div(i, a.ranges, a.inv_ranges) : a.split_units - 1 - i;
     range = split ? i - unit * a.ranges : 0;
   }
-  const int seq = n_hblk == 1 ? unit : div_by(unit, n_hblk, a.inv_hblk);
+  const int seq = n_hblk == 1 ? unit : mspr_div(unit, n_hblk, a.inv_hblk);
   const int hb = unit - seq * n_hblk;
-  const int b = div_by(seq, n_tokens, inv_tokens);
+  const int b = mspr_div(seq, n_tokens, inv_tokens);
   const int t = seq - b * n_tokens;
 
   // window rows and visible pool prefix, in the unsigned 32-bit arithmetic of the reference kernel
@@ -123,7 +115,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   // this workgroup's tiles: all of them, or its share of what the token has at most
   int t_begin = 0, t_share = 0x7FFFFFFF;
   if (CUT && split) {
-    t_share = div_by(wt + (n_idx + kTile - 1) / kTile + a.ranges - 1, a.ranges, a.inv_ranges);
+    t_share = mspr_div(wt + (n_idx + kTile - 1) / kTile + a.ranges - 1, a.ranges, a.inv_ranges);
     t_begin = range * t_share;
   }
   const uint64_t win_base = reinterpret_cast<uint64_t>(win) + (uint64_t)b * (uint64_t)n_raw * (kD * 2);
@@ -379,8 +371,8 @@ __global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(const float*
   const int c16 = lane & 15, kg = lane >> 4;
   const int piece = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
   const int unit = piece >> 7, wave = (piece >> 5) & 3, mt = piece & 31;
-  const int seq = div_by(unit, n_hblk, inv_hblk), hb = unit - seq * n_hblk;
-  const int b = div_by(seq, n_tokens, inv_tokens), t = seq - b * n_tokens;
+  const int seq = mspr_div(unit, n_hblk, inv_hblk), hb = unit - seq * n_hblk;
+  const int b = mspr_div(seq, n_tokens, inv_tokens), t = seq - b * n_tokens;
   const int head = hb * 64 + 16 * wave + c16;
   const float* po = parts + (int64_t)unit * ranges * (64 * kD) + ((wave * 32 + mt) * 64 + lane) * 4;
   const float* ml = parts + (int64_t)split_units * ranges * (64 * kD) + ((int64_t)unit * ranges * 64 + 16 * wave + c16) * 2;
@@ -428,10 +420,9 @@ int launch(const IndexedPrefillArgs& call, hipStream_t st) {
   IndexedPrefillArgs a = call;
   const int n_hblk = (a.n_heads + 63) / 64;
   const int64_t units = (int64_t)a.batch * a.n_tokens * n_hblk;
-  auto inverse = [](int n) -> uint32_t { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); };
-  a.inv_hblk = inverse(n_hblk);
-  a.inv_ranges = inverse(a.ranges);
-  const uint32_t inv_tokens = inverse(a.n_tokens);
+  a.inv_hblk = mspr_inverse(n_hblk);
+  a.inv_ranges = mspr_inverse(a.ranges);
+  const uint32_t inv_tokens = mspr_inverse(a.n_tokens);
   dim3 grid((unsigned)(units - a.split_units + a.split_units * a.ranges)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);

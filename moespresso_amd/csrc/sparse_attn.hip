@@ -89,7 +89,7 @@ struct SparseAttnArgs {
   // split: range sp of a sequence owns window slots [sp*win_per_split, +win_per_split) and gathered
   // ids [sp*idx_per_split, +idx_per_split)
   int n_splits;
-  uint32_t inv_splits, inv_hblk, inv_tokens;  // floor(2^32 / n) of n_splits, n_hblk, n_tokens
+  uint32_t inv_splits, inv_hblk, inv_tokens;  // mspr_inverse() of n_splits, n_hblk, n_tokens
   int win_per_split;
   int idx_per_split;
   int tiles_per_split;  // > 0: range sp owns this many consecutive tiles of the window's and the ids' tiles instead
@@ -180,8 +180,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Normalised output values of four consecutive columns -> output tensor, in the output element type
 // (the fused-decode form applies the inverse partial rope on the float16 values at float16 op rounding; `rope_cs` holds the
 // cosines of the columns' pairs and, eight further on, their negated sines, where they are known).
-template <int ODT, class Args>
-__device__ __forceinline__ void emit_output(Args& a, const float (&r)[4], int64_t ooff, int dim0,
+template <int ODT>
+__device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float (&r)[4], int64_t ooff, int dim0,
                                             const float* rope_cs = nullptr) {
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = f32x4_t{r[0], r[1], r[2], r[3]};
@@ -219,8 +219,7 @@ __device__ __forceinline__ void emit_output(Args& a, const float (&r)[4], int64_
   }
 }
 
-template <class Args>
-__device__ __forceinline__ float load_sink_log2(Args& a, int head) {
+__device__ __forceinline__ float load_sink_log2(const SparseAttnArgs& a, int head) {
   if (!a.sinks) return -__builtin_inff();
   return (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.sinks)[head])
                                     : reinterpret_cast<const float*>(a.sinks)[head]) * 1.4426950408889634f;
@@ -302,15 +301,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(const in
   // ---- workgroup -> (batch, head block, split); consecutive splits of one batch share an XCD
   int work = blockIdx.x;
   if ((total & 7) == 0) work = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
-  // (divisions by multiplication with floor(2^32 / n) and one correction step: a software division is a hundred
-  // instructions in front of the first memory request, four to five cycles each with two waves on a SIMD)
-  auto div_by = [](uint32_t x, uint32_t n, uint32_t inv) -> uint32_t {
-    if (n == 1u) return x;
-    uint32_t q = __umulhi(x, inv);  // true quotient or one less
-    if (x - q * n >= n) q++;
-    return q;
-  };
-  const int bh = (int)div_by((uint32_t)work, (uint32_t)n_splits, inv_splits);
+  const int bh = mspr_div(work, n_splits, inv_splits);
   const int sp = work - bh * n_splits;
 
   // range sp: its share of the window slots, then its share of the gathered ids. Window tiles come
@@ -352,9 +343,9 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(const in
   int seq_n_win = n_win, seq_win_first = a.win_first;
   int64_t seq_visible = a.visible;
   if (plain_stride < 0) {
-    seq = (int)div_by((uint32_t)bh, (uint32_t)a.n_hblk, a.inv_hblk);
+    seq = mspr_div(bh, a.n_hblk, a.inv_hblk);
     hb = bh - seq * a.n_hblk;
-    b = (int)div_by((uint32_t)seq, (uint32_t)a.n_tokens, a.inv_tokens);
+    b = mspr_div(seq, a.n_tokens, a.inv_tokens);
     t = seq - b * a.n_tokens;
     if (a.prefill) {
       const uint32_t qpos = a.pos0 + (uint32_t)t, n_raw = (uint32_t)a.raw_cap;
@@ -979,17 +970,11 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_prefill_kernel(Sparse
   int unit = (int)blockIdx.x;
   if (unit >= n_units) return;
 
-  auto div_by = [](uint32_t x, uint32_t n, uint32_t inv) -> uint32_t {
-    if (n == 1u) return x;
-    uint32_t q = __umulhi(x, inv);
-    if (x - q * n >= n) q++;
-    return q;
-  };
   auto unit_of = [&](int u) -> PrefillUnit {
     PrefillUnit m;
-    m.seq = (int)div_by((uint32_t)u, (uint32_t)a.n_hblk, a.inv_hblk);
+    m.seq = mspr_div(u, a.n_hblk, a.inv_hblk);
     m.hb = u - m.seq * a.n_hblk;
-    m.b = (int)div_by((uint32_t)m.seq, (uint32_t)a.n_tokens, a.inv_tokens);
+    m.b = mspr_div(m.seq, a.n_tokens, a.inv_tokens);
     m.t = m.seq - m.b * a.n_tokens;
     // window rows and visible pool prefix, in the unsigned 32-bit arithmetic of the reference kernel
     const uint32_t qpos = a.pos0 + (uint32_t)m.t, n_raw = (uint32_t)a.raw_cap;
@@ -1488,13 +1473,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   const int piece = work & 7;        // registers 8 piece .. +7 of the wave's 64: columns tile piece / 2
   const int wave = (work >> 3) & 7;  // wave of the split kernel whose registers this workgroup merges
   const int bh = work >> 6;
-  auto div_by = [](uint32_t x, uint32_t n, uint32_t inv) -> uint32_t {
-    if (n == 1u) return x;
-    uint32_t q = __umulhi(x, inv);
-    if (x - q * n >= n) q++;
-    return q;
-  };
-  const int seq = (int)div_by((uint32_t)bh, (uint32_t)a.n_hblk, a.inv_hblk);
+  const int seq = mspr_div(bh, a.n_hblk, a.inv_hblk);
   const int hb = bh - seq * a.n_hblk;
   const int hg = wave >> 2, dh = wave & 3;
   const int n = lane & 31, g = lane >> 5;
@@ -1581,7 +1560,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   }
   const float inv = l == 0.0f ? 0.0f : 1.0f / l;
   const float r[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
-  const int b = (int)div_by((uint32_t)seq, (uint32_t)a.n_tokens, a.inv_tokens);
+  const int b = mspr_div(seq, a.n_tokens, a.inv_tokens);
   const int t = seq - b * a.n_tokens;
   const int dim0 = dh * 128 + 32 * (piece >> 1) + 16 * (piece & 1) + 8 * w4 + 4 * g;
   const int64_t ooff = (int64_t)b * a.out_batch_stride + (int64_t)t * a.out_token_stride +
@@ -1734,9 +1713,8 @@ int run_sparse_attention(SparseAttnArgs a, int kv_dtype, int k_dim, void* worksp
     a.out_batch_stride = (int64_t)a.n_heads * kDV;
   }
   a.n_hblk = (a.n_heads + 63) / 64;
-  auto magic = [](int n) -> uint32_t { return n <= 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint32_t)n); };
-  a.inv_hblk = magic(a.n_hblk);
-  a.inv_tokens = magic(a.n_tokens);
+  a.inv_hblk = mspr_inverse(a.n_hblk);
+  a.inv_tokens = mspr_inverse(a.n_tokens);
   if (prefill_consumer_fits(a, kv_dtype, k_dim)) {
     if (a.q_dtype == MSPR_F32) {
       // (a.batch counts sequences = batch entries x tokens)
@@ -1777,7 +1755,7 @@ int run_sparse_attention(SparseAttnArgs a, int kv_dtype, int k_dim, void* worksp
   }
   MSPR_REQUIRE(table_slots <= 1024, "sparse attention: too many key slots (%d)", n_keys);
   a.direct = a.n_splits == 1;
-  a.inv_splits = magic(a.n_splits);
+  a.inv_splits = mspr_inverse(a.n_splits);
   size_t need = workspace_bytes(a.batch, a.n_heads, n_keys);
   MSPR_REQUIRE(workspace && workspace_bytes_given >= need, "sparse attention: workspace of %zu bytes needed, %zu given",
                need, workspace_bytes_given);
