@@ -42,38 +42,46 @@ constexpr int kDV = 512;
 constexpr int kThreads = 512;  // split kernel: eight waves, two per SIMD
 constexpr int kWaves = kThreads / 64;
 
-struct SparseAttnArgs {
-  // query
-  const void* q;
-  int q_dtype;
+// Where the output goes, and the inverse rope of its last columns.
+struct SparseOutArgs {
+  void* out;
+  int64_t out_batch_stride, out_head_stride, out_token_stride;  // elements
+  const float* inv_freq;
+  const int32_t* params;
+  int rope;
+  int out_dtype;
+};
+
+// What the split kernel reads behind its plain arguments. (A kernel is handed what it reads, once: with the whole of
+// SparseAttnArgs behind their plain words the split's block was 392 bytes and the merge's 384, now 312 and 112. One token's
+// launches 23.9 -> 23.4 us of the device's time, four captured layers of 16 sequences 188.8 -> 187.7.)
+struct SparseSplitArgs : SparseOutArgs {
   int64_t q_batch_stride;  // elements; q of (b, t, head) at b*q_batch_stride + t*q_token_stride + head*q_head_stride
   int64_t q_head_stride;
   int64_t q_token_stride;
   int n_heads;
-  int batch;               // sequences = batch entries x tokens
+  int n_hblk;
   int n_tokens;            // query tokens per batch entry; they share the window and pool tensors
+  uint32_t inv_hblk, inv_tokens;  // mspr_inverse() of n_hblk, n_tokens
   // prefill form: window range and visible pool prefix follow from the token's position pos0 + t
   int prefill;
   uint32_t pos0, window, ratio;
+  int direct;  // one key range per sequence: the split kernel normalises and stores, no partials
   // window segment (the split kernel reads win_first .. subst_slot, and check_stop .. scale_log2 below, with one load of four
   // words each; a word of such a load that it had no use for would be given away, and its next owner wait for the load)
   const void* win;
   int64_t win_batch_stride;
-  int n_win;
   int win_first;  // logical index of the first visited ring row
   int raw_start;
   int raw_cap;
   int subst_slot;          // window slot replaced by subst_row (-1: none)
-  int subst_from_params;   // take the slot from params[1] on the device instead
   const void* subst_row;
   // gathered segment
   const void* pool;
   int64_t pool_batch_stride;
   int64_t n_pool;
   const int32_t* pool_rows_dev;  // optional: rows of the pool in use, read on the device (<= n_pool, the capacity)
-  const int32_t* idx;
   int64_t idx_batch_stride;
-  int n_idx;
   int64_t visible;  // ids >= visible end the walk
   int check_stop;
   int row_mul;  // pool row = id * row_mul + row_add
@@ -82,25 +90,25 @@ struct SparseAttnArgs {
   float scale_log2;
   const void* sinks;
   int sinks_dtype;
-  // rope
-  const float* inv_freq;
-  const int32_t* params;
-  int rope;
+  int subst_from_params;   // take the substituted slot from params[1] on the device instead
+  uint16_t* ws_o;  // float16 partial rows, each normalised by its own range's denominator
+  float* ws_ml;
+};
+
+struct SparseAttnArgs : SparseSplitArgs {
+  const void* q;
+  int q_dtype;
+  int batch;  // sequences = batch entries x tokens
+  int n_win;
+  const int32_t* idx;
+  int n_idx;
   // split: range sp of a sequence owns window slots [sp*win_per_split, +win_per_split) and gathered
   // ids [sp*idx_per_split, +idx_per_split)
   int n_splits;
-  uint32_t inv_splits, inv_hblk, inv_tokens;  // mspr_inverse() of n_splits, n_hblk, n_tokens
+  uint32_t inv_splits;  // mspr_inverse(n_splits)
   int win_per_split;
   int idx_per_split;
   int tiles_per_split;  // > 0: range sp owns this many consecutive tiles of the window's and the ids' tiles instead
-  int n_hblk;
-  uint16_t* ws_o;  // float16 partial rows, each normalised by its own range's denominator
-  float* ws_ml;
-  // output
-  void* out;
-  int out_dtype;
-  int64_t out_batch_stride, out_head_stride, out_token_stride;  // elements
-  int direct;  // one key range per sequence: the split kernel normalises and stores, no partials
 };
 
 template <int KDT>
@@ -181,7 +189,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // (the fused-decode form applies the inverse partial rope on the float16 values at float16 op rounding; `rope_cs` holds the
 // cosines of the columns' pairs and, eight further on, their negated sines, where they are known).
 template <int ODT>
-__device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float (&r)[4], int64_t ooff, int dim0,
+__device__ __forceinline__ void emit_output(const SparseOutArgs& a, const float (&r)[4], int64_t ooff, int dim0,
                                             const float* rope_cs = nullptr) {
   if constexpr (ODT == MSPR_F32) {
     *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + ooff) = f32x4_t{r[0], r[1], r[2], r[3]};
@@ -219,7 +227,7 @@ __device__ __forceinline__ void emit_output(const SparseAttnArgs& a, const float
   }
 }
 
-__device__ __forceinline__ float load_sink_log2(const SparseAttnArgs& a, int head) {
+__device__ __forceinline__ float load_sink_log2(const SparseSplitArgs& a, int head) {
   if (!a.sinks) return -__builtin_inff();
   return (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.sinks)[head])
                                     : reinterpret_cast<const float*>(a.sinks)[head]) * 1.4426950408889634f;
@@ -276,7 +284,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_attn_split_kernel(const in
                                                                         int n_splits, uint32_t inv_splits,
                                                                         int tiles_per_split, int win_per_split,
                                                                         int idx_per_split, int n_win, int n_idx,
-                                                                        int plain_stride, SparseAttnArgs a) {
+                                                                        int plain_stride, SparseSplitArgs a) {
   using G = Geometry<DK>;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   unsigned char* kbuf = lds;                                                   // [kBufs][kTileBytes]
@@ -1451,17 +1459,10 @@ __global__ __launch_bounds__(256) void prefill_q_to_half_kernel(const float* q, 
 // the statistics, it took 6.2 us at 16 ranges (16 sequences; now 5.1) and 6.3 at 32 (one sequence; now 3.9).
 // (Plain arguments first: they come in registers with the wave.)
 template <int ODT>
-__global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, float* ws_ml, const void* sinks,
+__global__ __launch_bounds__(256) void sparse_attn_merge_kernel(const uint16_t* ws_o, const float* ws_ml, const void* sinks,
                                                                 int sinks_dtype, unsigned total, int n_splits, int n_hblk,
-                                                                uint32_t inv_hblk, int n_heads, SparseAttnArgs a) {
-  a.ws_o = ws_o;
-  a.ws_ml = ws_ml;
-  a.sinks = sinks;
-  a.sinks_dtype = sinks_dtype;
-  a.n_splits = n_splits;
-  a.n_hblk = n_hblk;
-  a.inv_hblk = inv_hblk;
-  a.n_heads = n_heads;
+                                                                uint32_t inv_hblk, int n_heads, int n_tokens,
+                                                                uint32_t inv_tokens, SparseOutArgs a) {
   __shared__ float xm[4][64], xl[4][64];
   __shared__ __attribute__((aligned(16))) float xo[4][2][64][4];
   __shared__ float rope_cs[16];  // of the workgroup's sixteen columns: eight cosines, eight negated sines
@@ -1473,21 +1474,21 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   const int piece = work & 7;        // registers 8 piece .. +7 of the wave's 64: columns tile piece / 2
   const int wave = (work >> 3) & 7;  // wave of the split kernel whose registers this workgroup merges
   const int bh = work >> 6;
-  const int seq = mspr_div(bh, a.n_hblk, a.inv_hblk);
-  const int hb = bh - seq * a.n_hblk;
+  const int seq = mspr_div(bh, n_hblk, inv_hblk);
+  const int hb = bh - seq * n_hblk;
   const int hg = wave >> 2, dh = wave & 3;
   const int n = lane & 31, g = lane >> 5;
   const int head = hb * 64 + hg * 32 + n;
-  const bool live = head < a.n_heads;
+  const bool live = head < n_heads;
 
-  const int64_t part0 = (int64_t)bh * a.n_splits;
-  const f32x2_t* ml0 = reinterpret_cast<const f32x2_t*>(a.ws_ml) + part0 * 64 + hg * 32 + n;
-  const f16x8_t* wo0 = reinterpret_cast<const f16x8_t*>(a.ws_o) + (part0 * kWaves + wave) * (int64_t)(8 * 64) + piece * 64 + lane;
+  const int64_t part0 = (int64_t)bh * n_splits;
+  const f32x2_t* ml0 = reinterpret_cast<const f32x2_t*>(ws_ml) + part0 * 64 + hg * 32 + n;
+  const f16x8_t* wo0 = reinterpret_cast<const f16x8_t*>(ws_o) + (part0 * kWaves + wave) * (int64_t)(8 * 64) + piece * 64 + lane;
   uint32_t sink_bits = 0;  // (on its way with the partials; made a number of behind them)
-  if (a.sinks) {
+  if (sinks) {
     const int h = live ? head : 0;
-    sink_bits = a.sinks_dtype == MSPR_F16 ? reinterpret_cast<const uint16_t*>(a.sinks)[h]
-                                          : reinterpret_cast<const uint32_t*>(a.sinks)[h];
+    sink_bits = sinks_dtype == MSPR_F16 ? reinterpret_cast<const uint16_t*>(sinks)[h]
+                                          : reinterpret_cast<const uint32_t*>(sinks)[h];
   }
   constexpr int kChunk = 8;
   // The inverse rope of the last 64 columns: waves 2 and 3 work out the workgroup's cosines and sines in float64 while the
@@ -1502,13 +1503,13 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   };
   float m_run = -__builtin_inff(), l = 0.0f;
   float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s0 = w4; s0 < a.n_splits; s0 += 4 * kChunk) {
+  for (int s0 = w4; s0 < n_splits; s0 += 4 * kChunk) {
     f32x2_t ml[kChunk];
     f16x8_t ov[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; j++) {
       const int sj = s0 + 4 * j;  // (the same in every lane: ranges past the end cost no load)
-      if (sj < a.n_splits) {
+      if (sj < n_splits) {
         ml[j] = ml0[(int64_t)sj * 64];
         ov[j] = wo0[(int64_t)sj * (kWaves * 8 * 64)];
       } else {
@@ -1534,7 +1535,7 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
     }
     m_run = m_new;
   }
-  if (w4 >= a.n_splits) rope_columns();  // (no range for this wave)
+  if (w4 >= n_splits) rope_columns();  // (no range for this wave)
   xm[w4][lane] = m_run;
   xl[w4][lane] = l;
 #pragma unroll
@@ -1543,8 +1544,8 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   __syncthreads();
   // waves 0 and 1 finish four of the eight columns each; the sink joins the maximum and the denominator once
   if (w4 >= 2 || !live) return;
-  const float sink = !a.sinks ? -__builtin_inff()
-                              : (a.sinks_dtype == MSPR_F16 ? f16_bits_to_f32((uint16_t)sink_bits)
+  const float sink = !sinks ? -__builtin_inff()
+                              : (sinks_dtype == MSPR_F16 ? f16_bits_to_f32((uint16_t)sink_bits)
                                                            : __uint_as_float(sink_bits)) * 1.4426950408889634f;
   float m_all = sink;
 #pragma unroll
@@ -1560,8 +1561,8 @@ __global__ __launch_bounds__(256) void sparse_attn_merge_kernel(uint16_t* ws_o, 
   }
   const float inv = l == 0.0f ? 0.0f : 1.0f / l;
   const float r[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
-  const int b = mspr_div(seq, a.n_tokens, a.inv_tokens);
-  const int t = seq - b * a.n_tokens;
+  const int b = mspr_div(seq, n_tokens, inv_tokens);
+  const int t = seq - b * n_tokens;
   const int dim0 = dh * 128 + 32 * (piece >> 1) + 16 * (piece & 1) + 8 * w4 + 4 * g;
   const int64_t ooff = (int64_t)b * a.out_batch_stride + (int64_t)t * a.out_token_stride +
                        (int64_t)head * a.out_head_stride + dim0;
@@ -1777,7 +1778,8 @@ int run_sparse_attention(SparseAttnArgs a, int kv_dtype, int k_dim, void* worksp
     const auto merge = a.out_dtype == MSPR_F32 ? &sparse_attn_merge_kernel<MSPR_F32>
                        : a.out_dtype == MSPR_BF16 ? &sparse_attn_merge_kernel<MSPR_BF16>
                                                   : &sparse_attn_merge_kernel<MSPR_F16>;
-    merge<<<grid, block, 0, st>>>(a.ws_o, a.ws_ml, a.sinks, a.sinks_dtype, grid.x, a.n_splits, a.n_hblk, a.inv_hblk, a.n_heads, a);
+    merge<<<grid, block, 0, st>>>(a.ws_o, a.ws_ml, a.sinks, a.sinks_dtype, grid.x, a.n_splits, a.n_hblk, a.inv_hblk, a.n_heads,
+                                 a.n_tokens, a.inv_tokens, a);
   }
   MSPR_CHECK_LAUNCH("sparse attention (merge)");
   return MSPR_OK;

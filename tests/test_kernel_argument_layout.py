@@ -39,3 +39,18 @@ def test_the_8_bit_split_requests_its_first_tiles_before_it_waits_for_an_argumen
     for name, lines in bodies.items():
         head = _first_lines(lines, r"s_waitcnt")
         assert sum(l.startswith("global_load_dwordx4 ") for l in head) >= 16, name
+
+
+def _argument_bytes(text):
+    """Size of every kernel's argument block, hidden arguments included."""
+    records = re.split(r"\n  - \.", text[text.index("amdhsa.kernels:"):])[1:]
+    return {re.search(r"\.name:\s+(_Z\S+)", r)[1]: int(re.search(r"\.kernarg_segment_size:\s+(\d+)", r)[1]) for r in records}
+
+
+# (a call that the host issues more slowly than the device runs it pays for long blocks)
+@pytest.mark.parametrize("source,kernel,count,most", [("sparse_attn.hip", "sparse_attn_split_kernel", 6, 312),
+                                                      ("sparse_attn.hip", "sparse_attn_merge_kernel", 3, 112),
+                                                      ("q8_decode.hip", "q8_decode_split_kernel", 6, 104)])
+def test_argument_blocks_hold_no_field_twice(source, kernel, count, most):
+    sizes = [n for name, n in _argument_bytes(build.device_assembly(os.path.join(build.CSRC, source))).items() if kernel in name]
+    assert len(sizes) == count and max(sizes) <= most, sizes
