@@ -67,15 +67,17 @@ __device__ __forceinline__ void async_row(uint64_t row, uint32_t lane_off, uint3
 }
 
 // CUT: the launch has units that are cut into key ranges (compiled in, the choice cost whole units 3 %).
-// (Plain arguments first: what the first copies and the ids take comes in registers with the wave, and the struct is loaded
-// meanwhile: it was loaded in three dependent steps with three software divisions between. One token behind 28000 rows 22.1 ->
-// 21.6 us with its merge, 255 tokens 43.8 -> 43.5; full rounds, which power bounds, are as they were.)
+// (Plain arguments first: what the first copies and the ids of up to 64 heads of one sequence take comes in registers with the
+// wave, and the struct is loaded meanwhile: it was loaded in three dependent steps with three software divisions between. One
+// token behind 28000 rows 22.1 -> 21.6 us with its merge, 255 tokens 43.8 -> 43.5; full rounds, which power bounds, are as they
+// were. With how the units are cut among the plain words, and the block 136 bytes instead of 224, whole calls of 1, 17 and 60
+// tokens 11.7 -> 11.5, 20.0 -> 19.9, 23.7 -> 23.5; calls that are not cut the same within 0.3 %. cut: split_units, and ranges from bit 16 on; inv_ranges: mspr_inverse(ranges).)
 template <int QDT, bool CUT>
 __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void* win, const int32_t* idx, int units,
-                                                                      int n_tokens, uint32_t inv_tokens, int n_hblk,
-                                                                      uint32_t pos0, uint32_t window, uint32_t n_raw,
-                                                                      int raw_start, int max_win, int n_idx,
-                                                                      IndexedPrefillArgs a) {
+                                                                      int n_tokens, int n_hblk, uint32_t pos0,
+                                                                      uint32_t window, uint32_t n_raw, int raw_start,
+                                                                      int n_idx, uint32_t cut, uint32_t inv_ranges,
+                                                                      IndexedPrefillRest a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int* ids = reinterpret_cast<int*>(lds + kOffIds);
   int* stop_sh = reinterpret_cast<int*>(lds + kOffStop);
@@ -86,19 +88,22 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   const int kg = lane >> 4;
 
   // The tokens with the most rows (the last ones, at the start of a context) are started first.
-  // The first a.split_units units, a part-filled last round, are cut into a.ranges key ranges each and come last.
+  // The first split_units units, a part-filled last round, are cut into that many key ranges each and come last.
+  const int split_units = (int)(cut & 0xFFFFu), ranges = (int)(cut >> 16);
   int unit = units - 1 - (int)blockIdx.x, range = 0;
   bool split = false;
   if constexpr (CUT) {
-    const int whole = units - a.split_units;
+    const int whole = units - split_units;
     split = (int)blockIdx.x >= whole;
     const int i = (int)blockIdx.x - whole;
-    unit = split ? mspr_div(i, a.ranges, a.inv_ranges) : a.split_units - 1 - i;
-    range = split ? i - unit * a.ranges : 0;
+    unit = split ? mspr_div(i, ranges, inv_ranges) : split_units - 1 - i;
+    range = split ? i - unit * ranges : 0;
   }
-  const int seq = n_hblk == 1 ? unit : mspr_div(unit, n_hblk, a.inv_hblk);
+  // (real divisions, but in branches that 64 heads of one sequence pass by: reciprocals of both in the struct were loaded, and
+  // waited for, in front of the branches)
+  const int seq = n_hblk == 1 ? unit : unit / n_hblk;
   const int hb = unit - seq * n_hblk;
-  const int b = mspr_div(seq, n_tokens, inv_tokens);
+  const int b = seq < n_tokens ? 0 : seq / n_tokens;
   const int t = seq - b * n_tokens;
 
   // window rows and visible pool prefix, in the unsigned 32-bit arithmetic of the reference kernel
@@ -108,14 +113,13 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   const uint32_t window_first = (window != 0u && qpos + 1u > window) ? qpos + 1u - window : 0u;
   const uint32_t first = first_raw_pos > window_first ? first_raw_pos : window_first;
   const uint32_t last = qpos < last_pos ? qpos : last_pos;
-  int n_win = first <= last ? (int)(last - first + 1u) : 0;
-  if (n_win > max_win) n_win = max_win;
+  const int n_win = first <= last ? (int)(last - first + 1u) : 0;
   const int win_first = first <= last ? (int)(first - first_raw_pos) : 0;
   const int wt = (n_win + kTile - 1) / kTile;
   // this workgroup's tiles: all of them, or its share of what the token has at most
   int t_begin = 0, t_share = 0x7FFFFFFF;
   if (CUT && split) {
-    t_share = mspr_div(wt + (n_idx + kTile - 1) / kTile + a.ranges - 1, a.ranges, a.inv_ranges);
+    t_share = mspr_div(wt + (n_idx + kTile - 1) / kTile + ranges - 1, ranges, inv_ranges);
     t_begin = range * t_share;
   }
   const uint64_t win_base = reinterpret_cast<uint64_t>(win) + (uint64_t)b * (uint64_t)n_raw * (kD * 2);
@@ -164,12 +168,12 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
 
   // ---- ids to LDS, position of the first one that ends the walk
   auto stage_ids = [&](int done) {
-    int64_t visible = a.ratio == 0u ? a.n_pool : (int64_t)((qpos + 1u) / a.ratio);
-    if (visible > a.n_pool) visible = a.n_pool;
+    uint32_t visible = a.ratio == 0u ? (uint32_t)a.n_pool : (qpos + 1u) / a.ratio;
+    if (visible > (uint32_t)a.n_pool) visible = (uint32_t)a.n_pool;
     int found = n_idx;
     auto look = [&](int i, int id) {
       ids[i] = id;
-      if (id >= 0 && (int64_t)id >= visible && i < found) found = i;
+      if (id >= 0 && (uint32_t)id >= visible && i < found) found = i;
     };
 #pragma unroll
     for (int j = 0; j < kEager; j++)
@@ -316,12 +320,12 @@ __global__ __launch_bounds__(kThreads, 2) void indexed_prefill_kernel(const void
   l += __shfl_xor(l, 16, MSPR_WAVE);
   l += __shfl_xor(l, 32, MSPR_WAVE);
   if (CUT && split) {  // unnormalised, as the registers hold it
-    const int part = unit * a.ranges + range;
+    const int part = unit * ranges + range;
     float* po = a.parts + (int64_t)part * (64 * kD) + (wave * 32 * 64 + lane) * 4;
 #pragma unroll
     for (int mt = 0; mt < 32; mt++) *reinterpret_cast<f32x4_t*>(po + mt * 256) = oacc[mt];
     if (kg == 0) {
-      float* ml = a.parts + (int64_t)a.split_units * a.ranges * (64 * kD) + ((int64_t)part * 64 + 16 * wave + c16) * 2;
+      float* ml = a.parts + (int64_t)split_units * ranges * (64 * kD) + ((int64_t)part * 64 + 16 * wave + c16) * 2;
       ml[0] = m_run;
       ml[1] = l;
     }
@@ -406,7 +410,7 @@ __global__ __launch_bounds__(256) void indexed_prefill_merge_kernel(const float*
 }
 
 template <int QDT, bool CUT>
-int launch(const IndexedPrefillArgs& call, hipStream_t st) {
+int launch(const IndexedPrefillArgs& a, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&indexed_prefill_kernel<QDT, CUT>),
@@ -417,24 +421,20 @@ int launch(const IndexedPrefillArgs& call, hipStream_t st) {
     }
     attr_set = true;
   }
-  IndexedPrefillArgs a = call;
   const int n_hblk = (a.n_heads + 63) / 64;
   const int64_t units = (int64_t)a.batch * a.n_tokens * n_hblk;
-  a.inv_hblk = mspr_inverse(n_hblk);
-  a.inv_ranges = mspr_inverse(a.ranges);
-  const uint32_t inv_tokens = mspr_inverse(a.n_tokens);
   dim3 grid((unsigned)(units - a.split_units + a.split_units * a.ranges)), block(kThreads);
   {
     MsprProfScope prof(MSPR_K_SPARSE_SPLIT, st);
-    indexed_prefill_kernel<QDT, CUT><<<grid, block, kLdsBytes, st>>>(a.win, a.idx, (int)units, a.n_tokens, inv_tokens, n_hblk, a.pos0,
-                                                                     a.window, (uint32_t)a.raw_cap, a.raw_start, a.max_win,
-                                                                     a.n_idx, a);
+    indexed_prefill_kernel<QDT, CUT><<<grid, block, kLdsBytes, st>>>(
+        a.win, a.idx, (int)units, a.n_tokens, n_hblk, a.pos0, a.window, (uint32_t)a.raw_cap, a.raw_start, a.n_idx,
+        (uint32_t)a.split_units | (uint32_t)a.ranges << 16, mspr_inverse(a.ranges), a);
   }
   MSPR_CHECK_LAUNCH("indexed prefill attention");
   if constexpr (CUT) {
     MsprProfScope prof(MSPR_K_SPARSE_MERGE, st);
     indexed_prefill_merge_kernel<<<dim3((unsigned)(a.split_units * 32)), block, 0, st>>>(
-        a.parts, a.sinks, a.split_units, a.ranges, a.n_heads, n_hblk, a.inv_hblk, a.n_tokens, inv_tokens, a.out,
+        a.parts, a.sinks, a.split_units, a.ranges, a.n_heads, n_hblk, mspr_inverse(n_hblk), a.n_tokens, mspr_inverse(a.n_tokens), a.out,
         a.q_batch_stride, a.q_token_stride, a.q_head_stride);
     MSPR_CHECK_LAUNCH("indexed prefill attention (merge)");
   }

@@ -2016,7 +2016,7 @@ extern "C" int mspr_indexed_mixed_attention_prefill(const void* q, int q_dtype, 
     p.raw_start = raw_start;
     p.max_win = (int)max_win;
     p.pool = comp_kv;
-    p.n_pool = n_comp;
+    p.n_pool = (int)n_comp;
     p.idx = topk;
     p.n_idx = top_k;
     p.pos0 = (uint32_t)pos0;

@@ -13,10 +13,35 @@ pytestmark = pytest.mark.skipif(not (os.path.exists(build.HIPCC) or shutil.which
 
 def _first_lines(lines, until):
     code = [l.split(";")[0].strip() for l in lines]
-    code = [l for l in code if l and not l.startswith(".")]
+    code = [l for l in code if l and (not l.startswith(".") or l.endswith(":"))]
     start = next(i for i, l in enumerate(code) if l.startswith("s_branch"))  # (in front: the form for firmware that preloads nothing)
     code = code[start + 1:]
     return code[:next(i for i, l in enumerate(code) if re.match(until, l))]
+
+
+def _waits_on_the_way(lines, until):
+    """Waits for arguments in front of the first instruction that matches `until`, but for those of blocks that load what they wait
+    for themselves and that a conditional branch passes by."""
+    found, passed_by, loads = [], False, False
+    for line in _first_lines(lines, until):
+        if line.startswith("s_cbranch"):
+            passed_by, loads = True, False
+        elif line.endswith(":"):
+            passed_by = loads = False
+        elif line.startswith("s_load"):
+            loads = True
+        elif line.startswith("s_waitcnt") and not (passed_by and loads):
+            found.append(line)
+    return found
+
+
+@pytest.mark.parametrize("source,kernel,count", [("prefill_attn.hip", "indexed_prefill_kernel", 4)])
+def test_the_first_copies_wait_for_no_argument(source, kernel, count):
+    text = build.device_assembly(os.path.join(build.CSRC, source))
+    bodies = {k: v for k, v in build.kernel_bodies(text).items() if kernel in k}
+    assert len(bodies) == count
+    for name, lines in bodies.items():
+        assert _waits_on_the_way(lines, r"global_load_lds") == [], name
 
 
 def test_the_split_kernel_requests_its_ids_before_it_waits_for_an_argument():
@@ -50,6 +75,7 @@ def _argument_bytes(text):
 # (a call that the host issues more slowly than the device runs it pays for long blocks)
 @pytest.mark.parametrize("source,kernel,count,most", [("sparse_attn.hip", "sparse_attn_split_kernel", 6, 312),
                                                       ("sparse_attn.hip", "sparse_attn_merge_kernel", 3, 112),
+                                                      ("prefill_attn.hip", "indexed_prefill_kernel", 4, 136),
                                                       ("q8_decode.hip", "q8_decode_split_kernel", 6, 104)])
 def test_argument_blocks_hold_no_field_twice(source, kernel, count, most):
     sizes = [n for name, n in _argument_bytes(build.device_assembly(os.path.join(build.CSRC, source))).items() if kernel in name]
