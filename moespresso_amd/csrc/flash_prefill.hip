@@ -13,6 +13,8 @@
 // Per wave and tile: S^T = K.Q^T on v_mfma_f32_32x32x16 (keys x queries: the softmax statistics of a
 // query live in one lane column), online softmax in the log2 domain with a lazily advanced reference
 // maximum, O^T += V^T.P^T. Q^T stays in registers (64 VGPRs), O^T in 128 accumulator registers.
+#include <type_traits>
+
 #include "common.h"
 #include "profile.h"
 
@@ -27,27 +29,18 @@ constexpr int kBufs = 4;
 constexpr int kThreads = 512;
 constexpr int kLdsBytes = kBufs * kStageBytes;  // 128 KB
 
-struct PrefillArgs {
-  const void* q;   // [B, Hq, L, 256]
-  const void* k;   // [B, Hkv, kv_rows, 256]
-  const void* v;
-  void* out;       // [B, Hq, L, 256]
-  int batch, n_q_heads, n_kv_heads;
-  int q_len;
-  int64_t past_len;
-  int64_t kv_rows;  // rows allocated per (batch, kv head); >= past_len + q_len
-  float scale_log2;
-  int rep_shift;    // log2(query heads per KV head), 0..3
-  int q_blocks;     // workgroups along the query axis
-  uint32_t inv_splits, inv_q_blocks, inv_kv_heads;  // mspr_inverse() of n_splits, q_blocks, n_kv_heads
-  // key-range splits (short chunks over deep prefixes do not fill the device otherwise): split sp of a
-  // query block takes every n_splits-th share of that block's tiles; partials are merged afterwards
-  int n_splits;
+// What the kernel reads behind its plain arguments,
+struct FlashRest {
+  void* out;        // [B, Hq, L, 256]
   float* ws_o;      // [n_splits][B][Hq][L][256] unnormalised O relative to ws_ml's maximum
   float* ws_ml;     // [n_splits][B][Hq][L][2]   (reference maximum in log2 units, denominator)
-  // quantised-prefix form only: tiles [0, q8_tiles) come from the affine 8-bit prefix below, the rest
-  // from k / v, which then hold float16 rows for keys [32 q8_tiles, past_len + q_len)
-  int q8_tiles;
+  int batch;
+  float scale_log2;
+};
+
+// and its quantised-prefix form besides: tiles [0, q8_tiles) come from the affine 8-bit prefix below, the rest
+// from k / v, which then hold float16 rows for keys [32 q8_tiles, past_len + q_len).
+struct FlashRestQ8 : FlashRest {
   int64_t past_rows;  // rows allocated per (batch, kv head) in the prefix tensors; >= past_len
   const void* pk_wq;  // [B, Hkv, past_rows, 256] codes
   const void* pk_s;   // [B, Hkv, past_rows, 4]
@@ -55,6 +48,22 @@ struct PrefillArgs {
   const void* pv_wq;
   const void* pv_s;
   const void* pv_b;
+  int q8_tiles;
+};
+
+struct PrefillArgs : FlashRestQ8 {
+  const void* q;   // [B, Hq, L, 256]
+  const void* k;   // [B, Hkv, kv_rows, 256]
+  const void* v;
+  int n_q_heads, n_kv_heads;
+  int q_len;
+  int64_t past_len;
+  int64_t kv_rows;  // rows allocated per (batch, kv head); >= past_len + q_len
+  int rep_shift;    // log2(query heads per KV head), 0..3
+  int q_blocks;     // workgroups along the query axis
+  // key-range splits (short chunks over deep prefixes do not fill the device otherwise): split sp of a
+  // query block takes every n_splits-th share of that block's tiles; partials are merged afterwards
+  int n_splits;
 };
 
 typedef __attribute__((ext_vector_type(2))) _Float16 h2_t;
@@ -178,14 +187,19 @@ __device__ __forceinline__ int swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 
 // gives; without it in packed float16 arithmetic.
 constexpr int kExactUnpack = 4;
 
-// (Plain arguments first: what the first tiles' addresses take comes in registers with the wave, and the struct is loaded
-// meanwhile. With that and without software divisions, 100 queries behind 1000 rows 18.5 -> 18.0 us, 203 behind 9001 42.7 -> 42.2,
-// and their merges 5.3 -> 5.1 and 9.3 -> 9.2. heads: n_kv_heads, and rep_shift from bit 28 on.)
+// (Plain arguments first: what the addresses of the first tiles and of the queries take comes in registers with the wave, and the
+// struct is loaded meanwhile, but where the first tiles are an 8-bit prefix's, whose addresses are in it. With that and without
+// software divisions, 100 queries behind 1000 rows 18.5 -> 18.0 us, 203 behind 9001 42.7 -> 42.2, and their merges 5.3 -> 5.1 and
+// 9.3 -> 9.2. The number of workgroups, which runs are dealt out by, was made of a word of the struct and waited for; with it
+// among the plain words in place of the blocks of queries, which follow from q_len, and 88 (152) bytes instead of 232, 203 dense
+// queries behind 9001 rows 49.0 -> 48.3 with their merge, 700 behind 9000 rows of 8 bits 136.1 -> 135.6, others the same. heads:
+// n_kv_heads, and rep_shift from bit 28 on; wgs: workgroups of the launch.)
 template <int KDT, bool Q8, int SDT, bool IO32, bool Q32, bool RUNS>
 __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsigned char* k, const unsigned char* v,
                                                                    const void* q, int q_len, int past, int kv_rows,
-                                                                   int n_splits, uint32_t inv_splits, int q_blocks,
-                                                                   uint32_t inv_q_blocks, uint32_t heads, PrefillArgs a) {
+                                                                   int n_splits, uint32_t inv_splits, uint32_t inv_q_blocks,
+                                                                   uint32_t heads, int wgs,
+                                                                   std::conditional_t<Q8, FlashRestQ8, FlashRest> a) {
   extern __shared__ __attribute__((aligned(256))) unsigned char lds[];  // tile bases: zero low bits under the address XORs
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -204,7 +218,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   const int blocks_per_group = 4 >> hpg_shift;
   const int halves_shift = rep_shift - hpg_shift;
   const int n_blocks = (q_len + 31) >> 5;
-  const int n_pairs = q_blocks >> halves_shift;
+  const int n_pairs = (n_blocks + 2 * blocks_per_group - 1) >> (3 - hpg_shift);  // (each of 2 blocks_per_group)
+  const int q_blocks = n_pairs << halves_shift;
   // RUNS (four ranges or more, of ten tiles or more): workgroup i, which is on XCD i % 8, takes the i / 8th of that XCD's run
   // of the list (batch, KV head, range, pair). An L2 then holds the keys of few ranges and one or two heads' queries, which
   // all pairs of a range pass together. Elsewhere the ranges go round the XCDs, as in runs the partials leave the L2s 2 us
@@ -213,7 +228,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   int work = blockIdx.x;
   int sp, q_block;
   if constexpr (RUNS) {
-    const int wgs = a.batch * n_kv_heads * q_blocks * n_splits, xcd = work & 7;
+    const int xcd = work & 7;
     work = xcd * (wgs >> 3) + (xcd < (wgs & 7) ? xcd : wgs & 7) + (work >> 3);
     const int rest = mspr_div(work, q_blocks, inv_q_blocks);
     q_block = work - rest * q_blocks;
@@ -229,7 +244,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   const int head_half = q_block & ((1 << halves_shift) - 1);
   int kvh = work, b = 0;
   if (work >= n_kv_heads) {
-    b = mspr_div(work, n_kv_heads, a.inv_kv_heads);
+    b = work / n_kv_heads;
     kvh = work - b * n_kv_heads;
   }
   const int wi = wave & 3;
@@ -260,7 +275,9 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSPR_LDS_PTR(unsigned char, lds);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds0) + wave * 1024;
   const int n_keys = past + q_len;  // keys that exist
-  const int t1 = Q8 ? a.q8_tiles : 0;        // first tile served from k / v; their row 0 is key 32 t1
+  FlashRestQ8 prefix = {};
+  if constexpr (Q8) prefix = a;
+  const int t1 = prefix.q8_tiles;  // first tile served from k / v; their row 0 is key 32 t1
   auto issue_tile = [&](int t_abs, int slot) {
     // rows past the last key (only in the last tile) are masked by the causal rule; read the last key instead
     const int t = t_abs - t1;
@@ -285,14 +302,14 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   constexpr int kRawBytes = 2 * kCodeBytes + 4 * 512;
   constexpr int kRawBase = 2 * kStageBytes;      // the unpacked stages use the lower 64 KB
   static_assert(kRawBase + 3 * kRawBytes <= kLdsBytes, "raw ring does not fit");
-  const int64_t raw_row0 = ((int64_t)b * n_kv_heads + kvh) * a.past_rows;
-  const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.pk_wq) + raw_row0 * kD;
-  const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.pv_wq) + raw_row0 * kD;
+  const int64_t raw_row0 = ((int64_t)b * n_kv_heads + kvh) * prefix.past_rows;
+  const uint8_t* kc = reinterpret_cast<const uint8_t*>(prefix.pk_wq) + raw_row0 * kD;
+  const uint8_t* vc = reinterpret_cast<const uint8_t*>(prefix.pv_wq) + raw_row0 * kD;
   // scale / bias copies: wave w moves array w & 3 (K scale, K bias, V scale, V bias), 4 bytes per lane; with
   // float32 scales waves 4-7 move the second 256 bytes, with 16-bit ones they repeat the copy of waves 0-3
   // (every wave then issues the same number of copies and the waits below are static counts)
   const int arr = wave & 3;
-  const uint8_t* sb_base = reinterpret_cast<const uint8_t*>(arr == 0 ? a.pk_s : arr == 1 ? a.pk_b : arr == 2 ? a.pv_s : a.pv_b) +
+  const uint8_t* sb_base = reinterpret_cast<const uint8_t*>(arr == 0 ? prefix.pk_s : arr == 1 ? prefix.pk_b : arr == 2 ? prefix.pv_s : prefix.pv_b) +
                            raw_row0 * 4 * kSB;
   const int sb_half = kSB == 4 ? (wave >> 2) * 256 : 0;
   const uint32_t code_off = (uint32_t)tid * 16;  // K / V codes: LDS slot tid of the tile's 512
@@ -325,7 +342,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
     // clocks for the eight waves' float32 rows, of the 13000 before the first tile. With the stores below, us: 203 float32
     // queries over 9001 quantised keys 78.5 -> 74.0 (whole operator with its append), 30 queries 46.4 -> 42.2, 203 bfloat16
     // ones over 9001 dense keys 56.5 -> 53. Tiles requested behind the queries 1 us more, behind their exchange the same.
-    const int64_t qbase = ((int64_t)b * a.n_q_heads + head) * q_len;
+    const int64_t qbase = ((int64_t)b * n_kv_heads * rep + head) * q_len;
     constexpr int kLanes = Q32 ? 32 : 16;  // lanes of a row
     constexpr int kRows = 64 / kLanes;      // rows of an instruction
     const int xr = lane / kLanes, xc = lane % kLanes;
@@ -585,7 +602,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_prefill_kernel(const unsign
   asm volatile("" : "+v"(tl));  // (the offsets below are made here, not carried through the tile loop)
   const int en = tl & 31, eg = (tl >> 5) & 1;
   unsigned char* xo = lds + (wave << 14);
-  const int64_t out_row = (((int64_t)(n_splits > 1 ? sp : 0) * a.batch + b) * a.n_q_heads + head) * q_len + q0;
+  const int64_t out_row = (((int64_t)(n_splits > 1 ? sp : 0) * a.batch + b) * n_kv_heads * rep + head) * q_len + q0;
   const int n_rows = active ? q_len - q0 : 0;  // (of the wave's 32, those below it)
   const float inv = n_splits > 1 ? 1.0f : l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
   if (n_splits > 1 && en < n_rows && eg == 0) {
@@ -883,19 +900,15 @@ int prefill_launch_flash(const PrefillArgs& a, hipStream_t st) {
     MsprProfScope prof(MSPR_K_FLASH_PREFILL, st);
     flash_prefill_kernel<KDT, Q8, SDT, IO32, Q32, RUNS><<<grid, block, kLdsBytes, st>>>(
         reinterpret_cast<const unsigned char*>(a.k), reinterpret_cast<const unsigned char*>(a.v), a.q, a.q_len,
-        (int)a.past_len, (int)a.kv_rows, a.n_splits, a.inv_splits, a.q_blocks, a.inv_q_blocks,
-        (uint32_t)a.n_kv_heads | (uint32_t)a.rep_shift << 28, a);
+        (int)a.past_len, (int)a.kv_rows, a.n_splits, mspr_inverse(a.n_splits), mspr_inverse(a.q_blocks),
+        (uint32_t)a.n_kv_heads | (uint32_t)a.rep_shift << 28, (int)grid.x, a);
   }
   MSPR_CHECK_LAUNCH("flash_prefill");
   return MSPR_OK;
 }
 
 template <int KDT, bool Q8, int SDT, bool IO32 = Q8>
-int prefill_launch(const PrefillArgs& call, hipStream_t st, bool q32 = false) {
-  PrefillArgs a = call;
-  a.inv_splits = mspr_inverse(a.n_splits);
-  a.inv_q_blocks = mspr_inverse(a.q_blocks);
-  a.inv_kv_heads = mspr_inverse(a.n_kv_heads);
+int prefill_launch(const PrefillArgs& a, hipStream_t st, bool q32 = false) {
   // (the line of the kernel's mapping; a template parameter because as a run-time branch it cost long chunks 0.5 %)
   const bool runs = a.n_splits >= 4 && (a.past_len + a.q_len) / kTile >= (int64_t)10 * a.n_splits;
   int rc;
