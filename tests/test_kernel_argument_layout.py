@@ -19,6 +19,28 @@ def _first_lines(lines, until):
     return code[:next(i for i, l in enumerate(code) if re.match(until, l))]
 
 
+def _preload_lengths(text):
+    """Words of arguments that come in registers, of every kernel whose descriptor names a number."""
+    found = {}
+    for name, descriptor in re.findall(r"^\s*\.amdhsa_kernel (\S+)\n(.*?)^\s*\.end_amdhsa_kernel", text, flags=re.S | re.M):
+        m = re.search(r"kernarg_preload_length (\d+)", descriptor)
+        found[name] = int(m[1]) if m else 0
+    return found
+
+
+def test_a_kernel_without_a_preload_length_is_not_given_the_next_ones():
+    text = ".amdhsa_kernel a\n.end_amdhsa_kernel\n.amdhsa_kernel b\n.amdhsa_user_sgpr_kernarg_preload_length 14\n.end_amdhsa_kernel\n"
+    assert _preload_lengths(text) == {"a": 0, "b": 14}
+
+
+def test_a_wait_is_seen_where_it_is_on_the_way():
+    start = ["s_waitcnt lgkmcnt(0)", "s_branch .LBB0_0", ".LBB0_0:"]
+    load, wait, copy, past = "s_load_dword s6, s[0:1], 0xd0", "s_waitcnt lgkmcnt(0)", "global_load_lds_dwordx4 v1, s[2:3]", "s_cbranch_scc1 .LBB0_1"
+    for lines, waits in (([load, copy], 0), ([load, wait, copy], 1), ([load, past, wait, ".LBB0_1:", copy], 1),
+                         ([past, load, wait, ".LBB0_1:", copy], 0), ([past, load, ".LBB0_1:", wait, copy], 1)):
+        assert len(_waits_on_the_way(start + lines, r"global_load_lds")) == waits, lines
+
+
 def _waits_on_the_way(lines, until):
     """Waits for arguments in front of the first instruction that matches `until`, but for those of blocks that load what they wait
     for themselves and that a conditional branch passes by."""
@@ -53,8 +75,9 @@ def test_the_split_kernel_requests_its_ids_before_it_waits_for_an_argument():
     for name, lines in bodies.items():
         head = _first_lines(lines, r"global_load_dword v")
         assert not any(l.startswith("s_waitcnt") for l in head), name
-    preload = dict(re.findall(r"\.amdhsa_kernel (\S+).*?kernarg_preload_length (\d+)", text, flags=re.S))
-    assert all(int(n) >= 11 for k, n in preload.items() if "split_kernel" in k or "merge_kernel" in k)
+    lengths = _preload_lengths(text)
+    assert sum("split_kernel" in k for k in lengths) == 6 and sum("merge_kernel" in k for k in lengths) == 3
+    assert all(n >= 11 for k, n in lengths.items() if "split_kernel" in k or "merge_kernel" in k), lengths
 
 
 def test_the_8_bit_split_requests_its_first_tiles_before_it_waits_for_an_argument():

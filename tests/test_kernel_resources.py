@@ -41,6 +41,30 @@ def test_sparse_attention_kernels_use_no_scratch(sparse_kernels):
         assert res["vgprs"] <= 256, (name, res)
 
 
+def test_the_fp4_scores_with_the_float16_form_inside_fit_three_waves():
+    """Three waves of a SIMD share 512 registers, in units of eight: 168 each, and nothing may be spilled to keep to that."""
+    (name, res), = [(k, v) for k, v in build.kernel_resources(os.path.join(build.CSRC, "indexer_tiled.hip")).items() if "scores_fp4_kernel" in k]
+    assert res["vgprs"] <= 168 and res["scratch_bytes"] == 0 and res["vgpr_spills"] == 0, (name, res)
+
+
+def test_flash_prefill_spills_one_value_in_one_form_and_none_around_its_copies():
+    """Float32 queries over an 8-bit prefix in fewer than four key ranges: one value is put away in front of the tile loops and
+    fetched once behind the loop over 8-bit tiles, where the kernel has waited for all its copies."""
+    source = os.path.join(build.CSRC, "flash_prefill.hip")
+    text = build.device_assembly(source)
+    bodies = build.kernel_bodies(text)
+    spilling = {k for k, v in build.kernel_resources(source, text).items() if v["scratch_bytes"] or v["vgpr_spills"]}
+    assert len(bodies) > 28 and all("flash_prefill_kernelILi1ELb1E" in k and "ELb1ELb1ELb0EEE" in k for k in spilling), sorted(spilling)
+    for name in spilling:
+        lines = [l.split(";")[0].strip() for l in bodies[name]]
+        ops = [i for i, l in enumerate(lines) if l.startswith("scratch_")]
+        first_tile = next(i for i, l in enumerate(lines) if l.startswith("v_mfma"))
+        assert [lines[i].split()[0] for i in ops] == ["scratch_store_dword", "scratch_load_dword"], name
+        assert ops[0] < first_tile < ops[1], name
+        in_front = [l for l in lines[ops[1] - 6:ops[1]] if l and not l.startswith(".")]
+        assert any(l.startswith("s_barrier") for l in in_front) and any("vmcnt(0)" in l for l in in_front), (name, in_front)
+
+
 def test_resource_query_sees_every_kernel_of_the_source(sparse_kernels):
     assert sum("sparse_attn_merge_kernel" in k for k in sparse_kernels) == 3
     for res in sparse_kernels.values():
