@@ -32,9 +32,9 @@ COMMON_FLAGS = [
     # The first plain arguments of a kernel, up to 14 words, arrive in registers with its waves instead of through a load at
     # their start (400 to 900 cycles where the argument block is in no cache yet, as at every launch): the score, QAT,
     # selection, rope and 8-bit quantisation kernels. DS4 decode of one sequence 24.1 -> 23.6 us, of five 30.5 -> 30.1, four
-    # captured layers of sixteen 211.6 -> 209.7, a 517-token chunk 160.5 -> 156.7. The attention, flash and
-    # 8-bit split kernels take what their first loads need this way and the rest in a struct, which is loaded; the 8-bit merge
-    # and append take structs only.
+    # captured layers of sixteen 211.6 -> 209.7, a 517-token chunk 160.5 -> 156.7. The attention, flash and 8-bit split kernels
+    # take what their first loads need this way and what they read later in a struct, which is loaded meanwhile; the 8-bit
+    # merge and append and the rows of a quantised prefill take structs only.
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument",
     # the asynchronous LDS loads set M0 by hand inside inline asm

@@ -461,10 +461,9 @@ __global__ __launch_bounds__(64 * kQ8Waves, 1) void q8_decode_split_kernel(const
 // Merge of the per-range partials: one workgroup per (batch, query head); 64 lanes cover the 256
 // dims four at a time, the 16 waves each take every 16th range and fetch up to 16 of them in one go
 // (one memory round trip for up to 256 ranges), the wave results are combined in LDS.
-// (Its arguments come in the struct: as plain ones, in registers, they take 0.6 us off the device's time, but 32 bytes of arguments
-// for the call's last launch leave the host 0.3 to 0.6 us behind, and one sequence's step is the host's: appended and attended
-// with 8192 keys 17.3 and 17.9 us, where the host keeps up 15.6 and 15.0. With both kernels on the struct and the merge's head
-// taken apart by a division, 16.0.)
+// (Its arguments come in the struct of 128 bytes: as plain ones, 36 bytes in registers, they take 0.3 us off the device's time, but
+// the host issues the call 0.3 us more slowly, for whatever reason, and one sequence's step is the host's: appended and attended
+// with 8191 keys, eight processes of each in turn, 16.7 to 17.1 and 17.1 to 17.3 us, on the device 15.0 to 15.4 and 14.8 to 15.1.)
 constexpr int kMergeWaves = 16;
 template <int ODT>
 __global__ __launch_bounds__(64 * kMergeWaves) void q8_decode_merge_kernel(Q8Args a) {

@@ -77,6 +77,34 @@ def test_every_tile_row_lies_in_its_tensor_and_the_walk_is_the_references(seed):
             assert got_pool == want and all(0 <= r < shape["n_pool"] for r in got_pool)
 
 
+def test_no_token_visits_more_ring_rows_than_the_host_counts():
+    """The host sizes ranges and scratch by host_n_win(); the kernel's own arithmetic stays within it, without a clamp."""
+    for pos0 in (*range(9), 2 ** 31 - 8):
+        for n_tokens in range(1, 6):
+            for raw_cap in range(1, 14):
+                for window in (0, 1, 2, 5, 9, 14):
+                    most = host_n_win(pos0, n_tokens, raw_cap, window)
+                    for t in range(n_tokens):
+                        _, _, n_win = unit_rows(t, pos0=pos0, n_tokens=n_tokens, raw_cap=raw_cap, raw_start=0, window=window, ratio=4,
+                                                n_pool=1, host_n_win=1 << 31)
+                        assert n_win <= most, (pos0, n_tokens, raw_cap, window, t)
+
+
+def test_division_by_reciprocal_is_division():
+    """mspr_div(x, n, mspr_inverse(n)) of common.h for every x below 2^31: the high half of x * floor(2^32 / n), corrected by one."""
+    rng = np.random.default_rng(2)
+    text = open(os.path.join(build.CSRC, "common.h")).read()
+    assert "int q = (int)__umulhi((uint32_t)x, inv);" in text and "if (x - q * n >= n) q++;" in text
+    for n in [*range(2, 700), *(2 ** k + d for k in range(10, 31) for d in (-1, 0, 1)), *rng.integers(2, 2 ** 31, 300).tolist()]:
+        inv = np.uint64(2 ** 32 // n)
+        top = 2 ** 31 // n * n
+        x = np.unique(np.clip(np.concatenate([rng.integers(0, 2 ** 31, 200), [0, 1, n - 1, n, n + 1, top - 1, top, 2 ** 31 - 1]]), 0, 2 ** 31 - 1))
+        x = x.astype(np.uint64)
+        q = x * inv >> np.uint64(32)
+        q += (x - q * np.uint64(n) >= np.uint64(n)).astype(np.uint64)
+        assert np.array_equal(q, x // np.uint64(n)), n
+
+
 # ------------------------------------------------------------------------------------------------ key ranges
 
 def test_key_ranges_of_a_cut_unit_hold_every_tile_once():
